@@ -267,6 +267,74 @@ def run(s):
     return _torch(m), _torch(K.var(s["x"], dims=_ints(case["over"]), mean=m, corrected=False))
 
 
+# ---- the same in 64 bits, by torch alone ----------------------------------------------------------------------------------------------
+
+def _updated(case, w, g, states):
+    """One parameter and its optimizer's state after the first step."""
+    if case["opt"] == "sgd":
+        return [w - 0.01 * g]
+    if case["opt"] == "momentum":
+        v = 0.9 * states[0] - 0.001 * g
+        return [w + v, v]
+    m, v = 0.9 * states[0] + 0.1 * g, 0.999 * states[1] + 0.001 * g * g
+    return [w - 0.0001 * (m / 0.1) / (torch.sqrt(v / 0.001) + 1e-8), m, v]
+
+
+def exact(case, seed):
+    """What run returns for these inputs; None where dropout draws from the library's own generator."""
+    kind = case["kind"]
+    if kind == "mlp" and case["pdrop"] > 0:
+        return None
+    s = prepare(case, seed)
+    torch.cuda.synchronize()
+
+    def double(a):
+        return _torch(K.value(a)).double()
+
+    if kind in ("mlp", "words"):
+        w = [double(p).requires_grad_() for p in s["params"]]
+        if kind == "mlp":
+            h = double(s["x"])
+            for i in range(0, len(w), 2):
+                h = w[i] @ h + w[i + 1]
+                h = torch.relu(h) if i < len(w) - 2 else h
+        else:
+            we, w1, b1, w2, b2 = w
+            h = w2 @ torch.relu(w1 @ we[:, torch.as_tensor(s["words"] - 1, device="cuda")] + b1) + b2
+        loss = torch.nn.functional.cross_entropy(h.t(), torch.as_tensor(s["labels"] - 1, device="cuda"))
+        grads = torch.autograd.grad(loss, w)
+        out, each = [loss.item()], len(s["kept"]) // len(w)
+        for i, (a, g) in enumerate(zip(w, grads)):
+            states = [t.double() for t in s["kept"][i * each + 1:(i + 1) * each]]
+            out += _updated(case, a.detach().t().reshape(-1), g.t().reshape(-1), states)
+        return out
+    if kind == "actback":
+        y, dy, act = double(s["y"]), double(s["dy"]), case["act"]
+        if act == "relu":
+            return dy * (y > 0)
+        if act == "sigm":
+            return dy * y * (1 - y)
+        if act == "tanh":
+            return dy * (1 - y) * (1 + y)
+        if act == "elu":
+            return torch.where(y >= 0, dy, dy * (1 + y))
+        scale, alpha = 1.0507009873554805, 1.6732632423543772
+        return torch.where(y >= 0, scale * dy, dy * (y + scale * alpha))
+    if kind == "xent":
+        x = double(s["scores"]).requires_grad_()
+        loss = torch.nn.functional.cross_entropy(x.t(), torch.as_tensor(s["labels"] - 1, device="cuda"))
+        return loss.item(), torch.autograd.grad(loss, x)[0]
+    x = double(s["x"])
+    over = [d - 1 for d in (_ints(case["over"]) if kind != "softmax" else [case["over"]])]
+    if kind == "unbroadcast":
+        return x.sum(over, keepdim=True)
+    if kind == "softmax":
+        x.requires_grad_()
+        y = torch.softmax(x, over[0]) if case["op"] == "softmax" else torch.log_softmax(x, over[0])
+        return y.detach(), torch.autograd.grad(y, x, double(s["dy"]))[0]
+    return x.mean(over, keepdim=True), x.var(over, correction=0, keepdim=True)
+
+
 # ---- what a pass cannot do without, and how far another correct implementation may be off ------------------------------------------------
 
 _STATE = {"sgd": 3, "momentum": 5, "adam": 7}                # arrays read or written by an update: gradient, weights twice, state twice each

@@ -1,0 +1,396 @@
+// Large fp32 matrix products on the bf16 matrix cores (column-major, C = alpha*op(A)*op(B) + beta*C [+ bias] [relu]).
+//
+// The fp32 matrix instructions run at 1/16 of the bf16 ones (157 against 2500 TFLOP/s nominal), and the vendor library's fp32 products sit at
+// their limit: 8192^3 reaches 153 TFLOP/s, 4096x2048x4096 149.  Here every element is cut into three bf16 parts, x = h + m + l, each the
+// rounding of what the ones before it leave: 3 x 8 bits and the signs hold all 24 bits of an fp32 number, so h + m + l = x exactly.  Of the nine
+// products of parts the six whose weight reaches 2^-24 of the whole are formed (hh, hm, mh, mm, hl, lh; what is left out is below 2^-26), hh in one
+// set of fp32 accumulators and the five small ones in another: the large sums see one rounding per 16 steps of k.  The result is more precise than the
+// fp32 instruction's.  2-norm of the error against 64 bits, this / vendor fp32, normal data: 512x256x64 4.9e-8/1.45e-7, 1000x237x784 1.6e-7/5.0e-7,
+// 4096x2048x4096 4.0e-7/1.15e-6; all-positive data 5.0e-8/1.2e-7, 1.5e-7/4.2e-7, 3.0e-7/8.4e-7.  (With all six in one set, which leaves room
+// for a 256x256 tile: 1.0e-6 at 4096x2048x4096, and 231 instead of 212 TFLOP/s at 8192^3.)
+//   * Small numbers: the lower parts of numbers below 2^-109 would leave bf16's range.  Both operands are multiplied by 2^24 on the way in and the
+//     sums by 2^-48 on the way out, which keeps every fp32 number, denormals included, whole.
+//   * Large numbers, infinities, NaN: a part or a sum that overflows leaves a NaN or an infinity in an accumulator (inf - inf in the split itself
+//     if not before).  A wave that finds one in its patch forms the patch again with the fp32 matrix instruction: results beyond
+//     2^80, and what is infinite or NaN, come out as that instruction gives them.
+//
+// The cut is made while a tile goes from global memory to LDS (6.5 vector instructions an element, in the shadow of the matrix instructions of the
+// SIMD's other wave): no extra pass over the operands, no scratch.  What bounds it: 256x128 tile, 8 waves of 64x64, 32 steps of k a stage, two
+// stages in LDS (149 KB): matrix cores 3072 cycles a stage, LDS about 2070, vector ALU about 2100.  Measured with the loads and the cut left out: 255 TFLOP/s
+// on normal data against 345 on zeros -- the card's power limit, not the pipes, ends at about 255.  TFLOP/s (of fp32 work), this / vendor:
+// 4096x2048x4096 206/149, TN 209/149, 4096x4096x2048 NT 195/149, 512x2048x32000 TN 206/140, 32000x512x2048 NT 189/140, 8192^3 212/153.
+#pragma once
+#include "knet8_device.h"
+#include "knet8_runtime.h"
+
+namespace knet8 {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+template <int N> struct __attribute__((packed, aligned(4))) FNu { float v[N]; };   // N elements at any element boundary, one load
+using F4u = FNu<4>;
+
+constexpr float kSplitScale = 16777216.0f;              // 2^24
+constexpr float kSplitUnscale = 1.0f / (16777216.0f * 16777216.0f);   // 2^-48: both operands are scaled
+
+template <int N> struct SplitParts { unsigned h[N / 2], m[N / 2], l[N / 2]; };
+
+__device__ __forceinline__ unsigned pack_bf16(float a, float b) {
+  const f32x2 v = {a, b};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));   // v_cvt_pk_bf16_f32, round to nearest even
+}
+template <int N>
+__device__ __forceinline__ SplitParts<N> split_bf16(const float* x) {
+  SplitParts<N> r;
+#pragma unroll
+  for (int i = 0; i < N; i += 2) {
+    const float a = x[i] * kSplitScale, b = x[i + 1] * kSplitScale;
+    const unsigned h = pack_bf16(a, b);
+    const float ra = a - __builtin_bit_cast(float, h << 16), rb = b - __builtin_bit_cast(float, h & 0xffff0000u);
+    const unsigned m = pack_bf16(ra, rb);
+    const float sa = ra - __builtin_bit_cast(float, m << 16), sb = rb - __builtin_bit_cast(float, m & 0xffff0000u);
+    r.h[i / 2] = h; r.m[i / 2] = m; r.l[i / 2] = pack_bf16(sa, sb);
+  }
+  return r;
+}
+
+// One operand's share of a tile: ROWS rows (of op(A), or columns of op(B)) by BK steps of k, fetched as fp32 and kept in LDS as three bf16 parts,
+// 16 bytes (8 steps of k) of one row at a time.
+// KC: k is the contiguous axis in memory (element (row,k) at p[row*ld + k]): a lane takes 4 steps of k of one row.
+// Otherwise the rows are (p[k*ld + row]): a lane takes 4 steps of k of kRows rows next to each other.
+template <int ROWS, int BK, int NT, bool KC>
+struct SplitLoader {
+  static constexpr int kVals = ROWS * BK / NT;
+  static constexpr int kRows = KC ? 1 : (kVals >= 16 ? 4 : 2);
+  static constexpr int kItems = kVals / (4 * kRows);
+  static_assert(kItems >= 1 && kVals % (4 * kRows) == 0 && ROWS % 64 == 0, "tile and workgroup do not match");
+  // Where the 16 bytes of a row stand (in units of 16 bytes): in order, or dealt out to four groups.  With the groups 32 bytes off the
+  // multiples of 128 (and likewise the octets of k of the first form) the writes of store() and the reads of the fragments meet no bank twice.
+  static constexpr int kGroup = ROWS / 4 + 2;
+  static constexpr int kStride = KC ? ROWS + 2 : 4 * kGroup;      // from one octet of k to the next
+  static constexpr int kPart = (BK / 8) * kStride;                // from one part to the next
+  static constexpr int kUnits = 3 * kPart;
+  static __device__ __forceinline__ int unit(int r) { return KC ? r : (r & 3) * kGroup + (r >> 2); }
+
+  float v[kVals];
+  int off[kItems];           // elements from the tile's first row and step (below it for a tile of fewer rows than a lane takes)
+  int to[kItems][kRows];     // in units of 8 bytes
+
+  __device__ __forceinline__ void init(int t, int rows, int ld) {   // rows: how many of the matrix are left here (the matrix itself has 4 or more)
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+      const int e = t + i * NT;
+      if (KC) {
+        const int r = e / (BK / 4), q = e % (BK / 4), rr = r < rows ? r : rows - 1;   // rows beyond the matrix: any valid row, nothing is made of them
+        off[i] = rr * ld + 4 * q;
+        to[i][0] = 2 * ((q >> 1) * kStride + r) + (q & 1);
+      } else {
+        const int g = (e >> 1) % (ROWS / kRows), q = 2 * ((e >> 1) / (ROWS / kRows)) + (e & 1);
+        const int r = kRows * g + kRows <= rows ? kRows * g : rows - kRows;           // the matrix's last rows (again) rather than rows beyond it
+        off[i] = 4 * q * ld + r;
+#pragma unroll
+        for (int j = 0; j < kRows; j++) to[i][j] = 2 * ((q >> 1) * kStride + (r + j < 0 ? ROWS / 4 : unit(r + j))) + (q & 1);   // rows before the tile: into the gap after the first group
+      }
+    }
+  }
+  // p: the operand at the tile's first row and step
+  __device__ __forceinline__ void load(const float* __restrict__ p, int ld) {
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+      if constexpr (KC) {
+        const F4u q = *reinterpret_cast<const F4u*>(p + off[i]);
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[4 * i + j] = q.v[j];
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          const FNu<kRows> q = *reinterpret_cast<const FNu<kRows>*>(p + (long)j * ld + off[i]);
+#pragma unroll
+          for (int r = 0; r < kRows; r++) v[4 * (kRows * i + r) + j] = q.v[r];
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ void load_tail(int t, const float* __restrict__ p, int ld, int kleft) {   // kleft of the BK steps exist
+#pragma unroll
+    for (int i = 0; i < kItems; i++) {
+      const int e = t + i * NT;
+      const int k = 4 * (KC ? e % (BK / 4) : 2 * ((e >> 1) / (ROWS / kRows)) + (e & 1));
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int r = 0; r < kRows; r++) v[4 * (kRows * i + r) + j] = k + j < kleft ? p[(long)off[i] + (KC ? (long)j : (long)j * ld + r)] : 0.0f;
+    }
+  }
+  __device__ __forceinline__ void store(uint4* __restrict__ s) const {
+    uint2* s2 = reinterpret_cast<uint2*>(s);
+#pragma unroll
+    for (int i = 0; i < kItems; i++)
+#pragma unroll
+      for (int r = 0; r < kRows; r++) {
+        const SplitParts<4> p = split_bf16<4>(v + 4 * (kRows * i + r));
+        uint2* d = s2 + to[i][r];
+        d[0] = make_uint2(p.h[0], p.h[1]);
+        d[2 * kPart] = make_uint2(p.m[0], p.m[1]);
+        d[4 * kPart] = make_uint2(p.l[0], p.l[1]);
+      }
+  }
+};
+
+// Workgroup -> (tile of m, tile of n, slice of k).  Workgroups go to the 8 XCDs in turn: give every XCD a run of neighbouring tiles, walked in
+// bands of kBand tiles of m, so that the operands' panels are shared in its L2.
+__device__ __forceinline__ void split_tile(unsigned b, unsigned total, unsigned tm, unsigned tn, unsigned& im, unsigned& in, unsigned& z) {
+  constexpr unsigned kXcd = 8, kBand = 8;
+  const unsigned q = total / kXcd, rem = total % kXcd, x = b % kXcd, y = b / kXcd;
+  unsigned id = x < rem ? x * (q + 1) + y : rem * (q + 1) + (x - rem) * q + y;
+  z = id / (tm * tn);
+  id -= z * (tm * tn);
+  const unsigned band = id / (kBand * tn), first = band * kBand, h = tm - first < kBand ? tm - first : kBand;
+  const unsigned in_band = id - band * (kBand * tn);
+  im = first + in_band % h;
+  in = in_band / h;
+}
+
+template <int BM, int BN, int WM, int WN, int BK, bool TA, bool TB>
+__global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2)
+void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb, float* __restrict__ C, int ldc,
+                       float alpha, float beta, const float* __restrict__ bias, int act, int kchunk, unsigned splits) {
+  constexpr int NT = 64 * (BM / WM) * (BN / WN), FM = WM / 32, FN = WN / 32;
+  using LA = SplitLoader<BM, BK, NT, TA>;
+  using LB = SplitLoader<BN, BK, NT, !TB>;
+  __shared__ uint4 lds[2][LA::kUnits + LB::kUnits];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, half = lane >> 5, l32 = lane & 31;
+  const int wm = (wave % (BM / WM)) * WM, wn = (wave / (BM / WM)) * WN;
+  unsigned im, in, z;
+  split_tile(blockIdx.x, gridDim.x, (unsigned)((m + BM - 1) / BM), (unsigned)((n + BN - 1) / BN), im, in, z);
+  const int i0 = (int)im * BM, j0 = (int)in * BN;
+  const int kbeg = (int)z * kchunk, kend = k - kbeg < kchunk ? k : kbeg + kchunk;
+  const long sa = TA ? 1 : lda, sb = TB ? ldb : 1;               // elements from one k to the next
+  const float* pa = A + (TA ? (long)i0 * lda : i0) + kbeg * sa;
+  const float* pb = B + (TB ? (long)j0 : (long)j0 * ldb) + kbeg * sb;
+  LA la;
+  LB lb;
+  la.init(t, m - i0, lda);
+  lb.init(t, n - j0, ldb);
+  f32x16 acc[FN][FM], low[FN][FM];   // hh, and the five products of lower weight
+#pragma unroll
+  for (int a = 0; a < FN; a++)
+#pragma unroll
+    for (int b = 0; b < FM; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) acc[a][b][r] = low[a][b][r] = 0.0f;
+  auto fetch_full = [&]() {
+    la.load(pa, lda);
+    lb.load(pb, ldb);
+    pa += BK * sa;
+    pb += BK * sb;
+  };
+  auto fetch = [&](int k0) {
+    if (kend - k0 >= BK) { fetch_full(); return; }
+    la.load_tail(t, pa, lda, kend - k0);
+    lb.load_tail(t, pb, ldb, kend - k0);
+  };
+  auto stage = [&](uint4* s) {
+    la.store(s);
+    lb.store(s + LA::kUnits);
+  };
+  int ua[FM], ub[FN];   // this lane's rows in the two halves of a buffer
+#pragma unroll
+  for (int i = 0; i < FM; i++) ua[i] = half * LA::kStride + LA::unit(wm + 32 * i + l32);
+#pragma unroll
+  for (int i = 0; i < FN; i++) ub[i] = LA::kUnits + half * LB::kStride + LB::unit(wn + 32 * i + l32);
+  auto multiply = [&](const uint4* s, int step) {   // 16 steps of k
+    bf16x8 fb[FN][3];
+#pragma unroll
+    for (int p = 0; p < 3; p++)
+#pragma unroll
+      for (int i = 0; i < FN; i++) fb[i][p] = __builtin_bit_cast(bf16x8, s[ub[i] + p * LB::kPart + 2 * step * LB::kStride]);
+#pragma unroll
+    for (int p = 2; p >= 0; p--) {
+      bf16x8 fa[FM];
+#pragma unroll
+      for (int i = 0; i < FM; i++) fa[i] = __builtin_bit_cast(bf16x8, s[ua[i] + p * LA::kPart + 2 * step * LA::kStride]);
+#pragma unroll
+      for (int q = 2 - p; q >= 0; q--)
+#pragma unroll
+        for (int a = 0; a < FN; a++)
+#pragma unroll
+          for (int b = 0; b < FM; b++) {
+            f32x16& c = p + q > 0 ? low[a][b] : acc[a][b];
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[a][q], fa[b], c, 0, 0, 0);
+          }
+    }
+  };
+  const int tiles = (kend - kbeg + BK - 1) / BK, full = (kend - kbeg) / BK;
+  fetch(kbeg);
+  stage(lds[0]);
+  if (tiles > 1) fetch(kbeg + BK);
+  int cur = 0, i = 0;
+  for (; i + 2 < full; i++, cur ^= 1) {
+    __syncthreads();
+    multiply(lds[cur], 0);
+    la.store(lds[cur ^ 1]);
+    la.load(pa, lda);
+    pa += BK * sa;
+    lb.store(lds[cur ^ 1] + LA::kUnits);
+    lb.load(pb, ldb);
+    pb += BK * sb;
+    multiply(lds[cur], 1);
+    __builtin_amdgcn_iglp_opt(0);   // spread the LDS traffic and the cut over the matrix instructions (8192^3 202 -> 212 TFLOP/s, 4096x2048x4096 165 -> 206)
+  }
+  for (; i < tiles; i++, cur ^= 1) {   // the last stages: nothing more to fetch, or less than a stage
+    __syncthreads();
+    multiply(lds[cur], 0);
+    if (i + 1 < tiles) stage(lds[cur ^ 1]);
+    if (i + 2 < tiles) fetch(kbeg + (i + 2) * BK);
+    multiply(lds[cur], 1);
+  }
+#pragma unroll
+  for (int a = 0; a < FN; a++)
+#pragma unroll
+    for (int b = 0; b < FM; b++) acc[a][b] += low[a][b];
+  float scale = kSplitUnscale;
+  float bad = 0.0f;
+#pragma unroll
+  for (int b = 0; b < FM; b++)
+    if (i0 + wm + 32 * b + l32 < m) {
+#pragma unroll
+      for (int a = 0; a < FN; a++)
+#pragma unroll
+        for (int r = 0; r < 16; r++)
+          if (j0 + wn + 32 * a + 8 * (r >> 2) + 4 * half + (r & 3) < n) bad += acc[a][b][r] * 0.0f;
+    }
+  if (__any(bad != 0.0f)) {   // (NaN: a sum was not finite)
+    scale = 1.0f;
+#pragma unroll
+    for (int a = 0; a < FN; a++)
+#pragma unroll
+      for (int b = 0; b < FM; b++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[a][b][r] = 0.0f;
+    long ra[FM], rb[FN];
+#pragma unroll
+    for (int f = 0; f < FM; f++) { const int i = i0 + wm + 32 * f + l32; ra[f] = (long)(i < m ? i : m - 1) * (TA ? lda : 1); }
+#pragma unroll
+    for (int f = 0; f < FN; f++) { const int j = j0 + wn + 32 * f + l32; rb[f] = (long)(j < n ? j : n - 1) * (TB ? 1 : ldb); }
+    for (int k0 = kbeg; k0 < kend; k0 += 2) {
+      const int kk = k0 + half;
+      const bool in_k = kk < kend;
+      float va[FM], vb[FN];
+#pragma unroll
+      for (int f = 0; f < FM; f++) va[f] = in_k ? A[ra[f] + kk * sa] : 0.0f;
+#pragma unroll
+      for (int f = 0; f < FN; f++) vb[f] = in_k ? B[rb[f] + kk * sb] : 0.0f;
+#pragma unroll
+      for (int a = 0; a < FN; a++)
+#pragma unroll
+        for (int b = 0; b < FM; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[a], va[b], acc[a][b], 0, 0, 0);
+    }
+  }
+  float* c = C;
+  const long ld = ldc;
+  if (splits > 1) c += (long)z * m * n;   // this slice's sums; gemm_split_sum_kernel applies the rest
+#pragma unroll
+  for (int b = 0; b < FM; b++) {
+    const int i = i0 + wm + 32 * b + l32;
+    if (i >= m) continue;
+    const float bi = (bias && splits == 1) ? bias[i] : 0.0f;
+#pragma unroll
+    for (int a = 0; a < FN; a++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const int j = j0 + wn + 32 * a + 8 * (r >> 2) + 4 * half + (r & 3);
+        if (j < n) {
+          float v = acc[a][b][r] * scale;
+          float* d = c + (long)j * ld + i;
+          if (splits == 1) {
+            v = alpha * v;
+            if (beta != 0.0f) v = v + beta * *d;
+            if (bias) v = v + bi;
+            if (act == 1) v = v > 0.0f ? v : 0.0f;
+          }
+          *d = v;
+        }
+      }
+  }
+}
+
+// How many slices of k an m x n x k product is cut into, and its estimated time in us: a stage of 32 steps takes 2.4 with all 256 CUs at work, starting
+// and storing a tile 5 (fitted to measurements); slices, which let few tiles fill the chip, cost a second launch that reads them.
+struct SplitPlan { int splits, kchunk; double us; };
+inline SplitPlan gemm_split_plan(int m, int n, int k) {
+  constexpr size_t kMostPartial = size_t(64) << 20;
+  const double ncu = tuning(kTuneNumCUs), tiles = double((m + 255) / 256) * ((n + 127) / 128), stages = (k + 31) / 32;
+  SplitPlan best = {1, k, 1e30};
+  for (int s = 1; s <= 16; s++) {
+    if (s > 1 && (stages / s < 4 || (size_t)s * m * n * sizeof(float) > kMostPartial)) break;
+    const double per = (double)(long)((stages + s - 1) / s), turns = (double)(long)((tiles * s + ncu - 1) / ncu);
+    double us = turns * (per * 2.4 + 5);
+    if (s > 1) us += 4 + (s + 1) * 4.0 * m * n / 5e6;
+    if (us < best.us) best = {s, (int)per * 32, us};
+  }
+  best.splits = (k + best.kchunk - 1) / best.kchunk;
+  return best;
+}
+// True if the product runs here: estimated faster than the vendor's fp32 kernels (140 TFLOP/s and 8 us for the call).  us, this / vendor: 2000x1000x2000 55/64,
+// 2000x2000x1000 NT 56/65, 1000x2048x4096 101/127; not taken: 1024^3 30/19, 512x512x2048 NT 27/15, 1000x237x784 21/11, 3000x3000x40 32/22.
+// The loaders' offsets within a tile have 32 bits: 255 * ld.
+inline bool gemm_split_fits(int m, int n, int k, int lda, int ldb, SplitPlan* plan) {
+  const int knob = tuning(kTuneGemmSplit);   // for tests and comparisons: 1 never, 2 wherever the kernel can
+  if (m < 4 || n < 4 || k < 1 || lda > (1 << 23) || ldb > (1 << 23) || knob == 1) return false;
+  const double flop = 2.0 * m * n * (double)k;
+  if (knob != 2 && (m < 64 || n < 64 || k < 64 || flop < 2e9)) return false;
+  *plan = gemm_split_plan(m, n, k);
+  return knob == 2 || plan->us < 0.95 * (flop / 140e6 + 8);
+}
+
+// C = act(alpha*sum of the slices [+ beta*C] [+ bias]), slices in order.
+__global__ __launch_bounds__(256) void gemm_split_sum_kernel(int m, int n, int splits, const float* __restrict__ partial, float* C, int ldc, float alpha,
+                                                             float beta, const float* __restrict__ bias, int act) {
+  const long mn = (long)m * n;
+  for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < mn; e += (long)gridDim.x * 256) {
+    float v = partial[e];
+    for (int z = 1; z < splits; z++) v = v + partial[z * mn + e];
+    const int i = (int)(e % m), j = (int)(e / m);
+    float* d = C + (long)j * ldc + i;
+    v = alpha * v;
+    if (beta != 0.0f) v = v + beta * *d;
+    if (bias) v = v + bias[i];
+    if (act == 1) v = v > 0.0f ? v : 0.0f;
+    *d = v;
+  }
+}
+
+inline int launch_gemm_split(hipStream_t stream, bool ta, bool tb, int m, int n, int k, float alpha, const float* A, int lda, const float* B, int ldb,
+                             float beta, float* C, int ldc, const float* bias, int act, const SplitPlan& plan) {
+  float* out = C;
+  int ldo = ldc;
+  if (plan.splits > 1) {
+    const Workspace ws = workspace_for(stream, (size_t)plan.splits * m * n * sizeof(float), 0);
+    if (ws.partial == nullptr) {
+      record_error("gemm (split): no scratch memory for the slices of k");
+      return -1;
+    }
+    out = static_cast<float*>(ws.partial);
+    ldo = m;
+  }
+  const long tiles = (long)((m + 255) / 256) * ((n + 127) / 128);
+  const dim3 grid((unsigned)(tiles * plan.splits)), block(512);
+#define KNET8_SP(TA, TB) hipLaunchKernelGGL((gemm_split_kernel<256, 128, 64, 64, 32, TA, TB>), grid, block, 0, stream, m, n, k, A, lda, B, ldb, out, ldo, alpha, beta, bias, act, plan.kchunk, (unsigned)plan.splits)
+  if (!ta && !tb) KNET8_SP(false, false);
+  else if (ta && !tb) KNET8_SP(true, false);
+  else if (!ta && tb) KNET8_SP(false, true);
+  else KNET8_SP(true, true);
+#undef KNET8_SP
+  if (plan.splits > 1) {
+    const long mn = (long)m * n, blocks = (mn + 255) / 256;
+    hipLaunchKernelGGL(gemm_split_sum_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream, m, n, plan.splits, out, C, ldc, alpha, beta, bias, act);
+  }
+  check_launch("gemm (split)");
+  return 0;
+}
+
+}  // namespace knet8

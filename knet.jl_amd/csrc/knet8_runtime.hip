@@ -2,6 +2,7 @@
 // storage, copies, stream/timer helpers and the hipBLASLt GEMM entry points.
 #include "knet8_runtime.h"
 #include "knet8_gemm_small.h"
+#include "knet8_gemm_split.h"
 #include "knet8_fused.h"
 
 #include <hipblaslt/hipblaslt.h>
@@ -82,7 +83,7 @@ void rng_take(unsigned long long blocks, unsigned long long* seed, unsigned long
   g_rng_offset += blocks;
 }
 
-static int g_tune[kTuneCount] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+static int g_tune[kTuneCount] = {};
 int tuning(int key) {
   if (key < 0 || key >= kTuneCount) return 0;
   if (key == kTuneNumCUs && g_tune[key] == 0) {  // compute units of the current device, asked once
@@ -891,6 +892,14 @@ static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T*
     launch_gemm_small<T>(stream, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, bias, act);
     check_launch("gemm (small)");
     return 0;
+  }
+  if constexpr (sizeof(T) == 4) {   // large fp32 products: on the bf16 matrix cores
+    SplitPlan plan;
+    if (batch.count == 1 && gemm_split_fits(m, n, k, lda, ldb, &plan)) {
+      if (bias == nullptr && act) { record_error("gemm_bias_act: an activation without a bias is not provided"); return -1; }
+      if (g_tune[kTuneGemmDryRun] != 0) return 0;
+      return launch_gemm_split(stream, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, bias, act, plan);
+    }
   }
   // Products the vendor library has no kernel for (seen with some fp64 shapes) run on the library's own tiles, whatever their size.
   auto plain = [&](T bt) {

@@ -1,0 +1,122 @@
+"""Large fp32 products on the bf16 matrix cores (three bf16 parts per element): edges of the tiles, remainders of k, slices of k, the epilogue,
+and what does not fit the parts (infinities, NaN, sums beyond 2^80, denormals)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def device(knet, a):
+    return knet.KnetArray(np.asfortranarray(a))
+
+
+def product(knet, ta, tb, A, B, alpha=1.0, beta=0.0, C=None):
+    m, n = (A.shape[1] if ta else A.shape[0]), (B.shape[0] if tb else B.shape[1])
+    C = np.zeros((m, n), np.float32) if C is None else C
+    out = device(knet, C)
+    knet.gemm("T" if ta else "N", "T" if tb else "N", alpha, device(knet, A), device(knet, B), beta, out)
+    return knet.Array(out)
+
+
+def operands(rng, ta, tb, m, n, k):
+    A, B = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
+    return A, B, (np.ascontiguousarray(A.T) if ta else A), (np.ascontiguousarray(B.T) if tb else B)
+
+
+@pytest.fixture
+def everywhere(knet):
+    """The kernel takes every product that it can (knet8_tune key 9), so that its edges are reached at small sizes."""
+    fn = knet.libknet8().fn
+    old = fn["knet8_tune"](9, 2)
+    yield
+    fn["knet8_tune"](9, old)
+
+
+# (m, n, k) around the 256x128 tile and its 32 steps of k: the smallest; one row or column less and more; 1 to 3 rows in the last tile (fewer than
+# one lane of the loader takes); k of less than a stage, whole stages, remainders; more than one slice of k
+SHAPES = [(4, 4, 1), (5, 7, 3), (63, 200, 33), (255, 127, 31), (256, 128, 32), (257, 129, 64), (258, 130, 65), (259, 131, 96), (129, 257, 127), (511, 385, 100),
+          (257, 131, 1000), (1024, 1024, 2048), (300, 260, 4111)]
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_every_element_against_64_bits(knet, everywhere, m, n, k, ta, tb):
+    rng = np.random.default_rng(m + 3 * n + 7 * k + 2 * ta + tb)
+    A, B, a, b = operands(rng, ta, tb, m, n, k)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    got = product(knet, ta, tb, a, b)
+    # k products with a rounding of 2^-24 of the running sum each (random signs: sqrt(k) of them, running sums up to sqrt(k)); 6 standard deviations
+    bound = 6 * 2.0 ** -24 * k ** 0.5 * max(1.0, k ** 0.5)
+    assert np.abs(got - want).max() <= bound
+    assert np.linalg.norm(got - want) <= 2.0 ** -24 * max(4.0, k ** 0.5) * np.linalg.norm(want)
+    knet.libknet8().check()
+
+
+@pytest.mark.parametrize("m,n,k", [(515, 390, 330), (1025, 771, 4100)])
+def test_scalars_bias_and_relu(knet, everywhere, m, n, k):
+    rng = np.random.default_rng(9)
+    lib = knet.libknet8()
+    A, B, _, _ = operands(rng, False, False, m, n, k)
+    C = rng.standard_normal((m, n)).astype(np.float32)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    got = product(knet, False, False, A, B, alpha=0.5, beta=2.0, C=C)
+    assert np.linalg.norm(got - (0.5 * want + 2.0 * C)) <= 2.0 ** -24 * k ** 0.5 * np.linalg.norm(want)
+    plain = product(knet, False, False, A, B)
+    bias = rng.standard_normal(m).astype(np.float32)
+    Ad, Bd, bd = device(knet, A), device(knet, B), device(knet, bias)
+    for act in (0, 1):
+        out = knet.KnetArray(np.zeros((m, n), np.float32))
+        assert lib.call("gemm_bias_act_32", b"N", b"N", m, n, k, 1.0, Ad.ptr, m, Bd.ptr, k, bd.ptr, act, out.ptr, m) == 0
+        chain = plain + bias[:, None]
+        assert np.array_equal(knet.Array(out), np.maximum(chain, 0) if act else chain)      # the product's bits, one rounded addition
+    lib.check()
+
+
+@pytest.mark.parametrize("m,n,k", [(4096, 1792, 545), (1000, 2048, 4096), (255, 3000, 8005), (64, 100, 784)])
+def test_the_rule_for_large_products(knet, m, n, k):
+    """Products that the rule gives to this kernel have the bits of the forced route; a small one stays where it was."""
+    fn = knet.libknet8().fn
+    rng = np.random.default_rng(12)
+    A, B, _, _ = operands(rng, False, False, m, n, k)
+    got = {}
+    for knob in (0, 1, 2):
+        old = fn["knet8_tune"](9, knob)
+        try:
+            got[knob] = product(knet, False, False, A, B)
+        finally:
+            fn["knet8_tune"](9, old)
+    assert np.array_equal(got[0], got[1] if m == 64 else got[2])
+    assert np.linalg.norm(got[1] - got[2]) <= 2.0 ** -24 * k ** 0.5 * np.linalg.norm(got[1])
+
+
+def test_what_the_parts_cannot_hold(knet, everywhere):
+    rng = np.random.default_rng(10)
+    m, n, k = 1024, 1024, 2048
+    A, B, _, _ = operands(rng, False, False, m, n, k)
+    A[3, 5], A[700, 9], A[300, 17] = np.inf, np.nan, 3.4e38
+    B[1, 400] = -np.inf
+    with np.errstate(all="ignore"):
+        want = A.astype(np.float64) @ B.astype(np.float64)
+    got = product(knet, False, False, A, B)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)].astype(np.float32))
+    fine = np.isfinite(want) & (np.abs(want) < 3e38)
+    with np.errstate(invalid="ignore"):
+        off = np.abs(got - want)
+    assert off[fine].max() <= 1e-5 * np.abs(want[fine]).max()
+    rest = np.ones(m, bool)
+    rest[[3, 700, 300]] = False
+    cols = np.ones(n, bool)
+    cols[400] = False
+    assert off[rest][:, cols].max() <= 6 * 2.0 ** -24 * k
+    # whole rows at the ends of the range: denormals and tiny numbers, numbers whose sums pass 2^80
+    A, B, _, _ = operands(rng, False, False, m, n, k)
+    s = np.ones(m)
+    s[:64], s[64:128], s[512:576] = 1e-36, 1e-42, 1e30
+    A = (A * s[:, None]).astype(np.float32)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    got = product(knet, False, False, A, B)
+    err = np.linalg.norm(got - want, axis=1)
+    least = 2.0 ** -149 * n ** 0.5        # the spacing of denormal results
+    assert np.all(err <= 2.0 ** -24 * k ** 0.5 * np.linalg.norm(want, axis=1) + least)
+    knet.libknet8().check()

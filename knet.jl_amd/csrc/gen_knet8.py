@@ -678,8 +678,8 @@ KNET8_API const char* knet8_build_id(void);
 KNET8_API void sum_32_21_noalloc(int nx, float* x, int sy, int ny, float* y, hipStream_t stream);
 /* launch-heuristic knobs; returns the old value; value 0 restores the default, a negative value only reads.  Key 0: number of compute units the reduction planner aims at (default: asked from the
    device); key 1: longest softmax column kept resident in registers, longer ones take the two-pass streaming kernel (default 0: the register capacity);
-   key 3: products of up to this many MFLOP (2*m*n*k/1e6) take the library's own small-product kernels instead of hipBLASLt (default 0: off,
-   products of gemm_S / gemm_bias_act_S go to hipBLASLt, or where key 9 says);
+   key 3: products of up to this many MFLOP (2*m*n*k/1e6) take the library's own small-product kernels instead of hipBLASLt (default 0: a rule on
+   type and sizes, up to 270 MFLOP, where the loaded hipBLASLt allows no prepared calls; 1 in effect switches them off);
    key 4: dense_back_S / dense_nll_back_S accept layers whose products have up to this many MFLOP each (default 270);
    key 5: non-zero makes the library behave as if the scratch memory of split launches could not be allocated (for tests of that error path);
    key 6: non-zero keeps softmax columns of 128 to 256 KB in registers alone instead of registers + LDS (for comparisons);

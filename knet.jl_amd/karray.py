@@ -174,6 +174,17 @@ def Array(x):
     return x.to_numpy() if isinstance(x, KnetArray) else np.asarray(x)
 
 
+def upload(data):
+    """Device array of a contiguous host vector for launches that follow on the current stream: the caller does not wait for the copy (``knet8_upload``).
+    For arrays that stay inside one operation; ``KnetArray(data)`` is ready on every stream."""
+    a = np.ascontiguousarray(data)
+    k = KnetArray(dtype=a.dtype, dims=a.shape)
+    lib = libknet8()
+    if lib.fn["knet8_upload"](k.ptr, a.ctypes.data, a.nbytes, lib.stream) != 0:
+        lib.check()
+    return k
+
+
 def synchronize():
     lib = libknet8()
     lib.fn["knet8_synchronize"](lib.stream)

@@ -7,7 +7,7 @@ Mirrors src/ops20/loss.jl:37-41,116-140 and the device side of ``x[indices]`` an
 import numpy as np
 
 from .autograd import drop, primitive, value
-from .karray import KnetArray
+from .karray import KnetArray, upload
 from .libknet8 import knet8
 from . import reduction as R
 from .softmax import logsoftmax
@@ -43,7 +43,7 @@ def _device_indices(x, indices):
     idx = np.asarray(indices, dtype=np.int64).ravel()
     if idx.size and (idx.min() < 1 or idx.max() > x.length):  # bounds check on the host, getindex.jl:277-287
         raise IndexError("BoundsError")
-    return KnetArray(idx.astype(np.int32))
+    return upload(idx.astype(np.int32))
 
 
 def ungetindex(x, dxi, indices):
@@ -97,7 +97,7 @@ def _nll_fused(scores, labels, dims=1, count=None):
         if lab.size and (lab.min() < 0 or lab.max() > m):
             raise IndexError("BoundsError")
         count = int(np.count_nonzero(lab))
-        dlab = KnetArray(lab.astype(np.int32))
+        dlab = upload(lab.astype(np.int32))
     dx = scores.similar()
     lossv = scores.similar((n,))
     scale = T(1) / T(count) if count else T(np.inf)
@@ -126,7 +126,7 @@ def _nll_fused(scores, labels, dims=1, count=None):
 
 def _nll_one_pass(scores, labels, dims):
     """``nll`` of host labels by ``nll_logsoftmax_back_S`` and one sum: loss and gradient in one read of the scores and one write, where logsoftmax, gather,
-    scatter and logsoftmaxback take seven passes and two uploads of indices (32000x512 fp32: 145 -> 82 us a pass).  None where the chain has to decide:
+    scatter and logsoftmaxback take seven passes and two uploads of indices (32000x512 fp32: 145 -> 82 us a pass, 62 with ``upload``).  None where the chain has to decide:
     labels that skip an instance or lie outside the classes, other dims, and scores whose loss is not finite (the chain then says which gradients are NaN)."""
     x = value(scores)
     if dims != 1 or not isinstance(x, KnetArray) or x.suffix is None or x.ndims < 1 or isinstance(labels, KnetArray):

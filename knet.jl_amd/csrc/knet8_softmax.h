@@ -630,27 +630,32 @@ __device__ __forceinline__ void maxsum_merge(T& m, T& s, T m2, T s2) {
   s = s1 + s3;
 }
 
-template <typename T, typename Algo, bool VEC>
+// Few columns leave compute units idle that way: then P workgroups share a column, `chunk` rows each, in two launches.  The first (PART 1) leaves each share's
+// max and sum in `part`, the second (PART 2) merges a column's P pairs in order and writes its share.  (100000 rows, 100 columns, fp32, P = 5:
+// logsoftmaxback 37.3 -> 25.4 us, logsoftmax 20.1 -> 19.6.)
+enum { kWhole = 0, kReducePart = 1, kApplyPart = 2 };
+template <typename T, typename Algo, bool VEC, int PART>
 __global__ __launch_bounds__(1024) void softmax_col_stream_kernel(long m, long n, const T* a, const T* b, T* out, const int* labels,
-                                                                  T scale, T* loss) {
+                                                                  T scale, T* loss, long chunk, unsigned P, T* part) {
   constexpr int NV = VEC ? Vec16<T>::N : 1;
   constexpr int U = 4;
   constexpr bool kTwo = Algo::kInputs == 2;
   constexpr long STEP = 1024L * NV;
   typedef typename Vec16<T>::type V;
   __shared__ T lds[2][1024 / kWave];
-  const long col = blockIdx.x;
+  const long col = PART == kWhole ? (long)blockIdx.x : (long)(blockIdx.x / P);
+  const long c0 = PART == kWhole ? 0 : (long)(blockIdx.x % P) * chunk, c1 = PART == kWhole || c0 + chunk > m ? m : c0 + chunk;
   const T* ac = a + col * m;
   const T* bc = kTwo ? b + col * m : nullptr;
   T* oc = out + col * m;
   const T ninf = T(-INFINITY);
   T mx = Algo::kNeedMax ? ninf : T(0), s = T(0);
-  for (long r0 = (long)threadIdx.x * NV; r0 < m; r0 += STEP * U) {
+  if (PART != kApplyPart) for (long r0 = c0 + (long)threadIdx.x * NV; r0 < c1; r0 += STEP * U) {
     T va[U][NV], vb[U][NV];
 #pragma unroll
     for (int q = 0; q < U; q++) {
       const long r = r0 + q * STEP;
-      if (r < m) {
+      if (r < c1) {
         if (VEC) {
           const V t = *reinterpret_cast<const V*>(ac + r);
 #pragma unroll
@@ -687,7 +692,15 @@ __global__ __launch_bounds__(1024) void softmax_col_stream_kernel(long m, long n
         for (int e = 0; e < NV; e++) s = s + Algo::term(va[q][e], kTwo ? vb[q][e] : T(0), T(0));
     }
   }
-  if (Algo::kNeedMax) {
+  if (PART == kApplyPart) {
+    const T* mine = part + 2 * col * P;
+    mx = mine[0];
+    s = mine[1];
+    for (unsigned w = 1; w < P; w++) {
+      if (Algo::kNeedMax) maxsum_merge(mx, s, mine[2 * w], mine[2 * w + 1]);
+      else s = s + mine[2 * w + 1];
+    }
+  } else if (Algo::kNeedMax) {
     {
       MaxSum<T> ms = {mx, s};
       ms = ms_wave_reduce(ms);
@@ -703,16 +716,20 @@ __global__ __launch_bounds__(1024) void softmax_col_stream_kernel(long m, long n
   } else {
     s = block_reduce<T, 1024 / kWave>(s, lds[0], AddFn(), T(0));
   }
+  if (PART == kReducePart) {
+    if (threadIdx.x == 0) { part[2 * (long)blockIdx.x] = mx; part[2 * (long)blockIdx.x + 1] = s; }
+    return;
+  }
   const T fin = Algo::finish(s);
   int lab = Algo::kNll ? labels[col] : 0;
   if (lab < 0 || lab > m) lab = 0;
   const T st = -scale;
-  for (long r0 = (long)threadIdx.x * NV; r0 < m; r0 += STEP * U) {
+  for (long r0 = c0 + (long)threadIdx.x * NV; r0 < c1; r0 += STEP * U) {
     T va[U][NV], vb[U][NV];
 #pragma unroll
     for (int q = 0; q < U; q++) {
       const long r = r0 + q * STEP;
-      if (r < m) {
+      if (r < c1) {
         if (VEC) {
           const V t = ld_stream(reinterpret_cast<const V*>(ac + r));
 #pragma unroll
@@ -731,7 +748,7 @@ __global__ __launch_bounds__(1024) void softmax_col_stream_kernel(long m, long n
 #pragma unroll
     for (int q = 0; q < U; q++) {
       const long r = r0 + q * STEP;
-      if (r < m) {
+      if (r < c1) {
         V vo;
 #pragma unroll
         for (int e = 0; e < NV; e++) {
@@ -750,7 +767,7 @@ __global__ __launch_bounds__(1024) void softmax_col_stream_kernel(long m, long n
       }
     }
   }
-  if (Algo::kNll && lab == 0 && threadIdx.x == 0) loss[col] = T(0);
+  if (Algo::kNll && lab == 0 && c0 == 0 && threadIdx.x == 0) loss[col] = T(0);
 }
 
 // ---- softmax along a non-leading axis: x viewed as (inner, d, outer), softmax over d -----------------------
@@ -1056,8 +1073,32 @@ inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const
     }
   }
   if ((resident_cap > 0 && m > resident_cap) || m > 1024L * kBig1024) {
-    if (vec_stream) hipLaunchKernelGGL((softmax_col_stream_kernel<T, Algo, true>), dim3((unsigned)n), dim3(1024), 0, stream, m, n, a, b, out, labels, scale, loss);
-    else hipLaunchKernelGGL((softmax_col_stream_kernel<T, Algo, false>), dim3((unsigned)n), dim3(1024), 0, stream, m, n, a, b, out, labels, scale, loss);
+    // Shares of a column: two workgroups per compute unit over all columns, 8192 rows or more each (a compute unit holds two of these workgroups, so that a
+    // column to a workgroup fills the chip from 257 columns on).
+    const long ncu = tuning(kTuneNumCUs);
+    long P = n <= ncu ? 2 * ncu / n : 1;
+    if (P > m / 8192) P = m / 8192;
+    if (P > 64) P = 64;
+    T* part = nullptr;
+    long chunk = m;
+    if (P > 1) {
+      chunk = ((m + P - 1) / P + N - 1) / N * N;
+      P = (m + chunk - 1) / chunk;
+      part = static_cast<T*>(workspace_for(stream, 2 * sizeof(T) * (size_t)n * P, 0).partial);   // without scratch: a workgroup per column
+    }
+#define KNET8_STREAM(VEC, PART, BLOCKS) \
+  hipLaunchKernelGGL((softmax_col_stream_kernel<T, Algo, VEC, PART>), dim3((unsigned)(BLOCKS)), dim3(1024), 0, stream, m, n, a, b, out, labels, scale, loss, chunk, (unsigned)P, part)
+    if (part == nullptr) {
+      if (vec_stream) KNET8_STREAM(true, kWhole, n);
+      else KNET8_STREAM(false, kWhole, n);
+    } else if (vec_stream) {
+      KNET8_STREAM(true, kReducePart, n * P);
+      KNET8_STREAM(true, kApplyPart, n * P);
+    } else {
+      KNET8_STREAM(false, kReducePart, n * P);
+      KNET8_STREAM(false, kApplyPart, n * P);
+    }
+#undef KNET8_STREAM
     return;
   }
   // Columns of 128 to 256 KB: two 512-lane workgroups per compute unit with part of the column in LDS (see softmax_col_body).

@@ -584,12 +584,14 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   // workgroup size by the work of one part: a wave for short runs, 512 lanes when there is plenty
   const int bt = chunk <= 2 * kWave ? 64 : chunk <= 4096 ? 256 : 512;
   const dim3 grid((unsigned)(ny * P));
+  // no more workgroups than compute units: twice the lanes keep twice the bytes in flight (sum over 29x29x193x64 fp32 15.6 -> 11.0 us)
+  const bool alone = (long)ny * P <= tuning(kTuneNumCUs);
 #define KNET8_RUN(NV, SINGLE, BT, U, ANY) \
   hipLaunchKernelGGL((reduce_run_kernel<T, Op, NV, SINGLE, BT, U, ANY>), grid, dim3(BT), 0, stream, x, sy, ny, units, chunk, P, y, partial, ws.counters, center KNET8_TL_ARG)
   // (the path with loads of one element, for short runs that do not start on 16-byte boundaries, keeps four times as many in flight per lane to move the same bytes)
 #define KNET8_RUN_BT(NV, SINGLE, ANY) \
   do { if (bt == 64) KNET8_RUN(NV, SINGLE, 64, (NV == 1 ? 16 : 8), ANY); else if (bt == 256) KNET8_RUN(NV, SINGLE, 256, (NV == 1 ? 16 : 4), ANY); \
-       else KNET8_RUN(NV, SINGLE, 512, (NV == 1 ? 16 : ANY ? 8 : 4), ANY); } while (0)
+       else if (ANY && alone) KNET8_RUN(NV, SINGLE, 1024, 8, ANY); else KNET8_RUN(NV, SINGLE, 512, (NV == 1 ? 16 : ANY ? 8 : 4), ANY); } while (0)
   if (vec)      { if (no == 1) KNET8_RUN_BT(N, true, false); else KNET8_RUN_BT(N, false, false); }
   else if (any) { if (no == 1) KNET8_RUN_BT(N, true, true); else KNET8_RUN_BT(N, false, true); }
   else          { if (no == 1) KNET8_RUN_BT(1, true, false); else KNET8_RUN_BT(1, false, false); }

@@ -55,7 +55,7 @@ def mean(x, dims=None, f=None):
 
 
 def _var_one_pass(x, m, dims, corrected):
-    """The sum of squares, its division and the subtraction before it as one launch (``sumsqdev_S_21``; 29x29x193x64 fp32: 98 us a pass with the mean, 36 us so), where nothing is recorded of ``x`` or ``m``, one
+    """The sum of squares, its division and the subtraction before it as one launch (``sumsqdev_S_21``; 29x29x193x64 fp32: 98 us a pass with the mean, 30 us so), where nothing is recorded of ``x`` or ``m``, one
     dimension of ``x`` remains and ``m`` has a value for each of its positions; None otherwise, and for shapes the kernel does not take."""
     if dims is None or track(x) is not None or track(m) is not None:
         return None

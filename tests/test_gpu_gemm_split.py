@@ -33,9 +33,10 @@ def everywhere(knet):
 
 
 # (m, n, k) around the 256x128 tile and its 32 steps of k: the smallest; one row or column less and more; 1 to 3 rows in the last tile (fewer than
-# one lane of the loader takes); k of less than a stage, whole stages, remainders; more than one slice of k
+# one lane of the loader takes); k of less than a stage, whole stages, remainders; more than one slice of k; more tiles than
+# compute units
 SHAPES = [(4, 4, 1), (5, 7, 3), (63, 200, 33), (255, 127, 31), (256, 128, 32), (257, 129, 64), (258, 130, 65), (259, 131, 96), (129, 257, 127), (511, 385, 100),
-          (257, 131, 1000), (1024, 1024, 2048), (300, 260, 4111)]
+          (257, 131, 1000), (1024, 1024, 2048), (300, 260, 4111), (4097, 2049, 70)]
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])

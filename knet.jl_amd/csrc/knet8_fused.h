@@ -248,7 +248,7 @@ inline void launch_actback_biasgrad(hipStream_t stream, long m, long n, const T*
   long jchunk = ceil_div(n, P);
   P = (unsigned)ceil_div(n, jchunk > 0 ? jchunk : 1);
   if (P < 1) P = 1;
-  Workspace ws = {nullptr, nullptr};
+  Workspace ws;
   if (P > 1) {
     ws = workspace_for(stream, sizeof(T) * (size_t)atiles * P * tile, (size_t)atiles * kTicketStride);
     if (!scratch_ready(ws, "activation gradient + bias gradient: no scratch memory for a split launch")) return;

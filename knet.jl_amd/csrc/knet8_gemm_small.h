@@ -248,7 +248,7 @@ inline void launch_gemm_small(hipStream_t stream, bool ta, bool tb, int m, int n
   if (kchunk < kGsTile) kchunk = kGsTile;
   P = (k + kchunk - 1) / kchunk;
   if (P < 1) P = 1;
-  Workspace ws = {nullptr, nullptr};
+  Workspace ws;
   if (P > 1) {
     ws = workspace_for(stream, sizeof(T) * (size_t)tiles * P * kGsTile * kGsTile, (size_t)tiles);
     if (!scratch_ready(ws, "gemm (small, k split): no scratch memory for a split launch")) return;

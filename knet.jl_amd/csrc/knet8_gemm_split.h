@@ -368,8 +368,9 @@ inline int launch_gemm_split(hipStream_t stream, bool ta, bool tb, int m, int n,
                              float beta, float* C, int ldc, const float* bias, int act, const SplitPlan& plan) {
   float* out = C;
   int ldo = ldc;
+  Workspace ws;
   if (plan.splits > 1) {
-    const Workspace ws = workspace_for(stream, (size_t)plan.splits * m * n * sizeof(float), 0);
+    ws = workspace_for(stream, (size_t)plan.splits * m * n * sizeof(float), 0);
     if (ws.partial == nullptr) {
       record_error("gemm (split): no scratch memory for the slices of k");
       return -1;

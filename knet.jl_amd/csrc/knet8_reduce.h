@@ -512,7 +512,7 @@ inline bool launch_reduce_stretch(hipStream_t stream, const T* x, long sy, long 
   if (P < 1 || !scratch_fits(scratch, sizeof(T) * (size_t)groups * P * g, (size_t)groups * kTicketStride)) P = 1;   // a provider of fixed size: no split beyond it
   long ipp = ceil_div(iters, P);
   P = ceil_div(iters, ipp);
-  Workspace ws = {nullptr, nullptr};
+  Workspace ws;
   if (P > 1) {
     ws = take_scratch(scratch, stream, sizeof(T) * (size_t)groups * P * g, (size_t)groups * kTicketStride);
     if (!scratch_ready(ws, "reduction: no scratch memory for a split launch")) { if (launched) *launched = false; return true; }
@@ -575,7 +575,7 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   long chunk = ceil_div(units, P);
   P = (unsigned)ceil_div(units, chunk > 0 ? chunk : 1);
   if (P < 1) P = 1;
-  Workspace ws = {nullptr, nullptr};
+  Workspace ws;
   if (P > 1) {
     ws = take_scratch(scratch, stream, sizeof(T) * (size_t)ny * P, (size_t)ny * kTicketStride);
     if (!scratch_ready(ws, "reduction: no scratch memory for a split launch")) return false;
@@ -626,7 +626,7 @@ inline bool launch_reduce_strided(hipStream_t stream, const T* x, long s1, long 
   long kchunk = ceil_div(d, P);
   P = (unsigned)ceil_div(d, kchunk > 0 ? kchunk : 1);
   if (P < 1) P = 1;
-  Workspace ws = {nullptr, nullptr};
+  Workspace ws;
   if (P > 1) {
     ws = take_scratch(scratch, stream, front + sizeof(T) * (size_t)groups * P * tile, (size_t)groups * kTicketStride);
     if (!scratch_ready(ws, "reduction: no scratch memory for a split launch")) return false;

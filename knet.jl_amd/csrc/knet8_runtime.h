@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include <mutex>
+
 #ifndef KNET8_API
 #define KNET8_API __attribute__((visibility("default")))
 #endif
@@ -17,11 +19,14 @@ void check_launch(const char* name);  // records hipGetLastError() if a launch f
 
 // Scratch that split reductions need beyond their inputs and outputs: `partial` holds the per-workgroup
 // partial results, `counters` the per-output-group tickets (all zero between launches; the kernel that
-// uses them resets them).  One Workspace per stream, so launches on different streams never share it;
-// launches on one stream are ordered and may.
+// uses them resets them).  One per stream, so launches on different streams never share it; launches on one stream are
+// ordered and may.  Where a first launch leaves sums there that a second one reads, another host thread's launch must not
+// come in between: a Workspace keeps the stream's scratch to its thread until it goes out of scope, so keep it until the
+// last launch that uses it is queued.
 struct Workspace {
-  void* partial;
-  unsigned* counters;
+  void* partial = nullptr;
+  unsigned* counters = nullptr;
+  std::unique_lock<std::recursive_mutex> held;
 };
 Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounters);
 // Where a split launch takes its scratch from: the per-stream buffers above (a null source) or a caller-supplied provider.  A provider

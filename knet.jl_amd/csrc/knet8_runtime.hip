@@ -130,6 +130,14 @@ static bool stream_is_capturing(hipStream_t stream) {
   return cap != hipStreamCaptureStatusNone;
 }
 
+// The lock a Workspace holds.  Of a fixed set, by stream: it outlives every stream, and two streams that meet in one only wait for each other's launches
+// to be queued.  Recursive, as the second pass of a two-pass reduction asks for scratch of its own.  Taken before g_scratch_mutex, never after it.
+constexpr size_t kScratchLocks = 61;
+static std::recursive_mutex g_scratch_locks[kScratchLocks];
+static std::unique_lock<std::recursive_mutex> hold_scratch(hipStream_t stream) {
+  return std::unique_lock<std::recursive_mutex>(g_scratch_locks[reinterpret_cast<uintptr_t>(stream) / 8 % kScratchLocks]);
+}
+
 // hipBLASLt workspaces, one per (device, stream), defined with the GEMM entry points below: release the one of a stream that is being
 // destroyed, or (every = true) all that no captured graph holds; returns the bytes released.
 static size_t gemm_release(int dev, hipStream_t stream, bool every);
@@ -153,10 +161,11 @@ __global__ __launch_bounds__(256) void zero_counters_kernel(unsigned* c, size_t 
 Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounters) {
   if (g_tune[kTuneFailScratch] != 0) {   // set by tests: behave as if the device were out of memory, without touching it
     record_error("reduction scratch: allocation refused (knet8_tune key 5 is set)");
-    Workspace none = {nullptr, nullptr};
-    return none;
+    return Workspace();
   }
   const bool capturing = stream_is_capturing(stream);
+  Workspace w;
+  w.held = hold_scratch(stream);
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
   StreamScratch& s = scratch_of(stream);
   if (capturing) s.in_graph = true;
@@ -183,7 +192,8 @@ Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounte
       if (ok(hipGetLastError(), "zero_counters_kernel")) s.ncounters = want;
     }
   }
-  Workspace w = {s.partial, s.counters};
+  w.partial = s.partial;
+  w.counters = s.counters;
   return w;
 }
 
@@ -216,24 +226,26 @@ static unsigned char* static_scratch_ptr() {
 }
 
 static Workspace static_scratch_get(void*, hipStream_t stream, size_t partial_bytes, size_t ncounters) {
-  Workspace none = {nullptr, nullptr};
+  Workspace w;
   if (partial_bytes > kStaticPartialBytes || ncounters > kStaticCounters) {
     char buf[256];
     snprintf(buf, sizeof(buf), "sum_32_21_noalloc: the split of this shape needs %zu bytes of partial results and %zu tickets; the library's fixed scratch "
              "holds %zu bytes and %zu tickets (use sum_32_21)", partial_bytes, ncounters, kStaticPartialBytes, kStaticCounters);
     record_error(buf);
-    return none;
+    return w;
   }
   unsigned char* base = static_scratch_ptr();
-  if (base == nullptr) return none;
+  if (base == nullptr) return w;
+  w.held = hold_scratch(stream);
   unsigned* counters = reinterpret_cast<unsigned*>(base + kStaticPartialBytes);
   // The array keeps whatever the last call on this GPU left in it: the tickets this launch draws start from zero by a fill kernel on
   // the same stream (a kernel, not a memset node, so the call can be captured into a graph).
   if (ncounters > 0) {
     hipLaunchKernelGGL(zero_counters_kernel, dim3((unsigned)((ncounters + 255) / 256)), dim3(256), 0, stream, counters, ncounters);
-    if (!ok(hipGetLastError(), "zero_counters_kernel")) return none;
+    if (!ok(hipGetLastError(), "zero_counters_kernel")) return w;
   }
-  Workspace w = {base, counters};
+  w.partial = base;
+  w.counters = counters;
   return w;
 }
 
@@ -402,6 +414,9 @@ KNET8_API void knet8_free(void* ptr) {
 }
 
 KNET8_API size_t knet8_trim(void) {
+  // no thread stands between being handed scratch and queueing the launches that use it
+  std::vector<std::unique_lock<std::recursive_mutex>> held;
+  for (auto& l : g_scratch_locks) held.emplace_back(l);
   (void)hipDeviceSynchronize();
   size_t released = 0;
   {

@@ -1079,13 +1079,14 @@ inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const
     long P = n <= ncu ? 2 * ncu / n : 1;
     if (P > m / 8192) P = m / 8192;
     if (P > 64) P = 64;
-    T* part = nullptr;
+    Workspace ws;
     long chunk = m;
     if (P > 1) {
       chunk = ((m + P - 1) / P + N - 1) / N * N;
       P = (m + chunk - 1) / chunk;
-      part = static_cast<T*>(workspace_for(stream, 2 * sizeof(T) * (size_t)n * P, 0).partial);   // without scratch: a workgroup per column
+      ws = workspace_for(stream, 2 * sizeof(T) * (size_t)n * P, 0);   // without scratch: a workgroup per column
     }
+    T* const part = static_cast<T*>(ws.partial);
 #define KNET8_STREAM(VEC, PART, BLOCKS) \
   hipLaunchKernelGGL((softmax_col_stream_kernel<T, Algo, VEC, PART>), dim3((unsigned)(BLOCKS)), dim3(1024), 0, stream, m, n, a, b, out, labels, scale, loss, chunk, (unsigned)P, part)
     if (part == nullptr) {

@@ -698,7 +698,8 @@ KNET8_API int knet8_tune(int key, int value);
    src/knetarrays/random.jl:14-18 (CUDA.seed!).  Unseeded, the stream starts from the operating system's entropy. */
 KNET8_API void knet8_seed(unsigned long long seed);
 /* replaces cublasSgemm_v2 / cublasDgemm_v2 at src/knetarrays/linalg.jl:26-52 (column-major, transa/transb in 'N','T'): hipBLASLt; large fp32 products run on the
-   library's own kernel, on the bf16 matrix cores with every element in three bf16 parts (no less precise than the fp32 matrix instruction) */
+   library's own kernel, on the bf16 matrix cores with every element in three bf16 parts (all 24 bits: dense sums come out more precise than from the fp32 matrix
+   instruction, a sum with one term that is not zero as precise) */
 KNET8_API int gemm_32_stream(char transa, char transb, int m, int n, int k, float alpha, float* A, int lda, float* B, int ldb, float beta, float* C, int ldc, hipStream_t stream);
 KNET8_API int gemm_32(char transa, char transb, int m, int n, int k, float alpha, float* A, int lda, float* B, int ldb, float beta, float* C, int ldc);
 KNET8_API int gemm_64_stream(char transa, char transb, int m, int n, int k, double alpha, double* A, int lda, double* B, int ldb, double beta, double* C, int ldc, hipStream_t stream);

@@ -1,13 +1,14 @@
 // Large fp32 matrix products on the bf16 matrix cores (column-major, C = alpha*op(A)*op(B) + beta*C [+ bias] [relu]).
 //
 // The fp32 matrix instructions run at 1/16 of the bf16 ones (157 against 2500 TFLOP/s nominal), and the vendor library's fp32 products sit at
-// their limit: 8192^3 reaches 153 TFLOP/s, 4096x2048x4096 149.  Here every element is cut into three bf16 parts, x = h + m + l, each the
-// rounding of what the ones before it leave: 3 x 8 bits and the signs hold all 24 bits of an fp32 number, so h + m + l = x exactly.  Of the nine
-// products of parts the six whose weight reaches 2^-24 of the whole are formed (hh, hm, mh, mm, hl, lh; what is left out is below 2^-26), hh in one
-// set of fp32 accumulators and the five small ones in another: the large sums see one rounding per 16 steps of k.  The result is more precise than the
-// fp32 instruction's.  2-norm of the error against 64 bits, this / vendor fp32, normal data: 512x256x64 4.9e-8/1.45e-7, 1000x237x784 1.6e-7/5.0e-7,
-// 4096x2048x4096 4.0e-7/1.15e-6; all-positive data 5.0e-8/1.2e-7, 1.5e-7/4.2e-7, 3.0e-7/8.4e-7.  (With all six in one set, which leaves room
-// for a 256x256 tile: 1.0e-6 at 4096x2048x4096, and 231 instead of 212 TFLOP/s at 8192^3.)
+// their limit: 8192^3 reaches 154 TFLOP/s, 4096x2048x4096 142-149.  Here every element is cut into three bf16 parts, x = h + m + l, each the
+// rounding of what the ones before it leave: 3 x 8 bits and the signs hold all 24 bits of an fp32 number, so h + m + l = x exactly, with
+// |m| <= 2^-8 |x| and |l| <= 2^-17 |x|.  Of the nine products of parts all but ll (at most 2^-34 of the whole) are formed, hh in one
+// set of fp32 accumulators and the seven small ones in another: the large sums see one rounding per 16 steps of k, and a sum with one term that is not
+// zero is rounded as the fp32 instruction rounds it.  (ml and lm reach 2^-24 of the whole together: without them such a sum is off by up to 2^-23.2, and sums
+// of equal numbers by as much; they cost a sixth of the speed.)  2-norm of the error against 64 bits, this / vendor fp32: normal data 1000x237x784 8.4e-8/5.0e-7,
+// 4096x2048x4096 4.0e-7/1.15e-6, 512x2048x32000 4.0e-7/3.2e-6; all-positive data 4.9e-8/3.8e-7, 3.5e-7/9.9e-7, 1.3e-7/2.8e-6; 2048^3 with one term a sum
+// 2.53e-8/2.53e-8 (largest 2^-23.995/2^-24.000), with two 3.2e-8/3.1e-8, with eight 3.8e-8/5.4e-8.
 //   * Small numbers: the lower parts of numbers below 2^-109 would leave bf16's range.  Both operands are multiplied by 2^24 on the way in and the
 //     sums by 2^-48 on the way out, which keeps every fp32 number, denormals included, whole.
 //   * Large numbers, infinities, NaN: a part or a sum that overflows leaves a NaN or an infinity in an accumulator (inf - inf in the split itself
@@ -16,9 +17,9 @@
 //
 // The cut is made while a tile goes from global memory to LDS (6.5 vector instructions an element, in the shadow of the matrix instructions of the
 // SIMD's other wave): no extra pass over the operands, no scratch.  What bounds it: 256x128 tile, 8 waves of 64x64, 32 steps of k a stage, two
-// stages in LDS (149 KB): matrix cores 3072 cycles a stage, LDS about 2070, vector ALU about 2100.  Measured with the loads and the cut left out: 255 TFLOP/s
-// on normal data against 345 on zeros -- the card's power limit, not the pipes, ends at about 255.  TFLOP/s (of fp32 work), this / vendor:
-// 4096x2048x4096 206/149, TN 209/149, 4096x4096x2048 NT 195/149, 512x2048x32000 TN 206/140, 32000x512x2048 NT 189/140, 8192^3 212/153.
+// stages in LDS (149 KB): matrix cores 4096 cycles a stage, LDS about 2070, vector ALU about 2100; and the clock, which normal data
+// holds further down than zeros do (with six products, loads and cut left out: 255 TFLOP/s against 345).  TFLOP/s (of fp32 work), this / vendor:
+// 4096x2048x4096 176/142, TN 171/149, 4096x4096x2048 NT 169/148, 32000x2048x512 150/137, 512x2048x32000 TN 165/143, 32000x512x2048 NT 163/145, 8192^3 177/154.
 #pragma once
 #include "knet8_device.h"
 #include "knet8_runtime.h"
@@ -175,7 +176,7 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
   LB lb;
   la.init(t, m - i0, lda);
   lb.init(t, n - j0, ldb);
-  f32x16 acc[FN][FM], low[FN][FM];   // hh, and the five products of lower weight
+  f32x16 acc[FN][FM], low[FN][FM];   // hh, and the seven products of lower weight
 #pragma unroll
   for (int a = 0; a < FN; a++)
 #pragma unroll
@@ -214,7 +215,7 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
 #pragma unroll
       for (int i = 0; i < FM; i++) fa[i] = __builtin_bit_cast(bf16x8, s[ua[i] + p * LA::kPart + 2 * step * LA::kStride]);
 #pragma unroll
-      for (int q = 2 - p; q >= 0; q--)
+      for (int q = p > 1 ? 1 : 2; q >= 0; q--)
 #pragma unroll
         for (int a = 0; a < FN; a++)
 #pragma unroll
@@ -239,7 +240,7 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
     lb.load(pb, ldb);
     pb += BK * sb;
     multiply(lds[cur], 1);
-    __builtin_amdgcn_iglp_opt(0);   // spread the LDS traffic and the cut over the matrix instructions (8192^3 202 -> 212 TFLOP/s, 4096x2048x4096 165 -> 206)
+    __builtin_amdgcn_iglp_opt(0);   // spread the LDS traffic and the cut over the matrix instructions (with six products: 8192^3 202 -> 212 TFLOP/s, 4096x2048x4096 165 -> 206)
   }
   for (; i < tiles; i++, cur ^= 1) {   // the last stages: nothing more to fetch, or less than a stage
     __syncthreads();
@@ -318,8 +319,8 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
   }
 }
 
-// How many slices of k an m x n x k product is cut into, and its estimated time in us: a stage of 32 steps takes 2.4 with all 256 CUs at work, starting
-// and storing a tile 5 (fitted to measurements); slices, which let few tiles fill the chip, cost a second launch that reads them.
+// How many slices of k an m x n x k product is cut into, and its estimated time in us: a stage of 32 steps takes 2.8 with most of the 256 CUs at work, starting
+// and storing a tile 7 (fitted to 90 products of 2 to 200 GFLOP); slices, which let few tiles fill the chip, cost a second launch that reads them.
 struct SplitPlan { int splits, kchunk; double us; };
 inline SplitPlan gemm_split_plan(int m, int n, int k) {
   constexpr size_t kMostPartial = size_t(64) << 20;
@@ -328,15 +329,16 @@ inline SplitPlan gemm_split_plan(int m, int n, int k) {
   for (int s = 1; s <= 16; s++) {
     if (s > 1 && (stages / s < 4 || (size_t)s * m * n * sizeof(float) > kMostPartial)) break;
     const double per = (double)(long)((stages + s - 1) / s), turns = (double)(long)((tiles * s + ncu - 1) / ncu);
-    double us = turns * (per * 2.4 + 5);
+    double us = turns * (per * 2.8 + 7);
     if (s > 1) us += 4 + (s + 1) * 4.0 * m * n / 5e6;
     if (us < best.us) best = {s, (int)per * 32, us};
   }
   best.splits = (k + best.kchunk - 1) / best.kchunk;
   return best;
 }
-// True if the product runs here: estimated faster than the vendor's fp32 kernels (140 TFLOP/s and 8 us for the call).  us, this / vendor: 2000x1000x2000 55/64,
-// 2000x2000x1000 NT 56/65, 1000x2048x4096 101/127; not taken: 1024^3 30/19, 512x512x2048 NT 27/15, 1000x237x784 21/11, 3000x3000x40 32/22.
+// True if the product runs here: estimated faster than the vendor's fp32 kernels (140 TFLOP/s and 8 us for the call, a little less at odd sizes).  us, this /
+// vendor: 1000x2048x4096 113/119, 4096x1792x545 62/79, 255x3000x8005 94/103, 3161x6756x1098 TN 334/408, 1217x1950x2863 TN 105/108; not taken:
+// 1024x2048x1024 42/33, 3000x3000x400 NT 92/66, 188x6336x1630 47/37, 1785x5130x7191 1174/950 (a last turn that is nearly empty).
 // The loaders' offsets within a tile have 32 bits: 255 * ld.
 inline bool gemm_split_fits(int m, int n, int k, int lda, int ldb, SplitPlan* plan) {
   const int knob = tuning(kTuneGemmSplit);   // for tests and comparisons: 1 never, 2 wherever the kernel can
@@ -344,7 +346,7 @@ inline bool gemm_split_fits(int m, int n, int k, int lda, int ldb, SplitPlan* pl
   const double flop = 2.0 * m * n * (double)k;
   if (knob != 2 && (m < 64 || n < 64 || k < 64 || flop < 2e9)) return false;
   *plan = gemm_split_plan(m, n, k);
-  return knob == 2 || plan->us < 0.95 * (flop / 140e6 + 8);
+  return knob == 2 || plan->us < 1.05 * (flop / 140e6 + 8);
 }
 
 // C = act(alpha*sum of the slices [+ beta*C] [+ bias]), slices in order.

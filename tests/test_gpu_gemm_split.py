@@ -121,3 +121,47 @@ def test_what_the_parts_cannot_hold(knet, everywhere):
     least = 2.0 ** -149 * n ** 0.5        # the spacing of denormal results
     assert np.all(err <= 2.0 ** -24 * k ** 0.5 * np.linalg.norm(want, axis=1) + least)
     knet.libknet8().check()
+
+
+def with_knob(knet, value, f):
+    fn = knet.libknet8().fn
+    old = fn["knet8_tune"](9, value)
+    try:
+        return f()
+    finally:
+        fn["knet8_tune"](9, old)
+
+
+@pytest.mark.parametrize("m,n,k", [(512, 384, 512), (300, 260, 4111)])
+def test_sums_with_one_term(knet, everywhere, m, n, k):
+    """One element to a row of A: each result is one product, rounded once (2^-24; the parts' own sums add at most a few roundings of numbers 2^-8 as large)."""
+    rng = np.random.default_rng(21)
+    A = np.zeros((m, k), np.float32)
+    A[np.arange(m), rng.integers(0, k, size=m)] = rng.standard_normal(m)
+    B = rng.standard_normal((k, n)).astype(np.float32)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    assert np.all(np.abs(product(knet, False, False, A, B) - want) <= 2.0 ** -24 * (1 + 2.0 ** -6) * np.abs(want))
+
+
+def test_sums_of_equal_numbers(knet, everywhere):
+    """Where what is left out has one sign in every term: 1.0038986^2, whose products of the middle and the last part make up 2^-24.01 of it.  784 of them are within
+    2^-25.7 of a number that fp32 has, and that is the result."""
+    v = np.array([0x3f807fc0], np.int32).view(np.float32)[0]
+    m, n, k = 512, 256, 784
+    want = np.float32(k * np.float64(v) * np.float64(v))
+    assert np.all(product(knet, False, False, np.full((m, k), v), np.full((k, n), v)) == want)
+
+
+@pytest.mark.parametrize("m,n,k", [(1000, 237, 784), (1024, 768, 2048), (512, 640, 32000)])
+@pytest.mark.parametrize("what", ["normal", "positive", "relu"])
+def test_no_less_precise_than_fp32(knet, m, n, k, what):
+    """The error of dense products against 64 bits, beside the same product on the vendor's fp32 kernels."""
+    rng = np.random.default_rng(22)
+    A, B, _, _ = operands(rng, False, False, m, n, k)
+    if what == "positive":
+        A, B = np.abs(A), np.abs(B)
+    if what == "relu":
+        B = np.maximum(B, 0)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    off = [np.linalg.norm(with_knob(knet, v, lambda: product(knet, False, False, A, B)) - want) for v in (1, 2)]
+    assert off[1] <= off[0]

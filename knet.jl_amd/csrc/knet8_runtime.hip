@@ -976,9 +976,9 @@ static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T*
     check_launch("gemm (small)");
     return 0;
   }
-  if constexpr (sizeof(T) == 4) {   // large fp32 products: on the bf16 matrix cores
+  if constexpr (sizeof(T) == 4) {   // large fp32 products: on the bf16 matrix cores (alpha = 0, where A and B are not read, stays with the vendor)
     SplitPlan plan;
-    if (batch.count == 1 && gemm_split_fits(m, n, k, lda, ldb, &plan)) {
+    if (batch.count == 1 && alpha != T(0) && gemm_split_fits(m, n, k, lda, ldb, &plan)) {
       if (bias == nullptr && act) { record_error("gemm_bias_act: an activation without a bias is not provided"); return -1; }
       if (g_tune[kTuneGemmDryRun] != 0) return 0;
       return launch_gemm_split(stream, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, bias, act, plan);

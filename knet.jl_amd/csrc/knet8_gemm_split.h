@@ -366,19 +366,20 @@ __global__ __launch_bounds__(256) void gemm_split_sum_kernel(int m, int n, int s
   }
 }
 
-inline int launch_gemm_split(hipStream_t stream, bool ta, bool tb, int m, int n, int k, float alpha, const float* A, int lda, const float* B, int ldb,
-                             float beta, float* C, int ldc, const float* bias, int act, const SplitPlan& plan) {
+inline void launch_gemm_split(hipStream_t stream, bool ta, bool tb, int m, int n, int k, float alpha, const float* A, int lda, const float* B, int ldb,
+                             float beta, float* C, int ldc, const float* bias, int act, SplitPlan plan) {
   float* out = C;
   int ldo = ldc;
   Workspace ws;
   if (plan.splits > 1) {
-    ws = workspace_for(stream, (size_t)plan.splits * m * n * sizeof(float), 0);
-    if (ws.partial == nullptr) {
-      record_error("gemm (split): no scratch memory for the slices of k");
-      return -1;
+    ws = workspace_for(stream, (size_t)plan.splits * m * n * sizeof(float), 0, true);
+    if (ws.partial != nullptr) {
+      out = static_cast<float*>(ws.partial);
+      ldo = m;
+    } else {   // no scratch: k in one piece, which needs none
+      plan.splits = 1;
+      plan.kchunk = k;
     }
-    out = static_cast<float*>(ws.partial);
-    ldo = m;
   }
   const long tiles = (long)((m + 255) / 256) * ((n + 127) / 128);
   const dim3 grid((unsigned)(tiles * plan.splits)), block(512);
@@ -393,7 +394,6 @@ inline int launch_gemm_split(hipStream_t stream, bool ta, bool tb, int m, int n,
     hipLaunchKernelGGL(gemm_split_sum_kernel, dim3((unsigned)(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream, m, n, plan.splits, out, C, ldc, alpha, beta, bias, act);
   }
   check_launch("gemm (split)");
-  return 0;
 }
 
 }  // namespace knet8

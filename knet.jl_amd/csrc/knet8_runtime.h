@@ -28,7 +28,8 @@ struct Workspace {
   unsigned* counters = nullptr;
   std::unique_lock<std::recursive_mutex> held;
 };
-Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounters);
+// optional: the caller does without when there is none, so a failure is not recorded.
+Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounters, bool optional = false);
 // Where a split launch takes its scratch from: the per-stream buffers above (a null source) or a caller-supplied provider.  A provider
 // that cannot serve the request records why and returns null pointers.
 struct ScratchSource {

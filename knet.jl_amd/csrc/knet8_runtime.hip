@@ -158,11 +158,16 @@ __global__ __launch_bounds__(256) void zero_counters_kernel(unsigned* c, size_t 
   if (i < n) c[i] = 0u;
 }
 
-Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounters) {
+Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounters, bool optional) {
   if (g_tune[kTuneFailScratch] != 0) {   // set by tests: behave as if the device were out of memory, without touching it
-    record_error("reduction scratch: allocation refused (knet8_tune key 5 is set)");
+    if (!optional) record_error("reduction scratch: allocation refused (knet8_tune key 5 is set)");
     return Workspace();
   }
+  auto allocate = [&](void** p, size_t bytes, const char* what) {
+    const hipError_t e = dev_malloc(p, bytes, true);
+    if (e != hipSuccess && optional) (void)hipGetLastError();
+    return optional ? e == hipSuccess : ok(e, what);
+  };
   const bool capturing = stream_is_capturing(stream);
   Workspace w;
   w.held = hold_scratch(stream);
@@ -173,27 +178,31 @@ Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounte
   // captured on it, keep using their addresses.  Sizes grow geometrically, so the retired ones add up to less than
   // the current one.  knet8_trim (after a device-wide wait) and knet8_stream_destroy release them.
   if (s.partial_bytes < partial_bytes) {
-    if (s.partial) { s.retired.push_back(s.partial); s.retired_bytes.push_back(s.partial_bytes); }
-    size_t want = partial_bytes < (size_t(1) << 20) ? (size_t(1) << 20) : 2 * partial_bytes;
-    s.partial = nullptr;
-    s.partial_bytes = ok(dev_malloc(&s.partial, want, true), "hipMalloc(reduction partials)") ? want : 0;
+    const size_t want = partial_bytes < (size_t(1) << 20) ? (size_t(1) << 20) : 2 * partial_bytes;
+    void* p = nullptr;
+    if (allocate(&p, want, "hipMalloc(reduction partials)")) {
+      if (s.partial) { s.retired.push_back(s.partial); s.retired_bytes.push_back(s.partial_bytes); }
+      s.partial = p;
+      s.partial_bytes = want;
+    }
   }
   if (s.ncounters < ncounters) {
-    if (s.counters) { s.retired.push_back(s.counters); s.retired_bytes.push_back(s.ncounters * sizeof(unsigned)); }
-    size_t want = ncounters < 4096 ? 4096 : 2 * ncounters;
-    s.counters = nullptr;
-    s.ncounters = 0;
+    const size_t want = ncounters < 4096 ? 4096 : 2 * ncounters;
+    void* p = nullptr;
     // Zeroed by a fill kernel on the launching stream itself, so that the zeroing is ordered before the kernel that is about to
     // use the counters.  (A hipMemset goes to the null stream, which a non-blocking stream does not wait for: on recycled memory
     // the first split kernel on a new stream could then count on top of garbage and leave its tickets non-zero for good.  A fill
     // kernel is also what a stream capture can record safely.)
-    if (ok(dev_malloc(reinterpret_cast<void**>(&s.counters), want * sizeof(unsigned), true), "hipMalloc(reduction counters)")) {
+    if (allocate(&p, want * sizeof(unsigned), "hipMalloc(reduction counters)")) {
+      if (s.counters) { s.retired.push_back(s.counters); s.retired_bytes.push_back(s.ncounters * sizeof(unsigned)); }
+      s.counters = static_cast<unsigned*>(p);
+      s.ncounters = 0;
       hipLaunchKernelGGL(zero_counters_kernel, dim3((unsigned)((want + 255) / 256)), dim3(256), 0, stream, s.counters, want);
       if (ok(hipGetLastError(), "zero_counters_kernel")) s.ncounters = want;
     }
   }
-  w.partial = s.partial;
-  w.counters = s.counters;
+  if (s.partial_bytes >= partial_bytes) w.partial = s.partial;
+  if (s.ncounters >= ncounters) w.counters = s.counters;
   return w;
 }
 
@@ -981,7 +990,8 @@ static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T*
     if (batch.count == 1 && alpha != T(0) && gemm_split_fits(m, n, k, lda, ldb, &plan)) {
       if (bias == nullptr && act) { record_error("gemm_bias_act: an activation without a bias is not provided"); return -1; }
       if (g_tune[kTuneGemmDryRun] != 0) return 0;
-      return launch_gemm_split(stream, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, bias, act, plan);
+      launch_gemm_split(stream, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, bias, act, plan);
+      return 0;
     }
   }
   // Products the vendor library has no kernel for (seen with some fp64 shapes) run on the library's own tiles, whatever their size.

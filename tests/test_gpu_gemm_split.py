@@ -165,3 +165,20 @@ def test_no_less_precise_than_fp32(knet, m, n, k, what):
     want = A.astype(np.float64) @ B.astype(np.float64)
     off = [np.linalg.norm(with_knob(knet, v, lambda: product(knet, False, False, A, B)) - want) for v in (1, 2)]
     assert off[1] <= off[0]
+
+
+def test_slices_of_k_without_scratch(knet, everywhere):
+    """A product that would be cut into slices of k runs in one piece when there is no memory for their sums (knet8_tune key 5): a result, and no error."""
+    lib = knet.libknet8()
+    rng = np.random.default_rng(23)
+    m, n, k = 300, 260, 4111
+    A, B, _, _ = operands(rng, False, False, m, n, k)
+    C, want = rng.standard_normal((m, n)).astype(np.float32), A.astype(np.float64) @ B.astype(np.float64)
+    old = lib.fn["knet8_tune"](5, 1)
+    try:
+        Ad, Bd, Cd = device(knet, A), device(knet, B), device(knet, C)
+        assert lib.call("gemm_32", b"N", b"N", m, n, k, 0.5, Ad.ptr, m, Bd.ptr, k, 2.0, Cd.ptr, m) == 0
+    finally:
+        lib.fn["knet8_tune"](5, old)
+    assert np.linalg.norm(knet.Array(Cd) - (0.5 * want + 2.0 * C)) <= 2.0 ** -24 * k ** 0.5 * np.linalg.norm(want)
+    lib.check()

@@ -178,7 +178,9 @@ Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounte
   // captured on it, keep using their addresses.  Sizes grow geometrically, so the retired ones add up to less than
   // the current one.  knet8_trim (after a device-wide wait) and knet8_stream_destroy release them.
   if (s.partial_bytes < partial_bytes) {
-    const size_t want = partial_bytes < (size_t(1) << 20) ? (size_t(1) << 20) : 2 * partial_bytes;
+    // (twice the request, but not beyond the 64 MB that the slices of a product may take)
+    constexpr size_t kLeast = size_t(1) << 20, kSlices = size_t(64) << 20;
+    const size_t want = partial_bytes < kLeast ? kLeast : partial_bytes > kSlices / 2 && partial_bytes <= kSlices ? kSlices : 2 * partial_bytes;
     void* p = nullptr;
     if (allocate(&p, want, "hipMalloc(reduction partials)")) {
       if (s.partial) { s.retired.push_back(s.partial); s.retired_bytes.push_back(s.partial_bytes); }

@@ -182,3 +182,24 @@ def test_slices_of_k_without_scratch(knet, everywhere):
         lib.fn["knet8_tune"](5, old)
     assert np.linalg.norm(knet.Array(Cd) - (0.5 * want + 2.0 * C)) <= 2.0 ** -24 * k ** 0.5 * np.linalg.norm(want)
     lib.check()
+
+
+def test_scratch_of_slices_is_bounded(knet, everywhere):
+    """The slices of a product (here three of 21 MB) hold at most 64 MB of their stream."""
+    import ctypes
+    lib = knet.libknet8()
+    m, n, k = 2304, 2304, 2048
+    A, B, C = (knet.KnetArray(np.ones(d, np.float32)) for d in ((m, k), (k, n), (m, n)))
+
+    def held():
+        out = (ctypes.c_ulonglong * 6)()
+        lib.fn["knet8_stats"](ctypes.addressof(out))
+        return out[2]
+    stream = lib.fn["knet8_stream_create"]()
+    before = held()
+    assert lib.fn["gemm_32_stream"](b"N", b"N", m, n, k, 1.0, A.ptr, m, B.ptr, k, 0.0, C.ptr, m, stream) == 0
+    lib.fn["knet8_synchronize"](stream)
+    assert 3 * 4 * m * n <= held() - before <= 64 << 20
+    lib.fn["knet8_stream_destroy"](stream)
+    assert held() == before and np.all(knet.Array(C) == k)
+    lib.check()

@@ -12,8 +12,9 @@
 //   * Small numbers: the lower parts of numbers below 2^-109 would leave bf16's range.  Both operands are multiplied by 2^24 on the way in and the
 //     sums by 2^-48 on the way out, which keeps every fp32 number, denormals included, whole.
 //   * Large numbers, infinities, NaN: a part or a sum that overflows leaves a NaN or an infinity in an accumulator (inf - inf in the split itself
-//     if not before).  A wave that finds one in its patch forms the patch again with the fp32 matrix instruction: results beyond
-//     2^80, and what is infinite or NaN, come out as that instruction gives them.
+//     if not before).  A wave that finds one in its patch forms these sums again with the fp32 matrix instruction: results beyond
+//     2^80, and what is infinite or NaN, come out as that instruction gives them; the others stay.  us, 4096x2048x4096 (vendor 470): 400 on finite data, 340 if all is NaN, 600 with
+//     one NaN in A and 800 with one infinity (a row of sums to form again), 1240 if every sum is beyond 2^80.
 //
 // The cut is made while a tile goes from global memory to LDS (6.5 vector instructions an element, in the shadow of the matrix instructions of the
 // SIMD's other wave): no extra pass over the operands, no scratch.  What bounds it: 256x128 tile, 8 waves of 64x64, 32 steps of k a stage, two
@@ -253,7 +254,6 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
   for (int a = 0; a < FN; a++)
 #pragma unroll
     for (int b = 0; b < FM; b++) acc[a][b] += low[a][b];
-  float scale = kSplitUnscale;
   float bad = 0.0f;
 #pragma unroll
   for (int b = 0; b < FM; b++)
@@ -264,36 +264,20 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
         for (int r = 0; r < 16; r++)
           if (j0 + wn + 32 * a + 8 * (r >> 2) + 4 * half + (r & 3) < n) bad += acc[a][b][r] * 0.0f;
     }
-  if (__any(bad != 0.0f)) {   // (NaN: a sum was not finite)
-    scale = 1.0f;
-#pragma unroll
-    for (int a = 0; a < FN; a++)
-#pragma unroll
-      for (int b = 0; b < FM; b++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) acc[a][b][r] = 0.0f;
-    long ra[FM], rb[FN];
-#pragma unroll
-    for (int f = 0; f < FM; f++) { const int i = i0 + wm + 32 * f + l32; ra[f] = (long)(i < m ? i : m - 1) * (TA ? lda : 1); }
-#pragma unroll
-    for (int f = 0; f < FN; f++) { const int j = j0 + wn + 32 * f + l32; rb[f] = (long)(j < n ? j : n - 1) * (TB ? 1 : ldb); }
-    for (int k0 = kbeg; k0 < kend; k0 += 2) {
-      const int kk = k0 + half;
-      const bool in_k = kk < kend;
-      float va[FM], vb[FN];
-#pragma unroll
-      for (int f = 0; f < FM; f++) va[f] = in_k ? A[ra[f] + kk * sa] : 0.0f;
-#pragma unroll
-      for (int f = 0; f < FN; f++) vb[f] = in_k ? B[rb[f] + kk * sb] : 0.0f;
-#pragma unroll
-      for (int a = 0; a < FN; a++)
-#pragma unroll
-        for (int b = 0; b < FM; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[a], va[b], acc[a][b], 0, 0, 0);
-    }
-  }
+  const bool again = __any(bad != 0.0f);   // (NaN: a sum is not finite)
   float* c = C;
   const long ld = ldc;
   if (splits > 1) c += (long)z * m * n;   // this slice's sums; gemm_split_sum_kernel applies the rest
+  auto store = [&](float v, int i, int j, float bi) {
+    float* d = c + (long)j * ld + i;
+    if (splits == 1) {
+      v = alpha * v;
+      if (beta != 0.0f) v = v + beta * *d;
+      if (bias) v = v + bi;
+      if (act == 1) v = v > 0.0f ? v : 0.0f;
+    }
+    *d = v;
+  };
 #pragma unroll
   for (int b = 0; b < FM; b++) {
     const int i = i0 + wm + 32 * b + l32;
@@ -304,18 +288,65 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         const int j = j0 + wn + 32 * a + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (j < n) {
-          float v = acc[a][b][r] * scale;
-          float* d = c + (long)j * ld + i;
-          if (splits == 1) {
-            v = alpha * v;
-            if (beta != 0.0f) v = v + beta * *d;
-            if (bias) v = v + bi;
-            if (act == 1) v = v > 0.0f ? v : 0.0f;
-          }
-          *d = v;
-        }
+        if (j < n && !(again && acc[a][b][r] * 0.0f != 0.0f)) store(acc[a][b][r] * kSplitUnscale, i, j, bi);
       }
+  }
+  if (!again) return;
+  // The sums that are not finite, by the fp32 instruction: 32x32 of the patch at a time, where there are any.  Lanes 0-31 take the first 16 of 32 steps of k and lanes
+  // 32-63 the others, so that an operand with k in a row comes in 16-byte loads.  Once all that are wanted are NaN, as in a training run that has diverged, what follows
+  // changes nothing.
+  constexpr int kStep = 16;
+  unsigned wanted[FN * FM];   // one bit a sum
+#pragma unroll
+  for (int f = 0; f < FN * FM; f++) {
+    wanted[f] = 0;
+#pragma unroll
+    for (int r = 0; r < 16; r++) wanted[f] |= (acc[f / FM][f % FM][r] * 0.0f != 0.0f ? 1u : 0u) << r;
+  }
+#pragma unroll 1
+  for (int f = 0; f < FN * FM; f++) {
+    unsigned want = 0;
+#pragma unroll
+    for (int g = 0; g < FN * FM; g++) want = f == g ? wanted[g] : want;
+    const int i = i0 + wm + 32 * (f % FM) + l32, ja = j0 + wn + 32 * (f / FM), jl = ja + l32;
+    if (i >= m) want = 0;
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+      if (ja + 8 * (r >> 2) + 4 * half + (r & 3) >= n) want &= ~(1u << r);
+    if (!__any(want != 0)) continue;
+    const float* p = A + (long)(i < m ? i : m - 1) * (TA ? lda : 1) + (kbeg + kStep * half) * sa;
+    const float* q = B + (long)(jl < n ? jl : n - 1) * (TB ? 1 : ldb) + (kbeg + kStep * half) * sb;
+    f32x16 sum;
+#pragma unroll
+    for (int r = 0; r < 16; r++) sum[r] = 0.0f;
+#pragma unroll 1
+    for (int k0 = kbeg; k0 < kend; k0 += 2 * kStep, p += 2 * kStep * sa, q += 2 * kStep * sb) {
+      float va[kStep], vb[kStep];
+      if (kend - k0 >= 2 * kStep) {
+#pragma unroll
+        for (int s = 0; s < kStep; s += 4) {
+          const float *ps = p + s * sa, *qs = q + s * sb;
+          const F4u x = TA ? *reinterpret_cast<const F4u*>(ps) : F4u{{ps[0], ps[sa], ps[2 * sa], ps[3 * sa]}};
+          const F4u y = TB ? F4u{{qs[0], qs[sb], qs[2 * sb], qs[3 * sb]}} : *reinterpret_cast<const F4u*>(qs);
+#pragma unroll
+          for (int e = 0; e < 4; e++) { va[s + e] = x.v[e]; vb[s + e] = y.v[e]; }
+        }
+      } else {
+        const int left = kend - k0 - kStep * half;
+#pragma unroll
+        for (int s = 0; s < kStep; s++) { va[s] = s < left ? p[s * sa] : 0.0f; vb[s] = s < left ? q[s * sb] : 0.0f; }
+      }
+#pragma unroll
+      for (int s = 0; s < kStep; s++) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(vb[s], va[s], sum, 0, 0, 0);
+      bool done = true;
+#pragma unroll
+      for (int r = 0; r < 16; r++) done = done && ((want >> r & 1u) == 0 || sum[r] != sum[r]);
+      if (__all(done)) break;
+    }
+    const float bi = (want != 0 && bias && splits == 1) ? bias[i] : 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+      if (want >> r & 1u) store(sum[r], i, ja + 8 * (r >> 2) + 4 * half + (r & 3), bi);
   }
 }
 

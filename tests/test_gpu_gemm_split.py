@@ -203,3 +203,35 @@ def test_scratch_of_slices_is_bounded(knet, everywhere):
     lib.fn["knet8_stream_destroy"](stream)
     assert held() == before and np.all(knet.Array(C) == k)
     lib.check()
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (True, False), (False, True), (True, True)])
+@pytest.mark.parametrize("m,n,k", [(257, 131, 31), (300, 260, 4111), (129, 257, 96)])
+def test_sums_formed_again(knet, everywhere, m, n, k, ta, tb):
+    """Sums that are not finite, or lie beyond 2^80, beside others: around a tile's edges, with a remainder of k and in slices, with beta, bias and relu.  They are those
+    of the fp32 instruction; the sums of rows and columns without one keep their bits."""
+    rng = np.random.default_rng(24)
+    A, B, _, _ = operands(rng, ta, tb, m, n, k)
+    C, bias = rng.standard_normal((m, n)).astype(np.float32), rng.standard_normal(m).astype(np.float32)
+    lib = knet.libknet8()
+
+    def both(A, B):
+        a, b = (np.ascontiguousarray(A.T) if ta else A), (np.ascontiguousarray(B.T) if tb else B)
+        Ad, Bd, bd, out = device(knet, a), device(knet, b), device(knet, bias), device(knet, C)
+        assert lib.call("gemm_bias_act_32", b"T" if ta else b"N", b"T" if tb else b"N", m, n, k, 1.0, Ad.ptr, a.shape[0], Bd.ptr, b.shape[0], bd.ptr, 1, out.ptr, m) == 0
+        return product(knet, ta, tb, a, b, alpha=0.5, beta=2.0, C=C), knet.Array(out)
+    clean = both(A, B)
+    A, B = A.copy(), B.copy()
+    A[0, k // 2], A[m - 1, k - 1], A[70], B[3, n - 1] = np.nan, np.inf, A[70] * 1e28, -np.inf
+    got, ref = both(A, B), with_knob(knet, 1, lambda: both(A, B))
+    rest = np.ix_([i for i in range(m) if i not in (0, 70, m - 1)], range(n - 1))
+    for g, r, c in zip(got, ref, clean):
+        assert np.array_equal(np.isnan(g), np.isnan(r)) and np.array_equal(g[np.isinf(r)], r[np.isinf(r)])
+        assert np.linalg.norm(g[70, :-1].astype(np.float64) - r[70, :-1]) <= 2.0 ** -24 * max(4.0, k ** 0.5) * np.linalg.norm(r[70, :-1].astype(np.float64))
+        assert np.array_equal(g[rest], c[rest])
+    lib.check()
+
+
+def test_all_nan(knet, everywhere):
+    got = product(knet, False, False, np.full((260, 300), np.nan, np.float32), np.ones((300, 140), np.float32))
+    assert np.isnan(got).all()

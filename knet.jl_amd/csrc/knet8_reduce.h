@@ -87,7 +87,7 @@ __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x,
         if (SINGLE) off = uu * NV;
         else { const unsigned o = (unsigned)uu / (unsigned)usy; off = o * slab + ((unsigned)uu - o * (unsigned)usy) * NV; }
         if (ANY) {
-          const long in_run = SINGLE ? uu * NV : (long)((unsigned)uu % (unsigned)usy) * NV;
+          const long in_run = (long)((unsigned)uu % (unsigned)usy) * NV;
           skip = in_run + NV > sy ? in_run + NV - sy : 0;
           typedef T V __attribute__((ext_vector_type(NV), aligned(sizeof(T))));
           const V t = __builtin_nontemporal_load(reinterpret_cast<const V*>(xj + off - skip));
@@ -568,10 +568,16 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   bool launched = true;
   if (!kCentered<Op> && !small_total && ny > 1 && (sy <= 8 || short_one_slab) && launch_reduce_stretch<T, Op>(stream, x, sy, ny, no, 1, 0, y, scratch, &launched)) return launched;
   constexpr int N = Vec16<T>::N;
+  // 16-byte loads off the 16-byte boundaries (ANY): in fp32 and over several slabs.  us, loads of 4 bytes / ANY: 841 over 193 outputs x 64 slabs 31.1/11.4, 65 over
+  // 130 x 248 11.2/5.4, 529 over 1024 x 3 5.0/4.2.  One slab walks its runs in a row, where loads of one element and sixteen of them in flight are as good or
+  // better (8193 over 300 4.8/6.5, 20001 over 512 8.5/9.7, 1000003 over 4 6.7/10.5), and so they are in fp64 (361 over 64 channels x 45 7.0/9.1, 841 over 193 x 32 10.3/11.4).
+  // Runs of fewer than eight vectors: the load that ends a run with few elements of its own costs more than it saves.
+  constexpr bool kAny = sizeof(T) == 4;
   const bool vec = aligned16(x) && (sy % N == 0);
-  const bool any = !vec && sy >= 8 * N;   // (below, the load that ends a run with few elements of its own costs more than loads of one element)
+  const bool any = kAny && !vec && no > 1 && sy >= 8 * N;
   const long units = (vec ? sy / N : any ? ceil_div(sy, N) : sy) * no;
-  unsigned P = plan_parts(ny, units, 2048);
+  // (parts of as many bytes as with loads of one element: with 2048 vectors to a part 841 over 16 outputs x 19 slabs takes 9.5 us, with 512 it is back at 5.8)
+  unsigned P = plan_parts(ny, units, any ? 2048 / N : 2048);
   long chunk = ceil_div(units, P);
   P = (unsigned)ceil_div(units, chunk > 0 ? chunk : 1);
   if (P < 1) P = 1;
@@ -584,7 +590,8 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   // workgroup size by the work of one part: a wave for short runs, 512 lanes when there is plenty
   const int bt = chunk <= 2 * kWave ? 64 : chunk <= 4096 ? 256 : 512;
   const dim3 grid((unsigned)(ny * P));
-  // no more workgroups than compute units: twice the lanes keep twice the bytes in flight (sum over 29x29x193x64 fp32 15.6 -> 11.0 us)
+  // no more workgroups than compute units: twice the lanes keep twice the bytes in flight.  us, 512 / 1024 lanes: 841 over 16 outputs x 25 MB 10.6/8.5, over 130 x 12 MB 8.6/6.3,
+  // over 193 x 43 MB 17.6/11.7, over 256 x 167 MB 49.5/31.6; from 10 to 168 MB, runs of 65 to 20001 and 16 to 256 outputs none is slower
   const bool alone = (long)ny * P <= tuning(kTuneNumCUs);
 #define KNET8_RUN(NV, SINGLE, BT, U, ANY) \
   hipLaunchKernelGGL((reduce_run_kernel<T, Op, NV, SINGLE, BT, U, ANY>), grid, dim3(BT), 0, stream, x, sy, ny, units, chunk, P, y, partial, ws.counters, center KNET8_TL_ARG)
@@ -592,9 +599,17 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
 #define KNET8_RUN_BT(NV, SINGLE, ANY) \
   do { if (bt == 64) KNET8_RUN(NV, SINGLE, 64, (NV == 1 ? 16 : 8), ANY); else if (bt == 256) KNET8_RUN(NV, SINGLE, 256, (NV == 1 ? 16 : 4), ANY); \
        else if (ANY && alone) KNET8_RUN(NV, SINGLE, 1024, 8, ANY); else KNET8_RUN(NV, SINGLE, 512, (NV == 1 ? 16 : ANY ? 8 : 4), ANY); } while (0)
-  if (vec)      { if (no == 1) KNET8_RUN_BT(N, true, false); else KNET8_RUN_BT(N, false, false); }
-  else if (any) { if (no == 1) KNET8_RUN_BT(N, true, true); else KNET8_RUN_BT(N, false, true); }
-  else          { if (no == 1) KNET8_RUN_BT(1, true, false); else KNET8_RUN_BT(1, false, false); }
+  if (vec) {
+    if (no == 1) KNET8_RUN_BT(N, true, false); else KNET8_RUN_BT(N, false, false);
+    return true;
+  }
+  if constexpr (kAny) {
+    if (any) {
+      KNET8_RUN_BT(N, false, true);
+      return true;
+    }
+  }
+  if (no == 1) KNET8_RUN_BT(1, true, false); else KNET8_RUN_BT(1, false, false);
 #undef KNET8_RUN_BT
 #undef KNET8_RUN
   return true;

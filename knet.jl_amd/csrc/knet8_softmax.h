@@ -1073,12 +1073,16 @@ inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const
     }
   }
   if ((resident_cap > 0 && m > resident_cap) || m > 1024L * kBig1024) {
-    // Shares of a column: two workgroups per compute unit over all columns, 8192 rows or more each (a compute unit holds two of these workgroups, so that a
-    // column to a workgroup fills the chip from 257 columns on).
+    // Shares of a column: two workgroups per compute unit over all columns, 8192 rows or more each.  They pay (us, a workgroup a column / shares, fp32 logsoftmax unless
+    // said) from five to a column on: 65537 rows x 50 columns 18.9/11.6, 100000 x 50 17.4/12.7, x 100 20.1/20.2 and its gradient 37.0/26.2, 300000 x 100 70.2/55.5, 2000000 x 1
+    // 290/17; or where all are resident at once: fp64 33000 x 64 22.6/18.5, x 72 22.7/25.4.  Four (104 to 128 columns) where the second read does not come from the caches or
+    // loads are narrow: 150000 x 128 49.1/40.3, 100001 x 128 35.2/30.9, but 100000 x 128 22.9/27.4, 65537 x 128 softmaxback 27.9/30.8.  Three and two do not: 100000 x 170 29.3/35.1, 300000 x 200 112/134.
     const long ncu = tuning(kTuneNumCUs);
     long P = n <= ncu ? 2 * ncu / n : 1;
     if (P > m / 8192) P = m / 8192;
     if (P > 64) P = 64;
+    const bool past_caches = sizeof(T) * (size_t)m * n > (size_t(64) << 20);
+    if (n * P > ncu && P < 5 && !(P == 4 && m >= 10 * 8192 && (past_caches || !vec_stream))) P = 1;
     Workspace ws;
     long chunk = m;
     if (P > 1) {

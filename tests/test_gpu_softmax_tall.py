@@ -29,3 +29,9 @@ def test_tall_columns_shared_by_workgroups(knet, oracle, m, n):
     wantb = d - np.exp(want) * d.sum(axis=0)
     assert np.abs(got[:, sel] - wantb).max() <= 1e-5 * np.abs(wantb).max()
     knet.libknet8().check()
+
+
+# four shares: loads of one element, an array beyond the caches; a smaller one and shorter columns, which keep a workgroup to a column
+@pytest.mark.parametrize("m,n", [(100001, 104), (170000, 104), (100000, 104), (65537, 104)])
+def test_four_shares(knet, oracle, m, n):
+    test_tall_columns_shared_by_workgroups(knet, oracle, m, n)

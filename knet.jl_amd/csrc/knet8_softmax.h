@@ -1088,7 +1088,7 @@ inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const
     if (P > 1) {
       chunk = ((m + P - 1) / P + N - 1) / N * N;
       P = (m + chunk - 1) / chunk;
-      ws = workspace_for(stream, 2 * sizeof(T) * (size_t)n * P, 0);   // without scratch: a workgroup per column
+      ws = workspace_for(stream, 2 * sizeof(T) * (size_t)n * P, 0, true);   // without scratch: a workgroup per column
     }
     T* const part = static_cast<T*>(ws.partial);
 #define KNET8_STREAM(VEC, PART, BLOCKS) \

@@ -35,3 +35,13 @@ def test_tall_columns_shared_by_workgroups(knet, oracle, m, n):
 @pytest.mark.parametrize("m,n", [(100001, 104), (170000, 104), (100000, 104), (65537, 104)])
 def test_four_shares(knet, oracle, m, n):
     test_tall_columns_shared_by_workgroups(knet, oracle, m, n)
+
+
+def test_tall_columns_without_scratch(knet, oracle):
+    """No memory for the shares' sums (knet8_tune key 5): a workgroup to a column gives the result, and there is no error to report."""
+    fn = knet.libknet8().fn
+    old = fn["knet8_tune"](5, 1)
+    try:
+        test_tall_columns_shared_by_workgroups(knet, oracle, 81921, 3)
+    finally:
+        fn["knet8_tune"](5, old)

@@ -686,14 +686,18 @@ KNET8_API void sum_32_21_noalloc(int nx, float* x, int sy, int ny, float* y, hip
 /* launch-heuristic knobs; returns the old value; value 0 restores the default, a negative value only reads.  Key 0: number of compute units the reduction planner aims at (default: asked from the
    device); key 1: longest softmax column kept resident in registers, longer ones take the two-pass streaming kernel (default 0: the register capacity);
    key 3: products of up to this many MFLOP (2*m*n*k/1e6) take the library's own small-product kernels instead of hipBLASLt (default 0: a rule on
-   type and sizes, up to 270 MFLOP, where the loaded hipBLASLt allows no prepared calls; 1 in effect switches them off);
+   type and sizes, up to 270 MFLOP, where the loaded hipBLASLt allows no prepared calls; see key 10);
    key 4: dense_back_S / dense_nll_back_S accept layers whose products have up to this many MFLOP each (default 270);
    key 5: non-zero makes the library behave as if the scratch memory of split launches could not be allocated (for tests of that error path);
    key 6: non-zero keeps softmax columns of 128 to 256 KB in registers alone instead of registers + LDS (for comparisons);
    key 7: non-zero makes the hipBLASLt route of gemm_S do everything but the vendor call itself (for measuring the library's own share of a call's host time);
    key 8: non-zero keeps repeated products on hipblasLtMatmul instead of the prepared calls of the vendor's extension interface (for comparisons);
-   key 9: which fp32 products run on the bf16 matrix cores in three parts: 0 those that are faster there, 1 none, 2 all with sides of at least 4 (for tests) */
+   key 9: which fp32 products run on the bf16 matrix cores in three parts: 0 those that are faster there, 1 none, 2 all with sides of at least 4 (for tests);
+   key 10: which small products run on the library's own kernels while key 3 is 0: 0 by the rule, where hipBLASLt allows no prepared calls, 1 none, 2 by the rule whatever hipBLASLt allows (for tests) */
 KNET8_API int knet8_tune(int key, int value);
+/* no counterpart in the reference: what the calling thread's last product (gemm_S, bmm_S, gemm_bias_act_S) ran on: 0 none yet, 1 hipBLASLt, 2 the library's small-product
+   kernels, 3 its bf16 kernel with three parts to an element */
+KNET8_API int knet8_product_route(void);
 /* Seed of the default random stream used by rand_S / randn_S (restarts it at counter 0): the device half of Knet.seed!,
    src/knetarrays/random.jl:14-18 (CUDA.seed!).  Unseeded, the stream starts from the operating system's entropy. */
 KNET8_API void knet8_seed(unsigned long long seed);

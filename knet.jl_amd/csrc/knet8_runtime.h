@@ -62,7 +62,7 @@ void fetch_scalar(hipStream_t stream, const void* dev, void* host, size_t nbytes
 // State of the default random stream (knet8_seed): hands out `blocks` consecutive generator counters under the current seed.
 void rng_take(unsigned long long blocks, unsigned long long* seed, unsigned long long* offset);
 
-enum { kTuneNumCUs = 0, kTuneSoftmaxResidentRows = 1, kTuneGemmSmallMflop = 3, kTuneDenseBackMflop = 4, kTuneFailScratch = 5, kTuneSoftmaxNoLdsSlots = 6, kTuneGemmDryRun = 7, kTuneGemmNoPrepared = 8, kTuneGemmSplit = 9, kTuneCount = 10 };
+enum { kTuneNumCUs = 0, kTuneSoftmaxResidentRows = 1, kTuneGemmSmallMflop = 3, kTuneDenseBackMflop = 4, kTuneFailScratch = 5, kTuneSoftmaxNoLdsSlots = 6, kTuneGemmDryRun = 7, kTuneGemmNoPrepared = 8, kTuneGemmSplit = 9, kTuneGemmSmallRule = 10, kTuneCount = 11 };
 int tuning(int key);
 
 #ifdef KNET8_TIMELINE

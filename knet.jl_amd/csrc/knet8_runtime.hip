@@ -966,6 +966,10 @@ static int gemm_lt(bool ta, bool tb, int m, int n, int k, T alpha, const T* A, i
   return lt_ok(hipblasLtMatmul(h, p.desc, &alpha, A, p.la, B, p.lb, &beta, C, p.lc, C, p.lc, &p.algo, ws, kGemmWorkspace, stream), "matmul") ? 0 : -1;
 }
 
+// Which kernels this thread's last product ran on, or would have (knet8_product_route).
+enum { kRouteNone = 0, kRouteVendor = 1, kRouteSmall = 2, kRouteSplit = 3 };
+static thread_local int t_route = kRouteNone;
+
 template <typename T>
 static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T* A, int lda, const T* B, int ldb, T beta, T* C, int ldc,
                 hipStream_t stream, const T* bias = nullptr, int act = 0, GemmBatch batch = GemmBatch()) {
@@ -980,8 +984,13 @@ static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T*
     return false;
   };
   // empty products (C = beta*C [+ bias]) and small ones: by the caller's limit (knet8_tune key 3), or by the rule where a vendor call costs its caller more
-  // than a launch
-  if (batch.count == 1 && (k <= 0 || (tuning(kTuneGemmSmallMflop) > 0 ? gemm_is_small(m, n, k) : gemm_is_small_by_rule<T>(m, n, k) && !vendor_prepares()))) {
+  // than a launch (key 10: never, or wherever the rule holds)
+  auto small_by_rule = [&]() {
+    const int knob = g_tune[kTuneGemmSmallRule];
+    return knob != 1 && (sizeof(T) == 8 || g_tune[kTuneGemmSplit] != 2) && gemm_is_small_by_rule<T>(m, n, k) && (knob == 2 || !vendor_prepares());
+  };
+  if (batch.count == 1 && (k <= 0 || (tuning(kTuneGemmSmallMflop) > 0 ? gemm_is_small(m, n, k) : small_by_rule()))) {
+    t_route = kRouteSmall;
     if (!own_kernels_reach()) return -1;
     launch_gemm_small<T>(stream, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, bias, act);
     check_launch("gemm (small)");
@@ -991,11 +1000,13 @@ static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T*
     SplitPlan plan;
     if (batch.count == 1 && alpha != T(0) && gemm_split_fits(m, n, k, lda, ldb, &plan)) {
       if (bias == nullptr && act) { record_error("gemm_bias_act: an activation without a bias is not provided"); return -1; }
+      t_route = kRouteSplit;
       if (g_tune[kTuneGemmDryRun] != 0) return 0;
       launch_gemm_split(stream, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, bias, act, plan);
       return 0;
     }
   }
+  t_route = kRouteVendor;
   // Products the vendor library has no kernel for (seen with some fp64 shapes) run on the library's own tiles, whatever their size.
   auto plain = [&](T bt) {
     int rc = gemm_lt<T>(ta, tb, m, n, k, alpha, A, lda, B, ldb, bt, C, ldc, stream, kEpiNone, nullptr, batch);
@@ -1003,6 +1014,7 @@ static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T*
     if (batch.count > 1) { record_error("hipBLASLt: no algorithm for this batched product"); return -1; }
     if (!own_kernels_reach()) return -1;
     g_gemm_left_vendor.fetch_add(1, std::memory_order_relaxed);
+    t_route = kRouteSmall;
     launch_gemm_small<T>(stream, ta, tb, m, n, k, alpha, A, lda, B, ldb, bt, C, ldc, nullptr, 0);
     check_launch("gemm (own kernel: no vendor algorithm)");
     return 0;
@@ -1075,6 +1087,8 @@ KNET8_API int bmm_64(char transa, char transb, int m, int n, int k, double alpha
                      double beta, double* C, int ldc, long long strideC, int batch) {
   return bmm_64_stream(transa, transb, m, n, k, alpha, A, lda, strideA, B, ldb, strideB, beta, C, ldc, strideC, batch, 0);
 }
+
+KNET8_API int knet8_product_route(void) { return knet8::t_route; }
 
 static int check_epilogue(int act) {
   if (act == 0 || act == 1) return 0;

@@ -21,3 +21,43 @@ def test_small_products_match_64_bits(knet, m, n, k, dt):
             eps = 2.0 ** -24 if dt == np.float32 else 2.0 ** -52
             assert np.linalg.norm(got - want) <= 2 * eps * max(2.0, k ** 0.5) * np.linalg.norm(want), (ta, tb)
     knet.libknet8().check()
+
+
+VENDOR, SMALL, SPLIT = 1, 2, 3
+
+
+@pytest.fixture
+def knobs(knet):
+    """Sets knet8_tune keys and restores them."""
+    fn = knet.libknet8().fn
+    old = {}
+
+    def put(key, value):
+        old.setdefault(key, fn["knet8_tune"](key, value))
+        fn["knet8_tune"](key, value)
+    yield put
+    for key, value in old.items():
+        fn["knet8_tune"](key, value)
+
+
+def test_the_other_routes(knet, knobs):
+    """A limit of the caller's (key 3) comes before the rule, the forced bf16 kernel (key 9) before both of its limits; large products by their own rule."""
+    lib = knet.libknet8()
+
+    def route(m, n, k, dt=np.float32):
+        A, B, C = (knet.KnetArray(np.ones(d, dt)) for d in ((m, k), (k, n), (m, n)))
+        knet.gemm("N", "N", 1, A, B, 0, C)
+        assert np.all(knet.Array(C) == k)
+        return lib.fn["knet8_product_route"]()
+    knobs(10, 1)
+    assert route(10, 64, 100) == VENDOR                        # however small
+    assert route(1000, 2048, 4096) == SPLIT
+    knobs(3, 270)
+    assert route(700, 300, 600) == SMALL and route(1000, 2048, 4096) == SPLIT
+    knobs(3, 0)
+    knobs(10, 2)
+    knobs(9, 2)
+    assert route(64, 100, 784) == SPLIT and route(64, 100, 784, np.float64) == SMALL
+    knobs(9, 1)
+    assert route(1000, 2048, 4096) == VENDOR
+    lib.check()

@@ -200,15 +200,25 @@ inline bool gemm_is_small(int m, int n, int k) {
   if (k > 8192) return flop <= limit && (long)m * n <= 262144;   // cross-workgroup split: its partial tiles live in the stream's scratch
   return flop <= limit;
 }
-// The same where the caller has set no limit.  us a call, back to back from a Python process (own / vendor; NN, TN, NT): fp32 64x100x784 4.2/26, 4.0/27, 4.6/26;
-// 100x237x1000 5.0/106, 4.7/107, 5.4/106 (the vendor's candidates for these give all of it to one workgroup); 300x500x300 5.5/10, 1000x237x500 8.0/10,
-// 512^3 8.1/10.5, 9.8/10.4, 8.5/10.4; a long walk of k turns it round: 16x2048x4096 15/10.5, 1000x16x4000 15/13.  fp64, whose vendor kernels are weak on short
-// sides: 1000x100x1000 14/23, 15/38, 14/21; 16x2048x4096 24/55, 31/115, 21/55; the other way round with many tiles and a short k: 640x640x320 18/13.
+// The same where the caller has set no limit: where these kernels are not slower than the vendor's, call for call, over 1400 products of 1 to 30000 x 30000 x 4096.
+// us a call, back to back from a Python process (own / vendor; NN, TN, NT).
+// fp32: 64x100x784 4.2/26, 4.0/27, 4.6/26; 100x237x1000 5.0/106, 4.7/107, 5.4/106 (the vendor's candidates for these give all of it to one workgroup);
+// 1024x1024x64 5.7/10.4, 6.2/10.3, 6.0/10.3; 512^3 8.3/10.1, 9.8/10.2, 8.6/10.4.  Against them:
+//   many tiles: 2048x2048x16 12.0/10.4, 3000x3000x4 23.6/16.2, 8192x8192x1 123/50 (a workgroup of one wave to a tile); from 4300 tiles on 30000x64x64 11.0/10.0;
+//   a short side, which leaves few tiles a long walk: 10000x16x784 11.6/10.4, NT 48x3000x600 12.0/10.6; k beyond 2048: 16x16x4096 12.4/10.2;
+//   an operand along k that does not come in 16-byte loads: TN 900x900x150 18.8/10.4, 4096x128x150 12.5/10.4.
+// fp64, whose vendor kernels are weak on short sides: 1000x100x1000 14/23, 15/38, 14/21; 16x2048x4096 24/55, 31/115, 21/55; 320x320x300 5.9/9.9; short k: 1024x1024x16 5.7/6.2.
+// The other way round with many tiles: 512^3 14.7/15.0, 17.1/13.8, 768x768x128 10.1/8.7, 100x8192x64 9.2/8.0, 100x2000x400 13.0/12.2.
 template <typename T>
-inline bool gemm_is_small_by_rule(int m, int n, int k) {
-  const double flop = 2.0 * ((m + 15) / 16 * 16.0) * ((n + 15) / 16 * 16.0) * k;   // with the padding of 16x16 tiles
+inline bool gemm_is_small_by_rule(bool ta, bool tb, int m, int n, int k, int lda, int ldb) {
+  const double tiles = (m + 15) / 16 * 1.0 * ((n + 15) / 16), flop = 512 * tiles * k;   // with the padding of 16x16 tiles
   if (k > 8192 || flop > 2.7e8) return false;
-  return sizeof(T) == 4 ? k <= 2048 : (k >= 400 || flop <= 1.6e8);
+  if (sizeof(T) == 8) return (flop <= 6e7 && tiles <= 4096) || (k >= 200 && (tiles <= 760 || (tiles <= 900 && flop <= 1.2e8)));
+  const int side = m < n ? m : n;
+  double limit = side >= 128 ? 2.7e8 : side > 64 ? 2.4e8 : tb ? 1.5e8 : 2.1e8;
+  if (tiles > 4300 && limit > 1.5e8) limit = 1.5e8;
+  if ((ta && lda % 4 != 0) || (!tb && ldb % 4 != 0)) limit = 1.2e8;
+  return k <= 2048 && tiles <= 8192 && flop <= limit;
 }
 
 template <typename T>

@@ -987,7 +987,7 @@ static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T*
   // than a launch (key 10: never, or wherever the rule holds)
   auto small_by_rule = [&]() {
     const int knob = g_tune[kTuneGemmSmallRule];
-    return knob != 1 && (sizeof(T) == 8 || g_tune[kTuneGemmSplit] != 2) && gemm_is_small_by_rule<T>(m, n, k) && (knob == 2 || !vendor_prepares());
+    return knob != 1 && (sizeof(T) == 8 || g_tune[kTuneGemmSplit] != 2) && gemm_is_small_by_rule<T>(ta, tb, m, n, k, lda, ldb) && (knob == 2 || !vendor_prepares());
   };
   if (batch.count == 1 && (k <= 0 || (tuning(kTuneGemmSmallMflop) > 0 ? gemm_is_small(m, n, k) : small_by_rule()))) {
     t_route = kRouteSmall;

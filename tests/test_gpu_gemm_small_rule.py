@@ -1,4 +1,5 @@
-"""Small products by default: on both sides of the rule's limits (padding, length of k, type) they match 64 bits, whichever kernel they took."""
+"""Small products by default: on both sides of the rule's limits (padding, length of k, type) they match 64 bits, whichever kernel they took; and each takes the kernel
+that the rule names."""
 import numpy as np
 import pytest
 
@@ -38,6 +39,33 @@ def knobs(knet):
     yield put
     for key, value in old.items():
         fn["knet8_tune"](key, value)
+
+
+# (m, n, k, form, the route where the rule decides): each of the rule's limits from both sides
+F32 = [(64, 100, 784, "NN", SMALL), (512, 512, 512, "NN", SMALL), (513, 512, 512, "NN", VENDOR), (1024, 1024, 64, "NN", SMALL),
+       (1408, 1456, 32, "NN", SMALL), (1456, 1456, 32, "NN", VENDOR), (8192, 8192, 1, "NN", VENDOR), (64, 4096, 200, "NN", SMALL), (1040, 1040, 128, "NN", VENDOR),
+       (32, 64, 2048, "NN", SMALL), (32, 64, 2052, "NN", VENDOR), (64, 2048, 804, "NN", VENDOR), (64, 2048, 800, "NN", SMALL), (64, 2048, 576, "NT", VENDOR), (64, 2048, 568, "NT", SMALL),
+       (112, 2048, 528, "NN", VENDOR), (112, 2048, 520, "NN", SMALL), (900, 900, 72, "TN", SMALL), (900, 900, 74, "TN", VENDOR), (900, 900, 74, "NT", SMALL)]
+F64 = [(64, 100, 784, "NN", SMALL), (512, 512, 112, "NN", SMALL), (512, 512, 116, "NN", VENDOR), (432, 440, 300, "NN", SMALL), (480, 480, 300, "NN", VENDOR), (480, 480, 256, "NN", SMALL),
+       (512, 512, 256, "NN", VENDOR), (1024, 1024, 16, "TN", SMALL), (1040, 1024, 4, "TN", VENDOR), (16, 24, 8192, "NN", SMALL), (16, 24, 8193, "NN", VENDOR)]
+
+
+@pytest.mark.parametrize("m,n,k,form,route,dt", [c + (np.float32,) for c in F32] + [c + (np.float64,) for c in F64])
+def test_each_product_takes_its_route(knet, knobs, m, n, k, form, route, dt):
+    rng = np.random.default_rng(m + n + k)
+    lib = knet.libknet8()
+    ta, tb = form[0] == "T", form[1] == "T"
+    A, B = rng.standard_normal((m, k)).astype(dt), rng.standard_normal((k, n)).astype(dt)
+    a, b = knet.KnetArray(np.asfortranarray(A.T if ta else A)), knet.KnetArray(np.asfortranarray(B.T if tb else B))
+    eps = 2.0 ** -24 if dt == np.float32 else 2.0 ** -52
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    for value, expect in ((2, route), (1, VENDOR)):
+        knobs(10, value)
+        got = knet.Array(knet.gemm(form[0], form[1], 1, a, b, 0, knet.KnetArray(np.zeros((m, n), dt))))
+        assert lib.fn["knet8_product_route"]() == expect, value
+        # one rounding a step of a running sum that grows like sqrt(k); the 64-bit reference has as many
+        assert np.linalg.norm(got - want) <= 2 * eps * max(2.0, k ** 0.5) * np.linalg.norm(want)
+    lib.check()
 
 
 def test_the_other_routes(knet, knobs):

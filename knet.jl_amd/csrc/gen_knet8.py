@@ -688,7 +688,7 @@ KNET8_API void sum_32_21_noalloc(int nx, float* x, int sy, int ny, float* y, hip
    key 3: products of up to this many MFLOP (2*m*n*k/1e6) take the library's own small-product kernels instead of hipBLASLt (default 0: a rule on
    type and sizes, up to 270 MFLOP, where the loaded hipBLASLt allows no prepared calls; see key 10);
    key 4: dense_back_S / dense_nll_back_S accept layers whose products have up to this many MFLOP each (default 270);
-   key 5: non-zero makes the library behave as if the scratch memory of split launches could not be allocated (for tests of that error path);
+   key 5: non-zero makes the library behave as if the scratch memory of split launches and the buffers of uploads could not be allocated (for tests of these paths);
    key 6: non-zero keeps softmax columns of 128 to 256 KB in registers alone instead of registers + LDS (for comparisons);
    key 7: non-zero makes the hipBLASLt route of gemm_S do everything but the vendor call itself (for measuring the library's own share of a call's host time);
    key 8: non-zero keeps repeated products on hipblasLtMatmul instead of the prepared calls of the vendor's extension interface (for comparisons);

@@ -492,7 +492,10 @@ KNET8_API int knet8_upload(void* dst, const void* src, size_t nbytes, hipStream_
   Stage& s = g_stages[std::make_pair(dev, stream)];
   if (!s.host) {
     void* p = nullptr;
-    if (!ok(hipHostMalloc(&p, kStageBytes, hipHostMallocDefault), "hipHostMalloc(upload)")) return -1;
+    if (g_tune[kTuneFailScratch] != 0 || hipHostMalloc(&p, kStageBytes, hipHostMallocDefault) != hipSuccess) {   // no page-locked memory: the copy needs none
+      (void)hipGetLastError();
+      return knet8_memcpy(dst, src, nbytes, 1, stream);
+    }
     s.host = static_cast<char*>(p);
   }
   if (s.used + nbytes > kStageBytes) {

@@ -65,3 +65,25 @@ def test_streams_and_threads(knet):
     fn["knet8_trim"]()
     assert float(knet.sum(knet.KnetArray(np.ones(100, np.float32)))) == 100.0
     lib.check()
+
+
+def test_upload_without_staging_memory(knet):
+    """No page-locked memory for a stream's buffer (knet8_tune key 5): the bytes arrive by the copy that waits, and there is no error."""
+    lib = knet.libknet8()
+    fn = lib.fn
+    a, back = np.arange(1000, dtype=np.int32), np.empty(1000, np.int32)
+    s, p = fn["knet8_stream_create"](), fn["knet8_malloc"](a.nbytes)
+    old = fn["knet8_tune"](5, 1)
+    try:
+        assert fn["knet8_upload"](p, a.ctypes.data, a.nbytes, s) == 0
+    finally:
+        fn["knet8_tune"](5, old)
+    fn["knet8_memcpy"](back.ctypes.data, p, a.nbytes, 2, s)
+    assert np.array_equal(a, back)
+    a += 5
+    assert fn["knet8_upload"](p, a.ctypes.data, a.nbytes, s) == 0
+    fn["knet8_memcpy"](back.ctypes.data, p, a.nbytes, 2, s)
+    assert np.array_equal(a, back)
+    fn["knet8_stream_destroy"](s)
+    fn["knet8_free"](p)
+    lib.check()

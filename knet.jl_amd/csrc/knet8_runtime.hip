@@ -483,8 +483,9 @@ KNET8_API int knet8_memcpy(void* dst, const void* src, size_t nbytes, int kind, 
 }
 
 KNET8_API int knet8_upload(void* dst, const void* src, size_t nbytes, hipStream_t stream) {
-  // larger ones, odd ones, and a stream under capture (where waiting is an error, as it was) take the copy that waits
-  if (nbytes == 0 || nbytes > kStageBytes / 4 || nbytes % 4 != 0 || reinterpret_cast<uintptr_t>(dst) % 4 != 0 || stream_is_capturing(stream))
+  // larger ones, odd ones, and a stream under capture (where waiting is an error, as it was) take the copy that waits; so does the per-thread stream, whose one
+  // handle stands for another stream in every thread: waiting for this thread's would not show that the others have read their part of the buffer
+  if (stream == hipStreamPerThread || nbytes == 0 || nbytes > kStageBytes / 4 || nbytes % 4 != 0 || reinterpret_cast<uintptr_t>(dst) % 4 != 0 || stream_is_capturing(stream))
     return knet8_memcpy(dst, src, nbytes, 1, stream);
   int dev = 0;
   (void)hipGetDevice(&dev);

@@ -87,3 +87,27 @@ def test_upload_without_staging_memory(knet):
     fn["knet8_stream_destroy"](s)
     fn["knet8_free"](p)
     lib.check()
+
+
+def test_per_thread_stream(knet):
+    """hipStreamPerThread is one handle (2) for a stream of each thread: uploads from several threads, enough to use a staging buffer up, keep their bytes."""
+    lib = knet.libknet8()
+    fn = lib.fn
+    wrong = []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        p, back = fn["knet8_malloc"](60000), np.empty(15000, np.int32)
+        for _ in range(30):
+            a = rng.integers(-1000, 1000, size=15000).astype(np.int32)
+            ok = fn["knet8_upload"](p, a.ctypes.data, a.nbytes, 2) == 0 and fn["knet8_memcpy"](back.ctypes.data, p, a.nbytes, 2, 2) == 0
+            if not ok or not np.array_equal(a, back):
+                wrong.append(seed)
+        fn["knet8_free"](p)
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    lib.check()

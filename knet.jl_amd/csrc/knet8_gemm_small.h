@@ -224,7 +224,6 @@ inline bool gemm_is_small_by_rule(bool ta, bool tb, int m, int n, int k, int lda
 template <typename T>
 inline void launch_gemm_small(hipStream_t stream, bool ta, bool tb, int m, int n, int k, T alpha, const T* A, int lda, const T* B, int ldb,
                               T beta, T* C, int ldc, const T* bias = nullptr, int act = 0) {
-  if (alpha == T(0)) k = 0;   // A and B are not read then, as in BLAS: no infinity or NaN of theirs reaches C
   const long tiles = (long)((m + kGsTile - 1) / kGsTile) * ((n + kGsTile - 1) / kGsTile);
   const long ksteps = (k + kGsTile - 1) / kGsTile;
   const long tiles16 = (long)((m + 15) / 16) * ((n + 15) / 16);

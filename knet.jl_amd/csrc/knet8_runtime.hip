@@ -987,6 +987,9 @@ static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T*
     record_error("gemm: an operand has 2^31 or more elements; the 32-bit indices of the library's own kernels do not reach that far");
     return false;
   };
+  // alpha = 0: A and B are not read, as in BLAS, so that no infinity or NaN of theirs reaches C.  (hipBLASLt's kernels that split k have left NaN in C then, with
+  // nothing but their workspace to have it from: 16x24x9000 fp32.)
+  if (batch.count == 1 && alpha == T(0) && (bias || !act) && (long long)m * n < (1LL << 31)) k = 0;
   // empty products (C = beta*C [+ bias]) and small ones: by the caller's limit (knet8_tune key 3), or by the rule where a vendor call costs its caller more
   // than a launch (key 10: never, or wherever the rule holds)
   auto small_by_rule = [&]() {
@@ -1000,7 +1003,7 @@ static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T*
     check_launch("gemm (small)");
     return 0;
   }
-  if constexpr (sizeof(T) == 4) {   // large fp32 products: on the bf16 matrix cores (alpha = 0, where A and B are not read, stays with the vendor)
+  if constexpr (sizeof(T) == 4) {   // large fp32 products: on the bf16 matrix cores
     SplitPlan plan;
     if (batch.count == 1 && alpha != T(0) && gemm_split_fits(m, n, k, lda, ldb, &plan)) {
       if (bias == nullptr && act) { record_error("gemm_bias_act: an activation without a bias is not provided"); return -1; }
@@ -1043,7 +1046,7 @@ template <typename T>
 static int bmm_entry(char transa, char transb, int m, int n, int k, T alpha, const T* A, int lda, long long sa, const T* B, int ldb, long long sb, T beta,
                      T* C, int ldc, long long sc, int batch, hipStream_t stream) {
   if (batch < 0 || sa < 0 || sb < 0 || sc < 0) { record_error("bmm: negative batch count or stride"); return -1; }
-  if (batch <= 1 || k <= 0) {   // nothing to batch, or empty products (C = beta*C): the plain entry handles both
+  if (batch <= 1 || k <= 0 || alpha == T(0)) {   // nothing to batch, or empty products (C = beta*C): the plain entry handles both
     for (int b = 0; b < batch; b++) {
       const int rc = gemm<T>(transa, transb, m, n, k, alpha, A + b * sa, lda, B + b * sb, ldb, beta, C + b * sc, ldc, stream);
       if (rc != 0) return rc;

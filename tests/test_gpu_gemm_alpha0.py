@@ -25,3 +25,25 @@ def test_alpha_zero(knet, m, n, k, S, dt, knob):
     finally:
         lib.fn["knet8_tune"](knob[0], old)
     lib.check()
+
+
+@pytest.mark.parametrize("S,dt", [("32", np.float32), ("64", np.float64)])
+def test_alpha_zero_in_batches(knet, S, dt):
+    lib = knet.libknet8()
+    m, n, k, batch = 16, 24, 9000, 3
+    A, B = knet.KnetArray(np.full((m, k, batch), np.nan, dt)), knet.KnetArray(np.full((k, n, batch), np.inf, dt))
+    C = np.arange(m * n * batch, dtype=dt).reshape(m, n, batch)
+    for beta in (0.0, -2.0):
+        out = knet.KnetArray(C)
+        assert lib.call("bmm_" + S, b"N", b"N", m, n, k, 0.0, A.ptr, m, m * k, B.ptr, k, k * n, beta, out.ptr, m, m * n, batch) == 0
+        assert np.array_equal(knet.Array(out), beta * C)
+    lib.check()
+
+
+def test_what_stays_refused(knet):
+    """An activation without a bias has no kernel on any route, alpha = 0 included."""
+    lib = knet.libknet8()
+    A, B, C = (knet.KnetArray(np.ones(d, np.float32)) for d in ((700, 700), (700, 700), (700, 700)))
+    assert lib.call("gemm_bias_act_32", b"N", b"N", 700, 700, 700, 0.0, A.ptr, 700, B.ptr, 700, None, 1, C.ptr, 700) == -1
+    with pytest.raises(RuntimeError):
+        lib.check()

@@ -1,7 +1,7 @@
 // Large fp32 matrix products on the bf16 matrix cores (column-major, C = alpha*op(A)*op(B) + beta*C [+ bias] [relu]).
 //
 // The fp32 matrix instructions run at 1/16 of the bf16 ones (157 against 2500 TFLOP/s nominal), and the vendor library's fp32 products sit at
-// their limit: 8192^3 reaches 154 TFLOP/s, 4096x2048x4096 142-149.  Here every element is cut into three bf16 parts, x = h + m + l, each the
+// their limit: 8192^3 reaches 154 TFLOP/s, 4096x2048x4096 151.  Here every element is cut into three bf16 parts, x = h + m + l, each the
 // rounding of what the ones before it leave: 3 x 8 bits and the signs hold all 24 bits of an fp32 number, so h + m + l = x exactly, with
 // |m| <= 2^-8 |x| and |l| <= 2^-17 |x|.  Of the nine products of parts all but ll (at most 2^-34 of the whole) are formed, hh in one
 // set of fp32 accumulators and the seven small ones in another: the large sums see one rounding per 16 steps of k, and a sum with one term that is not
@@ -19,8 +19,8 @@
 // The cut is made while a tile goes from global memory to LDS (6.5 vector instructions an element, in the shadow of the matrix instructions of the
 // SIMD's other wave): no extra pass over the operands, no scratch.  What bounds it: 256x128 tile, 8 waves of 64x64, 32 steps of k a stage, two
 // stages in LDS (149 KB): matrix cores 4096 cycles a stage, LDS about 2070, vector ALU about 2100; and the clock, which normal data
-// holds further down than zeros do (with six products, loads and cut left out: 255 TFLOP/s against 345).  TFLOP/s (of fp32 work), this / vendor:
-// 4096x2048x4096 176/142, TN 171/149, 4096x4096x2048 NT 169/148, 32000x2048x512 150/137, 512x2048x32000 TN 165/143, 32000x512x2048 NT 163/145, 8192^3 177/154.
+// holds down: 8192^3 175 TFLOP/s, and 239 on zeros or small whole numbers.  TFLOP/s (of fp32 work), this / vendor: 4096x2048x4096 167/151, TN 167/151,
+// 4096x4096x2048 NT 164/148, 32000x2048x512 146/137, 512x2048x32000 TN 161/140, 32000x512x2048 NT 162/145, 8192^3 175/154.
 #pragma once
 #include "knet8_device.h"
 #include "knet8_runtime.h"

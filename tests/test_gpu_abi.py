@@ -297,8 +297,8 @@ def test_transpose_and_batched_permutation(knet, dt, S):
 
 
 def test_product_routing_knob_both_routes_agree(knet, oracle):
-    """gemm_S goes to hipBLASLt unless a caller opts in: knet8_tune key 3 (products of up to that many MFLOP run on the library's own
-    small-product kernels) is 0 by default.  The same product through both routes gives the same matrix to rounding; the knob reads
+    """A small product goes to hipBLASLt with the rule for small products switched off (knet8_tune key 10) and to the library's own small-product kernels when a
+    caller sets key 3 (products of up to that many MFLOP; 0 by default).  The same product through both routes gives the same matrix to rounding; the knob reads
     back and restores."""
     fn = knet.libknet8().fn
     rng = np.random.default_rng(55)
@@ -306,12 +306,17 @@ def test_product_routing_knob_both_routes_agree(knet, oracle):
     A, B = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((k, n)).astype(np.float32)
     want = oracle.gemm(A, B)
     Ad, Bd = knet.KnetArray(A), knet.KnetArray(B)
-    assert fn["knet8_tune"](3, -1) == 0                       # default: every product goes to the vendor library
-    vendor = knet.Array(knet.gemm("N", "N", 1, Ad, Bd, 0, knet.KnetArray(np.zeros((m, n), np.float32))))
+    assert fn["knet8_tune"](3, -1) == 0 and fn["knet8_tune"](10, 1) == 0
+    try:
+        vendor = knet.Array(knet.gemm("N", "N", 1, Ad, Bd, 0, knet.KnetArray(np.zeros((m, n), np.float32))))
+        assert fn["knet8_product_route"]() == 1
+    finally:
+        fn["knet8_tune"](10, 0)
     old = fn["knet8_tune"](3, 270)                            # opt in: this product now runs on the library's own kernel
     try:
         assert old == 0 and fn["knet8_tune"](3, -1) == 270    # a negative value only reads
         own = knet.Array(knet.gemm("N", "N", 1, Ad, Bd, 0, knet.KnetArray(np.zeros((m, n), np.float32))))
+        assert fn["knet8_product_route"]() == 2
     finally:
         fn["knet8_tune"](3, 0)
     for got in (vendor, own):

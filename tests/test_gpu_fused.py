@@ -222,7 +222,7 @@ def test_gemm_bias_act_on_the_own_kernels_carries_the_bits_of_the_three_launch_c
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
 def test_gemm_bias_act_treats_nan_and_inf_alike_on_both_routes(knet, dt):
     """A NaN, a +Inf and a -Inf in A: without activation the rows they touch come out NaN / +-Inf; with relu every route of the entry point --
-    the vendor epilogue (key 3 = 0) and the library's own kernels (key 3 = 270) -- computes z > 0 ? z : 0, the device relu of the reference
+    the vendor epilogue (keys 3 = 0, 10 = 1) and the library's own kernels (key 3 = 270) -- computes z > 0 ? z : 0, the device relu of the reference
     (src/libknet8/ops.jl:63): the NaN row becomes 0, +Inf stays, -Inf becomes 0.  (relu_S, which follows the CPU path, keeps a NaN.)"""
     lib = knet.libknet8()
     fn = lib.fn
@@ -237,13 +237,14 @@ def test_gemm_bias_act_treats_nan_and_inf_alike_on_both_routes(knet, dt):
     clean = np.ones(m, bool)
     clean[[3, 7, 9]] = False
     want = A[clean].astype(np.float64) @ B.astype(np.float64) + b[clean, None]
-    old = fn["knet8_tune"](3, -1)
+    old, rule = fn["knet8_tune"](3, -1), fn["knet8_tune"](10, 1)
     try:
         for route in (0, 270):
             fn["knet8_tune"](3, route)
             for act in (0, 1):
                 C = knet.KnetArray(np.full((m, n), 5.0, dt))
                 assert fn["gemm_bias_act_%s_stream" % S](b"N", b"N", m, n, k, 1.0, Ad.ptr, m, Bd.ptr, k, bd.ptr, act, C.ptr, m, lib.stream) == 0
+                assert fn["knet8_product_route"]() == (2 if route else 1)
                 c = knet.Array(C)
                 ref = np.maximum(want, 0) if act else want
                 assert np.abs(c[clean] - ref).max() <= (1e-5 if dt == np.float32 else 1e-13) * np.abs(want).max(), (route, act)
@@ -253,6 +254,7 @@ def test_gemm_bias_act_treats_nan_and_inf_alike_on_both_routes(knet, dt):
                     assert np.all(c[3] == 0) and np.all(c[7] == np.inf) and np.all(c[9] == 0), (route, act, c[3, :4], c[7, :4], c[9, :4])
     finally:
         fn["knet8_tune"](3, old)
+        fn["knet8_tune"](10, rule)
     y = knet.Array(knet.relu(knet.KnetArray(np.array([np.nan, -1.0, 2.0], dt))))
     assert np.isnan(y[0]) and y[1] == 0 and y[2] == 2
     lib.check()

@@ -7,8 +7,8 @@
 // set of fp32 accumulators and the seven small ones in another: the large sums see one rounding per 16 steps of k, and a sum with one term that is not
 // zero is rounded as the fp32 instruction rounds it.  (ml and lm reach 2^-24 of the whole together: without them such a sum is off by up to 2^-23.2, and sums
 // of equal numbers by as much; they cost a sixth of the speed.)  2-norm of the error against 64 bits, this / vendor fp32: normal data 1000x237x784 8.4e-8/5.0e-7,
-// 4096x2048x4096 4.0e-7/1.15e-6, 512x2048x32000 4.0e-7/3.2e-6; all-positive data 4.9e-8/3.8e-7, 3.5e-7/9.9e-7, 1.3e-7/2.8e-6; 2048^3 with one term a sum
-// 2.53e-8/2.53e-8 (largest 2^-23.995/2^-24.000), with two 3.2e-8/3.1e-8, with eight 3.8e-8/5.4e-8.
+// 4096x2048x4096 4.0e-7/1.15e-6, 512x2048x32000 4.0e-7/2.3e-6; all-positive data 4.9e-8/3.8e-7, 3.5e-7/9.9e-7, 1.3e-7/1.4e-6; 2048^3 with one term a sum
+// 2.53e-8/2.53e-8 (largest 2^-23.99/2^-24.00), with two 3.14e-8/3.11e-8, with eight 3.8e-8/5.4e-8.
 //   * Small numbers: the lower parts of numbers below 2^-109 would leave bf16's range.  Both operands are multiplied by 2^24 on the way in and the
 //     sums by 2^-48 on the way out, which keeps every fp32 number, denormals included, whole.
 //   * Large numbers, infinities, NaN: a part or a sum that overflows leaves a NaN or an infinity in an accumulator (inf - inf in the split itself

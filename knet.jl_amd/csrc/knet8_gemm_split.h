@@ -4,7 +4,7 @@
 // their limit: 8192^3 reaches 154 TFLOP/s, 4096x2048x4096 151.  Here every element is cut into three bf16 parts, x = h + m + l, each the
 // rounding of what the ones before it leave: 3 x 8 bits and the signs hold all 24 bits of an fp32 number, so h + m + l = x exactly, with
 // |m| <= 2^-8 |x| and |l| <= 2^-17 |x|.  Of the nine products of parts all but ll (at most 2^-34 of the whole) are formed, hh in one
-// set of fp32 accumulators and the seven small ones in another: the large sums see one rounding per 16 steps of k, and a sum with one term that is not
+// set of fp32 accumulators and the seven small ones in another: the large sums see one rounding per 32 steps of k, and a sum with one term that is not
 // zero is rounded as the fp32 instruction rounds it.  (ml and lm reach 2^-24 of the whole together: without them such a sum is off by up to 2^-23.2, and sums
 // of equal numbers by as much; they cost a sixth of the speed.)  2-norm of the error against 64 bits, this / vendor fp32: normal data 1000x237x784 8.4e-8/5.0e-7,
 // 4096x2048x4096 4.0e-7/1.15e-6, 512x2048x32000 4.0e-7/2.3e-6; all-positive data 4.9e-8/3.8e-7, 3.5e-7/9.9e-7, 1.3e-7/1.4e-6; 2048^3 with one term a sum
@@ -13,14 +13,18 @@
 //     sums by 2^-48 on the way out, which keeps every fp32 number, denormals included, whole.
 //   * Large numbers, infinities, NaN: a part or a sum that overflows leaves a NaN or an infinity in an accumulator (inf - inf in the split itself
 //     if not before).  A wave that finds one in its patch forms these sums again with the fp32 matrix instruction: results beyond
-//     2^80, and what is infinite or NaN, come out as that instruction gives them; the others stay.  us, 4096x2048x4096 (vendor 470): 400 on finite data, 340 if all is NaN, 600 with
-//     one NaN in A and 800 with one infinity (a row of sums to form again), 1240 if every sum is beyond 2^80.
+//     2^80, and what is infinite or NaN, come out as that instruction gives them; the others stay.  us, 4096x2048x4096 (vendor 458): 352 on finite data, 324 if all is NaN, 542 with
+//     one NaN in A and 731 with one infinity (a row of sums to form again), 1130 if every sum is beyond 2^80.
 //
 // The cut is made while a tile goes from global memory to LDS (6.5 vector instructions an element, in the shadow of the matrix instructions of the
-// SIMD's other wave): no extra pass over the operands, no scratch.  What bounds it: 256x128 tile, 8 waves of 64x64, 32 steps of k a stage, two
-// stages in LDS (149 KB): matrix cores 4096 cycles a stage, LDS about 2070, vector ALU about 2100; and the clock, which normal data
-// holds down: 8192^3 175 TFLOP/s, and 239 on zeros or small whole numbers.  TFLOP/s (of fp32 work), this / vendor: 4096x2048x4096 167/151, TN 167/151,
-// 4096x4096x2048 NT 164/148, 32000x2048x512 146/137, 512x2048x32000 TN 161/140, 32000x512x2048 NT 162/145, 8192^3 175/154.
+// SIMD's other wave): no extra pass over the operands, no scratch.  256x128 tile, 8 waves of 64x64, 32 steps of k a stage, two stages in LDS (up to 158 KB):
+// matrix cores 4096 cycles a stage, LDS about 2070, vector ALU about 2100.  What bounds it is power: 8192^3 runs at 198 TFLOP/s on normal data and at 232 on zeros.
+// So the matrix instructions are chosen and ordered by the energy they take on normal data.  From registers alone 32x32x16 reaches 1822 TFLOP/s of bf16 work
+// and 16x16x32 2073 (both 2450 to 2480 on zeros): half the traffic to the accumulators.  All eight products of a 16x16 tile follow each other, so that the sums stay
+// where they are (3 % over taking the tiles in turn), in an order in which only one operand changes from one to the next (another 2 %; one that changes the first
+// operand more often instead is 1 to 2 % slower).  us, before (32x32x16, tiles in turn) / now, the same run: 4096x2048x4096 396/346, TN 410/352, 4096x4096x2048 NT 420/358, 8192^3 6650/5910,
+// 32000x2048x512 458/401, 512x2048x32000 TN 414/375, 32000x512x2048 NT 427/374.  TFLOP/s (of fp32 work), this / vendor: 4096x2048x4096 192/150, TN 195/150,
+// 4096x4096x2048 NT 194/148, 32000x2048x512 168/137, 512x2048x32000 TN 178/139, 32000x512x2048 NT 188/145, 8192^3 198/154.
 #pragma once
 #include "knet8_device.h"
 #include "knet8_runtime.h"
@@ -31,6 +35,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 template <int N> struct __attribute__((packed, aligned(4))) FNu { float v[N]; };   // N elements at any element boundary, one load
 using F4u = FNu<4>;
@@ -69,9 +74,10 @@ struct SplitLoader {
   static constexpr int kRows = KC ? 1 : (kVals >= 16 ? 4 : 2);
   static constexpr int kItems = kVals / (4 * kRows);
   static_assert(kItems >= 1 && kVals % (4 * kRows) == 0 && ROWS % 64 == 0, "tile and workgroup do not match");
-  // Where the 16 bytes of a row stand (in units of 16 bytes): in order, or dealt out to four groups.  With the groups 32 bytes off the
-  // multiples of 128 (and likewise the octets of k of the first form) the writes of store() and the reads of the fragments meet no bank twice.
-  static constexpr int kGroup = ROWS / 4 + 2;
+  // Where the 16 bytes of a row stand (in units of 16 bytes): in order, or dealt out to four groups, each 64 bytes off the multiples of 256, so that the 16 rows of a
+  // fragment lie in all banks once (32 bytes off, which suits reads of 32 rows: 4096x4096x2048 NT 372 us, so 365).  The octets of k of the first form stand
+  // 32 bytes off: eight lanes there write the 32 steps of a row.
+  static constexpr int kGroup = ROWS / 4 + 4;
   static constexpr int kStride = KC ? ROWS + 2 : 4 * kGroup;      // from one octet of k to the next
   static constexpr int kPart = (BK / 8) * kStride;                // from one part to the next
   static constexpr int kUnits = 3 * kPart;
@@ -160,11 +166,12 @@ template <int BM, int BN, int WM, int WN, int BK, bool TA, bool TB>
 __global__ __launch_bounds__(64 * (BM / WM) * (BN / WN), 2)
 void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda, const float* __restrict__ B, int ldb, float* __restrict__ C, int ldc,
                        float alpha, float beta, const float* __restrict__ bias, int act, int kchunk, unsigned splits) {
-  constexpr int NT = 64 * (BM / WM) * (BN / WN), FM = WM / 32, FN = WN / 32;
+  constexpr int NT = 64 * (BM / WM) * (BN / WN), FM = WM / 16, FN = WN / 16;
   using LA = SplitLoader<BM, BK, NT, TA>;
   using LB = SplitLoader<BN, BK, NT, !TB>;
   __shared__ uint4 lds[2][LA::kUnits + LB::kUnits];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, half = lane >> 5, l32 = lane & 31;
+  __shared__ unsigned long long odd[NT / 64][FN * 4 * FM];   // which sums are not finite (see the end)
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, half = lane >> 5, l32 = lane & 31, quad = lane >> 4, l16 = lane & 15;
   const int wm = (wave % (BM / WM)) * WM, wn = (wave / (BM / WM)) * WN;
   unsigned im, in, z;
   split_tile(blockIdx.x, gridDim.x, (unsigned)((m + BM - 1) / BM), (unsigned)((n + BN - 1) / BN), im, in, z);
@@ -177,13 +184,13 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
   LB lb;
   la.init(t, m - i0, lda);
   lb.init(t, n - j0, ldb);
-  f32x16 acc[FN][FM], low[FN][FM];   // hh, and the seven products of lower weight
+  f32x4 acc[FN][FM], low[FN][FM];   // hh, and the seven products of lower weight
 #pragma unroll
   for (int a = 0; a < FN; a++)
 #pragma unroll
     for (int b = 0; b < FM; b++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) acc[a][b][r] = low[a][b][r] = 0.0f;
+      for (int r = 0; r < 4; r++) acc[a][b][r] = low[a][b][r] = 0.0f;
   auto fetch_full = [&]() {
     la.load(pa, lda);
     lb.load(pb, ldb);
@@ -199,31 +206,33 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
     la.store(s);
     lb.store(s + LA::kUnits);
   };
-  int ua[FM], ub[FN];   // this lane's rows in the two halves of a buffer
+  int ua[FM], ub[FN];   // this lane's rows in the two halves of a buffer, at its octet of k
 #pragma unroll
-  for (int i = 0; i < FM; i++) ua[i] = half * LA::kStride + LA::unit(wm + 32 * i + l32);
+  for (int i = 0; i < FM; i++) ua[i] = quad * LA::kStride + LA::unit(wm + 16 * i + l16);
 #pragma unroll
-  for (int i = 0; i < FN; i++) ub[i] = LA::kUnits + half * LB::kStride + LB::unit(wn + 32 * i + l32);
-  auto multiply = [&](const uint4* s, int step) {   // 16 steps of k
-    bf16x8 fb[FN][3];
+  for (int i = 0; i < FN; i++) ub[i] = LA::kUnits + quad * LB::kStride + LB::unit(wn + 16 * i + l16);
+  bf16x8 fa[FM][3];
+  auto take_a = [&](const uint4* s) {
 #pragma unroll
     for (int p = 0; p < 3; p++)
 #pragma unroll
-      for (int i = 0; i < FN; i++) fb[i][p] = __builtin_bit_cast(bf16x8, s[ub[i] + p * LB::kPart + 2 * step * LB::kStride]);
+      for (int i = 0; i < FM; i++) fa[i][p] = __builtin_bit_cast(bf16x8, s[ua[i] + p * LA::kPart]);
+  };
+  auto multiply = [&](const uint4* s, int first, int last) {   // 32 steps of k, column tiles first .. last - 1 of the wave
 #pragma unroll
-    for (int p = 2; p >= 0; p--) {
-      bf16x8 fa[FM];
+    for (int a = first; a < last; a++) {
+      bf16x8 fb[3];
 #pragma unroll
-      for (int i = 0; i < FM; i++) fa[i] = __builtin_bit_cast(bf16x8, s[ua[i] + p * LA::kPart + 2 * step * LA::kStride]);
+      for (int p = 0; p < 3; p++) fb[p] = __builtin_bit_cast(bf16x8, s[ub[a] + p * LB::kPart]);
+      // ml, mm ... hh: one operand changes at a time
+      constexpr int kA[8] = {2, 2, 1, 1, 1, 0, 0, 0}, kB[8] = {1, 0, 0, 1, 2, 2, 1, 0};
 #pragma unroll
-      for (int q = p > 1 ? 1 : 2; q >= 0; q--)
+      for (int b = 0; b < FM; b++)
 #pragma unroll
-        for (int a = 0; a < FN; a++)
-#pragma unroll
-          for (int b = 0; b < FM; b++) {
-            f32x16& c = p + q > 0 ? low[a][b] : acc[a][b];
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[a][q], fa[b], c, 0, 0, 0);
-          }
+        for (int o = 0; o < 8; o++) {
+          f32x4& c = o < 7 ? low[a][b] : acc[a][b];
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[b][kA[o]], fb[kB[o]], c, 0, 0, 0);
+        }
     }
   };
   const int tiles = (kend - kbeg + BK - 1) / BK, full = (kend - kbeg) / BK;
@@ -233,22 +242,24 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
   int cur = 0, i = 0;
   for (; i + 2 < full; i++, cur ^= 1) {
     __syncthreads();
-    multiply(lds[cur], 0);
+    take_a(lds[cur]);
+    multiply(lds[cur], 0, FN / 2);
     la.store(lds[cur ^ 1]);
     la.load(pa, lda);
     pa += BK * sa;
     lb.store(lds[cur ^ 1] + LA::kUnits);
     lb.load(pb, ldb);
     pb += BK * sb;
-    multiply(lds[cur], 1);
-    __builtin_amdgcn_iglp_opt(0);   // spread the LDS traffic and the cut over the matrix instructions (with six products: 8192^3 202 -> 212 TFLOP/s, 4096x2048x4096 165 -> 206)
+    multiply(lds[cur], FN / 2, FN);
+    __builtin_amdgcn_iglp_opt(0);   // spread the LDS traffic and the cut over the matrix instructions (8192^3 181 -> 184 TFLOP/s, 512x2048x32000 TN 172 -> 174)
   }
   for (; i < tiles; i++, cur ^= 1) {   // the last stages: nothing more to fetch, or less than a stage
     __syncthreads();
-    multiply(lds[cur], 0);
+    take_a(lds[cur]);
+    multiply(lds[cur], 0, FN / 2);
     if (i + 1 < tiles) stage(lds[cur ^ 1]);
     if (i + 2 < tiles) fetch(kbeg + (i + 2) * BK);
-    multiply(lds[cur], 1);
+    multiply(lds[cur], FN / 2, FN);
   }
 #pragma unroll
   for (int a = 0; a < FN; a++)
@@ -256,13 +267,13 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
     for (int b = 0; b < FM; b++) acc[a][b] += low[a][b];
   float bad = 0.0f;
 #pragma unroll
-  for (int b = 0; b < FM; b++)
-    if (i0 + wm + 32 * b + l32 < m) {
+  for (int a = 0; a < FN; a++)
+    if (j0 + wn + 16 * a + l16 < n) {
 #pragma unroll
-      for (int a = 0; a < FN; a++)
+      for (int b = 0; b < FM; b++)
 #pragma unroll
-        for (int r = 0; r < 16; r++)
-          if (j0 + wn + 32 * a + 8 * (r >> 2) + 4 * half + (r & 3) < n) bad += acc[a][b][r] * 0.0f;
+        for (int r = 0; r < 4; r++)
+          if (i0 + wm + 16 * b + 4 * quad + r < m) bad += acc[a][b][r] * 0.0f;
     }
   const bool again = __any(bad != 0.0f);   // (NaN: a sum is not finite)
   float* c = C;
@@ -279,40 +290,69 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
     *d = v;
   };
 #pragma unroll
-  for (int b = 0; b < FM; b++) {
-    const int i = i0 + wm + 32 * b + l32;
+  for (int b = 0; b < FM; b++) {   // a lane's four sums are neighbours in a column: 16 bytes a store
+    const int i = i0 + wm + 16 * b + 4 * quad;
     if (i >= m) continue;
-    const float bi = (bias && splits == 1) ? bias[i] : 0.0f;
+    const bool whole = i + 4 <= m && !again;
+    float bi[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (bias && splits == 1) {
 #pragma unroll
-    for (int a = 0; a < FN; a++)
+      for (int r = 0; r < 4; r++) bi[r] = bias[i + r < m ? i + r : i];
+    }
 #pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int j = j0 + wn + 32 * a + 8 * (r >> 2) + 4 * half + (r & 3);
-        if (j < n && !(again && acc[a][b][r] * 0.0f != 0.0f)) store(acc[a][b][r] * kSplitUnscale, i, j, bi);
+    for (int a = 0; a < FN; a++) {
+      const int j = j0 + wn + 16 * a + l16;
+      if (j >= n) continue;
+      if (whole) {
+        float* d = c + (long)j * ld + i;
+        F4u v;
+#pragma unroll
+        for (int r = 0; r < 4; r++) v.v[r] = acc[a][b][r] * kSplitUnscale;
+        if (splits == 1) {
+          F4u old = {{0.0f, 0.0f, 0.0f, 0.0f}};
+          if (beta != 0.0f) old = *reinterpret_cast<const F4u*>(d);
+#pragma unroll
+          for (int r = 0; r < 4; r++) {
+            v.v[r] = alpha * v.v[r];
+            if (beta != 0.0f) v.v[r] = v.v[r] + beta * old.v[r];
+            if (bias) v.v[r] = v.v[r] + bi[r];
+            if (act == 1) v.v[r] = v.v[r] > 0.0f ? v.v[r] : 0.0f;
+          }
+        }
+        *reinterpret_cast<F4u*>(d) = v;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          if (i + r < m && acc[a][b][r] * 0.0f == 0.0f) store(acc[a][b][r] * kSplitUnscale, i + r, j, bi[r]);
       }
+    }
   }
   if (!again) return;
   // The sums that are not finite, by the fp32 instruction: 32x32 of the patch at a time, where there are any.  Lanes 0-31 take the first 16 of 32 steps of k and lanes
   // 32-63 the others, so that an operand with k in a row comes in 16-byte loads.  Once all that are wanted are NaN, as in a training run that has diverged, what follows
   // changes nothing.
   constexpr int kStep = 16;
-  unsigned wanted[FN * FM];   // one bit a sum
 #pragma unroll
-  for (int f = 0; f < FN * FM; f++) {
-    wanted[f] = 0;
+  for (int a = 0; a < FN; a++)
 #pragma unroll
-    for (int r = 0; r < 16; r++) wanted[f] |= (acc[f / FM][f % FM][r] * 0.0f != 0.0f ? 1u : 0u) << r;
-  }
+    for (int r = 0; r < 4; r++)
+#pragma unroll
+      for (int b = 0; b < FM; b++) {   // bit 16*q + l: column l of the 16x16 tile, row 4*q + r
+        const unsigned long long w = __ballot(acc[a][b][r] * 0.0f != 0.0f);
+        if (lane == 0) odd[wave][(a * 4 + r) * FM + b] = w;
+      }
+  __builtin_amdgcn_wave_barrier();   // (a wave reads back what it wrote itself)
 #pragma unroll 1
-  for (int f = 0; f < FN * FM; f++) {
+  for (int f = 0; f < FN * FM / 4; f++) {
+    const int fi = 32 * (f % (FM / 2)), fj = 32 * (f / (FM / 2));
+    const int i = i0 + wm + fi + l32, ja = j0 + wn + fj, jl = ja + l32;
     unsigned want = 0;
 #pragma unroll
-    for (int g = 0; g < FN * FM; g++) want = f == g ? wanted[g] : want;
-    const int i = i0 + wm + 32 * (f % FM) + l32, ja = j0 + wn + 32 * (f / FM), jl = ja + l32;
-    if (i >= m) want = 0;
-#pragma unroll
-    for (int r = 0; r < 16; r++)
-      if (ja + 8 * (r >> 2) + 4 * half + (r & 3) >= n) want &= ~(1u << r);
+    for (int r = 0; r < 16; r++) {
+      const int jw = 8 * (r >> 2) + 4 * half + (r & 3);   // the column of the 32x32 patch that the instruction below leaves in register r
+      const unsigned long long w = odd[wave][(((fj + jw) / 16) * 4 + (l32 & 3)) * FM + (fi + l32) / 16];
+      if (i < m && ja + jw < n) want |= (unsigned)(w >> (16 * (l16 / 4) + jw % 16) & 1u) << r;
+    }
     if (!__any(want != 0)) continue;
     const float* p = A + (long)(i < m ? i : m - 1) * (TA ? lda : 1) + (kbeg + kStep * half) * sa;
     const float* q = B + (long)(jl < n ? jl : n - 1) * (TB ? 1 : ldb) + (kbeg + kStep * half) * sb;
@@ -350,7 +390,7 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
   }
 }
 
-// How many slices of k an m x n x k product is cut into, and its estimated time in us: a stage of 32 steps takes 2.8 with most of the 256 CUs at work, starting
+// How many slices of k an m x n x k product is cut into, and its estimated time in us: a stage of 32 steps takes 2.5 with most of the 256 CUs at work, starting
 // and storing a tile 7 (fitted to 90 products of 2 to 200 GFLOP); slices, which let few tiles fill the chip, cost a second launch that reads them.
 struct SplitPlan { int splits, kchunk; double us; };
 inline SplitPlan gemm_split_plan(int m, int n, int k) {
@@ -360,16 +400,16 @@ inline SplitPlan gemm_split_plan(int m, int n, int k) {
   for (int s = 1; s <= 16; s++) {
     if (s > 1 && (stages / s < 4 || (size_t)s * m * n * sizeof(float) > kMostPartial)) break;
     const double per = (double)(long)((stages + s - 1) / s), turns = (double)(long)((tiles * s + ncu - 1) / ncu);
-    double us = turns * (per * 2.8 + 7);
+    double us = turns * (per * 2.5 + 7);
     if (s > 1) us += 4 + (s + 1) * 4.0 * m * n / 5e6;
     if (us < best.us) best = {s, (int)per * 32, us};
   }
   best.splits = (k + best.kchunk - 1) / best.kchunk;
   return best;
 }
-// True if the product runs here: estimated faster than the vendor's fp32 kernels (140 TFLOP/s and 8 us for the call, a little less at odd sizes).  us, this /
-// vendor: 1000x2048x4096 113/119, 4096x1792x545 62/79, 255x3000x8005 94/103, 3161x6756x1098 TN 334/408, 1217x1950x2863 TN 105/108; not taken:
-// 1024x2048x1024 42/33, 3000x3000x400 NT 92/66, 188x6336x1630 47/37, 1785x5130x7191 1174/950 (a last turn that is nearly empty).
+// True if the product runs here: estimated faster than the vendor's fp32 kernels (140 TFLOP/s and 8 us for the call).  us, this /
+// vendor: 1000x2048x4096 101/119, 4096x1792x545 54/80, 255x3000x8005 89/104, 689x8103x920 TN 82/95, 3161x6756x1098 TN 304/410; level: 1880x1085x4387 130/130; not taken:
+// 1024x2048x1024 41/35, 3000x3000x400 NT 81/66, 188x6336x1630 44/37, 1785x5130x7191 1094/953 (a last turn that is nearly empty).
 // The loaders' offsets within a tile have 32 bits: 255 * ld.
 inline bool gemm_split_fits(int m, int n, int k, int lda, int ldb, SplitPlan* plan) {
   const int knob = tuning(kTuneGemmSplit);   // for tests and comparisons: 1 never, 2 wherever the kernel can
@@ -377,7 +417,7 @@ inline bool gemm_split_fits(int m, int n, int k, int lda, int ldb, SplitPlan* pl
   const double flop = 2.0 * m * n * (double)k;
   if (knob != 2 && (m < 64 || n < 64 || k < 64 || flop < 2e9)) return false;
   *plan = gemm_split_plan(m, n, k);
-  return knob == 2 || plan->us < 1.05 * (flop / 140e6 + 8);
+  return knob == 2 || plan->us < flop / 140e6 + 8;
 }
 
 // C = act(alpha*sum of the slices [+ beta*C] [+ bias]), slices in order.

@@ -235,3 +235,28 @@ def test_sums_formed_again(knet, everywhere, m, n, k, ta, tb):
 def test_all_nan(knet, everywhere):
     got = product(knet, False, False, np.full((260, 300), np.nan, np.float32), np.ones((300, 140), np.float32))
     assert np.isnan(got).all()
+
+
+@pytest.mark.parametrize("m,n,pad,first", [(256, 128, 0, 0), (259, 131, 1, 1), (258, 130, 3, 2), (5, 7, 2, 3)])
+def test_stores_at_any_boundary_and_single_sums(knet, everywhere, m, n, pad, first):
+    """C from any element of its array on and with any column stride: four sums a store, nothing beside the columns is touched.  Single sums beyond 2^80, in every row
+    and column of a 16x16 tile, are those of the fp32 instruction; their neighbours are not formed again."""
+    k, ldc = 40, m + pad
+    rng = np.random.default_rng(m)
+    A, B = rng.uniform(0.5, 1.0, (m, k)).astype(np.float32), rng.uniform(0.5, 1.0, (k, n)).astype(np.float32)
+    # scaled by powers of two, so that a sum is beyond 2^80 only where a large row meets a large column
+    A[np.arange(0, m, 17) % m] *= np.float32(2.0 ** 45)
+    B[:, np.arange(0, n, 9) % n] *= np.float32(2.0 ** 45)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    C = np.full(first + ldc * n + 4, 7.0, np.float32)
+    Ad, Bd, Cd = device(knet, A), device(knet, B), device(knet, C)
+    lib = knet.libknet8()
+    for beta in (0.0, 1.0):
+        assert lib.call("gemm_32", b"N", b"N", m, n, k, 1.0, Ad.ptr, m, Bd.ptr, k, beta, Cd.ptr + 4 * first, ldc) == 0
+    out = knet.Array(Cd)
+    got = out[first:first + ldc * n].reshape(ldc, n, order="F")
+    assert np.all(out[:first] == 7) and np.all(out[first + ldc * n:] == 7) and np.all(got[m:] == 7)
+    # positive terms: k + 1 roundings of at most 2^-24 of the sum each in the product, one in the addition
+    assert np.abs(got[:m] - 2 * want).max(initial=0, where=want < 2.0 ** 80) <= 2.0 ** -24 * (k + 2) * 2 * want[want < 2.0 ** 80].max()
+    assert (np.abs(got[:m] / (2 * want) - 1)).max() <= 2.0 ** -24 * (k + 2)
+    lib.check()

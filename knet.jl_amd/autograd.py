@@ -96,12 +96,6 @@ def selective(back):
     return back
 
 
-def drop(x):
-    """Takes the newest node off the tape again: nothing has been made of ``x`` yet, and nothing will be."""
-    if isinstance(x, Node) and _TAPE is not None and _TAPE.nodes[-1] is x:
-        _TAPE.nodes.pop()
-
-
 def addto(a, b):
     """``addto!(a,b)``: accumulate a gradient (src/autograd_gpu/addto.jl:7-10: ``axpy!(1,b,a)``)."""
     if a is None:

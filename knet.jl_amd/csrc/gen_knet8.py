@@ -553,6 +553,11 @@ def gen_softmax():
                 [("int", "m"), ("int", "n"), (T + "*", "scores"), ("int*", "labels"), (T, "scale"), (T + "*", "dx"), (T + "*", "loss")],
                 "launch_softmax<%s, AlgoNll<%s>>(stream, m, n, scores, %s, dx, labels, scale, loss)" % (T, T, z),
                 "the chain nll -> getindex -> logsoftmax of src/ops20/loss.jl:37-41 (getents/addents + cuDNN LOG backward)")
+    o.decl.append("/* nll(scores, labels; dims=1) of n labels that the host holds (64-bit, 1 ... m): returns the mean loss when it is there and leaves the gradient in dx, in order with the\n"
+                  "   stream's launches.  NaN, dx untouched, if a label is not one of 1 ... m; NaN on an error too.  Cannot be recorded into a graph. */")
+    for T, S in TYPES:
+        o.entry("nll_host_%s" % S, T, [("int", "m"), ("int", "n"), (T + "*", "scores"), ("const long long*", "labels"), (T + "*", "dx")], None,
+                "nll(scores, labels) and its gradient, src/ops20/loss.jl:37-41", body="  return nll_host<%s>(stream, m, n, scores, labels, dx);" % T)
     o.decl.append("\n/* ---- 2-d transpose y(n,m) = x(m,n)' -- CUDA.jl permutedims / cublasSgeam at src/knetarrays/reshape.jl:18, linalg.jl:92-113 ---- */")
     for T, S in TYPES:
         o.entry("transpose_%s" % S, "void", [("int", "m"), ("int", "n"), (T + "*", "x"), (T + "*", "y")],

@@ -47,6 +47,12 @@ template <typename T> constexpr bool kCentered<RedSumSqDev<T>> = true;
 template <typename Op, typename T> __device__ __forceinline__ T red_item(T x, T mu) { return Op::item(kCentered<Op> ? x - mu : x); }
 template <typename Op, typename T> __device__ __forceinline__ T red_finish(T r, const Center<T>& c) { return kCentered<Op> ? r / c.denom : r; }
 
+// A single result may be a word of host memory that the host is looking at: it goes out at once.
+template <typename T> __device__ __forceinline__ void st_result(T* p, T v, bool single) {
+  if (single) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  else *p = v;
+}
+
 template <typename Op, typename T> struct MergeFn {
   __device__ __forceinline__ T operator()(T a, T b) const { return Op::merge(a, b); }
 };
@@ -117,7 +123,7 @@ __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x,
   r = block_reduce<T, NW>(r, lds, MergeFn<Op, T>(), Op::init());
   KNET8_TL_MID
   if (P == 1) {
-    if (threadIdx.x == 0) y[j] = red_finish<Op>(r, center);
+    if (threadIdx.x == 0) st_result(y + j, red_finish<Op>(r, center), ny == 1);
     KNET8_TL_END
     return;
   }
@@ -127,8 +133,8 @@ __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x,
   for (unsigned q = threadIdx.x; q < P; q += BT) s = Op::merge(s, ld_coherent(partial + j * P + q));
   s = block_reduce<T, NW>(s, lds, MergeFn<Op, T>(), Op::init());
   if (threadIdx.x == 0) {
-    y[j] = red_finish<Op>(s, center);
     st_coherent(counters + j * kTicketStride, 0u);
+    st_result(y + j, red_finish<Op>(s, center), ny == 1);
   }
   KNET8_TL_END
 }

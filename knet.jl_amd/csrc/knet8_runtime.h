@@ -55,9 +55,23 @@ inline bool scratch_ready(const Workspace& ws, const char* who) {
   record_error(who);   // the allocation's own failure, recorded first, is the message that is kept
   return false;
 }
-// Device slot for the result of a `_20` reduction on this stream, and the blocking copy that fetches it.
+// Slot for the result of a `_20` reduction on this stream (host memory that the kernel writes), and the wait that fetches it (4 or 8 bytes).
 void* scalar_slot(hipStream_t stream);
-void fetch_scalar(hipStream_t stream, const void* dev, void* host, size_t nbytes);
+void fetch_scalar(hipStream_t stream, const void* slot, void* host, size_t nbytes);
+
+// `n` 4-byte words of page-locked host memory that a kernel can read, for small arrays that go with one launch: fill `host`, queue the launch that reads it, let go.
+// No other thread is given the stream's buffer in between.  host is null where there is none (stream under capture, the per-thread stream, too many words, no memory).
+struct StagedWords {
+  unsigned* host = nullptr;
+  std::unique_lock<std::recursive_mutex> held;
+};
+StagedWords stage_words(hipStream_t stream, size_t n);
+// Copies n words that stand in the stream's staging buffer (staged; the caller still holds them) or anywhere in host memory to the device, in order with the stream's launches.
+bool bring_words(hipStream_t stream, void* dst, const void* src, size_t n, bool staged);
+
+// Blocks of the KnetArray pool (knet8_malloc, knet8_free).
+void* pool_take(size_t nbytes);
+void pool_give(void* p);
 
 // State of the default random stream (knet8_seed): hands out `blocks` consecutive generator counters under the current seed.
 void rng_take(unsigned long long blocks, unsigned long long* seed, unsigned long long* offset);

@@ -10,6 +10,7 @@
 #include <hipblaslt/hipblaslt-version.h>
 
 #include <atomic>
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -262,25 +263,40 @@ static Workspace static_scratch_get(void*, hipStream_t stream, size_t partial_by
 
 // One slot per (host thread, device, stream): two threads that call a `_20` entry point on the same stream (the plain twins all use the
 // null stream; the reference builds with --default-stream per-thread, src/libknet8/build.jl:5) must not read each other's result.
-// 256 bytes each of host memory that kernels can write, kept until the process ends: the result is there when the stream has been waited for, without a copy
-// behind the kernel.
+// 256 bytes each of host memory that kernels can write, kept until the process ends: the result needs no copy behind the kernel, and the host sees it when the
+// kernel has stored it, before the runtime has seen the kernel end (launch and hipStreamSynchronize 11.0 us, launch and a look at the slot until it has changed 5.9).
+// The slot starts from a pattern that no arithmetic makes, as a double and as a float in its first four bytes a signalling NaN.
+constexpr unsigned long long kUnwritten = 0x7ff4a5a57fa5a5a5ull;
 void* scalar_slot(hipStream_t stream) {
   thread_local std::map<std::pair<int, hipStream_t>, void*> slots;
   int dev = 0;
   (void)hipGetDevice(&dev);
   void*& p = slots[std::make_pair(dev, stream)];
-  if (!p && !ok(hipHostMalloc(&p, 256, hipHostMallocDefault), "hipHostMalloc(scalar slot)")) p = nullptr;
+  if (!p && !ok(hipHostMalloc(&p, 256, hipHostMallocCoherent), "hipHostMalloc(scalar slot)")) p = nullptr;
+  if (p) __atomic_store_n(static_cast<unsigned long long*>(p), kUnwritten, __ATOMIC_RELEASE);
   return p;
 }
 
+// Looks for 100 us; then (a long queue before the kernel, a launch that failed, a result that is the pattern itself) the stream is waited for.
 void fetch_scalar(hipStream_t stream, const void* slot, void* host, size_t nbytes) {
-  if (slot && ok(hipStreamSynchronize(stream), "hipStreamSynchronize(scalar)")) memcpy(host, slot, nbytes);
+  if (!slot) return;
+  const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(100);
+  unsigned long long v = kUnwritten;
+  const unsigned long long mask = nbytes == 4 ? 0xffffffffull : ~0ull;
+  do {
+    for (int i = 0; i < 16 && ((v ^ kUnwritten) & mask) == 0; i++) {
+      v = nbytes == 4 ? __atomic_load_n(static_cast<const unsigned*>(slot), __ATOMIC_ACQUIRE) : __atomic_load_n(static_cast<const unsigned long long*>(slot), __ATOMIC_ACQUIRE);
+    }
+  } while (((v ^ kUnwritten) & mask) == 0 && std::chrono::steady_clock::now() < until);
+  if (((v ^ kUnwritten) & mask) != 0) memcpy(host, &v, nbytes);
+  else if (ok(hipStreamSynchronize(stream), "hipStreamSynchronize(scalar)")) memcpy(host, slot, nbytes);
 }
 
 // ---- small uploads ------------------------------------------------------------------------------------------------
 // Index arrays and labels of a step are a few KB, and the launch that reads them follows on the same stream: a copy that the caller waits for costs more
-// (15-20 us) than the launch.  (With this and the slots above, nll and its gradient: 32000x512 fp32 81.9 -> 61.7 us a pass, 1000x4096 fp64 69 -> 50.)  The bytes go into a page-locked buffer of the stream and a kernel brings them over, in order with what follows.  The
-// buffer is used from one end to the other; before it starts again the stream is waited for, so that nothing unread is overwritten.
+// (15-20 us) than the launch.  (With this and the slots above, nll and its gradient: 32000x512 fp32 81.9 -> 61.7 us a pass, 1000x4096 fp64 69 -> 50.)  The bytes go into a page-locked buffer of the stream and a kernel brings them over, in order with what follows,
+// or the kernel that uses them reads them there.  The buffer is used from one end to the other; before it starts again the stream is waited for, so that nothing unread
+// is overwritten.  Who has been given a piece of it keeps the stream's lock until the launch that reads it is queued: no one else can start the buffer again before.
 constexpr size_t kStageBytes = size_t(256) << 10;
 struct Stage { char* host = nullptr; size_t used = 0; };
 static std::mutex g_stage_mutex;
@@ -289,6 +305,38 @@ static std::map<std::pair<int, hipStream_t>, Stage> g_stages;
 __global__ __launch_bounds__(256) void stage_copy_kernel(unsigned* __restrict__ dst, const unsigned* __restrict__ src, unsigned n) {
   const unsigned i = blockIdx.x * 256 + threadIdx.x;
   if (i < n) dst[i] = src[i];
+}
+
+StagedWords stage_words(hipStream_t stream, size_t n) {
+  StagedWords w;
+  const size_t nbytes = 4 * n;
+  // (waiting is an error for a stream under capture; the per-thread stream's one handle stands for another stream in every thread: waiting for this thread's would not
+  //  show that the others have read their part of the buffer)
+  if (n == 0 || nbytes > kStageBytes / 4 || stream == hipStreamPerThread || stream_is_capturing(stream)) return w;
+  auto held = hold_scratch(stream);
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  Stage* s = nullptr;
+  {
+    std::lock_guard<std::mutex> lock(g_stage_mutex);
+    s = &g_stages[std::make_pair(dev, stream)];
+    if (!s->host) {
+      void* p = nullptr;
+      if (g_tune[kTuneFailScratch] != 0 || hipHostMalloc(&p, kStageBytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return w;
+      }
+      s->host = static_cast<char*>(p);
+    }
+  }
+  if (s->used + nbytes > kStageBytes) {
+    if (!ok(hipStreamSynchronize(stream), "hipStreamSynchronize(upload)")) return w;
+    s->used = 0;
+  }
+  w.host = reinterpret_cast<unsigned*>(s->host + s->used);
+  s->used += (nbytes + 255) / 256 * 256;
+  w.held = std::move(held);
+  return w;
 }
 
 // (nothing on the stream may still read the buffer)
@@ -483,33 +531,27 @@ KNET8_API int knet8_memcpy(void* dst, const void* src, size_t nbytes, int kind, 
 }
 
 KNET8_API int knet8_upload(void* dst, const void* src, size_t nbytes, hipStream_t stream) {
-  // larger ones, odd ones, and a stream under capture (where waiting is an error, as it was) take the copy that waits; so does the per-thread stream, whose one
-  // handle stands for another stream in every thread: waiting for this thread's would not show that the others have read their part of the buffer
-  if (stream == hipStreamPerThread || nbytes == 0 || nbytes > kStageBytes / 4 || nbytes % 4 != 0 || reinterpret_cast<uintptr_t>(dst) % 4 != 0 || stream_is_capturing(stream))
-    return knet8_memcpy(dst, src, nbytes, 1, stream);
-  int dev = 0;
-  (void)hipGetDevice(&dev);
-  std::lock_guard<std::mutex> lock(g_stage_mutex);
-  Stage& s = g_stages[std::make_pair(dev, stream)];
-  if (!s.host) {
-    void* p = nullptr;
-    if (g_tune[kTuneFailScratch] != 0 || hipHostMalloc(&p, kStageBytes, hipHostMallocDefault) != hipSuccess) {   // no page-locked memory: the copy needs none
-      (void)hipGetLastError();
-      return knet8_memcpy(dst, src, nbytes, 1, stream);
-    }
-    s.host = static_cast<char*>(p);
-  }
-  if (s.used + nbytes > kStageBytes) {
-    if (!ok(hipStreamSynchronize(stream), "hipStreamSynchronize(upload)")) return -1;
-    s.used = 0;
-  }
-  char* at = s.host + s.used;
-  s.used += (nbytes + 255) / 256 * 256;
-  memcpy(at, src, nbytes);
-  const unsigned n = (unsigned)(nbytes / 4);
-  hipLaunchKernelGGL(stage_copy_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, static_cast<unsigned*>(dst), reinterpret_cast<const unsigned*>(at), n);
-  return ok(hipGetLastError(), "stage_copy_kernel") ? 0 : -1;
+  // odd ones, and those that get no piece of the buffer, take the copy that waits
+  if (nbytes % 4 != 0 || reinterpret_cast<uintptr_t>(dst) % 4 != 0) return knet8_memcpy(dst, src, nbytes, 1, stream);
+  const StagedWords w = stage_words(stream, nbytes / 4);
+  if (!w.host) return knet8_memcpy(dst, src, nbytes, 1, stream);
+  memcpy(w.host, src, nbytes);
+  return bring_words(stream, dst, w.host, nbytes / 4, true) ? 0 : -1;
 }
+
+}  // extern "C"
+
+namespace knet8 {
+bool bring_words(hipStream_t stream, void* dst, const void* src, size_t n, bool staged) {
+  if (!staged) return knet8_memcpy(dst, src, 4 * n, 1, stream) == 0;
+  hipLaunchKernelGGL(stage_copy_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, static_cast<unsigned*>(dst), static_cast<const unsigned*>(src), (unsigned)n);
+  return ok(hipGetLastError(), "stage_copy_kernel");
+}
+void* pool_take(size_t nbytes) { return knet8_malloc(nbytes); }
+void pool_give(void* p) { knet8_free(p); }
+}  // namespace knet8
+
+extern "C" {
 
 KNET8_API int knet8_device_count(void) {
   int n = 0;

@@ -16,6 +16,9 @@
 #pragma once
 #include "knet8_device.h"
 #include "knet8_runtime.h"
+#include "knet8_reduce.h"
+
+#include <vector>
 
 namespace knet8 {
 
@@ -365,9 +368,9 @@ __device__ __forceinline__ void nll_col_body(int m, long n, const T* a, T* out, 
   const int tpos = head + nb * NV + tl;
   const T ninf = T(-INFINITY);
 
-  int lab = colok ? labels[col] : 0;
-  if (lab < 0 || lab > m) lab = 0;  // callers check labels on the host; an out-of-range one is skipped, never dereferenced
-  const T alab = (tl == 0 && lab > 0) ? ac[lab - 1] : T(0);
+  // the label may stand in host memory: one request a column, made before the column's own loads and not waited for until they are under way
+  __shared__ int lds_lab;
+  int lab = colok && (NW == 1 || threadIdx.x < kWave) ? labels[col] : 0;
   V rv[RI];
   // the LDS slots are filled by loads that go from memory to LDS directly (lane t's 16 bytes land at the wave's base + 16 t), no register in between;
   // a slot beyond the lane's share stays unwritten and is never read
@@ -387,6 +390,8 @@ __device__ __forceinline__ void nll_col_body(int m, long n, const T* a, T* out, 
     }
   }
   T xh = hv ? ac[tl] : ninf, xt = tv ? ac[tpos] : ninf;  // -inf padding contributes exp(-inf) = 0
+  if (lab < 0 || lab > m) lab = 0;  // callers check labels on the host; an out-of-range one is skipped, never dereferenced
+  const T alab = (tl == 0 && lab > 0) ? ac[lab - 1] : T(0);
 
   T mt = ninf;
 #pragma unroll
@@ -434,7 +439,9 @@ __device__ __forceinline__ void nll_col_body(int m, long n, const T* a, T* out, 
   if (NW > 1) {
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     if (lane == 0) { lds_m[wave] = ms.m; lds_s[wave] = ms.s; }
+    if (threadIdx.x == 0) lds_lab = lab;
     __syncthreads();
+    lab = lds_lab;
     MaxSum<T> t = {lane < NW ? lds_m[lane] : ninf, lane < NW ? lds_s[lane] : T(0)};
     ms = ms_wave_reduce(t);
   }
@@ -994,6 +1001,14 @@ inline void launch_softmax_cfg(hipStream_t stream, bool vec, int m, long n, cons
   }
 }
 
+// True where columns of m rows go to softmax_short_kernel.  (A matrix too small for sixteen workgroups stays with one wave per column: one launch is 2.8 us
+// there against 3.5 us through LDS.)
+template <typename T, typename Algo>
+inline bool softmax_is_short(long m, long n) {
+  const long resident_cap = tuning(kTuneSoftmaxResidentRows);
+  return m <= (Algo::kNll ? kShortRowsNll : kShortRows) && n >= 64 && n * m >= 16L * 256 * 4 * Vec16<T>::N && !(resident_cap > 0 && m > resident_cap);
+}
+
 template <typename T, typename Algo>
 inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const T* b, T* out, const int* labels, T scale, T* loss) {
   if (m <= 0 || n <= 0) return;
@@ -1013,7 +1028,7 @@ inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const
   const bool vec_stream = (m % N == 0) && ma == 0 && mo == 0 && mb == 0;
   const long resident_cap = tuning(kTuneSoftmaxResidentRows);  // 0: no limit below the register capacity (tests lower it to reach the streaming kernel with short columns)
 #define KNET8_SM(TEAM, E) launch_softmax_cfg<T, Algo, TEAM, E>(stream, vec, (int)m, n, a, b, out, labels, scale, loss)
-  if (m <= (Algo::kNll ? kShortRowsNll : kShortRows) && n >= 64 && !(resident_cap > 0 && m > resident_cap)) {
+  if (softmax_is_short<T, Algo>(m, n)) {
     // stretches of whole columns (see softmax_short_kernel): G columns per workgroup, starting on 16-byte boundaries on the vector path
     constexpr int cap = 256 * short_stretch_vectors<T, Algo>() * N;
     const bool v16 = ma == 0 && mo == 0 && mb == 0;
@@ -1024,8 +1039,7 @@ inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const
         if ((t * m) % N == 0) { step = t; break; }
       G = G / step * step;
     }
-    // (a matrix too small for sixteen workgroups stays with one wave per column: one launch is 2.8 us there against 3.5 us through LDS)
-    if (G >= 1 && n * m >= 16L * 256 * 4 * N) {
+    if (G >= 1) {
       // lanes per column and elements per lane: cheapest passes over the workgroup's G columns, a pass costing its R slots plus about six slots' worth
       // of reductions and bookkeeping (measured: ten classes are faster as 2 lanes x 8 in four passes than as 4 x 3 in seven, and faster still as
       // one lane x 10 in one).  The stretch is cut to a whole number of passes when that costs less per column than a last pass with idle teams.
@@ -1144,6 +1158,48 @@ inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const
   else if (m <= 1024 * (kBig1024 / 2)) KNET8_SM(1024, kBig1024 / 2);
   else KNET8_SM(1024, kBig1024);
 #undef KNET8_SM
+}
+
+// nll of labels that the host holds: loss and gradient of one call (nll_logsoftmax_back_S and the sum over its losses), the labels read where the host left them,
+// the mean handed back as soon as it is there.  NaN, and nothing launched, if a label is not one of 1 ... m.  32000x512 fp32 a pass with a tape around it: 61.2 us as an
+// upload, the kernel, a sum and a wait for the stream, 41.8 so; 1000x4096 fp64 49.3, 38.4.
+// Labels are fetched over the bus, one a column: about 1700 to the us, hidden behind the loads of the columns; up to 4096 that costs no more than the kernel that
+// would bring them over first (3 us and its launch).  The stretches of short columns fetch theirs pass by pass, one wait each: they get a device copy.
+template <typename T>
+inline T nll_host(hipStream_t stream, int m, int n, const T* x, const long long* labels, T* dx) {
+  const T none = T(NAN);
+  if (m <= 0 || n <= 0) return none;
+  bool in = true;
+  for (int i = 0; i < n; i++) in = in && labels[i] >= 1 && labels[i] <= m;
+  if (!in) return none;
+  const T scale = T(1) / T(n);
+  T* const loss = static_cast<T*>(pool_take(sizeof(T) * (size_t)n));
+  int* dlab = nullptr;
+  T total = none;
+  if (loss) {
+    StagedWords w = stage_words(stream, (size_t)n);
+    std::vector<int> own;
+    int* to = reinterpret_cast<int*>(w.host);
+    if (!to) { own.resize(n); to = own.data(); }
+    for (int i = 0; i < n; i++) to[i] = (int)labels[i];
+    const int* from = to;
+    if (!w.host || n > 4096 || softmax_is_short<T, AlgoNll<T>>(m, n)) {
+      dlab = static_cast<int*>(pool_take(4 * (size_t)n));
+      if (!dlab || !bring_words(stream, dlab, to, n, w.host != nullptr)) from = nullptr;
+      else from = dlab;
+    }
+    T* const slot = from ? static_cast<T*>(scalar_slot(stream)) : nullptr;
+    if (slot) {
+      launch_softmax<T, AlgoNll<T>>(stream, m, n, x, (const T*)nullptr, dx, from, scale, loss);
+      const bool launched = launch_reduce_run<T, RedSum<T>>(stream, loss, (long)n, 1, 1, slot);
+      check_launch("nll_host");
+      if (w.held) w.held.unlock();
+      if (launched) fetch_scalar(stream, slot, &total, sizeof(T));
+    }
+  }
+  if (dlab) pool_give(dlab);
+  if (loss) pool_give(loss);
+  return total / T(n);
 }
 
 }  // namespace knet8

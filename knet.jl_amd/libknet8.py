@@ -19,7 +19,7 @@ HEADER_PATH = os.path.join(_ROOT, "include", "knet8.h")
 _CTYPES = {
     "void": None, "int": ctypes.c_int, "unsigned long long": ctypes.c_ulonglong, "long long": ctypes.c_longlong, "float": ctypes.c_float, "double": ctypes.c_double, "char": ctypes.c_char,
     "size_t": ctypes.c_size_t, "hipStream_t": ctypes.c_void_p, "float*": ctypes.c_void_p, "double*": ctypes.c_void_p,
-    "int*": ctypes.c_void_p, "const int*": ctypes.c_void_p, "void*": ctypes.c_void_p, "const void*": ctypes.c_void_p, "size_t*": ctypes.c_void_p, "unsigned long long*": ctypes.c_void_p,
+    "const long long*": ctypes.c_void_p, "int*": ctypes.c_void_p, "const int*": ctypes.c_void_p, "void*": ctypes.c_void_p, "const void*": ctypes.c_void_p, "size_t*": ctypes.c_void_p, "unsigned long long*": ctypes.c_void_p,
     "const char*": ctypes.c_char_p, "float**": ctypes.c_void_p, "double**": ctypes.c_void_p,
 }
 _DECL = re.compile(r"KNET8_API\s+(.+?)\s*\b(\w+)\s*\(([^)]*)\)\s*;")

@@ -6,9 +6,9 @@ Mirrors src/ops20/loss.jl:37-41,116-140 and the device side of ``x[indices]`` an
 """
 import numpy as np
 
-from .autograd import drop, primitive, value
+from .autograd import primitive, value
 from .karray import KnetArray, upload
-from .libknet8 import knet8
+from .libknet8 import knet8, libknet8
 from . import reduction as R
 from .softmax import logsoftmax
 
@@ -124,22 +124,35 @@ def _nll_fused(scores, labels, dims=1, count=None):
     return loss, back
 
 
+@primitive
+def _nll_known(scores, loss, dx):
+    """A loss whose gradient wrt ``scores`` is there already."""
+    def back(dy):
+        from .linalg import scal
+        if float(dy) != 1.0:
+            scal(float(dy), dx)
+        return (dx, None, None)
+    return loss, back
+
+
 def _nll_one_pass(scores, labels, dims):
-    """``nll`` of host labels by ``nll_logsoftmax_back_S`` and one sum: loss and gradient in one read of the scores and one write, where logsoftmax, gather,
-    scatter and logsoftmaxback take seven passes and two uploads of indices (32000x512 fp32: 145 -> 82 us a pass, 62 with ``upload``).  None where the chain has to decide:
-    labels that skip an instance or lie outside the classes, other dims, and scores whose loss is not finite (the chain then says which gradients are NaN)."""
+    """``nll`` of host labels by ``nll_host_S``: loss and gradient in one read of the scores and one write, where logsoftmax, gather, scatter and logsoftmaxback take
+    seven passes and two uploads of indices (32000x512 fp32: 145 us a pass, 42 so).  None where the chain has to decide: labels that skip an instance or lie outside
+    the classes, other dims, and scores whose loss is not finite (the chain then says which gradients are NaN)."""
     x = value(scores)
     if dims != 1 or not isinstance(x, KnetArray) or x.suffix is None or x.ndims < 1 or isinstance(labels, KnetArray):
         return None
     lab = np.asarray(labels)
-    m = x.size(1)
-    if not np.issubdtype(lab.dtype, np.integer) or lab.size == 0 or lab.size * m != x.length or lab.min() < 1 or lab.max() > m:
+    m, n = x.size(1), lab.size
+    if lab.dtype.kind not in "iu" or n == 0 or n * m != x.length:
         return None
-    loss = _nll_fused(scores, lab)
-    if np.isfinite(value(loss)):
-        return loss
-    drop(loss)
-    return None
+    if lab.dtype != np.int64 or not lab.flags.f_contiguous:
+        lab = np.asarray(lab.ravel(order="F"), dtype=np.int64)   # (an unsigned number beyond 2^63 turns negative, which is no class either)
+    dx = x.similar()
+    lib = libknet8()
+    loss = x.dtype.type(lib.call("nll_host_%s" % x.suffix, m, n, x.ptr, lab.ctypes.data, dx.ptr))
+    lib.check()
+    return _nll_known(scores, loss, dx) if np.isfinite(loss) else None
 
 
 def _over_data(fn, model, data, dims, average, kw):
@@ -165,12 +178,12 @@ def nll(scores, labels=None, dims=1, average=True, fused=False, count=None, data
         raise TypeError("MethodError: nll got unexpected keyword arguments %r" % sorted(kw))
     if isinstance(labels, KnetArray) and not fused:
         raise TypeError("MethodError: nll takes host labels (an integer array), as in the reference; device labels need fused=True")
-    if fused and average:
-        return _nll_fused(scores, labels, dims=dims, count=count)
     if average:
         one = _nll_one_pass(scores, labels, dims)
         if one is not None:
             return one
+        if fused:
+            return _nll_fused(scores, labels, dims=dims, count=count)
     indices = findindices(value(scores), labels, dims=dims)
     lp = getindex(logsoftmax(scores, dims=dims), indices)
     n = len(indices)

@@ -30,9 +30,11 @@ def _check(*arrays):
 
 def unary_op(name, x):
     """``y = similar(x); @knet8(F_S, (Cint,Ptr,Ptr), length(y), x, y)`` (src/ops20_gpu/activation.jl:20-24)."""
-    _check(x)
+    S = x.suffix if isinstance(x, KnetArray) else None
+    if S is None:
+        _check(x)
     y = x.similar()
-    knet8("%s_%s" % (name, x.suffix), x.length, x.ptr, y.ptr)
+    knet8("%s_%s" % (name, S), x.length, x.ptr, y.ptr)
     return y
 
 
@@ -47,7 +49,8 @@ def unary_op_with_degree(name, d, x):
 
 def back11_op(name, dy, y):
     """``z = similar(x); @knet8(Fback_S_11, ..., length(z), dy, y, z)`` (src/ops20_gpu/activation.jl:33-37)."""
-    _check(dy, y)
+    if not (isinstance(dy, KnetArray) and isinstance(y, KnetArray) and dy.dtype == y.dtype and dy.length == y.length and dy.suffix):
+        _check(dy, y)
     dx = dy.similar()
     knet8("%s_%s_11" % (name, dy.suffix), dx.length, dy.ptr, y.ptr, dx.ptr)
     return dx
@@ -101,17 +104,17 @@ def _activation(name, back):
     @primitive
     def f(x):
         y = unary_op(name, x)
-        return y, (lambda dy: (back(dy, y),))  # @primitive relu(x),dy,y reluback.(dy,y)  (src/ops20/activation.jl:28)
+        return y, (lambda dy: (back11_op(back, dy, y),))  # @primitive relu(x),dy,y reluback.(dy,y)  (src/ops20/activation.jl:28)
 
     f.__name__ = name
     return f
 
 
-relu = _activation("relu", reluback)
-sigm = _activation("sigm", sigmback)
-tanh = _activation("tanh", tanhback)
-elu = _activation("elu", eluback)
-selu = _activation("selu", seluback)
+relu = _activation("relu", "reluback")
+sigm = _activation("sigm", "sigmback")
+tanh = _activation("tanh", "tanhback")
+elu = _activation("elu", "eluback")
+selu = _activation("selu", "seluback")
 
 
 # ---- ops21: f(x) and fback(x,y,dy) ----------------------------------------------------------------------

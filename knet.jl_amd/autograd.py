@@ -75,14 +75,22 @@ def primitive(fwd):
     None) per positional argument; the wrapper records a node when any argument is tracked."""
 
     def wrapper(*args, **kw):
-        nodes = [track(a) for a in args]
-        vals = [value(a) for a in args]
-        if _TAPE is None or all(n is None for n in nodes):
-            out = fwd(*vals, **kw)
-            return out[0]
+        tape = _TAPE
+        nodes, vals, tracked = [], [], False
+        for a in args:
+            if isinstance(a, _HOLDERS):
+                n = None if isinstance(a, Result) else a if isinstance(a, Node) else None if tape is None else tape.leaf(a)
+                tracked = tracked or n is not None
+                nodes.append(n)
+                vals.append(a.value)
+            else:
+                nodes.append(None)
+                vals.append(a)
         y, back = fwd(*vals, **kw)
-        node = Node(y, tuple(nodes), back)
-        _TAPE.nodes.append(node)
+        if tape is None or not tracked:
+            return y
+        node = Node(y, nodes, back)
+        tape.nodes.append(node)
         return node
 
     wrapper.__name__ = getattr(fwd, "__name__", "primitive")
@@ -114,6 +122,9 @@ class Result:
         self.value, self.grads, self.params = value, grads, tuple(params)   # params: in order of first use (AutoGrad's params(J))
 
 
+_HOLDERS = (Node, Param, Result)
+
+
 def diff(f):
     global _TAPE
     if _TAPE is not None:
@@ -138,12 +149,12 @@ def diff(f):
         if getattr(node.back, "selective", False):
             # like AutoGrad, which evaluates a primitive's gradient expression only for the arguments that are tracked:
             # the input layer's product never computes the gradient wrt the data, a constant operand of .* is not summed
-            grads = node.back(node.outgrad, tuple(p is not None for p in node.parents))
+            grads = node.back(node.outgrad, [p is not None for p in node.parents])
         else:
             grads = node.back(node.outgrad)
         for parent, g in zip(node.parents, grads):
             if parent is not None and g is not None:
-                parent.outgrad = addto(parent.outgrad, g)
+                parent.outgrad = g if parent.outgrad is None else addto(parent.outgrad, g)
         if node.param is None:
             # Dead from here on: drop the gradient, the value and the closure that holds the saved activations, so their
             # device blocks go back to the pool while the sweep is still running -- what the reference's tape-aware

@@ -9,28 +9,29 @@ operand had size 1 and the result did not, then reshape to the operand's size.
 import numpy as np
 
 from .autograd import primitive, selective
-from .karray import KnetArray
+from .karray import KnetArray, number
 from .libknet8 import knet8
 from .reduction import sum as ksum
 
 def _scalar_array(name, s, y, scalar_first=True):
     z = y.similar()
-    c = y.ctype
+    if name != "sub" or scalar_first:
+        s = number(y, s)
     if scalar_first:
-        knet8("%s_%s_01" % (name, y.suffix), z.length, c(s), y.ptr, z.ptr)
+        knet8("%s_%s_01" % (name, y.suffix), z.length, s, y.ptr, z.ptr)
         return z
     # array (op) scalar: commutative ops reuse _01; a-s = a+(-s); comparisons swap sides (a>s is s<a); a/s = a*(1/s) is NOT
     # used (different rounding): div and pow fill a temporary with the scalar and go through _11
     swap = {"gt": "lt", "lt": "gt", "ge": "le", "le": "ge"}
     if name in ("add", "mul", "max", "min", "eq", "ne"):
-        knet8("%s_%s_01" % (name, y.suffix), z.length, c(s), y.ptr, z.ptr)
+        knet8("%s_%s_01" % (name, y.suffix), z.length, s, y.ptr, z.ptr)
     elif name in swap:
-        knet8("%s_%s_01" % (swap[name], y.suffix), z.length, c(s), y.ptr, z.ptr)
+        knet8("%s_%s_01" % (swap[name], y.suffix), z.length, s, y.ptr, z.ptr)
     elif name == "sub":
-        knet8("add_%s_01" % y.suffix, z.length, c(-s), y.ptr, z.ptr)
+        knet8("add_%s_01" % y.suffix, z.length, number(y, -s), y.ptr, z.ptr)
     else:
         t = y.similar()
-        knet8("fill_%s" % y.suffix, t.length, c(s), t.ptr)
+        knet8("fill_%s" % y.suffix, t.length, s, t.ptr)
         knet8("%s_%s_11" % (name, y.suffix), z.length, y.ptr, t.ptr, z.ptr)
     return z
 
@@ -59,7 +60,16 @@ def broadcast_op(name, x, y):
         return _scalar_array(name, y, x, False)
     if x.dtype != y.dtype:
         raise TypeError("MethodError: element types differ")
-    if x.dims == y.dims or (x.length == y.length and _squeeze(x.dims) == _squeeze(y.dims)):
+    xd, yd = x.dims, y.dims
+    if xd == yd:
+        z = x.similar()
+        knet8("%s_%s_11" % (name, x.suffix), z.length, x.ptr, y.ptr, z.ptr)
+        return z
+    if len(xd) == 2 and len(yd) == 2 and yd[1] == 1 and yd[0] == xd[0] != 1 and xd[1] > 1:   # a bias: a vector along the first dimension of a matrix
+        z = x.similar()
+        knet8("%s_%s_12" % (name, x.suffix), z.length, x.ptr, 1, x.length, y.ptr, 1, yd[0], z.ptr)
+        return z
+    if (x.length == y.length and _squeeze(x.dims) == _squeeze(y.dims)):
         z = x.similar(x.dims if len(x.dims) >= len(y.dims) else y.dims)
         knet8("%s_%s_11" % (name, x.suffix), z.length, x.ptr, y.ptr, z.ptr)
         return z
@@ -142,13 +152,16 @@ def unbroadcast(x, dx):
         return ksum(dx) if isinstance(dx, KnetArray) else dx  # x is a Number: sum(dx)
     if not isinstance(dx, KnetArray):
         return dx
+    if x.dims == dx.dims:
+        return dx
     nd = max(x.ndims, dx.ndims)
     xs = tuple(x.dims) + (1,) * (nd - x.ndims)
     ds = tuple(dx.dims) + (1,) * (nd - dx.ndims)
     if xs == ds:
         return dx
     d = [i + 1 for i in range(nd) if xs[i] == 1 and ds[i] > 1]
-    return ksum(dx, dims=d[0] if len(d) == 1 else d).reshape(x.dims)
+    g = ksum(dx, dims=d[0] if len(d) == 1 else d)
+    return g if g.dims == x.dims else g.reshape(x.dims)
 
 
 def _neg(a):
@@ -189,7 +202,7 @@ def div(x, y):
 
 def fill(x, v):
     """``fill!(x, v)`` (src/knetarrays/abstractarray.jl:13 -> ``fill_S``)."""
-    knet8("fill_%s" % x.suffix, x.length, x.ctype(v), x.ptr)
+    knet8("fill_%s" % x.suffix, x.length, number(x, v), x.ptr)
     return x
 
 

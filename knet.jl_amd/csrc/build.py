@@ -17,6 +17,8 @@ LIB = os.path.join(PKG, "lib", "libknet8.so")
 # The measurement build: the same sources with -DKNET8_TIMELINE, whose gradient kernels stamp the wall clock per workgroup
 # (`bench.py --timeline`).  Never loaded by the package unless KNET8_LIBRARY names it.
 LIB_TIMELINE = os.path.join(PKG, "lib", "libknet8_timeline.so")
+# The host mirror's native part: a CPython module (knet8_host.c and the generated calls), compiled by the host compiler.
+HOST = os.path.join(PKG, "lib", "_knet8_host.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["-O3", "--offload-arch=gfx950", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-ffp-contract=off", "-fno-fast-math",
@@ -28,7 +30,7 @@ def source_id():
     included).  build() bakes it into the library (knet8_build_id()); the loader compares the two and refuses a stale binary."""
     import hashlib
     h = hashlib.sha256()
-    names = sorted(f for f in os.listdir(HERE) if f.endswith((".h", ".hip")) or f in ("gen_knet8.py", "build.py"))
+    names = sorted(f for f in os.listdir(HERE) if f.endswith((".h", ".hip", ".c")) or f in ("gen_knet8.py", "build.py"))
     for name in names:
         h.update(name.encode())
         with open(os.path.join(HERE, name), "rb") as f:
@@ -56,11 +58,24 @@ def compile_one(job):
     return obj, out
 
 
+def build_host():
+    import sysconfig
+    cmd = [os.environ.get("CC", "gcc"), "-O2", "-std=gnu11", "-Wall", "-shared", "-fPIC", "-fvisibility=hidden", "-DKNET8_BUILD_ID=\"%s\"" % source_id(),
+           "-I" + sysconfig.get_paths()["include"], "-I" + HERE, os.path.join(HERE, "knet8_host.c"), "-o", HOST]
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("compiling knet8_host.c failed:\n" + r.stdout)
+    return r.stdout
+
+
 def build(verbose=False, timeline=True):
     """Compile and link libknet8.so and (timeline=True) the measurement build libknet8_timeline.so.  Returns the path of the former."""
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(os.path.dirname(LIB), exist_ok=True)
     srcs = sources()
+    host = build_host()
+    if verbose and host.strip():
+        print(host)
     jobs = [(s, False) for s in srcs] + ([(s, True) for s in srcs] if timeline else [])
     with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(jobs))) as ex:
         results = list(ex.map(compile_one, jobs))

@@ -739,6 +739,29 @@ HEADER_BOTTOM = """
 """
 
 
+# C types of the header as one letter each (and the member of Value in knet8_host.c that holds them); pointers are p
+CALL_LETTERS = {"void": "v", "int": "i", "unsigned long long": "u", "size_t": "u", "long long": "l", "float": "f", "double": "d", "char": "c"}
+
+
+def gen_calls(header):
+    """One call per distinct signature of the header's _stream entry points, for the native host layer."""
+    import re
+    ctype = {"v": "void", "i": "int", "u": "unsigned long long", "l": "long long", "f": "float", "d": "double", "c": "char", "p": "void*"}
+    text = re.sub(r"/\*.*?\*/", "", header, flags=re.S)
+    found = set()
+    for ret, name, params in re.findall(r"KNET8_API\s+(.+?)\s*\b(\w+)\s*\(([^)]*)\)\s*;", text):
+        if name.endswith("_stream") and ret.strip() in CALL_LETTERS:
+            found.add(CALL_LETTERS[ret.strip()] + "".join(CALL_LETTERS.get(p.strip().rsplit(" ", 1)[0].strip(), "p") for p in params.split(",")))
+    sigs = sorted(found)
+    out = ["/* Generated by gen_knet8.py: do not edit.  Return type and arguments of the entry points, one letter each, and a call for every combination. */",
+           "static const char* const kSignatures[] = {%s};" % ", ".join('"%s"' % s for s in sigs),
+           "static void invoke(int sig, void* fn, const Value* a, Value* r) {", "  switch (sig) {"]
+    for k, s in enumerate(sigs):
+        call = "((%s (*)(%s))fn)(%s)" % (ctype[s[0]], ", ".join(ctype[c] for c in s[1:]), ", ".join("a[%d].%s" % (i, c) for i, c in enumerate(s[1:])))
+        out.append("    case %d: %s%s; break;" % (k, "" if s[0] == "v" else "r->%s = " % s[0], call))
+    return "\n".join(out + ["    default: break;", "  }", "}", ""])
+
+
 def generate(write=True):
     units = {"knet8_elementwise_gen.hip": gen_elementwise(), "knet8_broadcast_gen.hip": gen_broadcast(), "knet8_reduce_gen.hip": gen_reduce(), "knet8_softmax_gen.hip": gen_softmax()}
     files = {}
@@ -746,6 +769,7 @@ def generate(write=True):
         files[os.path.join(GEN, fn)] = "\n".join(o.src) + "\n"
     header = HEADER_TOP + "\n".join("\n".join(o.decl) for o in units.values()) + "\n" + HEADER_RUNTIME + HEADER_BOTTOM
     files[HEADER] = header
+    files[os.path.join(GEN, "knet8_calls_gen.h")] = gen_calls(header)
     if write:
         os.makedirs(GEN, exist_ok=True)
         os.makedirs(os.path.dirname(HEADER), exist_ok=True)

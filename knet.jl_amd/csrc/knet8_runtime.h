@@ -66,6 +66,7 @@ struct StagedWords {
   std::unique_lock<std::recursive_mutex> held;
 };
 StagedWords stage_words(hipStream_t stream, size_t n);
+bool stream_is_capturing(hipStream_t stream);
 // Copies n words that stand in the stream's staging buffer (staged; the caller still holds them) or anywhere in host memory to the device, in order with the stream's launches.
 bool bring_words(hipStream_t stream, void* dst, const void* src, size_t n, bool staged);
 

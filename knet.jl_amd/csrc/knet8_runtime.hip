@@ -122,7 +122,7 @@ static StreamScratch& scratch_of(hipStream_t stream) {
   return g_scratch[std::make_pair(dev, stream)];
 }
 
-static bool stream_is_capturing(hipStream_t stream) {
+bool stream_is_capturing(hipStream_t stream) {
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (stream == nullptr || hipStreamIsCapturing(stream, &cap) != hipSuccess) {
     (void)hipGetLastError();

@@ -1172,6 +1172,7 @@ inline T nll_host(hipStream_t stream, int m, int n, const T* x, const long long*
   bool in = true;
   for (int i = 0; i < n; i++) in = in && labels[i] >= 1 && labels[i] <= m;
   if (!in) return none;
+  if (stream_is_capturing(stream)) { record_error("nll: labels in host memory cannot be recorded into a graph"); return none; }
   const T scale = T(1) / T(n);
   T* const loss = static_cast<T*>(pool_take(sizeof(T) * (size_t)n));
   int* dlab = nullptr;

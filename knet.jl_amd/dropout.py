@@ -9,19 +9,19 @@ the CPU path.
 import numpy as np
 
 from .autograd import primitive, recording
-from .karray import KnetArray
+from .karray import KnetArray, number
 from .libknet8 import knet8
 
 
 def dropout_(p, x, y):
     """``dropout!(p, x, y)``: ``y`` holds U[0,1) on entry and the result on return (in place)."""
-    knet8("dropout_%s" % x.suffix, y.length, x.ctype(p), x.ptr, y.ptr)
+    knet8("dropout_%s" % x.suffix, y.length, number(x, p), x.ptr, y.ptr)
     return y
 
 
 def dropback_(p, x, y, dy, dx):
     """``dropback!(p, x, y, dy, dx)``."""
-    knet8("dropback_%s" % x.suffix, dx.length, x.ctype(p), x.ptr, y.ptr, dy.ptr, dx.ptr)
+    knet8("dropback_%s" % x.suffix, dx.length, number(x, p), x.ptr, y.ptr, dy.ptr, dx.ptr)
     return dx
 
 

@@ -13,7 +13,7 @@ import ctypes
 import numpy as np
 
 from .autograd import primitive
-from .karray import KnetArray, upload
+from .karray import KnetArray, upload, number
 from .libknet8 import knet8, libknet8
 
 
@@ -71,7 +71,7 @@ def _put(kind, mode, x, y, i):
             raise TypeError("MethodError: add%s needs an array" % kind)
         if idx.size:
             d = upload(idx)
-            knet8("set%s1_%s" % (kind[:-1], x.suffix), xrows, xcols, idx.size, d.ptr, x.ptr, x.ctype(y))
+            knet8("set%s1_%s" % (kind[:-1], x.suffix), xrows, xcols, idx.size, d.ptr, x.ptr, number(x, y))
     return x
 
 
@@ -97,7 +97,7 @@ def addrows_(x, y, i):
 
 def _zeros_like(x):
     z = x.similar()
-    knet8("fill_%s" % x.suffix, z.length, x.ctype(0), z.ptr)
+    knet8("fill_%s" % x.suffix, z.length, 0, z.ptr)
     return z
 
 
@@ -134,7 +134,7 @@ def setents_(x, y, i):
             raise ValueError("DimensionMismatch")
         knet8("setents_%s" % x.suffix, idx.size, d.ptr, x.ptr, y.ptr)
     else:
-        knet8("setent1_%s" % x.suffix, idx.size, d.ptr, x.ptr, x.ctype(y))
+        knet8("setent1_%s" % x.suffix, idx.size, d.ptr, x.ptr, number(x, y))
     return x
 
 
@@ -206,9 +206,9 @@ def setindex2_(A, B, I1, I2):
         if nelts == 0:
             return A
         if ncols == 1:
-            knet8("fill_%s" % A.suffix, nelts, A.ctype(B), aptr)
+            knet8("fill_%s" % A.suffix, nelts, number(A, B), aptr)
         else:
-            knet8("xfill_%s" % A.suffix, nrows, ncols, A.ctype(B), aptr, astep)
+            knet8("xfill_%s" % A.suffix, nrows, ncols, number(A, B), aptr, astep)
         return A
     if B.length != nelts:
         raise ValueError("DimensionMismatch")
@@ -425,14 +425,14 @@ def _put_planned(A, v, kind, payload, rdims, A2, add=False):
             if v.length != n:
                 raise ValueError("DimensionMismatch")
             if add:
-                knet8("axpy_%s" % A.suffix, n, A.ctype(1), v.ptr, dst.ptr)
+                knet8("axpy_%s" % A.suffix, n, number(A, 1), v.ptr, dst.ptr)
             else:
                 libknet8().fn["knet8_memcpy"](dst.ptr, v.ptr, n * A.dtype.itemsize, 3, libknet8().stream)
         else:
             if add:
-                knet8("add_%s_01" % A.suffix, n, A.ctype(v), dst.ptr, dst.ptr)
+                knet8("add_%s_01" % A.suffix, n, number(A, v), dst.ptr, dst.ptr)
             else:
-                knet8("fill_%s" % A.suffix, n, A.ctype(v), dst.ptr)
+                knet8("fill_%s" % A.suffix, n, number(A, v), dst.ptr)
         return A
     if kind == "ents":
         if payload.size == 0:

@@ -9,138 +9,66 @@ import ctypes
 
 import numpy as np
 
-from .libknet8 import libknet8
+from .libknet8 import host, libknet8
 
-_SUFFIX = {np.dtype(np.float32): "32", np.dtype(np.float64): "64"}
-
-# While a launch sequence is being captured into a graph, device blocks released by the garbage collector must not go
-# back to the pool: the graph keeps using their addresses.  capture() parks them here and the Graph object owns them.
-_PARKED = None
+KnetPtr = host.KnetPtr   # owner of one device allocation; a block of a borrowed address if `keep` is given
 
 
-class KnetPtr:
-    """Owner of one device allocation (src/knetarrays/kptr.jl:10-15)."""
+class KnetArray(host.ArrayBase):
+    """Dense column-major device array.  ``KnetArray(np_array)`` copies to the device, ``Array(k)`` back.
 
-    __slots__ = ("ptr", "nbytes", "_keep", "__weakref__")
-
-    def __init__(self, nbytes=None, ptr=None, keep=None):
-        if ptr is not None:  # borrowed memory (e.g. a torch tensor kept alive through `keep`)
-            self.ptr, self.nbytes, self._keep = int(ptr), nbytes, keep
-            return
-        lib = libknet8()
-        p = lib.fn["knet8_malloc"](max(int(nbytes), 1))
-        if not p:
-            lib.check()
-            raise MemoryError("Out of gpu memory")  # the reference's message, kptr.jl:141
-        self.ptr, self.nbytes, self._keep = int(p), int(nbytes), None
-
-    def __del__(self):
-        if self._keep is None and self.ptr:
-            if _PARKED is not None:
-                _PARKED.append(self.ptr)
-                self.ptr = 0
-                return
-            try:
-                libknet8().fn["knet8_free"](self.ptr)
-            except Exception:
-                pass
-            self.ptr = 0
-
-
-class KnetArray:
-    """Dense column-major device array.  ``KnetArray(np_array)`` copies to the device, ``Array(k)`` back."""
+    The native base holds ``kptr, dims, dtype, offset`` and gives ``ptr, length, ndims, suffix, size, stride, similar``."""
 
     __array_priority__ = 1000
 
     def __init__(self, data=None, dtype=None, dims=None, _ptr=None, _offset=0):
         if _ptr is not None:
-            self.kptr, self.dims, self.dtype, self.offset = _ptr, tuple(int(d) for d in dims), np.dtype(dtype), int(_offset)
+            self._init(_ptr, dims, dtype, int(_offset))
             return
         if data is None:
-            self.dtype = np.dtype(dtype if dtype is not None else np.float32)
-            self.dims = tuple(int(d) for d in dims)
-            self.kptr = KnetPtr(self.length * self.dtype.itemsize)
-            self.offset = 0
+            self._init(None, dims, dtype if dtype is not None else np.float32)
             return
         a = np.asarray(data, dtype=dtype)
         if a.dtype not in (np.float32, np.float64, np.int32):
             raise TypeError("KnetArray supports Float32, Float64 and Int32 elements, got %s" % a.dtype)
-        self.dtype = a.dtype
-        self.dims = tuple(a.shape)
-        self.kptr = KnetPtr(a.size * a.itemsize)
-        self.offset = 0
+        self._init(None, a.shape, a.dtype)
         flat = np.ascontiguousarray(a.ravel(order="F"))
         lib = libknet8()
         lib.fn["knet8_memcpy"](self.ptr, flat.ctypes.data, flat.nbytes, 1, lib.stream)
         lib.check()
 
-    # -- Julia-style queries -------------------------------------------------------------------------
-    @property
-    def ptr(self):
-        return self.kptr.ptr + self.offset
-
-    @property
-    def length(self):
-        n = 1
-        for d in self.dims:
-            n *= d
-        return n
-
-    @property
-    def ndims(self):
-        return len(self.dims)
-
-    def size(self, i=None):
-        if i is None:
-            return self.dims
-        return self.dims[i - 1] if i <= len(self.dims) else 1
-
-    def stride(self, i):
-        s = 1
-        for d in self.dims[: i - 1]:
-            s *= d
-        return s
-
-    @property
-    def suffix(self):
-        return _SUFFIX.get(self.dtype)
-
     @property
     def ctype(self):
         return ctypes.c_float if self.dtype == np.float32 else ctypes.c_double
 
+    def __copy__(self):
+        return self._view(self.dims, self.offset)
+
     def __repr__(self):
         return "KnetArray{%s,%d}%r" % (self.dtype.name, self.ndims, self.dims)
-
-    # -- construction helpers -------------------------------------------------------------------------
-    def similar(self, dims=None, dtype=None):
-        """``similar(x, dims)`` (src/knetarrays/abstractarray.jl:13-35): uninitialised array of the same kind."""
-        return KnetArray(dtype=dtype or self.dtype, dims=self.dims if dims is None else dims)
 
     def reshape(self, *dims):
         """Shares the pointer (src/knetarrays/reshape.jl:3-11); one dim may be -1 (Julia's ``:``)."""
         if len(dims) == 1 and isinstance(dims[0], (tuple, list)):
-            dims = tuple(dims[0])
-        dims = list(dims)
+            dims = dims[0]
         if -1 in dims:
+            dims = list(dims)
             k = dims.index(-1)
             rest = 1
             for i, d in enumerate(dims):
                 if i != k:
                     rest *= d
             dims[k] = self.length // rest if rest else 0
-        n = 1
-        for d in dims:
-            n *= d
-        if n != self.length:
+        y = self._view(dims)
+        if y.length != self.length:
             raise ValueError("DimensionMismatch: new dimensions %r must be consistent with array size %d" % (tuple(dims), self.length))
-        return KnetArray(dtype=self.dtype, dims=dims, _ptr=self.kptr, _offset=self.offset)
+        return y
 
     def view1d(self, start, n):
         """Contiguous sub-array of ``n`` elements starting at 0-based linear index ``start`` (shares memory)."""
         if start < 0 or start + n > self.length:
             raise IndexError("BoundsError")
-        return KnetArray(dtype=self.dtype, dims=(n,), _ptr=self.kptr, _offset=self.offset + start * self.dtype.itemsize)
+        return self._view((n,), self.offset + start * self.dtype.itemsize)
 
     @classmethod
     def from_torch(cls, t, dims=None):
@@ -168,6 +96,14 @@ class KnetArray:
         return y
 
     # -- operators: defined in ops20 / binary and attached there --------------------------------------
+
+
+host.array_type(KnetArray)
+
+
+def number(x, v):
+    """``v`` as an argument of the element type of ``x``: numbers as they are, anything else as ctypes converts or refuses it."""
+    return v if isinstance(v, (float, int, np.floating)) else x.ctype(v)
 
 
 def Array(x):
@@ -244,7 +180,6 @@ def capture(fn):
     """Run ``fn()`` once eagerly (so that pool blocks, reduction scratch and GEMM plans exist), then once more under
     stream capture, and return a ``Graph``.  ``fn`` must not synchronise with the host (no ``Array(x)``, no ``dims=:``
     reductions, no host labels): it may only enqueue work."""
-    global _PARKED
     lib = libknet8()
     if lib.stream is None:
         # Capture needs a stream of its own.  Work already queued on the null stream (fills, copies and random draws that built the
@@ -255,16 +190,19 @@ def capture(fn):
         lib.stream = capture_stream()
     # Warm-up under the same parking rule as the capture itself, so that the pool ends up holding one block for every
     # allocation of the sequence (blocks freed while parked are not recycled within the run).
-    warm = _PARKED = []
+    warm = []
+    host.park(warm)
     try:
         fn()
     finally:
-        _PARKED = None
+        host.park(None)
     lib.fn["knet8_synchronize"](lib.stream)
     for p in warm:
         lib.fn["knet8_free"](p)
     lib.check()
-    parked = _PARKED = []
+    parked = []
+    # While the sequence is being captured, blocks that are released must not go back to the pool: the graph keeps using their addresses, and owns them.
+    host.park(parked)
     try:
         if lib.fn["knet8_graph_begin"](lib.stream) != 0:
             lib.check()
@@ -273,7 +211,7 @@ def capture(fn):
         finally:
             handle = lib.fn["knet8_graph_end"](lib.stream)
     finally:
-        _PARKED = None
+        host.park(None)
     if not handle:
         lib.check()
         raise RuntimeError("graph capture failed")

@@ -6,14 +6,21 @@ calls the ``<fun>_stream`` entry point with the current stream appended.  Argume
 ``include/knet8.h`` so the Python side cannot drift from the header.
 
 There is no CPU fallback: if the library is missing or a symbol is absent, loading fails with an error.
+
+The calls themselves, the arrays and their blocks are objects of a native module beside the library (``csrc/knet8_host.c``): a call converts its arguments
+by the signature in the header, which ctypes and Python classes did at 2 to 5 times the cost of the launch.  The 784-64-10 training step takes 95 us so, 172 with them.
 """
 import ctypes
+import importlib.util
 import os
 import re
+
+import numpy as np
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 _ROOT = os.path.dirname(_PKG)
 LIB_PATH = os.environ.get("KNET8_LIBRARY", os.path.join(_PKG, "lib", "libknet8.so"))
+HOST_PATH = os.path.join(_PKG, "lib", "_knet8_host.so")
 HEADER_PATH = os.path.join(_ROOT, "include", "knet8.h")
 
 _CTYPES = {
@@ -56,7 +63,23 @@ def source_build_id():
     return mod.source_id()
 
 
-class LibKnet8:
+def _load_host():
+    if not os.path.exists(HOST_PATH):
+        raise OSError("_knet8_host.so not found at %s -- build it first (python __graft_entry__.py build)" % HOST_PATH)
+    spec = importlib.util.spec_from_file_location("_knet8_host", HOST_PATH)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+host = _load_host()
+knet8 = host.knet8   # knet8(fun, *args): call() of the library that libknet8() loaded
+
+# the letters of csrc/gen/knet8_calls_gen.h; pointers are p
+_LETTERS = {"void": "v", "int": "i", "unsigned long long": "u", "size_t": "u", "long long": "l", "float": "f", "double": "d", "char": "c"}
+
+
+class LibKnet8(host.Library):
     def __init__(self, path=LIB_PATH):
         if not os.path.exists(path):
             raise OSError("libknet8.so not found at %s -- build it first (python __graft_entry__.py build); "
@@ -70,33 +93,39 @@ class LibKnet8:
             f.restype = _CTYPES[ret]
             f.argtypes = [_CTYPES[a] for a in args]
             self.fn[name] = f
+            if name.endswith("_stream"):
+                self._bind(name[:-len("_stream")], ctypes.cast(f, ctypes.c_void_p).value, _LETTERS.get(ret, "?") + "".join(_LETTERS.get(a, "p") for a in args))
         self.stream = None  # current stream handle (None = null stream), cf. CUDA.stream() in the reference
         self.build_id = self.fn["knet8_build_id"]().decode()
         want = source_build_id()
-        if want is not None and want != self.build_id and not os.environ.get("KNET8_ALLOW_STALE"):
-            raise OSError("libknet8.so at %s was built from other sources (library %s, working tree %s): rebuild it "
-                          "(python __graft_entry__.py build)" % (path, self.build_id, want))
+        for what, got in ((path, self.build_id), (HOST_PATH, host.build_id)):
+            if want is not None and want != got and not os.environ.get("KNET8_ALLOW_STALE"):
+                raise OSError("%s was built from other sources (library %s, working tree %s): rebuild it "
+                              "(python __graft_entry__.py build)" % (what, got, want))
 
     def check(self):
         msg = self.fn["knet8_last_error"]()
         if msg:
             raise RuntimeError("libknet8: " + msg.decode())
 
-    def call(self, fun, *args):
-        """``@knet8(fun, ...)``: asynchronous launch of ``<fun>_stream`` on the current stream."""
-        r = self.fn[fun + "_stream"](*args, self.stream)
-        return r
+    def slow_call(self, fun, *args):
+        """What ``call`` leaves: arguments that ctypes has to convert, or to refuse."""
+        return self.fn[fun + "_stream"](*args, self.stream)
 
 
 _LIB = None
 
 
+def _out_of_memory():
+    libknet8().check()
+    raise MemoryError("Out of gpu memory")  # the reference's message, src/knetarrays/kptr.jl:141
+
+
 def libknet8():
     global _LIB
     if _LIB is None:
-        _LIB = LibKnet8()
+        lib = LibKnet8()
+        address = lambda name: ctypes.cast(lib.fn[name], ctypes.c_void_p).value  # noqa: E731
+        host.setup(address("knet8_malloc"), address("knet8_free"), _out_of_memory, np.dtype, tuple(np.dtype(t) for t in (np.float32, np.float64, np.int32)), lib)
+        _LIB = lib
     return _LIB
-
-
-def knet8(fun, *args):
-    return libknet8().call(fun, *args)

@@ -7,7 +7,7 @@ and ``scal!`` (``:75-90``).
 import numpy as np
 
 from .autograd import primitive, selective
-from .karray import KnetArray
+from .karray import KnetArray, number
 from .libknet8 import knet8, libknet8
 
 
@@ -27,24 +27,43 @@ def gemm(transA, transB, alpha, A, B, beta, C):
         raise ValueError("DimensionMismatch: %r" % ((A.dims, B.dims, C.dims),))
     if A.dtype != B.dtype or A.dtype != C.dtype:
         raise TypeError("MethodError: element types differ")
-    c = A.ctype
+    return _gemm(transA.encode(), transB.encode(), alpha, A, B, beta, C, m, n, k, a1, b1, c1)
+
+
+def _gemm(ta, tb, alpha, A, B, beta, C, m, n, k, lda, ldb, ldc):
     lib = libknet8()
-    rc = lib.call("gemm_%s" % A.suffix, transA.encode(), transB.encode(), m, n, k, c(alpha), A.ptr, a1, B.ptr, b1, c(beta), C.ptr, c1)
+    rc = lib.call("gemm_%s" % A.suffix, ta, tb, m, n, k, alpha, A.ptr, lda, B.ptr, ldb, beta, C.ptr, ldc)
     if rc != 0:
         lib.check()
         raise RuntimeError("gemm failed")
     return C
 
 
+def _matrices(A, B):
+    return A.ndims == 2 and B.ndims == 2 and A.dtype == B.dtype
+
+
 def A_mul_B(A, B):
+    if _matrices(A, B):
+        (m, k), (kb, n) = A.dims, B.dims
+        if k == kb:
+            return _gemm(b"N", b"N", 1, A, B, 0, A.similar((m, n)), m, n, k, m, k, m)
     return gemm("N", "N", 1, A, B, 0, A.similar((A.size(1), B.size(2))))
 
 
 def A_mul_Bt(A, B):
+    if _matrices(A, B):
+        (m, k), (n, kb) = A.dims, B.dims
+        if k == kb:
+            return _gemm(b"N", b"T", 1, A, B, 0, A.similar((m, n)), m, n, k, m, n, m)
     return gemm("N", "T", 1, A, B, 0, A.similar((A.size(1), B.size(1))))
 
 
 def At_mul_B(A, B):
+    if _matrices(A, B):
+        (k, m), (kb, n) = A.dims, B.dims
+        if k == kb:
+            return _gemm(b"T", b"N", 1, A, B, 0, A.similar((m, n)), m, n, k, k, k, m)
     return gemm("T", "N", 1, A, B, 0, A.similar((A.size(2), B.size(2))))
 
 
@@ -68,8 +87,7 @@ def dense(w, x, b, act=None):
         raise ValueError("DimensionMismatch: %r" % ((w.dims, x2.dims, b.dims),))
     y = w.similar((m, n))
     lib = libknet8()
-    c = w.ctype
-    rc = lib.call("gemm_bias_act_%s" % w.suffix, b"N", b"N", m, n, k, c(1), w.ptr, m, x2.ptr, k, b.ptr, 1 if act == "relu" else 0, y.ptr, m)
+    rc = lib.call("gemm_bias_act_%s" % w.suffix, b"N", b"N", m, n, k, 1, w.ptr, m, x2.ptr, k, b.ptr, 1 if act == "relu" else 0, y.ptr, m)
     if rc != 0:
         lib.check()
         raise RuntimeError("gemm_bias_act failed")
@@ -107,7 +125,7 @@ def _dense_nll(w, x, b, labels, count):
     x2 = x if x.ndims == 2 else x.reshape(x.length // x.size(x.ndims), x.size(x.ndims))
     m, k, n = _size2(w, 1), _size2(w, 2), x2.size(2)
     lib = libknet8()
-    c = w.ctype
+    c = float
     dW, db, dx, mean = w.similar((m, k)), b.similar(), x2.similar(), w.similar((1,))
     T = w.dtype.type
     scale = T(1) / T(count) if count else T(np.inf)
@@ -229,13 +247,13 @@ def axpy(alpha, x, y):
     """``axpy!(alpha, x, y)``: y += alpha*x in place."""
     if x.length != y.length:
         raise ValueError("DimensionMismatch: %r" % ((x.dims, y.dims),))
-    knet8("axpy_%s" % x.suffix, x.length, x.ctype(alpha), x.ptr, y.ptr)
+    knet8("axpy_%s" % x.suffix, x.length, number(x, alpha), x.ptr, y.ptr)
     return y
 
 
 def scal(alpha, x):
     """``scal!(alpha, x)`` / ``lmul!``: x *= alpha in place."""
-    knet8("scal_%s" % x.suffix, x.length, x.ctype(alpha), x.ptr)
+    knet8("scal_%s" % x.suffix, x.length, number(x, alpha), x.ptr)
     return x
 
 

@@ -7,7 +7,7 @@ Mirrors src/ops20/loss.jl:37-41,116-140 and the device side of ``x[indices]`` an
 import numpy as np
 
 from .autograd import primitive, value
-from .karray import KnetArray, upload
+from .karray import KnetArray, upload, number
 from .libknet8 import knet8, libknet8
 from . import reduction as R
 from .softmax import logsoftmax
@@ -49,7 +49,7 @@ def _device_indices(x, indices):
 def ungetindex(x, dxi, indices):
     """Gradient of ``x[indices]``: zeros like ``x`` with ``dxi`` added at ``indices``."""
     dx = x.similar()
-    knet8("fill_%s" % x.suffix, dx.length, x.ctype(0), dx.ptr)
+    knet8("fill_%s" % x.suffix, dx.length, 0, dx.ptr)
     ents = _device_indices(x, indices)
     knet8("addents_%s" % x.suffix, ents.length, ents.ptr, dx.ptr, dxi.ptr)
     return dx
@@ -101,11 +101,11 @@ def _nll_fused(scores, labels, dims=1, count=None):
     dx = scores.similar()
     lossv = scores.similar((n,))
     scale = T(1) / T(count) if count else T(np.inf)
-    knet8("nll_logsoftmax_back_%s" % scores.suffix, m, n, scores.ptr, dlab.ptr, scores.ctype(scale), dx.ptr, lossv.ptr)
+    knet8("nll_logsoftmax_back_%s" % scores.suffix, m, n, scores.ptr, dlab.ptr, number(scores, scale), dx.ptr, lossv.ptr)
     if on_device:
         loss = scores.similar((1,))
         knet8("sum_%s_21" % scores.suffix, n, lossv.ptr, n, 1, loss.ptr)
-        knet8("scal_%s" % scores.suffix, 1, scores.ctype(scale), loss.ptr)
+        knet8("scal_%s" % scores.suffix, 1, number(scores, scale), loss.ptr)
     else:
         total = R.reduce_op("sum", lossv)
         loss = T(total) / T(count)
@@ -211,7 +211,7 @@ def _bce(scores, labels):
 
     def back(dy):
         ds = scores.similar()
-        knet8("bceback_%s" % scores.suffix, n, scores.ctype(T(dy) / T(n)), scores.ptr, y.ptr, ds.ptr)
+        knet8("bceback_%s" % scores.suffix, n, T(dy) / T(n), scores.ptr, y.ptr, ds.ptr)
         return (ds, None)
     return total / T(n), back
 

@@ -8,7 +8,7 @@ reduced dimensions as size 1.  ``dims`` are 1-based.
 import builtins
 
 from .autograd import primitive
-from .karray import KnetArray
+from .karray import KnetArray, number
 from .libknet8 import knet8, libknet8
 
 REDUCTION_OPS = ["sum", "prod", "maximum", "minimum", "sumabs", "sumabs2", "maxabs", "minabs", "countnz"]
@@ -34,6 +34,12 @@ def reduce_op(name, x, dims=None):
         lib.check()
         return x.dtype.type(r)
     nd = x.ndims
+    if nd == 2 and (dims == 1 or dims == 2) and isinstance(dims, int):   # a matrix over its rows or columns: the general case below, spelt out
+        m, n = x.dims
+        y = x.similar((1, n) if dims == 1 else (m, 1))
+        if y.length > 1:
+            knet8("%s_%s_21" % (name, S), x.length, x.ptr, m if dims == 1 else 1, y.length, y.ptr)
+            return y
     dims = _dims_list(dims, nd)
     rdims = tuple(1 if (i + 1) in dims else x.dims[i] for i in range(nd))
     vdims = nd - len(dims)
@@ -41,7 +47,7 @@ def reduce_op(name, x, dims=None):
         vdims = builtins.sum(1 for d in rdims if d > 1)
     if vdims == 0:  # falls back to Array->Scalar reduction
         y = x.similar(rdims)
-        knet8("fill_%s" % S, y.length, x.ctype(reduce_op(name, x)), y.ptr)
+        knet8("fill_%s" % S, y.length, reduce_op(name, x), y.ptr)
         return y
     if vdims == 1 and builtins.sum(1 for i in range(nd) if (i + 1) not in dims and x.dims[i] > 1) <= 1:
         i0 = [i + 1 for i in range(nd) if (i + 1) not in dims and x.dims[i] > 1]
@@ -67,16 +73,16 @@ def _sum_back(x, dims):
         z = x.similar()
         if isinstance(dy, KnetArray):
             if dy.length == z.length:
-                knet8("add_%s_01" % z.suffix, z.length, z.ctype(0), dy.ptr, z.ptr)
+                knet8("add_%s_01" % z.suffix, z.length, 0, dy.ptr, z.ptr)
             else:
                 from .binary import _vector_dim, broadcast_op
-                knet8("fill_%s" % z.suffix, z.length, z.ctype(0), z.ptr)
+                knet8("fill_%s" % z.suffix, z.length, 0, z.ptr)
                 v = _vector_dim(dy.dims, z.dims)
                 if v is None:  # reduced over several separate dimensions (or to one element): the general broadcast
                     return (broadcast_op("add", z, dy),)
                 knet8("add_%s_12" % z.suffix, z.length, z.ptr, 1, z.length, dy.ptr, v[0], v[1], z.ptr)
         else:
-            knet8("fill_%s" % z.suffix, z.length, z.ctype(dy), z.ptr)
+            knet8("fill_%s" % z.suffix, z.length, number(z, dy), z.ptr)
         return (z,)
     return back
 

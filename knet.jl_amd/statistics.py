@@ -70,7 +70,7 @@ def _var_one_pass(x, m, dims, corrected):
     y = xv.similar(rdims)
     lib = libknet8()
     rc = lib.call("sumsqdev_%s_21" % xv.suffix, xv.length, xv.ptr, xv.stride(kept[0]), xv.size(kept[0]), mv.ptr,
-                  xv.ctype(float(xv.length // y.length - corrected)), y.ptr)
+                  float(xv.length // y.length - corrected), y.ptr)
     if rc < 0:
         lib.check()
         raise RuntimeError("sumsqdev failed")

@@ -8,6 +8,7 @@ arrays, ``gclip`` gradient clipping, and one ``update_(w, g, p)`` per parameter.
 import math
 
 from .binary import zero
+from .autograd import Param
 from .karray import KnetArray
 from .libknet8 import knet8
 from .linalg import axpy, scal
@@ -76,14 +77,17 @@ def update_(w, g, p=None, lr=0.1, gclip=0):
     """``update!(w, g, p)``: one in-place step of optimizer ``p`` on the weight array ``w`` with gradient ``g``.
     ``update!(x::Param, g)`` uses the parameter's own optimizer ``x.opt``; without any optimizer the step is SGD with
     ``lr`` and ``gclip`` (src/train20/update.jl:470-476); a gradient of ``None`` (the parameter took no part) changes nothing."""
-    from .autograd import Param
-    if isinstance(w, dict):                      # update!(w::AbstractDict, g::AbstractDict, p::AbstractDict): g may have fewer keys (update.jl:497-503)
+    if isinstance(w, Param):
+        if p is None:
+            p = w.opt
+        w = w.value
+    elif isinstance(w, dict):                      # update!(w::AbstractDict, g::AbstractDict, p::AbstractDict): g may have fewer keys (update.jl:497-503)
         if not isinstance(g, dict) or not isinstance(p, dict):
             raise TypeError("MethodError: update! of a Dict needs Dicts of gradients and optimizers")
         for key in g:
             update_(w[key], g[key], p[key])
         return w
-    if isinstance(w, (list, tuple)):             # arrays, tuples, iterators in general (update.jl:479-494)
+    elif isinstance(w, (list, tuple)):             # arrays, tuples, iterators in general (update.jl:479-494)
         if g is None:
             return w
         ps = [p] * len(w) if (p is None or isinstance(p, _Opt)) else list(p)
@@ -94,10 +98,6 @@ def update_(w, g, p=None, lr=0.1, gclip=0):
         for wi, gi, pi in zip(w, g, ps):
             update_(wi, gi, pi, lr=lr, gclip=gclip)
         return w
-    if isinstance(w, Param):
-        if p is None:
-            p = w.opt
-        w = w.value
     if g is None:
         return w
     if p is None:
@@ -106,36 +106,37 @@ def update_(w, g, p=None, lr=0.1, gclip=0):
         raise TypeError("MethodError: update! needs KnetArray weights and gradients")
     if w.length != g.length or w.dtype != g.dtype:
         raise ValueError("DimensionMismatch")
-    gclip_(g, p.gclip)
-    c, S, n = w.ctype, w.suffix, w.length
+    if p.gclip != 0:
+        gclip_(g, p.gclip)
+    S, n = w.suffix, w.length
     if isinstance(p, SGD):
         axpy(-p.lr, g, w)
     elif isinstance(p, Momentum):
         if p.velocity is None:
             p.velocity = zero(w)
-        knet8("momentum_%s" % S, n, c(-p.lr), c(p.gamma), g.ptr, p.velocity.ptr, w.ptr)
+        knet8("momentum_%s" % S, n, -p.lr, p.gamma, g.ptr, p.velocity.ptr, w.ptr)
     elif isinstance(p, Nesterov):
         if p.velocity is None:
             p.velocity = zero(w)
-        knet8("nesterov_%s" % S, n, c(-p.lr), c(p.gamma), c(1 + p.gamma), g.ptr, p.velocity.ptr, w.ptr)
+        knet8("nesterov_%s" % S, n, -p.lr, p.gamma, 1 + p.gamma, g.ptr, p.velocity.ptr, w.ptr)
     elif isinstance(p, Adagrad):
         if p.G is None:
             p.G = zero(w)
-        knet8("adagrad_%s" % S, n, c(-p.lr), c(p.eps), g.ptr, p.G.ptr, w.ptr)
+        knet8("adagrad_%s" % S, n, -p.lr, p.eps, g.ptr, p.G.ptr, w.ptr)
     elif isinstance(p, Rmsprop):
         if p.G is None:
             p.G = zero(w)
-        knet8("rmsprop_%s" % S, n, c(-p.lr), c(p.rho), c(1 - p.rho), c(p.eps), g.ptr, p.G.ptr, w.ptr)
+        knet8("rmsprop_%s" % S, n, -p.lr, p.rho, 1 - p.rho, p.eps, g.ptr, p.G.ptr, w.ptr)
     elif isinstance(p, Adadelta):
         if p.G is None:
             p.G, p.delta = zero(w), zero(w)
-        knet8("adadelta_%s" % S, n, c(-p.lr), c(p.rho), c(1 - p.rho), c(p.eps), g.ptr, p.G.ptr, p.delta.ptr, w.ptr)
+        knet8("adadelta_%s" % S, n, -p.lr, p.rho, 1 - p.rho, p.eps, g.ptr, p.G.ptr, p.delta.ptr, w.ptr)
     elif isinstance(p, Adam):
         if p.fstm is None:
             p.fstm, p.scndm = zero(w), zero(w)
         p.t += 1
-        knet8("adam_%s" % S, n, c(-p.lr), c(p.beta1), c(1 - p.beta1), c(p.beta2), c(1 - p.beta2), c(1 - p.beta1 ** p.t), c(1 - p.beta2 ** p.t),
-              c(p.eps), g.ptr, p.fstm.ptr, p.scndm.ptr, w.ptr)
+        knet8("adam_%s" % S, n, -p.lr, p.beta1, 1 - p.beta1, p.beta2, 1 - p.beta2, 1 - p.beta1 ** p.t, 1 - p.beta2 ** p.t,
+              p.eps, g.ptr, p.fstm.ptr, p.scndm.ptr, w.ptr)
     else:
         raise TypeError("MethodError: unknown optimizer %r" % (p,))
     return w

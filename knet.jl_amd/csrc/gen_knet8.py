@@ -515,6 +515,13 @@ def gen_reduce():
         o.entry("sumsqdev_%s_21" % S, "int", [("int", "nx"), (T + "*", "x"), ("int", "sy"), ("int", "ny"), (T + "*", "mean"), (T, "denom"), (T + "*", "y")],
                 None, "sub_S_12, mul_S_11, sum_S_21, div at src/knetarrays/statistics.jl:11-16",
                 body="  const int rc = reduce_sqdev_21<%s>(stream, nx, x, sy, ny, mean, denom, y);\n  knet8::check_launch(\"sumsqdev_%s_21\");\n  return rc;" % (T, S))
+    o.decl.append("/* y[j] = factor * sum of the x[i] with (i/sy)%ny == j: the mean's sum and product, the same bits as sum_S_21 and mul_S_01 */")
+    o.src.append("template <typename T> struct OpFactor { T f; __device__ __forceinline__ T operator()(T v) const { return f * v; } };\n")
+    for T, S in TYPES:
+        o.entry("mean_%s_21" % S, "void", [("int", "nx"), (T + "*", "x"), ("int", "sy"), ("int", "ny"), (T, "factor"), (T + "*", "y")],
+                None, "sum_S_21, mul_S_01 at src/knetarrays/statistics.jl:4",
+                body="  reduce_mean_21<%s>(stream, nx, x, sy, ny, factor, y, [stream](%s* v, long n, %s f) {\n"
+                     "    launch_ew<%s, 1>(stream, n, v, (const %s*)nullptr, (const %s*)nullptr, v, OpFactor<%s>{f});\n  });\n  knet8::check_launch(\"mean_%s_21\");" % (T, T, T, T, T, T, T, S))
     return o
 
 

@@ -41,11 +41,15 @@ template <typename T> struct RedCountnz { typedef RedSum<T> Merged; __host__ __d
 // sum((x - mean)^2) / denom with one mean per output: the variance's second pass (src/knetarrays/statistics.jl:11-16) in one read of x, every step
 // rounded as the separate launches (subtract, multiply, sum, divide) round it.
 template <typename T> struct RedSumSqDev : RedSumabs2<T> {};
-template <typename T> struct Center { const T* mean; T denom; };   // (used by that operator only)
+// sum(x) * denom: the mean (src/knetarrays/statistics.jl:4) without a launch for its factor.
+template <typename T> struct RedMean : RedSum<T> {};
+template <typename T> struct Center { const T* mean; T denom; };   // (used by these two only)
 template <typename Op> constexpr bool kCentered = false;
 template <typename T> constexpr bool kCentered<RedSumSqDev<T>> = true;
+template <typename Op> constexpr bool kScaled = false;
+template <typename T> constexpr bool kScaled<RedMean<T>> = true;
 template <typename Op, typename T> __device__ __forceinline__ T red_item(T x, T mu) { return Op::item(kCentered<Op> ? x - mu : x); }
-template <typename Op, typename T> __device__ __forceinline__ T red_finish(T r, const Center<T>& c) { return kCentered<Op> ? r / c.denom : r; }
+template <typename Op, typename T> __device__ __forceinline__ T red_finish(T r, const Center<T>& c) { return kCentered<Op> ? r / c.denom : kScaled<Op> ? r * c.denom : r; }
 
 // A single result may be a word of host memory that the host is looking at: it goes out at once.
 template <typename T> __device__ __forceinline__ void st_result(T* p, T v, bool single) {
@@ -63,10 +67,10 @@ template <typename Op, typename T> struct MergeFn {
 // sy % NV == 0 so a vector never straddles two runs.  Workgroup (j,p) covers units [p*chunk, (p+1)*chunk)
 // of the K/NV units of output j.
 // ANY: runs of any length and at any element boundary, still 16 bytes a load: the last load of a run ends with it, and the elements that the one before
-// it has had already do not count.  (29x29 feature maps, 193 channels, 64 images, 41.5 MB fp32: 32.7 us with loads of 4 bytes, 15.6 us so.)
+// it has had already do not count.  (29x29 feature maps, 193 channels, 64 images, 41.5 MB fp32: 32.7 us with loads of 4 bytes, 9.0 us so.)
 template <typename T, typename Op, int NV, bool SINGLE, int BT, int U, bool ANY = false>
 __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x, long sy, long ny, long units, long chunk,
-                                                               unsigned P, T* __restrict__ y, T* partial, unsigned* counters, Center<T> center KNET8_TL_PARAM) {
+                                                               unsigned P, T* __restrict__ y, T* partial, unsigned* counters, Center<T> center, unsigned run_step, unsigned at_step KNET8_TL_PARAM) {
   KNET8_TL_BEGIN
   constexpr int NW = BT / kWave;
   __shared__ T lds[NW];
@@ -83,33 +87,42 @@ __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x,
   T acc[NV];
 #pragma unroll
   for (int e = 0; e < NV; e++) acc[e] = Op::init();
+  // A lane's units are BT apart: its place in its run moves by at_step = BT % usy, its run by run_step = BT / usy, and on by one where the place wraps round (with a division
+  // for each unit 784 over 200 outputs x 100 slabs takes 12.9 us, so 12.1).
+  const unsigned steps = (unsigned)usy, first = (unsigned)(u0 + threadIdx.x);
+  const unsigned run = SINGLE ? 0u : first / steps;
+  unsigned at = SINGLE ? 0u : first - run * steps;
+  const T* xp = xj + (SINGLE ? (u0 + threadIdx.x) * NV : (long)run * slab + (ANY ? 0 : (long)at * NV));   // (ANY: the start of the run)
+  const long xp_step = SINGLE ? (long)BT * NV : (long)run_step * slab + (ANY ? 0 : (long)at_step * NV), xp_wrap = slab - (ANY ? 0 : (long)usy * NV);
   for (long u = u0 + threadIdx.x; u < u1; u += BT * U) {
     T v[U][NV];
 #pragma unroll
     for (int q = 0; q < U; q++) {
       const long uu = u + q * BT;
       if (uu < u1) {
-        long off, skip = 0;
-        if (SINGLE) off = uu * NV;
-        else { const unsigned o = (unsigned)uu / (unsigned)usy; off = o * slab + ((unsigned)uu - o * (unsigned)usy) * NV; }
         if (ANY) {
-          const long in_run = (long)((unsigned)uu % (unsigned)usy) * NV;
-          skip = in_run + NV > sy ? in_run + NV - sy : 0;
+          // the run's last unit ends with it, and the elements that the one before has had already do not count
+          const int in_run = (int)at * NV, last = (int)sy - NV, from = in_run > last ? last : in_run;
           typedef T V __attribute__((ext_vector_type(NV), aligned(sizeof(T))));
-          const V t = __builtin_nontemporal_load(reinterpret_cast<const V*>(xj + off - skip));
+          const V t = __builtin_nontemporal_load(reinterpret_cast<const V*>(xp + from));
 #pragma unroll
-          for (int e = 0; e < NV; e++) v[q][e] = e >= skip ? red_item<Op>(T(t[e]), mu) : Op::init();
+          for (int e = 0; e < NV; e++) v[q][e] = from + e >= in_run ? red_item<Op>(T(t[e]), mu) : Op::init();
         } else if (NV > 1) {
           typedef typename Vec16<T>::type V;
-          V t = ld_stream(reinterpret_cast<const V*>(xj + off));
+          V t = ld_stream(reinterpret_cast<const V*>(xp));
 #pragma unroll
           for (int e = 0; e < NV; e++) v[q][e] = red_item<Op>(T(t[e]), mu);
         } else {
-          v[q][0] = red_item<Op>(T(__builtin_nontemporal_load(xj + off)), mu);
+          v[q][0] = red_item<Op>(T(__builtin_nontemporal_load(xp)), mu);
         }
       } else {
 #pragma unroll
         for (int e = 0; e < NV; e++) v[q][e] = Op::init();
+      }
+      xp += xp_step;
+      if (!SINGLE) {
+        at += at_step;
+        if (at >= steps) { at -= steps; xp += xp_wrap; }
       }
     }
 #pragma unroll
@@ -559,7 +572,7 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   const size_t two_pass_from = sy < 20 ? (size_t)sy * 1310720 : (size_t(24) << 20);
   const bool small_total = no > 1 && sy < kWave && total_bytes < two_pass_from;
   const size_t front = (sizeof(T) * (size_t)(sy * ny) + 255) / 256 * 256;
-  if (!kCentered<Op> && !small_total && ny > 1 && sy < kWave && no >= 8 && sy * ny >= kWave && front <= kTwoPassMaxBytes && scratch_fits(scratch, 2 * front, 0)) {
+  if (!kCentered<Op> && !kScaled<Op> && !small_total && ny > 1 && sy < kWave && no >= 8 && sy * ny >= kWave && front <= kTwoPassMaxBytes && scratch_fits(scratch, 2 * front, 0)) {
     Workspace tw = take_scratch(scratch, stream, front, 0);
     if (tw.partial == nullptr) { record_error("reduction: no scratch memory for the slab sums"); return false; }
     T* tmp = static_cast<T*>(tw.partial);
@@ -572,7 +585,7 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   constexpr int NR = Vec16<T>::N;
   const bool short_one_slab = no == 1 && (sy <= 256 || (sy <= kStretchMaxRun && (sy % NR != 0 || !aligned16(x))));
   bool launched = true;
-  if (!kCentered<Op> && !small_total && ny > 1 && (sy <= 8 || short_one_slab) && launch_reduce_stretch<T, Op>(stream, x, sy, ny, no, 1, 0, y, scratch, &launched)) return launched;
+  if (!kCentered<Op> && !kScaled<Op> && !small_total && ny > 1 && (sy <= 8 || short_one_slab) && launch_reduce_stretch<T, Op>(stream, x, sy, ny, no, 1, 0, y, scratch, &launched)) return launched;
   constexpr int N = Vec16<T>::N;
   // 16-byte loads off the 16-byte boundaries (ANY): in fp32 and over several slabs.  us, loads of 4 bytes / ANY: 841 over 193 outputs x 64 slabs 31.1/11.4, 65 over
   // 130 x 248 11.2/5.4, 529 over 1024 x 3 5.0/4.2.  One slab walks its runs in a row, where loads of one element and sixteen of them in flight are as good or
@@ -582,8 +595,14 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   const bool vec = aligned16(x) && (sy % N == 0);
   const bool any = kAny && !vec && no > 1 && sy >= 8 * N;
   const long units = (vec ? sy / N : any ? ceil_div(sy, N) : sy) * no;
+  const long ncu = tuning(kTuneNumCUs);
+  // A split costs a ticket and the combining pass, about 2 us: an output of up to 160 KB over several slabs stays with one workgroup of up to 1024 lanes, which takes 40 KB to the us.
+  // us, fp32, split (lanes 256 or 512) / so: 364 over 108 x 65 7.3/5.0, 292 over 127 x 89 7.9/5.3, 628 over 16 x 42 5.9/4.8, 1156 over 38 x 15 6.0/4.1, 289 over 61 x 130 (150 KB) 8.9/6.8,
+  // 2401 over 59 x 12 7.7/5.7; beyond: 2025 over 25 x 47 (380 KB) 6.2 in 16 parts, 12.0 in one.
+  const bool slabs = no > 1 && (vec || any);
+  const bool whole = slabs && ny >= 16 && ny <= ncu && (size_t)sy * no * sizeof(T) <= (size_t(160) << 10);
   // (parts of as many bytes as with loads of one element: with 2048 vectors to a part 841 over 16 outputs x 19 slabs takes 9.5 us, with 512 it is back at 5.8)
-  unsigned P = plan_parts(ny, units, any ? 2048 / N : 2048);
+  unsigned P = whole ? 1 : plan_parts(ny, units, any ? 2048 / N : 2048);
   long chunk = ceil_div(units, P);
   P = (unsigned)ceil_div(units, chunk > 0 ? chunk : 1);
   if (P < 1) P = 1;
@@ -593,29 +612,38 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
     if (!scratch_ready(ws, "reduction: no scratch memory for a split launch")) return false;
   }
   T* partial = static_cast<T*>(ws.partial);
-  // workgroup size by the work of one part: a wave for short runs, 512 lanes when there is plenty
-  const int bt = chunk <= 2 * kWave ? 64 : chunk <= 4096 ? 256 : 512;
-  const dim3 grid((unsigned)(ny * P));
-  // no more workgroups than compute units: twice the lanes keep twice the bytes in flight.  us, 512 / 1024 lanes: 841 over 16 outputs x 25 MB 10.6/8.5, over 130 x 12 MB 8.6/6.3,
-  // over 193 x 43 MB 17.6/11.7, over 256 x 167 MB 49.5/31.6; from 10 to 168 MB, runs of 65 to 20001 and 16 to 256 outputs none is slower
-  const bool alone = (long)ny * P <= tuning(kTuneNumCUs);
+  // Workgroup size by the work of one part: a wave for short runs, 512 lanes when there is plenty.  Over several slabs: 256 lanes up to 1024 units (4096 with more than two outputs to a compute unit), 512 up to 2048 and, with a
+  // workgroup to each compute unit or less, 1024 beyond (from 7/8 of the compute units on, on whole vectors, 512 lanes are as fast: 3136 over 256 x 64 31.3, 1024 lanes 32.4);
+  // 256 with more than three outputs to a compute unit (512 / 256 lanes: 3844 over 797 x 13 29.0/25.9, 1296 over 1070 x 28 28.3/26.6, 3481 over 1148 x 9 26.0/24.5).
+  // us, fp32, before (256 or 512 lanes, 1024 with unaligned runs) / so: 1024 over 158 x 12 4.7/3.7, 3136 over 153 x 83 30.3/26.2, 2500 over 210 x 76 25.8/24.8, 196 over 496 x 41 5.2/5.0.
+  const long wgs = ny * (long)P;
+  const int bt = chunk <= 2 * kWave ? 64 : !slabs ? (chunk <= 4096 ? 256 : 512) : chunk <= (ny > 2 * ncu ? 4096 : 1024) || ny > 3 * ncu ? 256 : chunk > 2048 && wgs <= (any ? ncu : ncu / 8 * 7) ? 1024 : 512;
+  const dim3 grid((unsigned)wgs);
+  const long usy = vec ? sy / N : any ? ceil_div(sy, N) : sy;   // units per run
 #define KNET8_RUN(NV, SINGLE, BT, U, ANY) \
-  hipLaunchKernelGGL((reduce_run_kernel<T, Op, NV, SINGLE, BT, U, ANY>), grid, dim3(BT), 0, stream, x, sy, ny, units, chunk, P, y, partial, ws.counters, center KNET8_TL_ARG)
+  hipLaunchKernelGGL((reduce_run_kernel<T, Op, NV, SINGLE, BT, U, ANY>), grid, dim3(BT), 0, stream, x, sy, ny, units, chunk, P, y, partial, ws.counters, center, (unsigned)(BT / usy), (unsigned)(BT % usy) KNET8_TL_ARG)
   // (the path with loads of one element, for short runs that do not start on 16-byte boundaries, keeps four times as many in flight per lane to move the same bytes)
-#define KNET8_RUN_BT(NV, SINGLE, ANY) \
-  do { if (bt == 64) KNET8_RUN(NV, SINGLE, 64, (NV == 1 ? 16 : 8), ANY); else if (bt == 256) KNET8_RUN(NV, SINGLE, 256, (NV == 1 ? 16 : 4), ANY); \
-       else if (ANY && alone) KNET8_RUN(NV, SINGLE, 1024, 8, ANY); else KNET8_RUN(NV, SINGLE, 512, (NV == 1 ? 16 : ANY ? 8 : 4), ANY); } while (0)
-  if (vec) {
-    if (no == 1) KNET8_RUN_BT(N, true, false); else KNET8_RUN_BT(N, false, false);
-    return true;
-  }
+#define KNET8_RUN_BT(NV, SINGLE) \
+  do { if (bt == 64) KNET8_RUN(NV, SINGLE, 64, (NV == 1 ? 16 : 8), false); else if (bt == 256) KNET8_RUN(NV, SINGLE, 256, (NV == 1 ? 16 : 4), false); \
+       else KNET8_RUN(NV, SINGLE, 512, (NV == 1 ? 16 : 4), false); } while (0)
+  // Two loads in flight a lane where runs are unaligned or there are more workgroups than compute units.  us, fp32, 8, 4 and 2 of them: 841 over 193 x 64 11.1/10.4/9.0, x 128 19.6/17.8/15.1
+  // (a run of whole vectors, 840: 8.8 whichever); whole vectors, 4 and 2: 1296 over 329 x 93 28.9/27.4, 4096 over 352 x 23 23.0/21.8, 2116 over 678 x 27 26.0/24.9.
   if constexpr (kAny) {
     if (any) {
-      KNET8_RUN_BT(N, false, true);
+      if (bt == 64) KNET8_RUN(N, false, 64, 2, true);
+      else if (bt == 256) KNET8_RUN(N, false, 256, 2, true);
+      else if (bt == 512) KNET8_RUN(N, false, 512, 2, true);
+      else KNET8_RUN(N, false, 1024, 2, true);
       return true;
     }
   }
-  if (no == 1) KNET8_RUN_BT(1, true, false); else KNET8_RUN_BT(1, false, false);
+  if (slabs && bt == 1024) KNET8_RUN(N, false, 1024, 2, false);
+  else if (slabs && bt == 512 && ny > ncu) KNET8_RUN(N, false, 512, 2, false);
+  else if (slabs && bt == 256 && chunk > 4096) KNET8_RUN(N, false, 256, 2, false);
+  else if (vec && no == 1) KNET8_RUN_BT(N, true);
+  else if (vec) KNET8_RUN_BT(N, false);
+  else if (no == 1) KNET8_RUN_BT(1, true);
+  else KNET8_RUN_BT(1, false);
 #undef KNET8_RUN_BT
 #undef KNET8_RUN
   return true;
@@ -634,7 +662,7 @@ inline bool launch_reduce_strided(hipStream_t stream, const T* x, long s1, long 
   // fp64: 16 x 16 MB 12.1 / 13.7; 24 x 16 MB 12.4 / 12.0, x 64 MB 21.6 / 23.1; 32 x 64 MB 21.3 / 20.1, x 134 MB 28.8 / 32.3; 48 x 134 MB 33.2 / 26.8.
   const size_t row_bytes = (size_t)s1 * sizeof(T), array_bytes = row_bytes * (size_t)d * (size_t)nb;
   const bool short_axis = row_bytes <= 128 || (row_bytes <= 192 && array_bytes >= (size_t(48) << 20)) || (row_bytes <= 256 && array_bytes >= (size_t(96) << 20));
-  if (!kCentered<Op> && short_axis && launch_reduce_stretch<T, Op>(stream, x, 1, s1, d, nb, s1 * d, y, scratch, &launched)) return launched;
+  if (!kCentered<Op> && !kScaled<Op> && short_axis && launch_reduce_stretch<T, Op>(stream, x, 1, s1, d, nb, s1 * d, y, scratch, &launched)) return launched;
   const bool vec = aligned16(x) && (s1 % N == 0);
   // rows that do not start on 16-byte boundaries: the same tile width from N interleaved 4- or 8-byte loads per lane
   const long tile = (long)kWave * N;
@@ -675,6 +703,23 @@ inline void reduce_21(hipStream_t stream, long nx, const T* x, long sy, long ny,
   if (ny == 1) launch_reduce_run<T, Op>(stream, x, nx, 1, 1, y, scratch);
   else if (sy == 1) launch_reduce_strided<T, Op>(stream, x, ny, no, 1, y, scratch);
   else launch_reduce_run<T, Op>(stream, x, sy, ny, no, y, scratch);
+}
+
+// y[j] = factor * sum over x[i], (i/sy)%ny == j: in one launch, or the sums and then their factor where the sums take the stretch kernel or the route through slab sums.
+template <typename T, typename Scale>
+inline void reduce_mean_21(hipStream_t stream, long nx, const T* x, long sy, long ny, T factor, T* y, Scale scale) {
+  if (ny <= 0 || sy <= 0 || nx < 0) return;
+  const bool own = ny > 1 && (sy == 1 ? ny * (long)sizeof(T) <= 256 : sy < (nx == sy * ny ? kStretchMaxRun : (long)kWave));
+  if (own || nx % (sy * ny) != 0) {   // (the sums report sizes that do not fit)
+    reduce_21<T, RedSum<T>>(stream, nx, x, sy, ny, y);
+    if (nx % (sy * ny) == 0) scale(y, ny, factor);
+    return;
+  }
+  const Center<T> c = {nullptr, factor};
+  const long no = nx / (sy * ny);
+  if (ny == 1) launch_reduce_run<T, RedMean<T>>(stream, x, nx, 1, 1, y, nullptr, c);
+  else if (sy == 1) launch_reduce_strided<T, RedMean<T>>(stream, x, ny, no, 1, y, nullptr, 0, c);
+  else launch_reduce_run<T, RedMean<T>>(stream, x, sy, ny, no, y, nullptr, c);
 }
 
 // y[j] = sum over x[i], (i/sy)%ny == j, of (x[i] - mean[j])^2, divided by denom.  1: declined, nothing was launched -- shapes whose sums take the stretch kernel or

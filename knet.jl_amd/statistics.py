@@ -9,7 +9,7 @@ from .autograd import primitive, track, value
 from .activation import unary_op
 from .binary import broadcast_op, sub, mul
 from .karray import KnetArray, Array
-from .libknet8 import libknet8
+from .libknet8 import knet8, libknet8
 from . import reduction as R
 
 
@@ -50,27 +50,51 @@ def mean(x, dims=None, f=None):
             raise ValueError("mean(f, x): f must be 'abs' or 'abs2'")
         total = (R.sumabs if f == "abs" else R.sumabs2)(x)
         return _divn(total, _len(x))
+    if dims is not None and isinstance(value(x), KnetArray) and track(x) is None:
+        xv, dims = value(x), dims if isinstance(dims, int) else list(dims)
+        kept = _one_kept(xv, dims)
+        if kept is not None:
+            y = xv.similar(kept[0])
+            knet8("mean_%s_21" % xv.suffix, xv.length, xv.ptr, kept[1], y.length, y.length / xv.length, y.ptr)
+            return y
     b = R.sum(x, dims=dims)
     return _scale(b, _len(b) / _len(x))
 
 
+def _one_kept(x, dims):
+    """(dims of the result, elements between neighbours of the kept dimension) of a reduction that leaves one dimension of more than one element; None for others."""
+    if x.suffix is None or x.length == 0:
+        return None
+    over = R._dims_list(dims, x.ndims)
+    rdims, n, found = [], 1, None
+    for i, d in enumerate(x.dims):
+        if i + 1 in over or d == 1:
+            rdims.append(1)
+        elif found is None:
+            rdims.append(d)
+            found = n
+        else:
+            return None
+        n *= d
+    if found is None or len(set(over)) != len(over):
+        return None
+    return tuple(rdims), found
+
+
 def _var_one_pass(x, m, dims, corrected):
-    """The sum of squares, its division and the subtraction before it as one launch (``sumsqdev_S_21``; 29x29x193x64 fp32: 98 us a pass with the mean, 30 us so), where nothing is recorded of ``x`` or ``m``, one
+    """The sum of squares, its division and the subtraction before it as one launch (``sumsqdev_S_21``; 29x29x193x64 fp32: 98 us a pass with the mean and its factor, 18 us so), where nothing is recorded of ``x`` or ``m``, one
     dimension of ``x`` remains and ``m`` has a value for each of its positions; None otherwise, and for shapes the kernel does not take."""
     if dims is None or track(x) is not None or track(m) is not None:
         return None
     xv, mv = value(x), value(m)
-    if not isinstance(xv, KnetArray) or not isinstance(mv, KnetArray) or xv.suffix is None or mv.dtype != xv.dtype or xv.length == 0:
+    if not isinstance(xv, KnetArray) or not isinstance(mv, KnetArray) or mv.dtype != xv.dtype:
         return None
-    over = R._dims_list(dims, xv.ndims)
-    rdims = tuple(1 if i + 1 in over else d for i, d in enumerate(xv.dims))
-    kept = [i + 1 for i, d in enumerate(rdims) if d > 1]
-    if mv.dims != rdims or len(kept) != 1 or len(set(over)) != len(over):
+    kept = _one_kept(xv, dims)
+    if kept is None or mv.dims != kept[0]:
         return None
-    y = xv.similar(rdims)
+    y = xv.similar(kept[0])
     lib = libknet8()
-    rc = lib.call("sumsqdev_%s_21" % xv.suffix, xv.length, xv.ptr, xv.stride(kept[0]), xv.size(kept[0]), mv.ptr,
-                  float(xv.length // y.length - corrected), y.ptr)
+    rc = lib.call("sumsqdev_%s_21" % xv.suffix, xv.length, xv.ptr, kept[1], y.length, mv.ptr, float(xv.length // y.length - corrected), y.ptr)
     if rc < 0:
         lib.check()
         raise RuntimeError("sumsqdev failed")

@@ -60,3 +60,46 @@ def test_variance_is_the_chain(knet, dims, over, corrected, dt):
         J = knet.diff(lambda: knet.sum(knet.var(p, dims=over, mean=m, corrected=corrected)))    # recorded: through its parts
         np.testing.assert_allclose(knet.Array(knet.grad(J, p)), 2 * d / dt(n - int(corrected)), rtol=20 * eps, atol=8 * eps)
     knet.libknet8().check()
+
+
+# shapes x(run, outputs, slabs) on both sides of the lines between workgroup sizes and splits: units a part 128/129, 1024/1025, 2048/2049; 160 KB an output; 224/225 and 256/257
+# workgroups; more outputs than compute units; runs of whole vectors and with 1 to 3 elements over
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("dims", [(64, 5, 8), (65, 5, 8), (516, 3, 8), (512, 40, 8), (513, 40, 8), (1024, 40, 8), (1028, 40, 8), (1029, 9, 40), (1024, 9, 41), (5120, 3, 9),
+                                  (260, 224, 33), (260, 225, 33), (261, 256, 33), (261, 257, 33), (400, 300, 4), (1100, 300, 9), (67, 900, 3), (3000, 60, 20)])
+def test_reductions_over_slabs(knet, dims, dt):
+    rng = np.random.default_rng(sum(dims))
+    x = rng.standard_normal(dims).astype(dt)
+    eps = 2.0 ** -24 if dt == np.float32 else 2.0 ** -53
+    n = dims[0] * dims[2]
+    want = x.astype(np.longdouble).sum(axis=(0, 2), keepdims=True)
+    bound = 16 * eps * np.abs(x).sum(axis=(0, 2), keepdims=True)     # lanes hold partial sums of some ten terms, log2 of the lanes more on the way together
+    for by in (0, 1):
+        xd = offset(knet, x, by)
+        got = knet.Array(knet.sum(xd, dims=(1, 3)))
+        assert np.all(np.abs(got - want) <= bound)
+        assert np.array_equal(knet.Array(knet.maximum(xd, dims=(1, 3))), x.max(axis=(0, 2), keepdims=True))
+        m = knet.mean(xd, dims=(1, 3))
+        assert np.array_equal(knet.Array(m), got * dt(1.0 / n))      # the bits of the sum and its factor
+        v = knet.Array(knet.var(xd, dims=(1, 3), mean=m, corrected=False))      # terms of one sign: the bound above is relative to the sum, two more roundings a term
+        np.testing.assert_allclose(v, ((x - knet.Array(m)).astype(np.longdouble) ** 2).mean(axis=(0, 2), keepdims=True), rtol=32 * eps)
+    y = np.zeros(dims, dt)
+    y[0, :, 0], y[-1, :, -1], y[dims[0] // 2, :, dims[2] // 2] = 1, 2, 4   # the ends of every run's walk, once
+    assert np.all(knet.Array(knet.sum(offset(knet, y, 1), dims=(1, 3))) == 7)
+    knet.libknet8().check()
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("dims,over", [((3, 3, 5, 4), (1, 2, 4)), ((20, 500), 2), ((64, 31), [2]), ((65, 31), (2,)), ((300, 700), 1), ((50, 1), (1,)), ((1, 9), (2,)), ((6, 5, 4), (1,)), ((6, 1, 4), (1,)),
+                                       ((6, 5, 4), (1, 2, 3)), ((2000, 40), 1), ((7, 3000), 2), ((5, 4), (1, 5)), ((4000, 3), 2)])
+def test_mean_is_sum_and_factor(knet, dims, over, dt):
+    rng = np.random.default_rng(sum(dims))
+    xd = offset(knet, rng.standard_normal(dims).astype(dt), 1)
+    m, s = knet.mean(xd, dims=over), knet.sum(xd, dims=over)
+    assert m.dims == s.dims and m.dtype == s.dtype
+    factor, eps = dt(s.length / xd.length), 2.0 ** -24 if dt == np.float32 else 2.0 ** -53
+    np.testing.assert_allclose(knet.Array(m), knet.Array(s) * factor, rtol=0, atol=16 * eps * float(np.abs(knet.Array(xd)).sum()) * float(factor))
+    p = knet.Param(xd)
+    J = knet.diff(lambda: knet.sum(knet.mean(p, dims=over)))
+    assert np.allclose(knet.Array(knet.grad(J, p)), float(factor))
+    knet.libknet8().check()

@@ -705,10 +705,12 @@ KNET8_API void sum_32_21_noalloc(int nx, float* x, int sy, int ny, float* y, hip
    key 7: non-zero makes the hipBLASLt route of gemm_S do everything but the vendor call itself (for measuring the library's own share of a call's host time);
    key 8: non-zero keeps repeated products on hipblasLtMatmul instead of the prepared calls of the vendor's extension interface (for comparisons);
    key 9: which fp32 products run on the bf16 matrix cores in three parts: 0 those that are faster there, 1 none, 2 all with sides of at least 4 (for tests);
-   key 10: which small products run on the library's own kernels while key 3 is 0: 0 by the rule, where hipBLASLt allows no prepared calls, 1 none, 2 by the rule whatever hipBLASLt allows (for tests) */
+   key 10: which small products run on the library's own kernels while key 3 is 0: 0 by the rule, where hipBLASLt allows no prepared calls, 1 none, 2 by the rule whatever hipBLASLt allows (for tests);
+   key 11: which products between the small and the large ones (in fp64 the large ones too) run on the library's 32x32 kernel: 0 by the rule, where hipBLASLt allows no prepared calls and keys 3
+   and 10 are 0, 1 none, 2 all with sides of at least 2, 3 by the rule whatever hipBLASLt allows (for tests) */
 KNET8_API int knet8_tune(int key, int value);
 /* no counterpart in the reference: what the calling thread's last product (gemm_S, bmm_S, gemm_bias_act_S) ran on: 0 none yet, 1 hipBLASLt, 2 the library's small-product
-   kernels, 3 its bf16 kernel with three parts to an element */
+   kernels, 3 its bf16 kernel with three parts to an element, 4 its 32x32 kernel for products between the two */
 KNET8_API int knet8_product_route(void);
 /* Seed of the default random stream used by rand_S / randn_S (restarts it at counter 0): the device half of Knet.seed!,
    src/knetarrays/random.jl:14-18 (CUDA.seed!).  Unseeded, the stream starts from the operating system's entropy. */

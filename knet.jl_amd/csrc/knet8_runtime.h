@@ -77,7 +77,7 @@ void pool_give(void* p);
 // State of the default random stream (knet8_seed): hands out `blocks` consecutive generator counters under the current seed.
 void rng_take(unsigned long long blocks, unsigned long long* seed, unsigned long long* offset);
 
-enum { kTuneNumCUs = 0, kTuneSoftmaxResidentRows = 1, kTuneGemmSmallMflop = 3, kTuneDenseBackMflop = 4, kTuneFailScratch = 5, kTuneSoftmaxNoLdsSlots = 6, kTuneGemmDryRun = 7, kTuneGemmNoPrepared = 8, kTuneGemmSplit = 9, kTuneGemmSmallRule = 10, kTuneCount = 11 };
+enum { kTuneNumCUs = 0, kTuneSoftmaxResidentRows = 1, kTuneGemmSmallMflop = 3, kTuneDenseBackMflop = 4, kTuneFailScratch = 5, kTuneSoftmaxNoLdsSlots = 6, kTuneGemmDryRun = 7, kTuneGemmNoPrepared = 8, kTuneGemmSplit = 9, kTuneGemmSmallRule = 10, kTuneGemmMid = 11, kTuneCount = 12 };
 int tuning(int key);
 
 #ifdef KNET8_TIMELINE

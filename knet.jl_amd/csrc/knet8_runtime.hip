@@ -3,6 +3,7 @@
 #include "knet8_runtime.h"
 #include "knet8_gemm_small.h"
 #include "knet8_gemm_split.h"
+#include "knet8_gemm_mid.h"
 #include "knet8_fused.h"
 
 #include <hipblaslt/hipblaslt.h>
@@ -1013,7 +1014,7 @@ static int gemm_lt(bool ta, bool tb, int m, int n, int k, T alpha, const T* A, i
 }
 
 // Which kernels this thread's last product ran on, or would have (knet8_product_route).
-enum { kRouteNone = 0, kRouteVendor = 1, kRouteSmall = 2, kRouteSplit = 3 };
+enum { kRouteNone = 0, kRouteVendor = 1, kRouteSmall = 2, kRouteSplit = 3, kRouteMid = 4 };
 static thread_local int t_route = kRouteNone;
 
 template <typename T>
@@ -1038,6 +1039,20 @@ static int gemm(char transa, char transb, int m, int n, int k, T alpha, const T*
     const int knob = g_tune[kTuneGemmSmallRule];
     return knob != 1 && (sizeof(T) == 8 || g_tune[kTuneGemmSplit] != 2) && gemm_is_small_by_rule<T>(ta, tb, m, n, k, lda, ldb) && (knob == 2 || !vendor_prepares());
   };
+  // those between the small and the large ones, and in fp64 the large ones too: by their rule, in the same processes (key 11: never, or wherever the kernel can)
+  auto mid = [&]() {
+    const int knob = g_tune[kTuneGemmMid];
+    if (batch.count != 1 || k <= 0 || alpha == T(0) || (!bias && act) || knob == 1 || (sizeof(T) == 4 && g_tune[kTuneGemmSplit] == 2)) return false;
+    if (knob == 2) return m >= 2 && n >= 2;
+    return g_tune[kTuneGemmSmallRule] == 0 && tuning(kTuneGemmSmallMflop) == 0 && gemm_mid_fits<T>(ta, tb, m, n, k, lda, ldb, gemm_is_small_by_rule<T>(ta, tb, m, n, k, lda, ldb)) &&
+           (knob == 3 || !vendor_prepares());
+  };
+  if (mid()) {
+    t_route = kRouteMid;
+    launch_gemm_mid<T>(stream, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, bias, act);
+    check_launch("gemm (mid)");
+    return 0;
+  }
   if (batch.count == 1 && (k <= 0 || (tuning(kTuneGemmSmallMflop) > 0 ? gemm_is_small(m, n, k) : small_by_rule()))) {
     t_route = kRouteSmall;
     if (!own_kernels_reach()) return -1;

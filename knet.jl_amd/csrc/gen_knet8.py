@@ -384,6 +384,15 @@ def gen_elementwise():
         o.entry("dropout_%s" % S, "void", [("int", "n"), (T, "p"), (T + "*", "x"), (T + "*", "y")],
                 "launch_ew<%s, 2>(stream, n, x, y, (const %s*)nullptr, y, OpDropout<%s>{p, %s(1) - p})" % (T, T, T, T),
                 "src/libknet8/cuda1.jl:459-484 (in place: y is the uniform buffer on entry)")
+        o.entry("dropout_rand_%s" % S, "void", [("int", "n"), (T, "p"), (T + "*", "x"), (T + "*", "y")], None,
+                "src/ops20_gpu/dropout.jl:11-16 (rand_S into y and dropout_S in one launch: the same numbers of the default stream, the same bits)",
+                body="  if (n <= 0) return;\n  unsigned long long seed, offset;\n  knet8::rng_take(rand_blocks<%s>(n), &seed, &offset);\n"
+                     "  launch_dropout_rand<%s>(stream, n, seed, offset, nullptr, x, y, OpDropout<%s>{p, %s(1) - p});\n"
+                     "  knet8::check_launch(\"dropout_rand_%s\");" % (T, T, T, T, S))
+        o.entry("dropout_rand_state_%s" % S, "void", [("int", "n"), (T, "p"), ("unsigned long long*", "state"), (T + "*", "x"), (T + "*", "y")],
+                "if (state == nullptr) { knet8::record_error(\"dropout_rand_state_%s: null state\"); return; }\n"
+                "  launch_dropout_rand<%s>(stream, n, 0, 0, state, x, y, OpDropout<%s>{p, %s(1) - p})" % (S, T, T, T),
+                "src/ops20_gpu/dropout.jl:11-16 with the position in device memory, moved forward by a second launch as in rand_state_S")
         o.entry("dropback_%s" % S, "void", [("int", "n"), (T, "p"), (T + "*", "x"), (T + "*", "y"), (T + "*", "dy"), (T + "*", "dx")],
                 "(void)x; launch_ew<%s, 2>(stream, n, y, dy, (const %s*)nullptr, dx, OpDropback<%s>{%s(1) - p})" % (T, T, T, T),
                 "src/libknet8/cuda1.jl:469-493")

@@ -2,15 +2,16 @@
 
 The reference fills ``y`` with uniforms from the device generator (``rand!(y)``, after ``CUDA.seed!(seed)`` for a
 non-zero ``seed``) and calls ``dropout_S`` in place; CPU and GPU draw from different streams, which is why its own test
-only compares them statistically (test/dropout.jl:8-17).  Here the buffer comes from the library's generator in the same
-way; it can also be passed explicitly (``uniform=``) so that the device result can be compared element by element with
-the CPU path.
+only compares them statistically (test/dropout.jl:8-17).  Here the uniforms come from the library's generator in the same
+way, drawn inside the dropout launch (``dropout_rand_S``: the bits of ``rand_S`` followed by ``dropout_S``); a buffer of them
+can also be passed explicitly (``uniform=``) so that the device result can be compared element by element with the CPU path.
 """
 import numpy as np
 
 from .autograd import primitive, recording
 from .karray import KnetArray, number
 from .libknet8 import knet8
+from .random import _check, seed_
 
 
 def dropout_(p, x, y):
@@ -39,14 +40,17 @@ def dropback(dy, y, x, p):
 @primitive
 def _dropout(x, p, uniform=None, seed=0, rng=None):
     if uniform is None:
-        from .random import rand_, seed_
+        y = x.similar()
+        _check(y)
         if rng is not None:
-            uniform = rand_(x.similar(), state=rng)   # position on the device: safe to capture into a graph
+            # position on the device: safe to capture into a graph
+            knet8("dropout_rand_state_%s" % x.suffix, y.length, number(x, p), rng.ptr, x.ptr, y.ptr)
         else:
             if seed != 0:
                 seed_(seed)   # if seed !== 0; CUDA.seed!(seed); end   (src/ops20_gpu/dropout.jl:13)
-            uniform = rand_(x.similar())
-    elif not isinstance(uniform, KnetArray):
+            knet8("dropout_rand_%s" % x.suffix, y.length, number(x, p), x.ptr, y.ptr)
+        return y, (lambda dy: (dropback(dy, y, x, p), None))
+    if not isinstance(uniform, KnetArray):
         uniform = KnetArray(np.asarray(uniform, dtype=x.dtype))
     else:
         uniform = uniform.copy()

@@ -94,12 +94,17 @@ inline void launch_bias_act(hipStream_t stream, long m, long n, const T* z, cons
 // P workgroups split the columns of a tile and the last one to finish adds their partial sums (same ticket
 // scheme as the strided reduction).  F(dy, y) is the element gradient.  dz may be dy or y itself (each element is read
 // before the same lane writes it).
-// SC: rows that do not start on 16-byte boundaries (m odd) -- the lane's NV elements are the rows lane, lane+64, ... of the tile,
-// each moved with its own 4- or 8-byte access (see strided_walk).
-template <typename T, typename F, int NV, int BT, int U, bool SC>
+// AL: every row of sixteen bytes starts on a 16-byte boundary (m a multiple of NV, aligned arrays).  Otherwise the same 16-byte accesses go to element
+// boundaries, which this hardware's vector memory instructions take, and the one lane that straddles the last row moves back to end on it: it does its
+// left neighbour's last rows a second time (both lanes read them with one instruction before either writes them, and write the same bits) and leaves
+// them out of its sums.  Where the neighbour is in another tile (a last tile of fewer than NV rows), the caller sees to it that dz is neither dy nor y.
+// Rows off the boundaries, fp32, moved one element at a time -> so: (1081,965) 18.1 -> 5.4 us, (3223,1103) 34.8 -> 9.9; against the flat gradient and the
+// row sums as two launches: (4095,2048), arrays not in cache, 26.4 -> 18.8, (1001,2048) 11.4 -> 7.5, (1002,2048) fp64 stays at 9.6; (10,100) 6.6 -> 4.7.
+template <typename T, typename F, int NV, int BT, int U, bool AL>
 __global__ __launch_bounds__(BT) void actback_biasgrad_kernel(const T* dy, const T* yv, long m, long n, long jchunk, unsigned P, T* dz, T* __restrict__ db,
                                                               T* partial, unsigned* counters, F f KNET8_TL_PARAM) {
   KNET8_TL_BEGIN
+  typedef T V __attribute__((ext_vector_type(NV), aligned(AL ? NV * sizeof(T) : sizeof(T))));
   constexpr int TILE = kWave * NV;
   constexpr int NW = BT / kWave;
   __shared__ T lds[NW][TILE];
@@ -107,65 +112,40 @@ __global__ __launch_bounds__(BT) void actback_biasgrad_kernel(const T* dy, const
   const long at = blockIdx.x / P;
   const unsigned p = blockIdx.x % P;
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const long a0 = at * TILE + (SC ? (long)lane : (long)lane * NV);
-  unsigned livemask = 0;
-#pragma unroll
-  for (int e = 0; e < NV; e++)
-    if (a0 + (SC ? e * kWave : e) < m) livemask |= 1u << e;   // vector path: m % NV == 0, all or nothing
+  const bool out = at * TILE + (long)lane * NV >= m;
+  const int again = AL || out || at * TILE + (long)(lane + 1) * NV <= m ? 0 : (int)(at * TILE + (long)(lane + 1) * NV - m);   // rows done twice
+  const long a0 = at * TILE + (long)lane * NV - again;
   const long j0 = (long)p * jchunk;
   long j1 = j0 + jchunk;
   if (j1 > n) j1 = n;
   T acc[NV];
 #pragma unroll
   for (int e = 0; e < NV; e++) acc[e] = T(0);
-  if (livemask) {
+  if (!out) {
     for (long j = j0 + wave; j < j1; j += NW * U) {
       T g[U][NV];
-      if constexpr (!SC && NV > 1) {
-        // Vector path: the loads of all U columns first, then the U results and stores.  Written column by column, the second column's loads sink
-        // below the first column's store (dz may be dy or y itself, so the compiler must keep that order), and every load then waits for the store
-        // before it as well: U dependent round trips instead of one.  A column past the end of the share reads the share's last column again.
-        typedef typename Vec16<T>::type V;
-        V d[U], o[U];
+      // The loads of all U columns first, then the U results and stores.  Written column by column, the second column's loads sink
+      // below the first column's store (dz may be dy or y itself, so the compiler must keep that order), and every load then waits for the store
+      // before it as well: U dependent round trips instead of one.  A column past the end of the share reads the share's last column again.
+      V d[U], o[U];
 #pragma unroll
-        for (int q = 0; q < U; q++) {
-          const long jj = j + q * NW < j1 ? j + q * NW : j;
-          const long off = jj * m + a0;
-          d[q] = ld_stream(reinterpret_cast<const V*>(dy + off));
-          o[q] = ld_stream(reinterpret_cast<const V*>(yv + off));
-        }
-#pragma unroll
-        for (int q = 0; q < U; q++) {
-          const long jj = j + q * NW;
-          V r;
-#pragma unroll
-          for (int e = 0; e < NV; e++) { r[e] = f(d[q][e], o[q][e]); g[q][e] = jj < j1 ? r[e] : T(0); }
-          // written through (sc1), not merely streamed: what a kernel leaves dirty in the L2s is written back after its last workgroup has ended,
-          // before the next launch may start; written through, dz drains while the partial sums are still being combined
-          // ((4096,2048) fp32 cold: 19.3 -> 18.4 us; nt sc1 19.9-20.0, sc0 sc1 18.6, plain 19.3)
-          if (jj < j1) st_through(reinterpret_cast<V*>(dz + jj * m + a0), r);
-        }
-      } else {
+      for (int q = 0; q < U; q++) {
+        const long jj = j + q * NW < j1 ? j + q * NW : j;
+        const long off = jj * m + a0;
+        d[q] = ld_stream(reinterpret_cast<const V*>(dy + off));
+        o[q] = ld_stream(reinterpret_cast<const V*>(yv + off));
+      }
 #pragma unroll
       for (int q = 0; q < U; q++) {
         const long jj = j + q * NW;
-        if (jj < j1) {
-          const long off = jj * m + a0;
+        const long off = jj * m + a0;
+        V r;
 #pragma unroll
-          for (int e = 0; e < NV; e++) {
-            if (livemask & (1u << e)) {
-              const T r = f(__builtin_nontemporal_load(dy + off + e * kWave), __builtin_nontemporal_load(yv + off + e * kWave));
-              g[q][e] = r;
-              __builtin_nontemporal_store(r, dz + off + e * kWave);
-            } else {
-              g[q][e] = T(0);
-            }
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < NV; e++) g[q][e] = T(0);
-        }
-      }
+        for (int e = 0; e < NV; e++) { r[e] = f(d[q][e], o[q][e]); g[q][e] = jj < j1 && e >= again ? r[e] : T(0); }
+        // written through (sc1), not merely streamed: what a kernel leaves dirty in the L2s is written back after its last workgroup has ended,
+        // before the next launch may start; written through, dz drains while the partial sums are still being combined
+        // ((4096,2048) fp32 cold: 19.3 -> 18.4 us; nt sc1 19.9-20.0, sc0 sc1 18.6, plain 19.3)
+        if (jj < j1) st_through(reinterpret_cast<V*>(dz + off), r);
       }
 #pragma unroll
       for (int q = 0; q < U; q++)
@@ -173,10 +153,11 @@ __global__ __launch_bounds__(BT) void actback_biasgrad_kernel(const T* dy, const
         for (int e = 0; e < NV; e++) acc[e] = acc[e] + g[q][e];
     }
   }
+  auto slot = [&](int e) { return lane * NV + (e >= again ? e - again : e - again + NV); };   // where row a0 + e belongs in the tile
   KNET8_TL_MID
   if (P > 1) {
 #pragma unroll
-    for (int e = 0; e < NV; e++) lds[wave][SC ? e * kWave + lane : lane * NV + e] = acc[e];
+    for (int e = 0; e < NV; e++) lds[wave][slot(e)] = acc[e];
     __syncthreads();
     if (threadIdx.x < TILE) {
       T r = T(0);
@@ -188,11 +169,11 @@ __global__ __launch_bounds__(BT) void actback_biasgrad_kernel(const T* dy, const
 #pragma unroll
     for (int e = 0; e < NV; e++) acc[e] = T(0);
     const T mu[NV] = {};
-    strided_walk<T, RedSum<T>, NV, false, NW, kCombineU, SC>(partial + at * P * TILE + (SC ? lane : lane * NV), TILE, 0, P, wave, acc, mu);
+    strided_walk<T, RedSum<T>, NV, false, NW, kCombineU, false>(partial + at * P * TILE + lane * NV, TILE, 0, P, wave, acc, mu);
     if (threadIdx.x == 0) st_coherent(counters + at * kTicketStride, 0u);
   }
 #pragma unroll
-  for (int e = 0; e < NV; e++) lds[wave][SC ? e * kWave + lane : lane * NV + e] = acc[e];
+  for (int e = 0; e < NV; e++) lds[wave][P > 1 ? lane * NV + e : slot(e)] = acc[e];
   __syncthreads();
   const long a = at * TILE + threadIdx.x;
   if (threadIdx.x < TILE && a < m) {
@@ -226,25 +207,28 @@ inline void launch_actback_biasgrad(hipStream_t stream, long m, long n, const T*
   if (m <= 0) return;
   if (n > 0 && m * n >= (1L << 31)) { record_error("activation gradient + bias gradient: 2^31 or more elements are not supported"); return; }
   constexpr int N = Vec16<T>::N;
-  const bool flat16 = (m * n) % N == 0 && aligned16(dy) && aligned16(y) && aligned16(dz);
-  if ((m < kWave || (m % N != 0 && flat16)) && n > 0) {
-    // A layer of few units (ten classes): a 256-row tile would idle nearly all its lanes ((2, 4M): 531 us, (10, 839K): 132 us for 100 MB).
-    // Two launches instead: the element gradient over the flat array, then the row sums of dz by the reduction family -- one more read of dz,
-    // 4/3 of the bytes, same bits for dz and the same kind of fixed-order sum for db.  Also for a number of units that is not a multiple of the
-    // vector width (1001) when the flat array can still move in 16-byte accesses: the tiled kernel falls back on 4-byte ones there.
-    const long count = m * n;
-    const bool v = flat16;
+  const bool vec = (m % N == 0) && aligned16(dy) && aligned16(y) && aligned16(dz);
+  const long count = m * n, tile = (long)kWave * N, over = m % tile;
+  // A last tile of fewer than N rows starts by doing rows of the tile before it again (see AL above), so another workgroup must not have replaced their inputs.
+  auto apart = [&](const T* a) { return a + count <= dz || dz + count <= a; };
+  const bool tiles = vec || over == 0 || over >= N || (m > tile && apart(dy) && apart(y));
+  if (n > 0 && (!tiles || (m < kWave && n > 8192))) {
+    // Very many columns of a few rows: a tile's sixteen-column trips are then nearly all idle lanes, and what counts is their number ((2, 4M): 531 us, (10, 839K):
+    // 132 us for 100 MB).  Two launches instead: the element gradient over the flat array, then the row sums of dz by the reduction family -- one more read
+    // of dz, 4/3 of the bytes, same bits for dz and the same kind of fixed-order sum for db.  The line: fp32, tiles against two launches, (10, 8192) 7.2 us
+    // against 8.6, (10, 16384) 9.9 against 8.9, (10, 100000) 17.4 against 12.2; (48, 2048) 5.2 against 7.8, (63, 16384) 10.1 against 11.1, (48, 100000) 24.2
+    // against 23.5.  Fewer rows than a vector come here too.
+    const bool v = count % N == 0 && aligned16(dy) && aligned16(y) && aligned16(dz);
     if (v) hipLaunchKernelGGL((actback_flat_kernel<T, F, N>), dim3((unsigned)ceil_div(count / N, 256)), dim3(256), 0, stream, dy, y, count, dz, f);
     else hipLaunchKernelGGL((actback_flat_kernel<T, F, 1>), dim3((unsigned)ceil_div(count, 256)), dim3(256), 0, stream, dy, y, count, dz, f);
     launch_reduce_strided<T, RedSum<T>>(stream, dz, m, n, 1, db);
     return;
   }
-  const bool vec = (m % N == 0) && aligned16(dy) && aligned16(y) && aligned16(dz);
-  const long tile = (long)kWave * N;
   const long atiles = ceil_div(m, tile);
-  // (parts by memory round trips, as in the strided reduction; a part's waves take sixteen columns per trip here: (256, 8192) fp32 13.9 us with 256 parts of
-  //  32 columns, whose 256 partial rows one four-wave workgroup then combines)
-  unsigned P = n > 0 ? plan_parts_by_trips(atiles, n, 16, 64) : 1;
+  // Parts by memory round trips, as in the strided reduction: sixteen columns per trip, by four waves of four columns where one trip is all, else by sixteen waves
+  // of one; joining costs a trip and the partial rows.  (At least eight columns a part; sixteen and two trips for joining, with four waves up to 63 columns:
+  // fp32 (64,100) 5.2 -> 4.2 us, (1024,237) 5.6 -> 4.4, (3223,1103) 11.5 -> 9.8; (66, 8192) 7.3 us with 128 parts, 9.1 with 256.)
+  unsigned P = n > 0 ? plan_parts_by_trips(atiles, n, 16, 17, 8, 1, 64) : 1;
   long jchunk = ceil_div(n, P);
   P = (unsigned)ceil_div(n, jchunk > 0 ? jchunk : 1);
   if (P < 1) P = 1;
@@ -255,13 +239,13 @@ inline void launch_actback_biasgrad(hipStream_t stream, long m, long n, const T*
   }
   const dim3 grid((unsigned)(atiles * P));
   T* partial = static_cast<T*>(ws.partial);
-  const bool big = jchunk >= 64;
-#define KNET8_ABG(BT, U, SC) \
-  hipLaunchKernelGGL((actback_biasgrad_kernel<T, F, N, BT, U, SC>), grid, dim3(BT), 0, stream, dy, y, m, n, jchunk, P, dz, db, partial, ws.counters, f KNET8_TL_ARG)
+  const bool big = jchunk > 16;
+#define KNET8_ABG(BT, U, AL) \
+  hipLaunchKernelGGL((actback_biasgrad_kernel<T, F, N, BT, U, AL>), grid, dim3(BT), 0, stream, dy, y, m, n, jchunk, P, dz, db, partial, ws.counters, f KNET8_TL_ARG)
   // (sixteen waves, one column at a time each: (4096,2048) fp32 cold 19.2-19.4 us against 20.1-20.4 with two columns per wave and step, 20.8 with four or
   //  eight; 512 lanes x 32 parts 19.5, 256 lanes x 64 parts 22.1)
-  if (vec) { if (big) KNET8_ABG(1024, 1, false); else KNET8_ABG(256, 4, false); }
-  else     { if (big) KNET8_ABG(1024, 2, true); else KNET8_ABG(256, 4, true); }
+  if (vec) { if (big) KNET8_ABG(1024, 1, true); else KNET8_ABG(256, 4, true); }
+  else     { if (big) KNET8_ABG(1024, 1, false); else KNET8_ABG(256, 4, false); }
 #undef KNET8_ABG
 }
 

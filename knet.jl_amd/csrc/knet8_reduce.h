@@ -451,14 +451,14 @@ inline unsigned plan_parts(long groups, long units_per_group, long min_units_per
 // Parts of a split along an axis of d rows (or columns) per group, chosen by counting dependent memory round trips: a part's waves walk `per_trip` rows
 // per trip (sixteen waves with two rows in flight, or four with eight), the ticket costs two trips, and the workgroup that combines reads 128 partial rows
 // per trip when it has sixteen waves (parts of at least `big_from` rows) and 32 with four.  At most one workgroup per compute unit, parts of at least 16 rows.
-inline unsigned plan_parts_by_trips(long groups, long d, long per_trip, long big_from) {
+inline unsigned plan_parts_by_trips(long groups, long d, long per_trip, long big_from, long least = 16, long join = 2, long joined = 128) {
   const long ncu = tuning(kTuneNumCUs);
   long pmax = groups * 2 <= ncu ? ncu / groups : 1;
-  if (pmax > d / 16) pmax = d / 16;
+  if (pmax > d / least) pmax = d / least;
   if (pmax > 65535) pmax = 65535;
   auto trips = [&](long p) {
     const long rows = ceil_div(d, p);
-    return ceil_div(rows, per_trip) + (p > 1 ? ceil_div(p, rows >= big_from ? 128 : 32) + 2 : 0);
+    return ceil_div(rows, per_trip) + (p > 1 ? ceil_div(p, rows >= big_from ? joined : 32) + join : 0);
   };
   long best = trips(1);
   unsigned P = 1;

@@ -50,3 +50,21 @@ def test_few_rows_and_very_many_columns_on_both_sides_of_the_line(knet):
         z, u = dz.reshape(n, m).astype(np.float64), 2.0 ** -24
         assert (np.abs(knet.Array(db) - z.sum(axis=0)) <= n * u / (1 - n * u) * np.abs(z).sum(axis=0)).all()
     knet.libknet8().check()
+
+
+@pytest.mark.parametrize("m,n", [(64, 100), (10, 100), (300, 64), (33, 255)])
+def test_short_splits_without_scratch_go_unsplit(knet, m, n):
+    fn = knet.libknet8().fn
+    rng = np.random.default_rng(m)
+    dy, y = rng.integers(-9, 10, size=(2, m * n)).astype(np.float32)      # whole numbers: every order of the sum gives the same bits
+    dz = np.where(y > 0, dy, np.float32(0))
+    a, b, c = knet.KnetArray(dy), knet.KnetArray(y), knet.KnetArray(dtype=np.float32, dims=(m * n,))
+    for refuse in (1, 0):
+        db = knet.KnetArray(np.full(m, -777, np.float32))
+        fn["knet8_tune"](5, refuse)
+        try:
+            knet.knet8("reluback_biasgrad_32", m, n, a.ptr, b.ptr, c.ptr, db.ptr)
+            knet.libknet8().check()
+        finally:
+            fn["knet8_tune"](5, 0)
+        assert knet.Array(c).tobytes() == dz.tobytes() and np.array_equal(knet.Array(db), dz.reshape(n, m).sum(axis=0))

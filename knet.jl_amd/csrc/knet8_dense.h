@@ -74,7 +74,7 @@ template <typename T, int MODE>
 __global__ __launch_bounds__(kDbWaves * kWave) void dense_back_kernel(int act, int m, int n, int k, const T* __restrict__ W, const T* __restrict__ x,
                                                                       const T* __restrict__ y, const T* __restrict__ dy, T* __restrict__ dW,
                                                                       T* __restrict__ db, T* __restrict__ dx, int tiles_w, int tiles_w_m, int tiles_x_m,
-                                                                      int kslice_w, int kslice_x, bool vecw, bool vecz, const int* __restrict__ labels, T scale,
+                                                                      int kslice_w, int kslice_x, const int* __restrict__ labels, T scale,
                                                                       T* __restrict__ loss, T* __restrict__ mean, const T* __restrict__ bias, T* __restrict__ zout) {
   constexpr int TS = kDbTile, KS = kDbWaves;
   constexpr bool NLL = MODE >= 1, HEAD = MODE == 2;
@@ -117,8 +117,8 @@ __global__ __launch_bounds__(kDbWaves * kWave) void dense_back_kernel(int act, i
 #pragma unroll 4
       for (int kc = 0; kc < k; kc += 16) {
         T a[4], b[4];
-        mfma_load4<T, false>(a, wp, m, kc + 4 * kq, k, rok, false);   // W(class, kk): contiguous along the classes
-        mfma_load4<T, true>(b, xp, 1, kc + 4 * kq, k, cok, vecz);     // x(kk, col): contiguous along kk
+        mfma_load4<T, false>(a, wp, m, kc + 4 * kq, k, rok);   // W(class, kk): contiguous along the classes
+        mfma_load4<T, true>(b, xp, 1, kc + 4 * kq, k, cok);     // x(kk, col): contiguous along kk
 #pragma unroll
         for (int c = 0; c < 4; c++) za = Mfma16<T>::run(a[c], b[c], za);
       }
@@ -235,12 +235,12 @@ __global__ __launch_bounds__(kDbWaves * kWave) void dense_back_kernel(int act, i
 #pragma unroll 2
     for (int kc = kbeg; kc < kend; kc += 16) {
       T a[4], b[4];
-      mfma_load4<T, true>(a, wp, 1, kc + 4 * kq, kend, iok, vecw);
+      mfma_load4<T, true>(a, wp, 1, kc + 4 * kq, kend, iok);
       if (HEAD) {
 #pragma unroll
         for (int c = 0; c < 4; c++) b[c] = (jok && kc + 4 * kq + c < kend) ? zs[r16 * TS + kc + 4 * kq + c] : T(0);
       } else {
-        mfma_load4<T, true>(b, gp, 1, kc + 4 * kq, kend, jok, vecz);
+        mfma_load4<T, true>(b, gp, 1, kc + 4 * kq, kend, jok);
       }
       if (NLL) {
         // m <= 16: this one step holds every class of column j, four per lane in the lanes j, j+16, j+32, j+48
@@ -261,7 +261,7 @@ __global__ __launch_bounds__(kDbWaves * kWave) void dense_back_kernel(int act, i
       }
       if (relu) {
         T yy[4];
-        mfma_load4<T, true>(yy, yp, 1, kc + 4 * kq, kend, jok, vecz);
+        mfma_load4<T, true>(yy, yp, 1, kc + 4 * kq, kend, jok);
 #pragma unroll
         for (int c = 0; c < 4; c++) b[c] = yy[c] > T(0) ? b[c] : T(0);   // masked-out lanes hold zeros in both
       }
@@ -312,22 +312,25 @@ template <typename T, int MODE>
 inline int launch_dense_back_impl(hipStream_t stream, int act, int m, int n, int k, const T* W, const T* x, const T* y, const T* dy, T* dW, T* db, T* dx,
                                   const int* labels, T scale, T* loss, T* mean, const T* bias = nullptr, T* zout = nullptr) {
   constexpr bool NLL = MODE >= 1;
-  // both products have 2*m*n*k flop; kernel durations against reluback_biasgrad + two gemm launches (us, kernel trace): 64x100x784
-  // 3.6/11.3, 256^3 5.2/12.6, 300^3 7.3/14.8, 512x128x512 9.6/14.1, 400^3 11.9/18.8, 512^3 20.8/26.2 -- one launch wins over the whole range of
-  // the small-product kernels (2.7e8 flop); beyond it the separate launches reach the vendor library's large tiles
-  if (2.0 * m * n * (double)k > 1.0e6 * tuning(kTuneDenseBackMflop) || (db != nullptr && dW == nullptr)) return 1;
+  // Both products have 2*m*n*k flop; kernel durations against reluback_biasgrad + two gemm launches (us, kernel trace): 64x100x784
+  // 3.6/11.3, 256^3 5.2/12.6, 300^3 7.3/14.8, 512x128x512 9.6/14.1, 400^3 11.9/18.8, 512^3 20.8/26.2; beyond 2.7e8 flop the separate launches reach the
+  // vendor library's large tiles.
+  const double flop = 2.0 * m * n * (double)k;
+  if (flop > 1.0e6 * tuning(kTuneDenseBackMflop) || (db != nullptr && dW == nullptr)) return 1;
   const int tw_m = (m + kDbTile - 1) / kDbTile, tw_n = (k + kDbTile - 1) / kDbTile;
   const int tx_m = (k + kDbTile - 1) / kDbTile, tx_n = (n + kDbTile - 1) / kDbTile;
   const int tiles_w = dW ? tw_m * tw_n : 0, tiles_x = dx ? tx_m * tx_n : 0;
+  // A tile walks its whole inner dimension in one workgroup, and every tile reads its edges afresh.  So layers that have much of both, or very many tiles, are
+  // quicker in separate launches.  us a call over 326 layers up to the limit above (one launch / three; with dx): 33x1538x819 27.3/20.4, 3293x198x166 48.5/28.3,
+  // 1539x19x2714 (16830 tiles) 55.7/24.7; without dx 347x1741x77 27.5/16.5.  Inside the lines: 1265x146x232 14.6/17.8, 400^3 as above, fp64 96x1146x65 13.3/18.2.
+  // (The loss forms have no separate launches to fall back on here and keep their range.)
+  const int inner = tiles_x > 0 && m > n ? m : n;
+  if (!NLL && (flop * inner > 1.4e11 || (dW != nullptr && n > 1500) || (long)tiles_w + tiles_x > 8192)) return 1;
   if (tiles_w + tiles_x == 0) return 0;
   // inner dimension per wave, in whole 16-deep steps
   auto slice = [](int K) { const int steps = (K + 15) / 16; return ((steps + kDbWaves - 1) / kDbWaves) * 16; };
-  // 16-byte (fp64: 32-byte) loads along the inner dimension of dx = W'*dz need columns of W, dy and y that start on such a boundary
-  const bool vecw = W != nullptr && mfma_vec_ok(W, m);
-  // (head form: the flag covers the loads of x along its inner dimension instead)
-  const bool vecz = MODE == 2 ? mfma_vec_ok(x, k) : NLL ? mfma_vec_ok(y, m) : (mfma_vec_ok(dy, m) && (act != 1 || mfma_vec_ok(y, m)));
   hipLaunchKernelGGL((dense_back_kernel<T, MODE>), dim3((unsigned)(tiles_w + tiles_x)), dim3(kDbWaves * kWave), 0, stream, act, m, n, k, W, x, y, dy, dW, db, dx,
-                     tiles_w, tw_m, tx_m, slice(n), slice(m), vecw, vecz, labels, scale, loss, mean, bias, zout);
+                     tiles_w, tw_m, tx_m, slice(n), slice(m), labels, scale, loss, mean, bias, zout);
   return 0;
 }
 

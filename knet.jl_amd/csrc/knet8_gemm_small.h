@@ -110,7 +110,8 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(int m, int n, int k, T 
 // 4*r + l/16 in fp64 (r = 0..3).  The operands go from global memory straight into the instruction's registers -- no LDS staging, no
 // barrier inside the k walk.  Which k a lane feeds to which of the four instructions of a 16-deep step is free as long as A and B
 // agree: lane (.., q = l/16) takes k = 4q .. 4q+3, so an operand that is contiguous along k is read with one 16-byte (fp64: 32-byte)
-// load per lane and step -- with 4-byte loads the sixteen lines a wave touches per instruction keep the CU's address unit busy four
+// load per lane and step, wherever its columns start (odd leading dimensions in fp32, one element a load -> so: TN 450x79x1125 13.2 -> 5.4 us, 221x1259x431 22.8 -> 9.0;
+// over 109 products of 10 to 2000 each way TN 1.41x, NN 1.25x) -- with 4-byte loads the sixteen lines a wave touches per instruction keep the CU's address unit busy four
 // times as long, and the sixteen waves of a workgroup share it.  The KS waves of a workgroup take KS slices of k (every wave of
 // the product has all its loads in flight at once) and their partial tiles meet in LDS: no combine leaves the workgroup.
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -129,9 +130,9 @@ template <> struct Mfma16<double> {
 
 // Four consecutive k of one operand column (or row) for a lane: p points at k = 0 of it, `step` is the distance between consecutive k.
 template <typename T, bool KCONT>
-__device__ __forceinline__ void mfma_load4(T (&v)[4], const T* __restrict__ p, long step, int kk0, int kend, bool ok, bool vec) {
-  typedef T V4 __attribute__((ext_vector_type(4)));
-  if (KCONT && vec && ok && kk0 + 3 < kend) {
+__device__ __forceinline__ void mfma_load4(T (&v)[4], const T* __restrict__ p, long step, int kk0, int kend, bool ok) {
+  typedef T V4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));   // at any element boundary
+  if (KCONT && ok && kk0 + 3 < kend) {
     const V4 q = *reinterpret_cast<const V4*>(p + kk0);
 #pragma unroll
     for (int c = 0; c < 4; c++) v[c] = q[c];
@@ -140,12 +141,10 @@ __device__ __forceinline__ void mfma_load4(T (&v)[4], const T* __restrict__ p, l
     for (int c = 0; c < 4; c++) v[c] = (ok && kk0 + c < kend) ? p[(kk0 + c) * step] : T(0);
   }
 }
-template <typename T>
-inline bool mfma_vec_ok(const T* p, int ld) { return (reinterpret_cast<uintptr_t>(p) % (4 * sizeof(T))) == 0 && ld % 4 == 0; }
 
 template <typename T, bool TA, bool TB, int KS>
 __global__ __launch_bounds__(KS * kWave) void gemm_mfma_kernel(int m, int n, int k, T alpha, const T* __restrict__ A, int lda, const T* __restrict__ B,
-                                                              int ldb, T beta, T* C, int ldc, const T* bias, int act, int kslice, bool veca, bool vecb) {
+                                                              int ldb, T beta, T* C, int ldc, const T* bias, int act, int kslice) {
   constexpr int TS = 16;
   __shared__ T part[KS > 1 ? KS : 1][TS * TS];   // part[w][j*16 + i]
   const int tiles_m = (m + TS - 1) / TS;
@@ -166,8 +165,8 @@ __global__ __launch_bounds__(KS * kWave) void gemm_mfma_kernel(int m, int n, int
 #pragma unroll 4
   for (int kc = kbeg; kc < kend; kc += 16) {
     T a[4], b[4];
-    mfma_load4<T, TA>(a, ap, astep, kc + 4 * kq, kend, iok, veca);
-    mfma_load4<T, !TB>(b, bp, bstep, kc + 4 * kq, kend, jok, vecb);
+    mfma_load4<T, TA>(a, ap, astep, kc + 4 * kq, kend, iok);
+    mfma_load4<T, !TB>(b, bp, bstep, kc + 4 * kq, kend, jok);
 #pragma unroll
     for (int c = 0; c < 4; c++) acc = Mfma16<T>::run(a[c], b[c], acc);
   }
@@ -206,7 +205,8 @@ inline bool gemm_is_small(int m, int n, int k) {
 // 1024x1024x64 5.7/10.4, 6.2/10.3, 6.0/10.3; 512^3 8.3/10.1, 9.8/10.2, 8.6/10.4.  Against them:
 //   many tiles: 2048x2048x16 12.0/10.4, 3000x3000x4 23.6/16.2, 8192x8192x1 123/50 (a workgroup of one wave to a tile); from 4300 tiles on 30000x64x64 11.0/10.0;
 //   a short side, which leaves few tiles a long walk: 10000x16x784 11.6/10.4, NT 48x3000x600 12.0/10.6; k beyond 2048: 16x16x4096 12.4/10.2;
-//   an operand along k that does not come in 16-byte loads: TN 900x900x150 18.8/10.4, 4096x128x150 12.5/10.4.
+//   an operand along k whose columns start off the 16-byte boundaries and short k, which is then many tiles: 753x594x279 10.6/7.2, 1746x78x635 NN 9.6/7.3; from k = 400 on it is
+//   ahead further up: TN 828x60x1309 6.1/10.8, 83x553x1651 7.4/10.8.
 // fp64, whose vendor kernels are weak on short sides: 1000x100x1000 14/23, 15/38, 14/21; 16x2048x4096 24/55, 31/115, 21/55; 320x320x300 5.9/9.9; short k: 1024x1024x16 5.7/6.2.
 // The other way round with many tiles: 512^3 14.7/15.0, 17.1/13.8, 768x768x128 10.1/8.7, 100x8192x64 9.2/8.0, 100x2000x400 13.0/12.2.
 template <typename T>
@@ -217,7 +217,7 @@ inline bool gemm_is_small_by_rule(bool ta, bool tb, int m, int n, int k, int lda
   const int side = m < n ? m : n;
   double limit = side >= 128 ? 2.7e8 : side > 64 ? 2.4e8 : tb ? 1.5e8 : 2.1e8;
   if (tiles > 4300 && limit > 1.5e8) limit = 1.5e8;
-  if ((ta && lda % 4 != 0) || (!tb && ldb % 4 != 0)) limit = 1.2e8;
+  if (((ta && lda % 4 != 0) || (!tb && ldb % 4 != 0)) && limit > (k >= 400 ? 2.1e8 : 1.2e8)) limit = k >= 400 ? 2.1e8 : 1.2e8;
   return k <= 2048 && tiles <= 8192 && flop <= limit;
 }
 
@@ -237,8 +237,7 @@ inline void launch_gemm_small(hipStream_t stream, bool ta, bool tb, int m, int n
     while (ks < 16 && ks < ksteps) ks *= 2;
     const int kslice = (int)((ksteps + ks - 1) / ks) * kGsTile;
     const dim3 grid16((unsigned)tiles16);
-    const bool veca = ta && mfma_vec_ok(A, lda), vecb = !tb && mfma_vec_ok(B, ldb);
-#define KNET8_GM16K(TA, TB, KSX) hipLaunchKernelGGL((gemm_mfma_kernel<T, TA, TB, KSX>), grid16, dim3(KSX * kWave), 0, stream, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, bias, act, kslice, veca, vecb)
+#define KNET8_GM16K(TA, TB, KSX) hipLaunchKernelGGL((gemm_mfma_kernel<T, TA, TB, KSX>), grid16, dim3(KSX * kWave), 0, stream, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, bias, act, kslice)
 #define KNET8_GM16(TA, TB) do { if (ks == 1) KNET8_GM16K(TA, TB, 1); else if (ks == 2) KNET8_GM16K(TA, TB, 2); else if (ks == 4) KNET8_GM16K(TA, TB, 4); \
                                 else if (ks == 8) KNET8_GM16K(TA, TB, 8); else KNET8_GM16K(TA, TB, 16); } while (0)
     if (!ta && !tb) KNET8_GM16(false, false);

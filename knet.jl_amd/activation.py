@@ -100,11 +100,23 @@ eluback = _second_order("eluback", _negative_part)
 seluback = _second_order("seluback", _negative_part)
 
 
+class ActBack:
+    """``@primitive relu(x),dy,y reluback.(dy,y)`` (src/ops20/activation.jl:28) and the other four."""
+    __slots__ = ("name", "y")
+    ends_layer = True
+
+    def __init__(self, name, y):
+        self.name, self.y = name, y
+
+    def __call__(self, dy):
+        return (back11_op(self.name, dy, self.y),)
+
+
 def _activation(name, back):
     @primitive
     def f(x):
         y = unary_op(name, x)
-        return y, (lambda dy: (back11_op(back, dy, y),))  # @primitive relu(x),dy,y reluback.(dy,y)  (src/ops20/activation.jl:28)
+        return y, ActBack(back, y)
 
     f.__name__ = name
     return f

@@ -104,6 +104,11 @@ def selective(back):
     return back
 
 
+def layer_back(nodes, i):
+    """Set by the module of the matrix products: the gradients of a layer's end ``nodes[i]`` and of what it rests on, in fewer launches.  False: not one it knows."""
+    return False
+
+
 def addto(a, b):
     """``addto!(a,b)``: accumulate a gradient (src/autograd_gpu/addto.jl:7-10: ``axpy!(1,b,a)``)."""
     if a is None:
@@ -113,6 +118,11 @@ def addto(a, b):
         from .binary import broadcast_op
         return broadcast_op("add", a, b)
     return a + b
+
+
+def give(node, g):
+    """One more gradient of a node."""
+    node.outgrad = g if node.outgrad is None else addto(node.outgrad, g)
 
 
 class Result:
@@ -143,8 +153,12 @@ def diff(f):
         out.outgrad = 1.0  # a scalar kept on the device (1-element array): see nll(..., fused=True) with device labels
     else:
         out.outgrad = type(v)(1) if isinstance(v, (np.floating, float)) else 1.0
-    for node in reversed(tape.nodes):
+    nodes = tape.nodes
+    for i in range(len(nodes) - 1, -1, -1):
+        node = nodes[i]
         if node.outgrad is None or node.back is None:
+            continue
+        if getattr(node.back, "ends_layer", False) and layer_back(nodes, i):
             continue
         if getattr(node.back, "selective", False):
             # like AutoGrad, which evaluates a primitive's gradient expression only for the arguments that are tracked:
@@ -154,7 +168,7 @@ def diff(f):
             grads = node.back(node.outgrad)
         for parent, g in zip(node.parents, grads):
             if parent is not None and g is not None:
-                parent.outgrad = g if parent.outgrad is None else addto(parent.outgrad, g)
+                give(parent, g)
         if node.param is None:
             # Dead from here on: drop the gradient, the value and the closure that holds the saved activations, so their
             # device blocks go back to the pool while the sweep is still running -- what the reference's tape-aware

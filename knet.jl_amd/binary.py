@@ -168,10 +168,21 @@ def _neg(a):
     return broadcast_op("mul", -1, a) if isinstance(a, KnetArray) else -a
 
 
+class AddBack:
+    __slots__ = ("x", "y")
+    selective = True
+
+    def __init__(self, x, y):
+        self.x, self.y = x, y
+
+    def __call__(self, dy, need=(True, True)):
+        return unbroadcast(self.x, dy) if need[0] else None, unbroadcast(self.y, dy) if need[1] else None
+
+
 @primitive
 def add(x, y):
     """``x .+ y``; gradients ``unbroadcast(x,dy)``, ``unbroadcast(y,dy)``."""
-    return broadcast_op("add", x, y), selective(lambda dy, need=(True, True): (unbroadcast(x, dy) if need[0] else None, unbroadcast(y, dy) if need[1] else None))
+    return broadcast_op("add", x, y), AddBack(x, y)
 
 
 @primitive

@@ -341,7 +341,7 @@ template <typename T> __device__ __forceinline__ MaxSum<T> ms_wave_reduce(MaxSum
 // The labelled logit is re-read by lane 0 of the team (one scalar load, issued with the others) instead of being
 // fished out of the register that happens to hold it.  Columns are cut into head / vectors / tail as in softmax_col_kernel.
 // LV > 0: the last LV vectors of each lane live in LDS, as in softmax_col_body.
-template <typename T, int TEAM, int E, bool VEC, int LV>
+template <typename T, int TEAM, int E, bool VEC, int LV, bool LATE>
 __device__ __forceinline__ void nll_col_body(int m, long n, const T* a, T* out, const int* labels, T scale, T* loss KNET8_TL_PARAM) {
   KNET8_TL_BEGIN
   constexpr int BT = TEAM == kWave ? kWaveTeamBlock : TEAM;
@@ -368,9 +368,14 @@ __device__ __forceinline__ void nll_col_body(int m, long n, const T* a, T* out, 
   const int tpos = head + nb * NV + tl;
   const T ninf = T(-INFINITY);
 
-  // the label may stand in host memory: one request a column, made before the column's own loads and not waited for until they are under way
+  // LATE: the label may stand in host memory: one request a column, made before the column's own loads and not waited for until they are under way
   __shared__ int lds_lab;
-  int lab = colok && (NW == 1 || threadIdx.x < kWave) ? labels[col] : 0;
+  int lab = colok && (!LATE || NW == 1 || threadIdx.x < kWave) ? labels[col] : 0;
+  T alab;
+  if constexpr (!LATE) {
+    if (lab < 0 || lab > m) lab = 0;  // callers check labels on the host; an out-of-range one is skipped, never dereferenced
+    alab = (tl == 0 && lab > 0) ? ac[lab - 1] : T(0);
+  }
   V rv[RI];
   // the LDS slots are filled by loads that go from memory to LDS directly (lane t's 16 bytes land at the wave's base + 16 t), no register in between;
   // a slot beyond the lane's share stays unwritten and is never read
@@ -390,8 +395,10 @@ __device__ __forceinline__ void nll_col_body(int m, long n, const T* a, T* out, 
     }
   }
   T xh = hv ? ac[tl] : ninf, xt = tv ? ac[tpos] : ninf;  // -inf padding contributes exp(-inf) = 0
-  if (lab < 0 || lab > m) lab = 0;  // callers check labels on the host; an out-of-range one is skipped, never dereferenced
-  const T alab = (tl == 0 && lab > 0) ? ac[lab - 1] : T(0);
+  if constexpr (LATE) {
+    if (lab < 0 || lab > m) lab = 0;
+    alab = (tl == 0 && lab > 0) ? ac[lab - 1] : T(0);
+  }
 
   T mt = ninf;
 #pragma unroll
@@ -439,16 +446,20 @@ __device__ __forceinline__ void nll_col_body(int m, long n, const T* a, T* out, 
   if (NW > 1) {
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     if (lane == 0) { lds_m[wave] = ms.m; lds_s[wave] = ms.s; }
-    if (threadIdx.x == 0) lds_lab = lab;
+    if (LATE && threadIdx.x == 0) lds_lab = lab;
     __syncthreads();
-    lab = lds_lab;
+    if (LATE) lab = lds_lab;
     MaxSum<T> t = {lane < NW ? lds_m[lane] : ninf, lane < NW ? lds_s[lane] : T(0)};
     ms = ms_wave_reduce(t);
   }
   const T logS = dev_log(ms.s);
   // softmax_i = e_i * exp(m_t - M) / S; fold the upstream scale in: one multiply per element
   const T f = (mt == ninf ? T(0) : dev_exp(mt - ms.m) / ms.s) * scale;
-  if (colok && tl == 0) loss[col] = lab > 0 ? -((alab - ms.m) - logS) : T(0);
+  // (asked for late, the labelled logit arrives last: in fp32 the loss waits for it behind the output, (1000,4096) 7.03 -> 6.85 us; fp64 has no registers to keep it, (1000,512) 5.3 -> 5.7)
+  constexpr bool kLossLast = LATE && sizeof(T) == 4;
+  if constexpr (!kLossLast) {
+    if (colok && tl == 0) loss[col] = lab > 0 ? -((alab - ms.m) - logS) : T(0);
+  }
   KNET8_TL_MID
 #pragma unroll
   for (int i = 0; i < ITEMS; i++) {
@@ -471,19 +482,24 @@ __device__ __forceinline__ void nll_col_body(int m, long n, const T* a, T* out, 
     if (hv) oc[tl] = lab == 0 ? T(0) : ((tl + 1 == lab) ? -scale : T(0)) + xh * f;
     if (tv) oc[tpos] = lab == 0 ? T(0) : ((tpos + 1 == lab) ? -scale : T(0)) + xt * f;
   }
+  if constexpr (kLossLast) {
+    if (colok && tl == 0) loss[col] = lab > 0 ? -((alab - ms.m) - logS) : T(0);
+  }
   KNET8_TL_END
 }
 
-template <typename T, int TEAM, int E, bool VEC>
+// LATE costs where the labels are on the device: (1000,4096) fp64 13.0 us, 12.4 without.
+template <typename T, int TEAM, int E, bool VEC, bool LATE>
 __global__ __launch_bounds__(TEAM == kWave ? kWaveTeamBlock : TEAM) void nll_col_kernel(int m, long n, const T* a, T* out, const int* labels,
                                                                             T scale, T* loss KNET8_TL_PARAM) {
-  nll_col_body<T, TEAM, E, VEC, 0>(m, n, a, out, labels, scale, loss KNET8_TL_PASS);
+  nll_col_body<T, TEAM, E, VEC, 0, LATE>(m, n, a, out, labels, scale, loss KNET8_TL_PASS);
 }
-// four waves per SIMD (two 512-lane workgroups per compute unit): at most 128 registers per lane
-template <typename T, int TEAM, int E, int LV>
+// four waves per SIMD (two 512-lane workgroups per compute unit): at most 128 registers per lane.  Labels on the device are read first here: (32000,512) fp64 44.2 us
+// with the label waited for late, 42.2 so.
+template <typename T, int TEAM, int E, int LV, bool LATE>
 __global__ __launch_bounds__(TEAM) __attribute__((amdgpu_waves_per_eu(4, 4))) void nll_col_lds_kernel(int m, long n, const T* a, T* out,
                                                                                                       const int* labels, T scale, T* loss) {
-  nll_col_body<T, TEAM, E, true, LV>(m, n, a, out, labels, scale, loss KNET8_TL_NONE);
+  nll_col_body<T, TEAM, E, true, LV, LATE>(m, n, a, out, labels, scale, loss KNET8_TL_NONE);
 }
 
 // ---- many short columns -----------------------------------------------------------------------------------
@@ -984,7 +1000,7 @@ inline void launch_softmax_strided(hipStream_t stream, long inner, long d, long 
 
 template <typename T, typename Algo, int TEAM, int E>
 inline void launch_softmax_cfg(hipStream_t stream, bool vec, int m, long n, const T* a, const T* b, T* out, const int* labels,
-                               T scale, T* loss) {
+                               T scale, T* loss, bool host_labels) {
   constexpr int BT = TEAM == kWave ? kWaveTeamBlock : TEAM;
   constexpr int TEAMS = BT / TEAM;
   const dim3 block(BT);
@@ -993,8 +1009,10 @@ inline void launch_softmax_cfg(hipStream_t stream, bool vec, int m, long n, cons
   // between them.)
   const dim3 grid((unsigned)((n + TEAMS - 1) / TEAMS));
   if constexpr (Algo::kNll) {
-    if (vec) hipLaunchKernelGGL((nll_col_kernel<T, TEAM, E, true>), grid, block, 0, stream, m, n, a, out, labels, scale, loss KNET8_TL_ARG);
-    else hipLaunchKernelGGL((nll_col_kernel<T, TEAM, E, false>), grid, block, 0, stream, m, n, a, out, labels, scale, loss KNET8_TL_ARG);
+#define KNET8_NLL(VEC, LATE) hipLaunchKernelGGL((nll_col_kernel<T, TEAM, E, VEC, LATE>), grid, block, 0, stream, m, n, a, out, labels, scale, loss KNET8_TL_ARG)
+    if (host_labels) { if (vec) KNET8_NLL(true, true); else KNET8_NLL(false, true); }
+    else { if (vec) KNET8_NLL(true, false); else KNET8_NLL(false, false); }
+#undef KNET8_NLL
   } else {
     if (vec) hipLaunchKernelGGL((softmax_col_kernel<T, Algo, TEAM, E, true>), grid, block, 0, stream, m, n, a, b, out KNET8_TL_ARG);
     else hipLaunchKernelGGL((softmax_col_kernel<T, Algo, TEAM, E, false>), grid, block, 0, stream, m, n, a, b, out KNET8_TL_ARG);
@@ -1010,7 +1028,7 @@ inline bool softmax_is_short(long m, long n) {
 }
 
 template <typename T, typename Algo>
-inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const T* b, T* out, const int* labels, T scale, T* loss) {
+inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const T* b, T* out, const int* labels, T scale, T* loss, bool host_labels = false) {
   if (m <= 0 || n <= 0) return;
   constexpr int N = Vec16<T>::N;
   // Per-lane capacity: the 1024-lane workgroup is limited to 128 registers per lane, i.e. 64 fp32 / 32 fp64 held elements (half with two held
@@ -1027,7 +1045,7 @@ inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const
   const bool vec = ma == mo && ma == mb && ma % sizeof(T) == 0;
   const bool vec_stream = (m % N == 0) && ma == 0 && mo == 0 && mb == 0;
   const long resident_cap = tuning(kTuneSoftmaxResidentRows);  // 0: no limit below the register capacity (tests lower it to reach the streaming kernel with short columns)
-#define KNET8_SM(TEAM, E) launch_softmax_cfg<T, Algo, TEAM, E>(stream, vec, (int)m, n, a, b, out, labels, scale, loss)
+#define KNET8_SM(TEAM, E) launch_softmax_cfg<T, Algo, TEAM, E>(stream, vec, (int)m, n, a, b, out, labels, scale, loss, host_labels)
   if (softmax_is_short<T, Algo>(m, n)) {
     // stretches of whole columns (see softmax_short_kernel): G columns per workgroup, starting on 16-byte boundaries on the vector path
     constexpr int cap = 256 * short_stretch_vectors<T, Algo>() * N;
@@ -1129,7 +1147,10 @@ inline void launch_softmax(hipStream_t stream, long m, long n, const T* a, const
   if constexpr (Algo::kInputs == 1 && (!Algo::kNll || sizeof(T) == 8)) {
     constexpr int kLdsE = 32 * N;   // 32 vectors per lane, 512 lanes: columns of up to 256 KB (32768 fp64 or 65536 fp32 rows)
     if (vec && m > 1024 * (kBig1024 / 2) && m <= 512 * kLdsE && tuning(kTuneSoftmaxNoLdsSlots) == 0) {
-      if constexpr (Algo::kNll) hipLaunchKernelGGL((nll_col_lds_kernel<T, 512, kLdsE, 9>), dim3((unsigned)n), dim3(512), 0, stream, (int)m, n, a, out, labels, scale, loss);
+      if constexpr (Algo::kNll) {
+        if (host_labels) hipLaunchKernelGGL((nll_col_lds_kernel<T, 512, kLdsE, 9, true>), dim3((unsigned)n), dim3(512), 0, stream, (int)m, n, a, out, labels, scale, loss);
+        else hipLaunchKernelGGL((nll_col_lds_kernel<T, 512, kLdsE, 9, false>), dim3((unsigned)n), dim3(512), 0, stream, (int)m, n, a, out, labels, scale, loss);
+      }
       else hipLaunchKernelGGL((softmax_col_lds_kernel<T, Algo, 512, kLdsE, 9>), dim3((unsigned)n), dim3(512), 0, stream, (int)m, n, a, b, out);
       return;
     }
@@ -1191,7 +1212,7 @@ inline T nll_host(hipStream_t stream, int m, int n, const T* x, const long long*
     }
     T* const slot = from ? static_cast<T*>(scalar_slot(stream)) : nullptr;
     if (slot) {
-      launch_softmax<T, AlgoNll<T>>(stream, m, n, x, (const T*)nullptr, dx, from, scale, loss);
+      launch_softmax<T, AlgoNll<T>>(stream, m, n, x, (const T*)nullptr, dx, from, scale, loss, from == to);
       const bool launched = launch_reduce_run<T, RedSum<T>>(stream, loss, (long)n, 1, 1, slot);
       check_launch("nll_host");
       if (w.held) w.held.unlock();

@@ -234,9 +234,10 @@ inline void launch_actback_biasgrad(hipStream_t stream, long m, long n, const T*
   if (P < 1) P = 1;
   Workspace ws;
   if (P > 1) {
-    // Up to 255 columns a split only saves time: without scratch one workgroup walks them all.  More are refused: out of memory is an error to report.
+    // Up to 255 columns a split only saves time: without scratch, and in the first such launch of a stream if that is being captured, one workgroup walks them all.  More
+    // are refused without it: out of memory is an error to report.
     const bool optional = n < 256;
-    ws = workspace_for(stream, sizeof(T) * (size_t)atiles * P * tile, (size_t)atiles * kTicketStride, optional);
+    ws = workspace_for(stream, sizeof(T) * (size_t)atiles * P * tile, (size_t)atiles * kTicketStride, optional, optional);
     if (optional && (ws.partial == nullptr || ws.counters == nullptr)) { P = 1; jchunk = n; }
     else if (!scratch_ready(ws, "activation gradient + bias gradient: no scratch memory for a split launch")) return;
   }

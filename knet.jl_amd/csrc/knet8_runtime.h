@@ -29,7 +29,8 @@ struct Workspace {
   std::unique_lock<std::recursive_mutex> held;
 };
 // optional: the caller does without when there is none, so a failure is not recorded.
-Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounters, bool optional = false);
+// (spare_capture: nothing is allocated for a stream under capture, where an allocation may end the capture; what it has already is given out)
+Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounters, bool optional = false, bool spare_capture = false);
 // Where a split launch takes its scratch from: the per-stream buffers above (a null source) or a caller-supplied provider.  A provider
 // that cannot serve the request records why and returns null pointers.
 struct ScratchSource {

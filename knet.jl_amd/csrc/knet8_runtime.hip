@@ -160,7 +160,7 @@ __global__ __launch_bounds__(256) void zero_counters_kernel(unsigned* c, size_t 
   if (i < n) c[i] = 0u;
 }
 
-Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounters, bool optional) {
+Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounters, bool optional, bool spare_capture) {
   if (g_tune[kTuneFailScratch] != 0) {   // set by tests: behave as if the device were out of memory, without touching it
     if (!optional) record_error("reduction scratch: allocation refused (knet8_tune key 5 is set)");
     return Workspace();
@@ -175,6 +175,7 @@ Workspace workspace_for(hipStream_t stream, size_t partial_bytes, size_t ncounte
   w.held = hold_scratch(stream);
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
   StreamScratch& s = scratch_of(stream);
+  if (spare_capture && capturing && (s.partial_bytes < partial_bytes || s.ncounters < ncounters)) return w;
   if (capturing) s.in_graph = true;
   // Buffers that have become too small are retired, not freed: launches already queued on the stream, and graphs
   // captured on it, keep using their addresses.  Sizes grow geometrically, so the retired ones add up to less than

@@ -1,4 +1,6 @@
 """``Fback_biasgrad_S`` where rows do not start on 16-byte boundaries: the straddling lane, the last tile of one to three rows, few rows, in place."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -68,3 +70,38 @@ def test_short_splits_without_scratch_go_unsplit(knet, m, n):
         finally:
             fn["knet8_tune"](5, 0)
         assert knet.Array(c).tobytes() == dz.tobytes() and np.array_equal(knet.Array(db), dz.reshape(n, m).sum(axis=0))
+
+
+def test_the_first_call_of_a_stream_may_be_captured(knet):
+    """A stream's first short split, under capture: nothing is allocated there, one workgroup walks the columns, and replays between eager splits keep their results."""
+    fn = knet.libknet8().fn
+    m, n = 64, 100
+    rng = np.random.default_rng(8)
+    dy, y = rng.integers(-9, 10, size=(2, m * n)).astype(np.float32)
+    dz = np.where(y > 0, dy, np.float32(0))
+    a, b, c, db = knet.KnetArray(dy), knet.KnetArray(y), knet.KnetArray(dtype=np.float32, dims=(m * n,)), knet.KnetArray(dtype=np.float32, dims=(m,))
+    knet.synchronize()
+    stream = fn["knet8_stream_create"]()
+    try:
+        stats = (ctypes.c_ulonglong * 6)()
+        fn["knet8_stats"](ctypes.cast(stats, ctypes.c_void_p))
+        before = stats[0]
+        assert fn["knet8_graph_begin"](stream) == 0
+        fn["reluback_biasgrad_32_stream"](m, n, a.ptr, b.ptr, c.ptr, db.ptr, stream)
+        graph = fn["knet8_graph_end"](stream)
+        fn["knet8_stats"](ctypes.cast(stats, ctypes.c_void_p))
+        assert graph and stats[0] == before
+        for turn in range(3):
+            knet.fill(db, -777)
+            knet.fill(c, -777)
+            knet.synchronize()
+            assert fn["knet8_graph_launch"](graph, stream) == 0 and fn["knet8_synchronize"](stream) == 0
+            assert np.array_equal(knet.Array(db), dz.reshape(n, m).sum(axis=0)) and knet.Array(c).tobytes() == dz.tobytes()
+            knet.fill(db, -777)
+            knet.synchronize()
+            fn["reluback_biasgrad_32_stream"](m, n, a.ptr, b.ptr, c.ptr, db.ptr, stream)      # eager, split: the stream's scratch is made now
+            assert fn["knet8_synchronize"](stream) == 0 and np.array_equal(knet.Array(db), dz.reshape(n, m).sum(axis=0))
+        fn["knet8_graph_destroy"](graph)
+    finally:
+        fn["knet8_stream_destroy"](stream)
+    knet.libknet8().check()

@@ -619,7 +619,7 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   const long wgs = ny * (long)P;
   const int bt = chunk <= 2 * kWave ? 64 : !slabs ? (chunk <= 4096 ? 256 : 512) : chunk <= (ny > 2 * ncu ? 4096 : 1024) || ny > 3 * ncu ? 256 : chunk > 2048 && wgs <= (any ? ncu : ncu / 8 * 7) ? 1024 : 512;
   const dim3 grid((unsigned)wgs);
-  const long usy = vec ? sy / N : any ? ceil_div(sy, N) : sy;   // units per run
+  const long usy = sy == 0 ? 1 : vec ? sy / N : any ? ceil_div(sy, N) : sy;   // units per run (no elements at all: none is walked, any number will do)
 #define KNET8_RUN(NV, SINGLE, BT, U, ANY) \
   hipLaunchKernelGGL((reduce_run_kernel<T, Op, NV, SINGLE, BT, U, ANY>), grid, dim3(BT), 0, stream, x, sy, ny, units, chunk, P, y, partial, ws.counters, center, (unsigned)(BT / usy), (unsigned)(BT % usy) KNET8_TL_ARG)
   // (the path with loads of one element, for short runs that do not start on 16-byte boundaries, keeps four times as many in flight per lane to move the same bytes)

@@ -134,14 +134,18 @@ typedef struct {
 enum { kOther = 2 };
 static PyTypeObject ArrayType;
 
-/* The dtype object for what the caller named (a new reference): one of the three, or what numpy makes of it. */
+/* The dtype object for what the caller named (a new reference): one of the three, or what numpy makes of it.  numpy has several objects for one type (every dtype that comes
+ * out of a pickle is a new one, and what is made of such an array carries it on): they count as the one they are equal to. */
 static PyObject* as_dtype(PyObject* d, int* type, Py_ssize_t* itemsize) {
   for (int i = 0; i < 3; i++)
     if (d == g_dtypes[i]) { *type = i; *itemsize = g_itemsize[i]; Py_INCREF(d); return d; }
   PyObject* n = PyObject_CallFunctionObjArgs(g_dtype_class, d, NULL);
   if (!n) return NULL;
-  for (int i = 0; i < 3; i++)
-    if (n == g_dtypes[i]) { *type = i; *itemsize = g_itemsize[i]; return n; }
+  for (int i = 0; i < 3; i++) {
+    const int same = n == g_dtypes[i] ? 1 : PyObject_RichCompareBool(n, g_dtypes[i], Py_EQ);
+    if (same < 0) { Py_DECREF(n); return NULL; }
+    if (same) { *type = i; *itemsize = g_itemsize[i]; Py_INCREF(g_dtypes[i]); Py_DECREF(n); return g_dtypes[i]; }
+  }
   PyObject* size = PyObject_GetAttrString(n, "itemsize");
   *itemsize = size ? PyLong_AsSsize_t(size) : -1;
   *type = kOther;

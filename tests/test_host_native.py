@@ -3,6 +3,7 @@ import copy
 import ctypes
 import gc
 import itertools
+import pickle
 import sys
 
 import numpy as np
@@ -129,3 +130,31 @@ def test_similar_refuses_what_it_refused(knet):
     for args, kw in (((1, 2, 3), {}), ((), {"shape": (2,)}), ((5,), {}), ((("a",),), {})):
         with pytest.raises((TypeError, ValueError)):
             x.similar(*args, **kw)
+
+
+@pytest.mark.parametrize("dt,suffix", [(np.float32, "32"), (np.float64, "64"), (np.int32, None)])
+def test_element_types_are_told_by_equality(knet, monkeypatch, dt, suffix):
+    """A pickled array comes back with a dtype object of its own, and slices, products and transposes of it carry that on."""
+    a = pickle.loads(pickle.dumps(np.ones((3, 4), dt)))
+    assert a.dtype == dt and a.dtype is not np.dtype(dt)
+    ptr = knet.KnetPtr(nbytes=4096, ptr=0x10000, keep=object())
+    for d in (a.dtype, a[1:].dtype, (a * dt(2)).dtype, a.T.dtype, pickle.loads(pickle.dumps(np.dtype(dt)))):
+        x = knet.KnetArray(dtype=d, dims=(3, 4), _ptr=ptr)
+        for y in (x, x.reshape(12), x.view1d(2, 5)):
+            assert y.suffix == suffix and y.dtype is np.dtype(dt)
+    other = knet.KnetArray(dtype=np.uint8, dims=(2,), _ptr=ptr)
+    blocks, address = itertools.count(0x100000, 0x1000), lambda f: ctypes.cast(f, ctypes.c_void_p).value  # noqa: E731
+    alloc, free = ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_size_t)(lambda n: next(blocks)), ctypes.CFUNCTYPE(None, ctypes.c_void_p)(lambda p: None)
+    lk, real, dtypes = native(knet), knet.libknet8(), tuple(np.dtype(t) for t in (np.float32, np.float64, np.int32))
+    lk.host.setup(address(alloc), address(free), lk._out_of_memory, np.dtype, dtypes, real)
+    try:
+        monkeypatch.setitem(real.fn, "knet8_memcpy", lambda *args: 0)
+        monkeypatch.setattr(real, "check", lambda: None)
+        x = knet.KnetArray(a)
+        assert x.suffix == suffix and x.similar().suffix == suffix and x.similar((2,)).suffix == suffix
+        assert other.similar((2, 2), dtype=a.dtype).suffix == suffix and x.kptr.nbytes == 12 * np.dtype(dt).itemsize
+        assert knet.KnetArray(dtype=">f4", dims=(2,)).suffix is None                  # another byte order is another type
+        del x
+    finally:
+        gc.collect()
+        lk.host.setup(address(real.fn["knet8_malloc"]), address(real.fn["knet8_free"]), lk._out_of_memory, np.dtype, dtypes, real)

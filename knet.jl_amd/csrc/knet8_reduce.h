@@ -694,25 +694,26 @@ inline bool launch_reduce_strided(hipStream_t stream, const T* x, long s1, long 
   return true;
 }
 
-// `_21` contract: x[i] goes into y[(i/sy)%ny]  (src/libknet8/cuda21.jl:23).
+// `_21` contract: x[i] goes into y[(i/sy)%ny]  (src/libknet8/cuda21.jl:23).  False, and the error recorded, if y was left untouched.
 template <typename T, typename Op>
-inline void reduce_21(hipStream_t stream, long nx, const T* x, long sy, long ny, T* y, const ScratchSource* scratch = nullptr) {
-  if (ny <= 0 || sy <= 0 || nx < 0) return;
-  if (nx % (sy * ny) != 0) { record_error("reduce _21: nx is not a multiple of sy*ny"); return; }
+inline bool reduce_21(hipStream_t stream, long nx, const T* x, long sy, long ny, T* y, const ScratchSource* scratch = nullptr) {
+  if (ny <= 0 || sy <= 0 || nx < 0) return false;
+  if (nx % (sy * ny) != 0) { record_error("reduce _21: nx is not a multiple of sy*ny"); return false; }
   const long no = nx / (sy * ny);
-  if (ny == 1) launch_reduce_run<T, Op>(stream, x, nx, 1, 1, y, scratch);
-  else if (sy == 1) launch_reduce_strided<T, Op>(stream, x, ny, no, 1, y, scratch);
-  else launch_reduce_run<T, Op>(stream, x, sy, ny, no, y, scratch);
+  if (ny == 1) return launch_reduce_run<T, Op>(stream, x, nx, 1, 1, y, scratch);
+  if (sy == 1) return launch_reduce_strided<T, Op>(stream, x, ny, no, 1, y, scratch);
+  return launch_reduce_run<T, Op>(stream, x, sy, ny, no, y, scratch);
 }
 
-// y[j] = factor * sum over x[i], (i/sy)%ny == j: in one launch, or the sums and then their factor where the sums take the stretch kernel or the route through slab sums.
+// y[j] = factor * sum over x[i], (i/sy)%ny == j: in one launch, or the sums and then their factor where the sums take the stretch kernel or the route through slab sums,
+// so that the sum's bits come out either way.  (The line covers all of these shapes and a few more.  One slab of runs of just kStretchMaxRun elements: the stretch kernel
+// has them where x is off the 16-byte boundaries.)
 template <typename T, typename Scale>
 inline void reduce_mean_21(hipStream_t stream, long nx, const T* x, long sy, long ny, T factor, T* y, Scale scale) {
   if (ny <= 0 || sy <= 0 || nx < 0) return;
-  const bool own = ny > 1 && (sy == 1 ? ny * (long)sizeof(T) <= 256 : sy < (nx == sy * ny ? kStretchMaxRun : (long)kWave));
+  const bool own = ny > 1 && (sy == 1 ? ny * (long)sizeof(T) <= 256 : nx != sy * ny ? sy < kWave : sy < kStretchMaxRun || (sy == kStretchMaxRun && !aligned16(x)));
   if (own || nx % (sy * ny) != 0) {   // (the sums report sizes that do not fit)
-    reduce_21<T, RedSum<T>>(stream, nx, x, sy, ny, y);
-    if (nx % (sy * ny) == 0) scale(y, ny, factor);
+    if (reduce_21<T, RedSum<T>>(stream, nx, x, sy, ny, y)) scale(y, ny, factor);
     return;
   }
   const Center<T> c = {nullptr, factor};

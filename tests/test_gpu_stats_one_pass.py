@@ -103,3 +103,31 @@ def test_mean_is_sum_and_factor(knet, dims, over, dt):
     J = knet.diff(lambda: knet.sum(knet.mean(p, dims=over)))
     assert np.allclose(knet.Array(knet.grad(J, p)), float(factor))
     knet.libknet8().check()
+
+
+# one slab round the longest run of the stretch kernel (1024), on and off the 16-byte boundary; short runs over slabs (slab sums); rows of 256 bytes and more
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("dims,over", [((1023, 37), 1), ((1024, 37), 1), ((1024, 5000), 1), ((1025, 37), 1), ((63, 40, 50), (1, 3)), ((64, 40, 50), (1, 3)), ((32, 9000), 2), ((64, 9000), 2), ((65, 9000), 2)])
+def test_mean_has_the_bits_of_the_sum_and_its_factor(knet, dims, over, dt):
+    x = np.random.default_rng(sum(dims)).standard_normal(dims).astype(dt)
+    for by in (0, 1):
+        xd = offset(knet, x, by)
+        s = knet.sum(xd, dims=over)
+        assert np.array_equal(knet.Array(knet.mean(xd, dims=over)), knet.Array(s) * dt(s.length / xd.length)), by
+    knet.libknet8().check()
+
+
+def test_mean_without_scratch_leaves_its_output(knet):
+    lib = knet.libknet8()
+    x, y = knet.KnetArray(np.ones((10, 25000), np.float32)), knet.KnetArray(np.full(10, 3, np.float32))
+    lib.fn["knet8_tune"](5, 1)
+    try:
+        knet.knet8("mean_32_21", x.length, x.ptr, 1, 10, 0.5, y.ptr)
+        with pytest.raises(RuntimeError):
+            lib.check()
+    finally:
+        lib.fn["knet8_tune"](5, 0)
+    assert (knet.Array(y) == 3).all()
+    knet.knet8("mean_32_21", x.length, x.ptr, 1, 10, 0.5, y.ptr)
+    assert (knet.Array(y) == 12500).all()
+    lib.check()

@@ -68,7 +68,8 @@ template <typename Op, typename T> struct MergeFn {
 // of the K/NV units of output j.
 // ANY: runs of any length and at any element boundary, still 16 bytes a load: the last load of a run ends with it, and the elements that the one before
 // it has had already do not count.  (29x29 feature maps, 193 channels, 64 images, 41.5 MB fp32: 32.7 us with loads of 4 bytes, 9.0 us so.)
-template <typename T, typename Op, int NV, bool SINGLE, int BT, int U, bool ANY = false>
+// DIVIDE: a unit's place by a division instead of a step from the one before (see below).
+template <typename T, typename Op, int NV, bool SINGLE, int BT, int U, bool ANY = false, bool DIVIDE = false>
 __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x, long sy, long ny, long units, long chunk,
                                                                unsigned P, T* __restrict__ y, T* partial, unsigned* counters, Center<T> center, unsigned run_step, unsigned at_step KNET8_TL_PARAM) {
   KNET8_TL_BEGIN
@@ -87,8 +88,11 @@ __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x,
   T acc[NV];
 #pragma unroll
   for (int e = 0; e < NV; e++) acc[e] = Op::init();
-  // A lane's units are BT apart: its place in its run moves by at_step = BT % usy, its run by run_step = BT / usy, and on by one where the place wraps round (with a division
-  // for each unit 784 over 200 outputs x 100 slabs takes 12.9 us, so 12.1).
+  // A lane's units are BT apart: its place in its run moves by at_step = BT % usy, its run by run_step = BT / usy, and on by one where the place wraps round.  It moves only
+  // where there was a unit: a lane with two of them and sixteen loads to its trip is not kept by the steps of the other fourteen (us, all steps / so: fp64 25 over 286 x 12
+  // 3.9/3.75, 289 over 300 x 30 7.2/6.2; fp32 3136 over 153 x 83 27.6/26.9).  With a division for each unit 784 over 200 outputs x 100 slabs takes 11.8 us, so 11.4; 256 over 64 x 128 4.2/3.7.
+  // DIVIDE is for large arrays with an output to a compute unit, where addresses that wait for one another delay the loads (see the launch).
+  static_assert(!DIVIDE || (!SINGLE && !ANY && NV > 1), "reduce_run_kernel: division is for whole vectors over several slabs");
   const unsigned steps = (unsigned)usy, first = (unsigned)(u0 + threadIdx.x);
   const unsigned run = SINGLE ? 0u : first / steps;
   unsigned at = SINGLE ? 0u : first - run * steps;
@@ -109,20 +113,21 @@ __global__ __launch_bounds__(BT) void reduce_run_kernel(const T* __restrict__ x,
           for (int e = 0; e < NV; e++) v[q][e] = from + e >= in_run ? red_item<Op>(T(t[e]), mu) : Op::init();
         } else if (NV > 1) {
           typedef typename Vec16<T>::type V;
-          V t = ld_stream(reinterpret_cast<const V*>(xp));
+          const unsigned o = DIVIDE ? (unsigned)uu / steps : 0u;
+          V t = ld_stream(reinterpret_cast<const V*>(DIVIDE ? xj + (o * slab + (long)((unsigned)uu - o * steps) * NV) : xp));
 #pragma unroll
           for (int e = 0; e < NV; e++) v[q][e] = red_item<Op>(T(t[e]), mu);
         } else {
           v[q][0] = red_item<Op>(T(__builtin_nontemporal_load(xp)), mu);
         }
+        xp += xp_step;
+        if (!SINGLE && !DIVIDE) {
+          at += at_step;
+          if (at >= steps) { at -= steps; xp += xp_wrap; }
+        }
       } else {
 #pragma unroll
         for (int e = 0; e < NV; e++) v[q][e] = Op::init();
-      }
-      xp += xp_step;
-      if (!SINGLE) {
-        at += at_step;
-        if (at >= steps) { at -= steps; xp += xp_wrap; }
       }
     }
 #pragma unroll
@@ -613,34 +618,39 @@ inline bool launch_reduce_run(hipStream_t stream, const T* x, long sy, long ny, 
   }
   T* partial = static_cast<T*>(ws.partial);
   // Workgroup size by the work of one part: a wave for short runs, 512 lanes when there is plenty.  Over several slabs: 256 lanes up to 1024 units (4096 with more than two outputs to a compute unit), 512 up to 2048 and, with a
-  // workgroup to each compute unit or less, 1024 beyond (from 7/8 of the compute units on, on whole vectors, 512 lanes are as fast: 3136 over 256 x 64 31.3, 1024 lanes 32.4);
+  // workgroup to each compute unit or less, 1024 beyond (from 7/8 of the compute units on, on whole vectors, 512 lanes are as fast: 3136 over 256 x 64 31.1, 1024 lanes 32.4);
   // 256 with more than three outputs to a compute unit (512 / 256 lanes: 3844 over 797 x 13 29.0/25.9, 1296 over 1070 x 28 28.3/26.6, 3481 over 1148 x 9 26.0/24.5).
   // us, fp32, before (256 or 512 lanes, 1024 with unaligned runs) / so: 1024 over 158 x 12 4.7/3.7, 3136 over 153 x 83 30.3/26.2, 2500 over 210 x 76 25.8/24.8, 196 over 496 x 41 5.2/5.0.
   const long wgs = ny * (long)P;
   const int bt = chunk <= 2 * kWave ? 64 : !slabs ? (chunk <= 4096 ? 256 : 512) : chunk <= (ny > 2 * ncu ? 4096 : 1024) || ny > 3 * ncu ? 256 : chunk > 2048 && wgs <= (any ? ncu : ncu / 8 * 7) ? 1024 : 512;
   const dim3 grid((unsigned)wgs);
   const long usy = sy == 0 ? 1 : vec ? sy / N : any ? ceil_div(sy, N) : sy;   // units per run (no elements at all: none is walked, any number will do)
-#define KNET8_RUN(NV, SINGLE, BT, U, ANY) \
-  hipLaunchKernelGGL((reduce_run_kernel<T, Op, NV, SINGLE, BT, U, ANY>), grid, dim3(BT), 0, stream, x, sy, ny, units, chunk, P, y, partial, ws.counters, center, (unsigned)(BT / usy), (unsigned)(BT % usy) KNET8_TL_ARG)
+#define KNET8_RUN(NV, SINGLE, BT, U, ANY, DIVIDE) \
+  hipLaunchKernelGGL((reduce_run_kernel<T, Op, NV, SINGLE, BT, U, ANY, DIVIDE>), grid, dim3(BT), 0, stream, x, sy, ny, units, chunk, P, y, partial, ws.counters, center, (unsigned)(BT / usy), (unsigned)(BT % usy) KNET8_TL_ARG)
   // (the path with loads of one element, for short runs that do not start on 16-byte boundaries, keeps four times as many in flight per lane to move the same bytes)
 #define KNET8_RUN_BT(NV, SINGLE) \
-  do { if (bt == 64) KNET8_RUN(NV, SINGLE, 64, (NV == 1 ? 16 : 8), false); else if (bt == 256) KNET8_RUN(NV, SINGLE, 256, (NV == 1 ? 16 : 4), false); \
-       else KNET8_RUN(NV, SINGLE, 512, (NV == 1 ? 16 : 4), false); } while (0)
+  do { if (bt == 64) KNET8_RUN(NV, SINGLE, 64, (NV == 1 ? 16 : 8), false, false); else if (bt == 256) KNET8_RUN(NV, SINGLE, 256, (NV == 1 ? 16 : 4), false, false); \
+       else KNET8_RUN(NV, SINGLE, 512, (NV == 1 ? 16 : 4), false, false); } while (0)
   // Two loads in flight a lane where runs are unaligned or there are more workgroups than compute units.  us, fp32, 8, 4 and 2 of them: 841 over 193 x 64 11.1/10.4/9.0, x 128 19.6/17.8/15.1
-  // (a run of whole vectors, 840: 8.8 whichever); whole vectors, 4 and 2: 1296 over 329 x 93 28.9/27.4, 4096 over 352 x 23 23.0/21.8, 2116 over 678 x 27 26.0/24.9.
+  // (a run of whole vectors, 840: 8.8 whichever); whole vectors, 4 and 2: 1296 over 329 x 93 29.7/26.8, 4096 over 352 x 23 22.9/21.7, 2304 over 303 x 20 11.7/11.3.
+  // Places by division (us, in steps / so), where all but a few compute units have an output each, from 128 MB on: 3136 over 256 x 64 31.3/31.1, x 90 43.0/42.6, over 254 x 64 31.4/31.0,
+  // 6400 over 256 x 32 31.7/31.3, fp64 1600 over 256 x 64 31.8/31.5; but 3136 over 250 x 64 30.6/30.6, over 230 x 72 31.4/31.8, 3844 over 234 x 44 24.9/25.3; smaller: 3136 over 256 x 40
+  // 20.5/20.5, 784 over 256 x 128 17.2/17.3, 784 over 227 x 30 4.3/4.5, 1024 over 256 x 20 3.8/4.1.
+  const bool divide = slabs && P == 1 && bt == 512 && ny <= ncu && ny > ncu / 64 * 62 && total_bytes >= (size_t(128) << 20);
   if constexpr (kAny) {
     if (any) {
-      if (bt == 64) KNET8_RUN(N, false, 64, 2, true);
-      else if (bt == 256) KNET8_RUN(N, false, 256, 2, true);
-      else if (bt == 512) KNET8_RUN(N, false, 512, 2, true);
-      else KNET8_RUN(N, false, 1024, 2, true);
+      if (bt == 64) KNET8_RUN(N, false, 64, 2, true, false);
+      else if (bt == 256) KNET8_RUN(N, false, 256, 2, true, false);
+      else if (bt == 512) KNET8_RUN(N, false, 512, 2, true, false);
+      else KNET8_RUN(N, false, 1024, 2, true, false);
       return true;
     }
   }
-  if (slabs && bt == 1024) KNET8_RUN(N, false, 1024, 2, false);
-  else if (slabs && bt == 512 && ny > ncu) KNET8_RUN(N, false, 512, 2, false);
-  else if (slabs && bt == 256 && chunk > 4096) KNET8_RUN(N, false, 256, 2, false);
+  if (slabs && bt == 1024) KNET8_RUN(N, false, 1024, 2, false, false);
+  else if (slabs && bt == 512 && ny > ncu) KNET8_RUN(N, false, 512, 2, false, false);
+  else if (slabs && bt == 256 && chunk > 4096) KNET8_RUN(N, false, 256, 2, false, false);
   else if (vec && no == 1) KNET8_RUN_BT(N, true);
+  else if (divide) KNET8_RUN(N, false, 512, 4, false, true);
   else if (vec) KNET8_RUN_BT(N, false);
   else if (no == 1) KNET8_RUN_BT(1, true);
   else KNET8_RUN_BT(1, false);

@@ -131,3 +131,20 @@ def test_mean_without_scratch_leaves_its_output(knet):
     knet.knet8("mean_32_21", x.length, x.ptr, 1, 10, 0.5, y.ptr)
     assert (knet.Array(y) == 12500).all()
     lib.check()
+
+
+# whole vectors over several slabs, one workgroup an output, an output to (nearly) every compute unit, 128 MB and just less: places in the runs by division and in steps
+@pytest.mark.parametrize("dt,dims", [(np.float32, (1024, 256, 128)), (np.float32, (1024, 256, 127)), (np.float32, (2500, 249, 55)), (np.float32, (2500, 248, 55)), (np.float64, (1026, 253, 67)), (np.float64, (514, 257, 130))])
+def test_large_reductions_with_an_output_to_a_compute_unit(knet, dt, dims):
+    x = np.random.default_rng(dims[2]).integers(-3, 4, dims).astype(dt)
+    f = np.asfortranarray(x)
+    xd = knet.KnetArray(f)
+    total, squares, n = f.sum(axis=(0, 2), dtype=np.float64), (f * f).sum(axis=(0, 2), dtype=np.float64), dims[0] * dims[2]
+    assert squares.max() < 2 ** 24                                                        # whole numbers below that: sums in any order are exact
+    assert np.array_equal(knet.Array(knet.sum(xd, dims=(1, 3))).ravel(), total)
+    assert np.array_equal(knet.Array(knet.sumabs2(xd, dims=(1, 3))).ravel(), squares)
+    assert np.array_equal(knet.Array(knet.countnz(xd, dims=(1, 3))).ravel(), np.count_nonzero(f, axis=(0, 2)))
+    m = knet.mean(xd, dims=(1, 3))
+    assert np.array_equal(knet.Array(m).ravel(), total.astype(dt) * dt(1.0 / n))
+    np.testing.assert_allclose(knet.Array(knet.var(xd, dims=(1, 3), mean=m, corrected=False)).ravel(), squares / n - (total / n) ** 2, rtol=1e-5 if dt == np.float32 else 1e-12)
+    knet.libknet8().check()

@@ -139,7 +139,10 @@ inline int gemm_mid_waves(long tiles, int k) {
 // Where vendor calls cost more than a launch: true if the product is faster here.  small: the rule for small products would have it.  us a call, back to back from a Python process:
 // fp32 against the 16x16 kernel: faster with 160 tiles and more (1000x237x100 TN 3.7/4.2, 512^3 6.8/8.6), sooner where that kernel's loads along k start off the 16-byte
 //   boundaries (277x454x558 6.5/7.9); with fewer its waves are too few (100x237x1000 9.8/4.9, 399x651x243 6.6/5.5).  Against hipBLASLt: 291x460x433 TN 6.0/10.4, 307x706x605 TN 7.4/10.6, 1000x237x1000 TN 9.0/11.0; beyond 5.3e8 flop or long k
-//   its larger tiles are ahead (1719x183x930 TN 14.4/12.3, 512x512x2048 NT 16.4/14.9, 152x1600x1600 13.3/11.0).
+//   its larger tiles are ahead (1719x183x930 TN 14.4/12.3, 512x512x2048 NT 16.4/14.9, 152x1600x1600 13.3/11.0).  Short k over many tiles is nearly all stores of C.  Where m comes in whole
+//   128s and n in whole 16s, as its tiles do, hipBLASLt's are ahead from about 6500 tiles on, fewer with more steps of k to each: 8192x8192x1 59/51, 4096x4096x4 20.7/17.9, 8704x1536x8 TN
+//   21.7/15.9, 14592x640x20 TN 18.7/14.2, 10496x448x48 NT 14.4/11.5; at other sizes they do work for padding: 3000x3000x4 14.1/19.0, 7256x12328x2 NT 96/104, 108054x84x14 17.5/30.8.  (764 products
+//   with k up to 260: the sum of log(time / the better time) is 25.7 without this line, 11.0 with it.)
 // fp64, where hipBLASLt's kernels (the copy that PyTorch brings) reach 25 TFLOP/s: 979x200x870 TN 12.8/39.7, 1392x1234x1194 79/185, 2549x2683x1193 TN 330/847, 906x1912x63 11.8/13.0;
 //   not short k over many tiles: 2973x1218x64 TN 24.9/21.2.  Against the 16x16 kernel 120x1026x946 TN 14.6/31.3, 531x295x494 8.6/12.9, 204x859x279 TN 7.5/10.9; level: 968x122x376 7.0/6.9;
 //   few tiles: 212x155x1981 NT 21.9/13.4.
@@ -151,7 +154,7 @@ inline bool gemm_mid_fits(bool ta, bool tb, int m, int n, int k, int lda, int ld
     return small ? tiles >= 128 && k >= 150 : tiles >= 32 && !(k < 100 && tiles > 3500);
   }
   if (m < 32 || n < 32 || k > 1500 || flop > (k <= 1000 ? 5.3e8 : 3.5e8)) return false;
-  if (!small) return tiles >= 64;
+  if (!small) return tiles >= 64 && !(k <= 64 && m % 128 == 0 && n % 16 == 0 && tiles + 80.0 * k > 6500);
   const double padded = 512.0 * ((m + 15) / 16) * ((n + 15) / 16) * k;
   const bool narrow = (ta && lda % 4 != 0) || (!tb && ldb % 4 != 0);
   return tiles >= 160 && padded >= (narrow ? 6e7 : 1.3e8);

@@ -81,7 +81,9 @@ def test_scalars_bias_and_relu(knet, knob, dt):
 
 VENDOR, SMALL, SPLIT, MID = 1, 2, 3, 4
 F32 = [(1000, 237, 1000, "NN", MID), (1000, 237, 1500, "NN", VENDOR), (1000, 128, 1001, "NN", MID), (250, 250, 1501, "NN", VENDOR), (512, 512, 512, "NN", MID), (100, 237, 1000, "NN", SMALL), (512, 512, 32, "NN", SMALL),
-       (256, 256, 517, "TN", SMALL), (512, 320, 185, "TN", MID), (512, 320, 183, "TN", SMALL), (512, 320, 188, "TN", SMALL), (31, 4000, 500, "TN", SMALL), (1000, 1000, 252, "NT", MID), (1000, 1000, 253, "NT", VENDOR), (1000, 2048, 4096, "NN", SPLIT)]
+       (256, 256, 517, "TN", SMALL), (512, 320, 185, "TN", MID), (512, 320, 183, "TN", SMALL), (512, 320, 188, "TN", SMALL), (31, 4000, 500, "TN", SMALL), (1000, 1000, 252, "NT", MID), (1000, 1000, 253, "NT", VENDOR), (1000, 2048, 4096, "NN", SPLIT),
+       # short k over many tiles: the line on tiles and k, m off the 128s, n off the 16s, k beyond 64
+       (256, 24576, 8, "NN", VENDOR), (256, 24576, 4, "TN", MID), (264, 24576, 8, "NN", MID), (256, 24584, 8, "NT", MID), (512, 3712, 64, "NN", VENDOR), (512, 3712, 65, "NN", MID)]
 F64 = [(512, 512, 512, "NN", MID), (1100, 1200, 600, "TN", MID), (100, 64, 784, "NN", SMALL), (360, 340, 149, "NN", SMALL), (360, 380, 150, "NN", MID), (2000, 2000, 90, "NN", VENDOR), (2000, 2000, 100, "NN", MID),
        (60, 60, 8193, "NN", VENDOR), (900, 1, 900, "NN", SMALL)]
 

@@ -453,8 +453,8 @@ def gen_elementwise():
     o.decl.append("/* dense_back_S: the backward pass of one small dense layer y = f(W*x + b) in one launch.  W is m x k, x is k x n, y and dy\n"
                   "   are m x n (column-major, no padding); act 0: dz = dy, act 1: dz = y > 0 ? dy : 0 (relu).  Writes dW = dz*x' (m x k),\n"
                   "   db = sum(dz; dims=2) (m) and dx = W'*dz (k x n); any of the three may be NULL (db needs dW).  Returns 0 when done, 1 when\n"
-                  "   the layer is too large for the small-matrix kernels -- nothing is launched then and the caller uses Fback_biasgrad_S\n"
-                  "   and gemm_S instead --, -1 on bad arguments.  No libknet8 counterpart: replaces reluback + sum(dz;dims=2) + two gemm!\n"
+                  "   the layer is too large for the small-matrix kernels, or quicker in separate launches (see knet8_tune key 4) -- nothing is launched then and the\n"
+                  "   caller uses Fback_biasgrad_S and gemm_S instead --, -1 on bad arguments.  No libknet8 counterpart: replaces reluback + sum(dz;dims=2) + two gemm!\n"
                   "   calls (src/ops20_gpu/activation.jl:30-37, src/knetarrays/reduction.jl:21-77, src/knetarrays/linalg.jl:11-18). */")
     for T, S in TYPES:
         o.entry("dense_back_%s" % S, "int",
@@ -708,7 +708,8 @@ KNET8_API void sum_32_21_noalloc(int nx, float* x, int sy, int ny, float* y, hip
    device); key 1: longest softmax column kept resident in registers, longer ones take the two-pass streaming kernel (default 0: the register capacity);
    key 3: products of up to this many MFLOP (2*m*n*k/1e6) take the library's own small-product kernels instead of hipBLASLt (default 0: a rule on
    type and sizes, up to 270 MFLOP, where the loaded hipBLASLt allows no prepared calls; see key 10);
-   key 4: dense_back_S / dense_nll_back_S accept layers whose products have up to this many MFLOP each (default 270);
+   key 4: dense_back_S / dense_nll_back_S accept layers whose products have up to this many MFLOP each (default 0: 270, and dense_back_S leaves those to separate launches that are
+   quicker so, with long inner dimensions or many 16x16 tiles; with a value set here, which may be 270, it is the only limit);
    key 5: non-zero makes the library behave as if the scratch memory of split launches and the buffers of uploads could not be allocated (for tests of these paths);
    key 6: non-zero keeps softmax columns of 128 to 256 KB in registers alone instead of registers + LDS (for comparisons);
    key 7: non-zero makes the hipBLASLt route of gemm_S do everything but the vendor call itself (for measuring the library's own share of a call's host time);

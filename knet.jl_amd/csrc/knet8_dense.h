@@ -323,10 +323,10 @@ inline int launch_dense_back_impl(hipStream_t stream, int act, int m, int n, int
   // A tile walks its whole inner dimension in one workgroup, and every tile reads its edges afresh.  So layers that have much of both, or very many tiles, are
   // quicker in separate launches.  us a call over 326 layers up to the limit above (one launch / three; with dx): 33x1538x819 27.3/20.4, 3293x198x166 48.5/28.3,
   // 1539x19x2714 (16830 tiles) 55.7/24.7; without dx 347x1741x77 27.5/16.5.  Inside the lines: 1265x146x232 14.6/17.8, 400^3 as above, fp64 96x1146x65 13.3/18.2.
-  // (The loss forms have no separate launches to fall back on here and keep their range.)
-  const int inner = tiles_x > 0 && m > n ? m : n;
-  if (!NLL && (flop * inner > 1.4e11 || (dW != nullptr && n > 1500) || (long)tiles_w + tiles_x > 8192)) return 1;
+  // (The loss forms have no separate launches to fall back on here and keep their range.  A caller that sets the limit itself has it as the only one.)
   if (tiles_w + tiles_x == 0) return 0;
+  const int inner = tiles_x > 0 && m > n ? m : n;
+  if (!NLL && !tuned(kTuneDenseBackMflop) && (flop * inner > 1.4e11 || (dW != nullptr && n > 1500) || (long)tiles_w + tiles_x > 8192)) return 1;
   // inner dimension per wave, in whole 16-deep steps
   auto slice = [](int K) { const int steps = (K + 15) / 16; return ((steps + kDbWaves - 1) / kDbWaves) * 16; };
   hipLaunchKernelGGL((dense_back_kernel<T, MODE>), dim3((unsigned)(tiles_w + tiles_x)), dim3(kDbWaves * kWave), 0, stream, act, m, n, k, W, x, y, dy, dW, db, dx,

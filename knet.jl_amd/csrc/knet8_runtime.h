@@ -80,6 +80,7 @@ void rng_take(unsigned long long blocks, unsigned long long* seed, unsigned long
 
 enum { kTuneNumCUs = 0, kTuneSoftmaxResidentRows = 1, kTuneGemmSmallMflop = 3, kTuneDenseBackMflop = 4, kTuneFailScratch = 5, kTuneSoftmaxNoLdsSlots = 6, kTuneGemmDryRun = 7, kTuneGemmNoPrepared = 8, kTuneGemmSplit = 9, kTuneGemmSmallRule = 10, kTuneGemmMid = 11, kTuneCount = 12 };
 int tuning(int key);
+bool tuned(int key);   // set by the caller, not at its default (of keys whose default is not remembered: all but kTuneNumCUs)
 
 #ifdef KNET8_TIMELINE
 struct TlStamp;

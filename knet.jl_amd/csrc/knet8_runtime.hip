@@ -99,9 +99,10 @@ int tuning(int key) {
   }
   // kTuneGemmSmallMflop stays 0 unless a caller sets it: small products go by gemm_is_small_by_rule.  A positive value sends products of up to that many
   // MFLOP (2mnk) to the library's own small-product kernels, whatever their shape.
-  if (key == kTuneDenseBackMflop && g_tune[key] == 0) g_tune[key] = 270;  // dense_back_S and its relatives accept layers whose products have up to this many MFLOP each
+  if (key == kTuneDenseBackMflop && g_tune[key] == 0) return 270;  // dense_back_S and its relatives accept layers whose products have up to this many MFLOP each
   return g_tune[key];
 }
+bool tuned(int key) { return key >= 0 && key < kTuneCount && g_tune[key] != 0; }
 
 // ---- per-stream scratch for split reductions ------------------------------------------------------------
 struct StreamScratch {

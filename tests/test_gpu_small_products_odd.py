@@ -59,3 +59,28 @@ def test_layers_beyond_the_lines_are_left_to_separate_launches(knet):
     # declined on the host, nothing is read: much work over a long inner dimension, very many columns, very many tiles
     for m, n, k, dx in ((33, 1538, 819, ptr), (3293, 198, 166, ptr), (64, 1501, 100, None), (1539, 19, 2714, None)):
         assert call("dense_back_32", 1, m, n, k, ptr, ptr, ptr, ptr, ptr, ptr, dx) == 1
+
+
+@pytest.mark.parametrize("m,n,k,wants", [(33, 1538, 819, True), (64, 1501, 100, False), (1539, 19, 2714, False)])
+def test_a_limit_of_the_callers_own_is_the_only_one(knet, m, n, k, wants):
+    """knet8_tune key 4: 0 leaves layers that are quicker so to separate launches, a value takes every layer up to it."""
+    lib, u = knet.libknet8(), 2.0 ** -24
+    rng = np.random.default_rng(n)
+    W, x, y, dy = (rng.standard_normal(d).astype(np.float32) for d in ((m, k), (k, n), (m, n), (m, n)))
+    arrays = [knet.KnetArray(a) for a in (W, x, y, dy)]
+    dW, db, dx = (knet.KnetArray(np.full(d, 7, np.float32)) for d in ((m, k), (m,), (k, n)))
+    call = lambda: lib.call("dense_back_32", 1, m, n, k, *[a.ptr for a in arrays], dW.ptr, db.ptr, dx.ptr if wants else None)  # noqa: E731
+    assert lib.fn["knet8_tune"](4, -1) == 0 and call() == 1 and (knet.Array(dW) == 7).all()
+    old = lib.fn["knet8_tune"](4, 270)
+    try:
+        assert call() == 0
+    finally:
+        lib.fn["knet8_tune"](4, old)
+    assert call() == 1 and lib.call("dense_back_32", 0, m, n, k, *[a.ptr for a in arrays], None, None, None) == 0   # nothing wanted: nothing to decline
+    dz = np.where(y > 0, dy, 0).astype(np.float64)
+    pairs = [(dW, dz @ x.T.astype(np.float64), np.abs(dz) @ np.abs(x).T, n), (db, dz.sum(axis=1), np.abs(dz).sum(axis=1), n)]
+    if wants:
+        pairs.append((dx, W.T.astype(np.float64) @ dz, np.abs(W).T @ np.abs(dz), m))
+    for got, want, size, terms in pairs:        # terms products and additions in any order, as above
+        assert (np.abs(knet.Array(got) - want) <= terms * u / (1 - terms * u) * size).all()
+    lib.check()

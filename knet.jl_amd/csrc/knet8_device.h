@@ -32,10 +32,16 @@ template <> struct Vec16<int> {
 // Streaming (read-once / write-once) accesses.
 template <typename V> __device__ __forceinline__ V ld_stream(const V* p) { return __builtin_nontemporal_load(p); }
 template <typename V> __device__ __forceinline__ void st_stream(V* p, V v) { __builtin_nontemporal_store(v, p); }
+// ... of 16 bytes at any element boundary.  (An alignment that is an attribute of a type is lost where the type is a template argument, so an address that is not on
+// a 16-byte boundary must not go through ld_stream: the type is made here.)
+template <typename T> __device__ __forceinline__ typename Vec16<T>::type ld_stream_any(const T* p) {
+  typedef T V __attribute__((ext_vector_type(Vec16<T>::N), aligned(sizeof(T))));
+  return __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
+}
 
 // A 16-byte store written through to the device-coherent level (sc1) instead of staying dirty in this XCD's L2.  The compiler has no form of
-// it for vectors; the inline instruction is an ordinary vector store (the "memory" clobber keeps later loads of the same address behind it).
-template <typename V> __device__ __forceinline__ void st_through(V* p, V v) {
+// it for vectors; the inline instruction is an ordinary vector store at any element boundary (the "memory" clobber keeps later loads of the same address behind it).
+template <typename V> __device__ __forceinline__ void st_through(void* p, V v) {
   static_assert(sizeof(V) == 16, "st_through: 16-byte vectors");
   asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(p), "v"(v) : "memory");
 }

@@ -104,7 +104,8 @@ template <typename T, typename F, int NV, int BT, int U, bool AL>
 __global__ __launch_bounds__(BT) void actback_biasgrad_kernel(const T* dy, const T* yv, long m, long n, long jchunk, unsigned P, T* dz, T* __restrict__ db,
                                                               T* partial, unsigned* counters, F f KNET8_TL_PARAM) {
   KNET8_TL_BEGIN
-  typedef T V __attribute__((ext_vector_type(NV), aligned(AL ? NV * sizeof(T) : sizeof(T))));
+  typedef typename Vec16<T>::type V;
+  static_assert(NV == Vec16<T>::N, "actback_biasgrad_kernel: rows come 16 bytes at a time");
   constexpr int TILE = kWave * NV;
   constexpr int NW = BT / kWave;
   __shared__ T lds[NW][TILE];
@@ -132,8 +133,13 @@ __global__ __launch_bounds__(BT) void actback_biasgrad_kernel(const T* dy, const
       for (int q = 0; q < U; q++) {
         const long jj = j + q * NW < j1 ? j + q * NW : j;
         const long off = jj * m + a0;
-        d[q] = ld_stream(reinterpret_cast<const V*>(dy + off));
-        o[q] = ld_stream(reinterpret_cast<const V*>(yv + off));
+        if constexpr (AL) {
+          d[q] = ld_stream(reinterpret_cast<const V*>(dy + off));
+          o[q] = ld_stream(reinterpret_cast<const V*>(yv + off));
+        } else {
+          d[q] = ld_stream_any(dy + off);
+          o[q] = ld_stream_any(yv + off);
+        }
       }
 #pragma unroll
       for (int q = 0; q < U; q++) {
@@ -145,7 +151,7 @@ __global__ __launch_bounds__(BT) void actback_biasgrad_kernel(const T* dy, const
         // written through (sc1), not merely streamed: what a kernel leaves dirty in the L2s is written back after its last workgroup has ended,
         // before the next launch may start; written through, dz drains while the partial sums are still being combined
         // ((4096,2048) fp32 cold: 19.3 -> 18.4 us; nt sc1 19.9-20.0, sc0 sc1 18.6, plain 19.3)
-        if (jj < j1) st_through(reinterpret_cast<V*>(dz + off), r);
+        if (jj < j1) st_through(dz + off, r);
       }
 #pragma unroll
       for (int q = 0; q < U; q++)

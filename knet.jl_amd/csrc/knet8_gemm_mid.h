@@ -151,6 +151,7 @@ inline bool gemm_mid_fits(bool ta, bool tb, int m, int n, int k, int lda, int ld
   const double tiles = (m + 31) / 32 * 1.0 * ((n + 31) / 32), flop = 2048 * tiles * k;
   if (sizeof(T) == 8) {
     if (m < 2 || n < 2 || k < 16 || k > 8192) return false;
+    if (tiles * gemm_mid_waves<T>((long)tiles, k) * kWave >= 4294967296.0) return false;   // a grid has fewer than 2^32 threads (131072^2 outputs, k >= 500); in fp32 the flop are far below that
     return small ? tiles >= 128 && k >= 150 : tiles >= 32 && !(k < 100 && tiles > 3500);
   }
   if (m < 32 || n < 32 || k > 1500 || flop > (k <= 1000 ? 5.3e8 : 3.5e8)) return false;

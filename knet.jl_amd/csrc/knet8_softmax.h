@@ -18,7 +18,8 @@
 #include "knet8_runtime.h"
 #include "knet8_reduce.h"
 
-#include <vector>
+#include <memory>
+#include <new>
 
 namespace knet8 {
 
@@ -1200,12 +1201,13 @@ inline T nll_host(hipStream_t stream, int m, int n, const T* x, const long long*
   T total = none;
   if (loss) {
     StagedWords w = stage_words(stream, (size_t)n);
-    std::vector<int> own;
+    std::unique_ptr<int[]> own;
     int* to = reinterpret_cast<int*>(w.host);
-    if (!to) { own.resize(n); to = own.data(); }
-    for (int i = 0; i < n; i++) to[i] = (int)labels[i];
+    if (!to) { own.reset(new (std::nothrow) int[n]); to = own.get(); }
+    if (!to) record_error("nll_host: no host memory for the labels");
+    for (int i = 0; to && i < n; i++) to[i] = (int)labels[i];
     const int* from = to;
-    if (!w.host || n > 4096 || softmax_is_short<T, AlgoNll<T>>(m, n)) {
+    if (to && (!w.host || n > 4096 || softmax_is_short<T, AlgoNll<T>>(m, n))) {
       dlab = static_cast<int*>(pool_take(4 * (size_t)n));
       if (!dlab || !bring_words(stream, dlab, to, n, w.host != nullptr)) from = nullptr;
       else from = dlab;

@@ -18,3 +18,22 @@ assert shim.shim_most_threads() < 2 ** 32, shim.shim_most_threads()
 assert (shim.shim_launches() == 1) == own
 print("done")
 """ % ((m, n, k, own),))
+
+
+def test_labels_that_no_host_memory_is_left_for_are_an_error(knet, tmp_path):
+    launch_shim.run(knet, tmp_path, """
+import math, resource, numpy as np
+n = 1 << 26
+labels = np.ones(n, np.int64)
+p = ctypes.c_void_p(0x7f0000000000)
+lib.nll_host_32_stream.restype = ctypes.c_float
+lib.nll_host_32_stream(1, 16, p, labels.ctypes.data_as(ctypes.c_void_p), p, None)     # (what a first call sets up)
+before = shim.shim_launches()
+error = lib.knet8_last_error()
+assert error is None, error
+size = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (size + (64 << 20), resource.RLIM_INFINITY))     # the labels as 32 bits take 256 MB
+loss = lib.nll_host_32_stream(1, n, p, labels.ctypes.data_as(ctypes.c_void_p), p, None)
+assert math.isnan(loss) and shim.shim_launches() == before and b"host memory" in lib.knet8_last_error()
+print("done")
+""")

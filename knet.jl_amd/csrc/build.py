@@ -9,6 +9,7 @@ import concurrent.futures
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG = os.path.dirname(HERE)
@@ -17,8 +18,9 @@ LIB = os.path.join(PKG, "lib", "libknet8.so")
 # The measurement build: the same sources with -DKNET8_TIMELINE, whose gradient kernels stamp the wall clock per workgroup
 # (`bench.py --timeline`).  Never loaded by the package unless KNET8_LIBRARY names it.
 LIB_TIMELINE = os.path.join(PKG, "lib", "libknet8_timeline.so")
-# The host mirror's native part: a CPython module (knet8_host.c and the generated calls), compiled by the host compiler.
-HOST = os.path.join(PKG, "lib", "_knet8_host.so")
+# The host mirror's native part: a CPython module (knet8_host.c and the generated calls), compiled by the host compiler.  Its name carries the interpreter's tag:
+# a module that was built for another one is not found, rather than loaded.
+HOST = os.path.join(PKG, "lib", "_knet8_host" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["-O3", "--offload-arch=gfx950", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-ffp-contract=off", "-fno-fast-math",
@@ -59,7 +61,6 @@ def compile_one(job):
 
 
 def build_host():
-    import sysconfig
     cmd = [os.environ.get("CC", "gcc"), "-O2", "-std=gnu11", "-Wall", "-shared", "-fPIC", "-fvisibility=hidden", "-DKNET8_BUILD_ID=\"%s\"" % source_id(),
            "-I" + sysconfig.get_paths()["include"], "-I" + HERE, os.path.join(HERE, "knet8_host.c"), "-o", HOST]
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

@@ -11,6 +11,7 @@ The calls themselves, the arrays and their blocks are objects of a native module
 by the signature in the header, which ctypes and Python classes did at 2 to 5 times the cost of the launch.  The 784-64-10 training step takes 95 us so, 172 with them.
 """
 import ctypes
+import importlib.machinery
 import importlib.util
 import os
 import re
@@ -20,7 +21,7 @@ import numpy as np
 _PKG = os.path.dirname(os.path.abspath(__file__))
 _ROOT = os.path.dirname(_PKG)
 LIB_PATH = os.environ.get("KNET8_LIBRARY", os.path.join(_PKG, "lib", "libknet8.so"))
-HOST_PATH = os.path.join(_PKG, "lib", "_knet8_host.so")
+HOST_PATH = os.path.join(_PKG, "lib", "_knet8_host" + importlib.machinery.EXTENSION_SUFFIXES[0])   # for this interpreter
 HEADER_PATH = os.path.join(_ROOT, "include", "knet8.h")
 
 _CTYPES = {
@@ -65,7 +66,7 @@ def source_build_id():
 
 def _load_host():
     if not os.path.exists(HOST_PATH):
-        raise OSError("_knet8_host.so not found at %s -- build it first (python __graft_entry__.py build)" % HOST_PATH)
+        raise OSError("native part of the host mirror not found at %s -- build it first, with this interpreter (python __graft_entry__.py build)" % HOST_PATH)
     spec = importlib.util.spec_from_file_location("_knet8_host", HOST_PATH)
     mod = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mod)

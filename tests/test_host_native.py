@@ -2,6 +2,7 @@
 import copy
 import ctypes
 import gc
+import importlib.machinery
 import itertools
 import pickle
 import sys
@@ -130,6 +131,14 @@ def test_similar_refuses_what_it_refused(knet):
     for args, kw in (((1, 2, 3), {}), ((), {"shape": (2,)}), ((5,), {}), ((("a",),), {})):
         with pytest.raises((TypeError, ValueError)):
             x.similar(*args, **kw)
+
+
+def test_module_is_for_this_interpreter(knet, monkeypatch):
+    lk = native(knet)
+    assert lk.HOST_PATH.endswith(importlib.machinery.EXTENSION_SUFFIXES[0]) and sys.implementation.cache_tag in lk.HOST_PATH
+    monkeypatch.setattr(lk, "HOST_PATH", lk.HOST_PATH.replace(sys.implementation.cache_tag, "cpython-399"))
+    with pytest.raises(OSError, match="not found"):
+        lk._load_host()
 
 
 @pytest.mark.parametrize("dt,suffix", [(np.float32, "32"), (np.float64, "64"), (np.int32, None)])

@@ -30,8 +30,7 @@ static PyObject* g_library = NULL;        /* the Library that knet8() calls */
 typedef struct {
   PyObject_HEAD
   unsigned long long ptr;
-  int owned;             /* goes back to the pool with this object */
-  PyObject *nbytes, *keep, *weak;
+  PyObject *nbytes, *keep, *weak;   /* keep None: the block is this object's and goes back to the pool with it */
 } Ptr;
 static PyTypeObject PtrType;
 
@@ -53,7 +52,7 @@ static int ptr_init(Ptr* s, PyObject* args, PyObject* kw) {
   static char* names[] = {"nbytes", "ptr", "keep", NULL};
   PyObject *nbytes = Py_None, *ptr = Py_None, *keep = Py_None;
   if (!PyArg_ParseTupleAndKeywords(args, kw, "|OOO", names, &nbytes, &ptr, &keep)) return -1;
-  if (s->nbytes) { PyErr_SetString(PyExc_RuntimeError, "KnetPtr is initialised once"); return -1; }
+  if (s->keep) { PyErr_SetString(PyExc_RuntimeError, "KnetPtr is initialised once"); return -1; }
   if (ptr != Py_None) {   /* borrowed memory, kept alive through keep */
     PyObject* i = PyNumber_Long(ptr);
     if (!i) return -1;
@@ -62,7 +61,6 @@ static int ptr_init(Ptr* s, PyObject* args, PyObject* kw) {
     if (PyErr_Occurred()) return -1;
     Py_INCREF(nbytes); s->nbytes = nbytes;
     Py_INCREF(keep); s->keep = keep;
-    s->owned = keep == Py_None;
     return 0;
   }
   PyObject* n = PyNumber_Long(nbytes);
@@ -72,7 +70,6 @@ static int ptr_init(Ptr* s, PyObject* args, PyObject* kw) {
   const size_t p = take_block(want > 0 ? (size_t)want : 0);
   if (!p) { Py_DECREF(n); return -1; }
   s->ptr = p;
-  s->owned = 1;
   s->nbytes = n;
   Py_INCREF(Py_None); s->keep = Py_None;
   return 0;
@@ -84,7 +81,6 @@ static Ptr* ptr_new(size_t nbytes) {
   Ptr* s = (Ptr*)PtrType.tp_alloc(&PtrType, 0);
   if (!s) { g_free((void*)p); return NULL; }
   s->ptr = p;
-  s->owned = 1;
   s->nbytes = PyLong_FromSize_t(nbytes);
   Py_INCREF(Py_None); s->keep = Py_None;
   if (!s->nbytes) { Py_DECREF(s); return NULL; }
@@ -92,12 +88,16 @@ static Ptr* ptr_new(size_t nbytes) {
 }
 
 static int ptr_traverse(Ptr* s, visitproc visit, void* arg) { Py_VISIT(s->nbytes); Py_VISIT(s->keep); return 0; }
-static int ptr_clear(Ptr* s) { Py_CLEAR(s->nbytes); Py_CLEAR(s->keep); return 0; }
+static int ptr_clear(Ptr* s) {
+  Py_CLEAR(s->nbytes);
+  if (s->keep != Py_None) Py_CLEAR(s->keep);   /* (None says whose the block is, until the end) */
+  return 0;
+}
 
 static void ptr_dealloc(Ptr* s) {
   PyObject_GC_UnTrack(s);
   if (s->weak) PyObject_ClearWeakRefs((PyObject*)s);
-  if (s->ptr && s->owned) {
+  if (s->ptr && s->keep == Py_None) {
     int parked = 0;
     if (g_parked) {
       PyObject *t, *v, *tb;
@@ -110,12 +110,13 @@ static void ptr_dealloc(Ptr* s) {
     if (!parked && g_free) g_free((void*)(size_t)s->ptr);
   }
   ptr_clear(s);
+  Py_CLEAR(s->keep);
   Py_TYPE(s)->tp_free((PyObject*)s);
 }
 
 static PyMemberDef ptr_members[] = {{"ptr", T_ULONGLONG, offsetof(Ptr, ptr), 0, "device address"},
-                                    {"nbytes", T_OBJECT, offsetof(Ptr, nbytes), READONLY, "size in bytes"},
-                                    {"_keep", T_OBJECT, offsetof(Ptr, keep), READONLY, "owner of borrowed memory"},
+                                    {"nbytes", T_OBJECT, offsetof(Ptr, nbytes), 0, "size in bytes"},
+                                    {"_keep", T_OBJECT, offsetof(Ptr, keep), 0, "owner of borrowed memory; None: the block belongs to this object"},
                                     {NULL}};
 static PyTypeObject PtrType = {PyVarObject_HEAD_INIT(NULL, 0).tp_name = "knet8.KnetPtr",
                                .tp_doc = "Owner of one device allocation (src/knetarrays/kptr.jl:10-15), or a borrowed address and what keeps it alive.",
@@ -311,6 +312,28 @@ static int array_set_dims(Array* s, PyObject* v, void* c) {
   return 0;
 }
 
+static PyObject* array_get_dtype(Array* s, void* c) { (void)c; if (!ready(s)) return NULL; Py_INCREF(s->dtype); return s->dtype; }
+static int array_set_dtype(Array* s, PyObject* v, void* c) {   /* other elements in the same memory */
+  (void)c;
+  int type;
+  Py_ssize_t itemsize;
+  if (!v) { PyErr_SetString(PyExc_AttributeError, "dtype cannot be deleted"); return -1; }
+  PyObject* t = as_dtype(v, &type, &itemsize);
+  if (!t) return -1;
+  s->type = type; s->itemsize = itemsize;
+  Py_XSETREF(s->dtype, t);
+  return 0;
+}
+
+static PyObject* array_get_kptr(Array* s, void* c) { (void)c; if (!ready(s)) return NULL; Py_INCREF(s->kptr); return (PyObject*)s->kptr; }
+static int array_set_kptr(Array* s, PyObject* v, void* c) {   /* other memory; offset stays */
+  (void)c;
+  if (!v || !PyObject_TypeCheck(v, &PtrType)) { PyErr_SetString(PyExc_TypeError, "a KnetPtr is needed"); return -1; }
+  Py_INCREF(v);
+  Py_XSETREF(s->kptr, (Ptr*)v);
+  return 0;
+}
+
 static int array_traverse(Array* s, visitproc visit, void* arg) { Py_VISIT(s->kptr); Py_VISIT(s->dims); Py_VISIT(s->dtype); return 0; }
 static int array_clear(Array* s) { Py_CLEAR(s->kptr); Py_CLEAR(s->dims); Py_CLEAR(s->dtype); return 0; }
 static void array_dealloc(Array* s) {
@@ -327,14 +350,14 @@ static PyMethodDef array_methods[] = {
     {"size", (PyCFunction)(void*)array_size, METH_FASTCALL | METH_KEYWORDS, "size(x) and size(x, i)"},
     {"stride", (PyCFunction)array_stride, METH_O, "stride(x, i) in elements"},
     {NULL}};
-static PyMemberDef array_members[] = {{"kptr", T_OBJECT_EX, offsetof(Array, kptr), READONLY, "the block"},
-                                      {"dtype", T_OBJECT_EX, offsetof(Array, dtype), READONLY, "element type"},
-                                      {"offset", T_PYSSIZET, offsetof(Array, offset), 0, "bytes from the start of the block"},
+static PyMemberDef array_members[] = {{"offset", T_PYSSIZET, offsetof(Array, offset), 0, "bytes from the start of the block"},
                                       {"length", T_PYSSIZET, offsetof(Array, length), READONLY, "number of elements"},
                                       {NULL}};
 static PyGetSetDef array_getset[] = {{"ptr", (getter)array_get_ptr, NULL, "device address of the first element", NULL},
                                      {"ndims", (getter)array_get_ndims, NULL, "number of dimensions", NULL},
                                      {"dims", (getter)array_get_dims, (setter)array_set_dims, "Julia dims: the first varies fastest in memory", NULL},
+                                     {"kptr", (getter)array_get_kptr, (setter)array_set_kptr, "the block", NULL},
+                                     {"dtype", (getter)array_get_dtype, (setter)array_set_dtype, "element type", NULL},
                                      {"suffix", (getter)array_get_suffix, NULL, "\"32\" or \"64\": the element type in the names of entry points; None for Int32", NULL},
                                      {NULL}};
 static PyTypeObject ArrayType = {PyVarObject_HEAD_INIT(NULL, 0).tp_name = "knet8.ArrayBase",

@@ -113,6 +113,10 @@ def test_blocks_go_back_once_or_are_parked(knet):
         knet.KnetPtr(nbytes=4, ptr=0x5000, keep=object())
         knet.KnetPtr(nbytes=4, ptr=0x6000)                     # an address without an owner is the caller's to give away
         assert freed == [p, 0x6000]
+        late = knet.KnetPtr(nbytes=4, ptr=0x8000)
+        late._keep = object()                                  # somebody else's after all
+        del late
+        assert freed == [p, 0x6000]
         # a cycle through what keeps borrowed memory alive is collected, and the memory is not given back
         class Keep:
             pass
@@ -131,6 +135,30 @@ def test_similar_refuses_what_it_refused(knet):
     for args, kw in (((1, 2, 3), {}), ((), {"shape": (2,)}), ((5,), {}), ((("a",),), {})):
         with pytest.raises((TypeError, ValueError)):
             x.similar(*args, **kw)
+
+
+def test_block_and_element_type_can_be_replaced(knet):
+    """As of the attributes they were before there was a native class."""
+    a, b = (knet.KnetPtr(nbytes=64, ptr=p, keep=object()) for p in (0x10000, 0x20000))
+    x = knet.KnetArray(dtype=np.float32, dims=(2, 3), _ptr=a, _offset=8)
+    x.kptr = b
+    assert x.kptr is b and x.ptr == 0x20008 and x.reshape(6).ptr == 0x20008
+    x.dtype = np.float64
+    assert x.dtype == np.float64 and x.suffix == "64" and x.view1d(1, 2).ptr == 0x20010
+    x.dtype = "int32"
+    assert x.suffix is None
+    with pytest.raises(TypeError):
+        x.kptr = 5
+    with pytest.raises(TypeError):
+        x.dtype = "no such type"
+    assert x.kptr is b and x.dtype == np.int32
+    a.nbytes = 32
+    assert a.nbytes == 32
+    empty = knet.KnetArray.__new__(knet.KnetArray)
+    with pytest.raises(RuntimeError):
+        empty.dtype
+    with pytest.raises(RuntimeError):
+        empty.kptr
 
 
 def test_module_is_for_this_interpreter(knet, monkeypatch):

@@ -22,6 +22,7 @@ from .loss import nll, findindices, accuracy, zeroone, ungetindex, bce, logistic
 from .indexing import (getcols, getrows, setcols_, setrows_, addcols_, addrows_, setents_, getindex2, setindex2_, icat, concat,
                        getindex, setindex_)
 from .dropout import dropout, dropback, dropout_, dropback_
+from . import layers
 from .update import SGD, Momentum, Nesterov, Adagrad, Rmsprop, Adadelta, Adam, update_, gclip_
 from .train import (Data, minibatch, param, param0, params, gaussian, xavier, xavier_uniform, xavier_normal, Minimize, minimize, minimize_,
                     sgd, sgd_, momentum, momentum_, nesterov, nesterov_, adagrad, adagrad_, rmsprop, rmsprop_, adadelta, adadelta_,

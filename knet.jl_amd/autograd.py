@@ -105,7 +105,7 @@ def selective(back):
 
 
 def layer_back(nodes, i):
-    """Set by the module of the matrix products: the gradients of a layer's end ``nodes[i]`` and of what it rests on, in fewer launches.  False: not one it knows."""
+    """Replaced by ``layers.py``: the gradients of a layer's end ``nodes[i]`` and of what it rests on, in fewer launches.  False: not one it knows."""
     return False
 
 

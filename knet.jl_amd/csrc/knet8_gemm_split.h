@@ -17,8 +17,8 @@
 //     one NaN in A and 731 with one infinity (a row of sums to form again), 1130 if every sum is beyond 2^80.
 //
 // The cut is made while a tile goes from global memory to LDS (6.5 vector instructions an element, in the shadow of the matrix instructions of the
-// SIMD's other wave): no extra pass over the operands, no scratch.  256x128 tile, 8 waves of 64x64, 32 steps of k a stage, two stages in LDS (up to 158 KB):
-// matrix cores 4096 cycles a stage, LDS about 2070, vector ALU about 2100.  What bounds it is power: 8192^3 runs at 198 TFLOP/s on normal data and at 232 on zeros.
+// SIMD's other wave): no extra pass over the operands, no scratch.  256x128 tile, 8 waves of 64x64, 32 steps of k a stage.  LDS: two stages and the masks
+// of sums that are not finite, 153088 bytes (TN), 158464 (NN, TT) or 163840 (NT, all that a compute unit has).  Matrix cores 4096 cycles a stage, LDS about 2070, vector ALU about 2100.  What bounds it is power: 8192^3 runs at 198 TFLOP/s on normal data and at 232 on zeros.
 // So the matrix instructions are chosen and ordered by the energy they take on normal data.  From registers alone 32x32x16 reaches 1822 TFLOP/s of bf16 work
 // and 16x16x32 2073 (both 2450 to 2480 on zeros): half the traffic to the accumulators.  All eight products of a 16x16 tile follow each other, so that the sums stay
 // where they are (3 % over taking the tiles in turn), in an order in which only one operand changes from one to the next (another 2 %; one that changes the first
@@ -171,6 +171,7 @@ void gemm_split_kernel(int m, int n, int k, const float* __restrict__ A, int lda
   using LB = SplitLoader<BN, BK, NT, !TB>;
   __shared__ uint4 lds[2][LA::kUnits + LB::kUnits];
   __shared__ unsigned long long odd[NT / 64][FN * 4 * FM];   // which sums are not finite (see the end)
+  static_assert(sizeof(lds) + sizeof(odd) <= 160 * 1024, "gemm_split_kernel: more LDS than a compute unit has");
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, half = lane >> 5, l32 = lane & 31, quad = lane >> 4, l16 = lane & 15;
   const int wm = (wave % (BM / WM)) * WM, wn = (wave / (BM / WM)) * WN;
   unsigned im, in, z;

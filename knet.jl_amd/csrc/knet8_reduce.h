@@ -454,8 +454,9 @@ inline unsigned plan_parts(long groups, long units_per_group, long min_units_per
 }
 
 // Parts of a split along an axis of d rows (or columns) per group, chosen by counting dependent memory round trips: a part's waves walk `per_trip` rows
-// per trip (sixteen waves with two rows in flight, or four with eight), the ticket costs two trips, and the workgroup that combines reads 128 partial rows
-// per trip when it has sixteen waves (parts of at least `big_from` rows) and 32 with four.  At most one workgroup per compute unit, parts of at least 16 rows.
+// per trip (in the strided reduction sixteen waves with two rows in flight, or four with eight), the ticket costs `join` trips, and the workgroup that combines reads `joined`
+// partial rows per trip when it has sixteen waves (parts of at least `big_from` rows) and 32 with four.  At most one workgroup per compute unit, parts of at least `least` rows.
+// (The defaults are the strided reduction's; the activation + bias gradient, whose columns take two loads and a store each, has its own.)
 inline unsigned plan_parts_by_trips(long groups, long d, long per_trip, long big_from, long least = 16, long join = 2, long joined = 128) {
   const long ncu = tuning(kTuneNumCUs);
   long pmax = groups * 2 <= ncu ? ncu / groups : 1;

@@ -312,26 +312,25 @@ static int array_set_dims(Array* s, PyObject* v, void* c) {
   return 0;
 }
 
-static PyObject* array_get_dtype(Array* s, void* c) { (void)c; if (!ready(s)) return NULL; Py_INCREF(s->dtype); return s->dtype; }
-static int array_set_dtype(Array* s, PyObject* v, void* c) {   /* other elements in the same memory */
-  (void)c;
-  int type;
-  Py_ssize_t itemsize;
-  if (!v) { PyErr_SetString(PyExc_AttributeError, "dtype cannot be deleted"); return -1; }
-  PyObject* t = as_dtype(v, &type, &itemsize);
-  if (!t) return -1;
-  s->type = type; s->itemsize = itemsize;
-  Py_XSETREF(s->dtype, t);
-  return 0;
-}
-
-static PyObject* array_get_kptr(Array* s, void* c) { (void)c; if (!ready(s)) return NULL; Py_INCREF(s->kptr); return (PyObject*)s->kptr; }
-static int array_set_kptr(Array* s, PyObject* v, void* c) {   /* other memory; offset stays */
-  (void)c;
-  if (!v || !PyObject_TypeCheck(v, &PtrType)) { PyErr_SetString(PyExc_TypeError, "a KnetPtr is needed"); return -1; }
-  Py_INCREF(v);
-  Py_XSETREF(s->kptr, (Ptr*)v);
-  return 0;
+/* kptr and dtype are members, which read fastest; they are set here, so that what goes with them is too. */
+static int array_setattro(PyObject* o, PyObject* name, PyObject* v) {
+  Array* s = (Array*)o;
+  if (v && PyUnicode_Check(name) && PyUnicode_CompareWithASCIIString(name, "dtype") == 0) {   /* other elements in the same memory */
+    int type;
+    Py_ssize_t itemsize;
+    PyObject* t = as_dtype(v, &type, &itemsize);
+    if (!t) return -1;
+    s->type = type; s->itemsize = itemsize;
+    Py_XSETREF(s->dtype, t);
+    return 0;
+  }
+  if (v && PyUnicode_Check(name) && PyUnicode_CompareWithASCIIString(name, "kptr") == 0) {   /* other memory; offset stays */
+    if (!PyObject_TypeCheck(v, &PtrType)) { PyErr_SetString(PyExc_TypeError, "a KnetPtr is needed"); return -1; }
+    Py_INCREF(v);
+    Py_XSETREF(s->kptr, (Ptr*)v);
+    return 0;
+  }
+  return PyObject_GenericSetAttr(o, name, v);
 }
 
 static int array_traverse(Array* s, visitproc visit, void* arg) { Py_VISIT(s->kptr); Py_VISIT(s->dims); Py_VISIT(s->dtype); return 0; }
@@ -350,21 +349,21 @@ static PyMethodDef array_methods[] = {
     {"size", (PyCFunction)(void*)array_size, METH_FASTCALL | METH_KEYWORDS, "size(x) and size(x, i)"},
     {"stride", (PyCFunction)array_stride, METH_O, "stride(x, i) in elements"},
     {NULL}};
-static PyMemberDef array_members[] = {{"offset", T_PYSSIZET, offsetof(Array, offset), 0, "bytes from the start of the block"},
+static PyMemberDef array_members[] = {{"kptr", T_OBJECT_EX, offsetof(Array, kptr), READONLY, "the block"},
+                                      {"dtype", T_OBJECT_EX, offsetof(Array, dtype), READONLY, "element type"},
+                                      {"offset", T_PYSSIZET, offsetof(Array, offset), 0, "bytes from the start of the block"},
                                       {"length", T_PYSSIZET, offsetof(Array, length), READONLY, "number of elements"},
                                       {NULL}};
 static PyGetSetDef array_getset[] = {{"ptr", (getter)array_get_ptr, NULL, "device address of the first element", NULL},
                                      {"ndims", (getter)array_get_ndims, NULL, "number of dimensions", NULL},
                                      {"dims", (getter)array_get_dims, (setter)array_set_dims, "Julia dims: the first varies fastest in memory", NULL},
-                                     {"kptr", (getter)array_get_kptr, (setter)array_set_kptr, "the block", NULL},
-                                     {"dtype", (getter)array_get_dtype, (setter)array_set_dtype, "element type", NULL},
                                      {"suffix", (getter)array_get_suffix, NULL, "\"32\" or \"64\": the element type in the names of entry points; None for Int32", NULL},
                                      {NULL}};
 static PyTypeObject ArrayType = {PyVarObject_HEAD_INIT(NULL, 0).tp_name = "knet8.ArrayBase",
                                  .tp_doc = "Storage side of KnetArray: block, dims, element type.",
                                  .tp_basicsize = sizeof(Array), .tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_BASETYPE | Py_TPFLAGS_HAVE_GC, .tp_new = array_new,
                                  .tp_dealloc = (destructor)array_dealloc, .tp_traverse = (traverseproc)array_traverse, .tp_clear = (inquiry)array_clear,
-                                 .tp_methods = array_methods, .tp_members = array_members, .tp_getset = array_getset};
+                                 .tp_setattro = array_setattro, .tp_methods = array_methods, .tp_members = array_members, .tp_getset = array_getset};
 
 /* ---- Library ------------------------------------------------------------------------------------------------------------------- */
 typedef struct {

@@ -154,11 +154,15 @@ def test_block_and_element_type_can_be_replaced(knet):
     assert x.kptr is b and x.dtype == np.int32
     a.nbytes = 32
     assert a.nbytes == 32
-    empty = knet.KnetArray.__new__(knet.KnetArray)
-    with pytest.raises(RuntimeError):
-        empty.dtype
-    with pytest.raises(RuntimeError):
-        empty.kptr
+    x.note, x.offset = "kept", 16                 # any other attribute as ever
+    assert x.note == "kept" and x.ptr == 0x20010
+    for name in ("dtype", "kptr", "ptr", "length"):
+        with pytest.raises((AttributeError, TypeError)):
+            delattr(x, name)
+    with pytest.raises(AttributeError):
+        x.length = 5
+    with pytest.raises(AttributeError):
+        knet.KnetArray.__new__(knet.KnetArray).dtype
 
 
 def test_module_is_for_this_interpreter(knet, monkeypatch):

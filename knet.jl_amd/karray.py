@@ -5,6 +5,7 @@ src/knetarrays/kptr.jl: the pointer comes from ``knet8_malloc`` (a size-class po
 and goes back to the pool when the last array sharing it is collected, as the reference's finalizer
 does (kptr.jl:105-142).  ``dims`` are Julia dims: the first varies fastest in memory.
 """
+import copy
 import ctypes
 
 import numpy as np
@@ -41,8 +42,26 @@ class KnetArray(host.ArrayBase):
     def ctype(self):
         return ctypes.c_float if self.dtype == np.float32 else ctypes.c_double
 
+    # -- the copy and pickle protocols: the native base has no state that they could take by themselves ---
     def __copy__(self):
-        return self._view(self.dims, self.offset)
+        """The same memory, as ``reshape`` shares it."""
+        y = type(self).__new__(type(self))
+        y._init(self.kptr, self.dims, self.dtype, self.offset)
+        y.__dict__.update(self.__dict__)
+        return y
+
+    def __deepcopy__(self, memo):
+        """Memory of its own with the same contents, as ``copy()``."""
+        y = type(self).__new__(type(self))
+        memo[id(self)] = y
+        y._init(None, self.dims, self.dtype)
+        libknet8().fn["knet8_memcpy"](y.ptr, self.ptr, self.length * self.dtype.itemsize, 3, libknet8().stream)
+        y.__dict__.update(copy.deepcopy(self.__dict__, memo))
+        return y
+
+    def __reduce_ex__(self, protocol):
+        """Through the host: the elements, which are uploaded where it is read."""
+        return type(self), (self.to_numpy(),), self.__dict__ or None
 
     def __repr__(self):
         return "KnetArray{%s,%d}%r" % (self.dtype.name, self.ndims, self.dims)

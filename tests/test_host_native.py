@@ -199,3 +199,49 @@ def test_element_types_are_told_by_equality(knet, monkeypatch, dt, suffix):
     finally:
         gc.collect()
         lk.host.setup(address(real.fn["knet8_malloc"]), address(real.fn["knet8_free"]), lk._out_of_memory, np.dtype, dtypes, real)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64, np.int32])
+@pytest.mark.parametrize("dims", [(3, 4), (5,), (2, 3, 2), (0, 4), ()])
+def test_arrays_are_copied_and_pickled(knet, monkeypatch, dims, dt):
+    """copy, deepcopy and pickle of arrays and of what holds them, over host memory in the place of the device's."""
+    lk, real, dtypes = native(knet), knet.libknet8(), tuple(np.dtype(t) for t in (np.float32, np.float64, np.int32))
+    held, address = {}, lambda f: ctypes.cast(f, ctypes.c_void_p).value  # noqa: E731
+
+    def take(n):
+        b = ctypes.create_string_buffer(n)
+        held[ctypes.addressof(b)] = b
+        return ctypes.addressof(b)
+    alloc, free = ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_size_t)(take), ctypes.CFUNCTYPE(None, ctypes.c_void_p)(lambda p: held.pop(p))
+    lk.host.setup(address(alloc), address(free), lk._out_of_memory, np.dtype, dtypes, real)
+    try:
+        monkeypatch.setitem(real.fn, "knet8_memcpy", lambda to, of, n, kind, stream: ctypes.memmove(to, of, n))
+        monkeypatch.setattr(real, "check", lambda: None)
+        want = np.arange(np.prod(dims, dtype=int)).reshape(dims).astype(dt)
+        x = knet.KnetArray(want)
+        x.note = ["mine"]
+        same = copy.copy(x)
+        assert same.kptr is x.kptr and same.dims == dims and same.note is x.note
+        for y in (copy.deepcopy(x), *(pickle.loads(pickle.dumps(x, p)) for p in range(2, pickle.HIGHEST_PROTOCOL + 1))):
+            assert type(y) is knet.KnetArray and y.ptr != x.ptr and y.dtype is x.dtype and y.suffix == x.suffix and y.dims == dims
+            assert np.array_equal(y.to_numpy(), want) and y.note == x.note and y.note is not x.note
+        if len(dims) == 2 and want.size:                  # a part of a block: its own elements, in a block of their size
+            part = x.view1d(4, 3)
+            y = copy.deepcopy(part)
+            assert y.kptr.nbytes == 3 * want.itemsize and np.array_equal(y.to_numpy(), want.ravel(order="F")[4:7])
+        if dt != np.int32:                                # a model and its optimizer: arrays shared within stay shared, and the copy lives by itself
+            w = knet.Param(x)
+            w.opt = knet.Momentum(lr=0.5)
+            w.opt.velocity = x
+            v = copy.deepcopy([w, w])
+            assert v[0] is v[1] and v[0].value is v[0].opt.velocity and v[0].value.ptr != x.ptr
+            del w, x, same
+            gc.collect()
+            assert np.array_equal(v[0].value.to_numpy(), want)
+            del v
+        x = same = y = part = None
+        gc.collect()
+        assert not held
+    finally:
+        gc.collect()
+        lk.host.setup(address(real.fn["knet8_malloc"]), address(real.fn["knet8_free"]), lk._out_of_memory, np.dtype, dtypes, real)
